@@ -307,11 +307,10 @@ int sem2d_fetch_info(sem2d_solver *h, double *rows, int *nrows);
 int sem2d_field_info(sem2d_solver *h, double *vmax, double *dmax, int *nonfinite);
 
 /* Launch configuration of the structured-grid tile kernel (no counterpart in the
-   reference, whose loop is serial): threads per workgroup (256 = 10-element batches,
-   512 = 20-element batches) and persistent workgroups per CU (0: one workgroup per
-   tile; < 0: automatic, the persistent kernel with 2 (FP64) or 3 (FP32) workgroups
-   per CU once there are >= 4 tiles per workgroup).  Results do not depend on it (same
-   summation order). */
+   reference, whose loop is serial): persistent workgroups per CU (0: one workgroup per
+   tile; < 0: automatic, 2, or 4 for SH with FP32 fields).  threads is 256 or 512 and is
+   kept for sem2d_batch_config: the kernel has one workgroup shape.  Results do not depend
+   on either (same summation order). */
 int sem2d_set_tile_config(sem2d_solver *h, int threads, int wg_per_cu);
 
 /* Current step index (number of steps taken). */
@@ -382,12 +381,12 @@ typedef struct sem2d_batch sem2d_batch;
 int sem2d_batch_create(int n, sem2d_solver *const *members, sem2d_batch **out);
 
 /* Advance every member by nsteps.  The loop runs as replays of a captured hipGraph of
-   a chunk of up to 64 steps (the step index is kept in device memory). */
+   a chunk of up to 64 steps (the step index is kept in device memory) between the call's
+   first and last step. */
 int sem2d_batch_step(sem2d_batch *b, int nsteps);
 
 /* Autotuner: time trial_steps steps of each tile-kernel launch configuration
-   (threads per workgroup = elements per batch x 25, workgroups per CU, persistent or
-   one workgroup per tile), keep the fastest and restore the state.  *choice receives
+   (persistent workgroups per CU, or one workgroup per tile), keep the fastest and restore the state.  *choice receives
    the index of the chosen configuration. */
 int sem2d_batch_tune(sem2d_batch *b, int trial_steps, int *choice);
 

@@ -14,6 +14,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "sem2d_kernels.hpp"
 #include "sem2d_libm.hpp"
 
 namespace sem2d {
@@ -42,6 +43,11 @@ struct FaultDev {
   // the fault, zeroed in the force of node 1 (bits 0-1) and node 2 (bits 2-3) before the
   // corrector (null: none)
   const unsigned char* dmask = nullptr;
+  // structured grids: d and v after the step at both nodes of every pair, bulk type,
+  // [d, v][node 1, node 2][ndof][np] (k_fault; the field arrays hold the next step's
+  // predicted values), and the recorded nodes (bit 0: node 1, bit 1: node 2; null: none)
+  void* side = nullptr;
+  const unsigned char* rmark = nullptr;
   // time-weakening friction (BC_DYNFLT_TWF): kind (0: none; law 3: time weakening alone),
   // parameters MuS, MuD, Mu0, X, Z, V, L, T, Dc and the fault node coordinates [2][np]
   int twf = 0;
@@ -68,13 +74,25 @@ __host__ __device__ inline double normal_sigma(int kind, double coef, double vc,
 
 // Corrector of one split-fault node after the fault solve (a = f * rmass, then v and d;
 // SRC/solver.f90:78-82), in the bulk precision and outside the no-contraction region
-// below, like the corrector of every other node.
+// below, like the corrector of every other node; sd, sv: where d and v after the step go
+// for the jumps the fault outputs are made of.
 template <typename R>
-__device__ __forceinline__ void fault_node_correct(R* d, R* v, R* a, size_t i, R rm, R c3, R c4) {
+__device__ __forceinline__ void fault_node_correct(R* d, R* v, R* a, size_t i, R rm, R dt, R c1, R c2, R c3, R c4,
+                                                   const StepOut& so, R* recp, R* sd, R* sv) {
   const R ak = a[i] * rm;
-  a[i] = ak;
-  v[i] = v[i] + c3 * ak;
-  d[i] = d[i] + c4 * ak;
+  const R vn = v[i] + c3 * ak;
+  const R dn = d[i] + c4 * ak;
+  *sd = dn;
+  *sv = vn;
+  if (so.final) {
+    a[i] = ak;
+    v[i] = vn;
+    d[i] = dn;
+  } else {
+    v[i] = vn + c2 * ak;
+    d[i] = dn + dt * vn + c1 * ak;
+    if (recp && so.rec >= 0) recp[i] = so.rec == 0 ? dn : (so.rec == 1 ? vn : ak);
+  }
 }
 
 #pragma clang fp contract(off)
@@ -238,8 +256,8 @@ __device__ inline double f_rsf_v(const FaultDev& F, int k, double tstick, double
 // capped by the 1024-lane default (which spilled them to scratch).  time = it*dt of the
 // step (SRC/main.f90:53), read by time-weakening friction only.
 template <typename R, bool CORR = false>
-__global__ __launch_bounds__(64) void k_fault(FaultDev F, R* __restrict__ d, R* __restrict__ v, R* __restrict__ f,
-                                              int npoin, R c3 = 0, R c4 = 0, double time = 0.0) {
+__global__ __launch_bounds__(64) void k_fault(FaultDev F, R* d, R* v, R* f, int npoin, R dt = 0, R c1 = 0, R c2 = 0, R c3 = 0, R c4 = 0,
+                                              StepOut so = {}, R* recp = nullptr, double time = 0.0) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= F.np) return;
   const int np = F.np, nd = F.ndof;
@@ -341,8 +359,14 @@ __global__ __launch_bounds__(64) void k_fault(FaultDev F, R* __restrict__ d, R* 
       const size_t o = (size_t)c * npoin;
       if (dm >> c & 1) f[o + i1] = 0;
       if (i2 >= 0 && (dm >> (2 + c) & 1)) f[o + i2] = 0;
-      fault_node_correct<R>(d, v, f, o + i1, (R)F.rmn1[c * np + k], c3, c4);
-      if (i2 >= 0) fault_node_correct<R>(d, v, f, o + i2, (R)F.rmn2[c * np + k], c3, c4);
+      R* sd = (R*)F.side + (size_t)c * np + k;
+      R* sv = sd + (size_t)2 * nd * np;
+      const int rec = F.rmark ? F.rmark[k] : 0;
+      fault_node_correct<R>(d, v, f, o + i1, (R)F.rmn1[c * np + k], dt, c1, c2, c3, c4, so, rec & 1 ? recp : nullptr,
+                            sd, sv);
+      if (i2 >= 0)
+        fault_node_correct<R>(d, v, f, o + i2, (R)F.rmn2[c * np + k], dt, c1, c2, c3, c4, so, rec & 2 ? recp : nullptr,
+                              sd + (size_t)nd * np, sv + (size_t)nd * np);
     }
   }
 }
@@ -365,9 +389,10 @@ __global__ void k_fault_record(FaultDev F, int oix1, int oixd, int nout, double*
 // the fault frame (t, n) for P-SV (rotate, SRC/bc_dynflt.f90:722-739); side 2 of a
 // fault with one side is -(side 1).  FP64, no contraction, like the fault solve.
 #pragma clang fp contract(off)
+// side: from F.side instead of the fields.
 template <typename R>
 __global__ void k_fault_sides(FaultDev F, const R* __restrict__ d, const R* __restrict__ v, size_t stride,
-                              int oix1, int oixd, int nout, double* __restrict__ out) {
+                              int oix1, int oixd, int nout, double* __restrict__ out, int side_arrays) {
   const int o = blockIdx.x * blockDim.x + threadIdx.x;
   if (o >= nout) return;
   const int k = oix1 - 1 + o * oixd;
@@ -379,6 +404,11 @@ __global__ void k_fault_sides(FaultDev F, const R* __restrict__ d, const R* __re
       const R* u = w == 0 ? d : v;
       double x[2] = {0.0, 0.0};
       for (int c = 0; c < nd; ++c) {
+        if (side_arrays) {
+          const R* sc = (const R*)F.side + ((size_t)(w * 2) * nd + c) * F.np + k;
+          x[c] = side == 1 ? (double)sc[0] : (i2 >= 0 ? (double)sc[(size_t)nd * F.np] : -(double)sc[0]);
+          continue;
+        }
         const R* uc = u + (size_t)c * stride;
         x[c] = side == 1 ? (double)uc[i1] : (i2 >= 0 ? (double)uc[i2] : -(double)uc[i1]);
       }
@@ -399,11 +429,12 @@ __global__ void k_fault_sides(FaultDev F, const R* __restrict__ d, const R* __re
 // then of v, one row of 2*(ndof+1) values, over the fault pairs k0 .. k0+n-1.  One
 // workgroup of 256 lanes: lane t sums pairs k0+t, k0+t+256, ..., then a fixed-shape
 // tree, so the result is run-to-run identical and the same for a fault alone (k0 = 0)
-// and inside a batch (its pairs at k0 of the concatenated arrays).
+// and inside a batch (its pairs at k0 of the concatenated arrays).  side_arrays: the
+// jumps are taken from F.side instead of the fields.
 template <typename R>
 __device__ __forceinline__ void potency_row(const FaultDev& F, int k0, int n, const R* __restrict__ d,
                                             const R* __restrict__ v, size_t stride, double* __restrict__ out,
-                                            double (*red)[256]) {
+                                            double (*red)[256], int side_arrays) {
   const int t = threadIdx.x, np = F.np;
   double s[6] = {0, 0, 0, 0, 0, 0};
   for (int kl = t; kl < n; kl += 256) {
@@ -411,13 +442,23 @@ __device__ __forceinline__ void potency_row(const FaultDev& F, int k0, int n, co
     const int i1 = F.n1[k], i2 = F.n2[k];
     const double nx = F.nrm[k], nz = F.nrm[np + k], b = F.B[k];
     // get_jump (SRC/bc_dynflt.f90:692-704): x2 - x1, or -2 x1 on a one-sided fault
-    auto jump = [&](const R* x) {
-      return i2 >= 0 ? (double)x[i2] - (double)x[i1] : -2.0 * (double)x[i1];
+    auto jump = [&](int w, int c) {
+      double x1, x2 = 0.0;
+      if (side_arrays) {
+        const R* sc = (const R*)F.side + ((size_t)(w * 2) * F.ndof + c) * np + k;
+        x1 = (double)sc[0];
+        if (i2 >= 0) x2 = (double)sc[(size_t)F.ndof * np];
+      } else {
+        const R* x = (w == 0 ? d : v) + (size_t)c * stride;
+        x1 = (double)x[i1];
+        if (i2 >= 0) x2 = (double)x[i2];
+      }
+      return i2 >= 0 ? x2 - x1 : -2.0 * x1;
     };
-    const double jd0 = jump(d), jv0 = jump(v);
+    const double jd0 = jump(0, 0), jv0 = jump(1, 0);
     if (F.ndof == 2) {
-      const double jd1 = jump(d + stride);
-      const double jv1 = jump(v + stride);
+      const double jd1 = jump(0, 1);
+      const double jv1 = jump(1, 1);
       s[0] += nx * jd0 * b;
       s[1] += nz * jd1 * b;
       s[2] += (nx * jd1 + nz * jd0) * b;
@@ -457,9 +498,9 @@ __device__ __forceinline__ void potency_row(const FaultDev& F, int k0, int n, co
 
 template <typename R>
 __global__ __launch_bounds__(256) void k_fault_potency(FaultDev F, const R* __restrict__ d, const R* __restrict__ v,
-                                                       size_t stride, double* __restrict__ out) {
+                                                       size_t stride, double* __restrict__ out, int side_arrays) {
   __shared__ double red[6][256];
-  potency_row<R>(F, 0, F.np, d, v, stride, out, red);
+  potency_row<R>(F, 0, F.np, d, v, stride, out, red, side_arrays);
 }
 
 // Batched potency: workgroup m writes member m's row for the state after the current
@@ -476,7 +517,8 @@ __global__ __launch_bounds__(256) void k_batch_potency(FaultDev F, const int* __
   const int row = row_shift + *itp;
   if (row < 0 || row >= cap) return;  // uniform over the workgroup; the host reserves the rows
   const int k0 = fbase[m];
-  potency_row<R>(F, k0, fbase[m + 1] - k0, d, v, stride, pot + ((size_t)m * cap + row) * (2 * (F.ndof + 1)), red);
+  potency_row<R>(F, k0, fbase[m + 1] - k0, d, v, stride, pot + ((size_t)m * cap + row) * (2 * (F.ndof + 1)), red,
+                 1);
 }
 
 #pragma clang fp contract(on)

@@ -17,15 +17,41 @@ constexpr int NGMAX = 10;  // largest NGLL of the general element kernel
 // h'_i(x_j) stored at H[i*5+j], and wgll(i)*wgll(j) at W2[j*5+i] (they only depend on NGLL)
 __constant__ double c_H[NP];
 __constant__ double c_W2[NP];
+__constant__ float c_Hf[NP];  // c_H in single precision
 
 // Coefficient storage modes (sem2d_desc.coef_mode).  COEF_NODE is internal to the
 // structured tile kernel: the compact moduli stored once per global node (in the field
 // layout) when every element sharing a node holds the same values there.
 enum { COEF_PER_ELEM = 0, COEF_SHARED = 1, COEF_COMPACT = 2, COEF_NODE = 3 };
 
+// h'_i(x_j) at [i*NG + j] in the bulk type, by a pointer the compiler cannot look through:
+// read at compile-time indices, the entries are scalar operands, loaded where this is
+// called and not held in scalar registers throughout
+template <typename R>
+__device__ __forceinline__ const __attribute__((address_space(4))) R* hconst() {
+  using P = const __attribute__((address_space(4))) R*;
+  P p;
+  if constexpr (sizeof(R) == 4) p = (P)c_Hf;
+  else p = (P)c_H;
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
 template <typename R>
 struct Coef {
   static __device__ __forceinline__ R h(int a, int b) { return (R)c_H[a * NG + b]; }
+};
+
+// What a step stores.  final: the state (d, v, a) after the step, as callers see it.
+// Otherwise the state the next step starts from: its predicted displacement and velocity,
+// dp = d + dt v + c1 a and vp = v + c2 a (SRC/solver.f90:59-60) formed from the values the
+// step has just computed, in place of d and v; a is not stored (the next step needs no
+// other than through dp and vp), so a step of a run moves two field arrays each way
+// instead of three.  accel: a is stored as well.  rec: nodes marked as recorded take the
+// recorded field (0: d, 1: v, 2: a; -1: none) into their place of a field array of its
+// own (the a array, where that is not stored).
+struct StepOut {
+  int final = 1, accel = 0, rec = -1;
 };
 
 // ---------------------------------------------------------------------------

@@ -67,16 +67,16 @@ struct StructState {
   int nvl = 0;                    // vertical tile-edge lines (stored column-contiguous)
   size_t NS = 0;                  // field component stride: ROW*NZ1 + nvl*NZ1
   std::vector<int4> tiles;
-  int ntiles = 0, per_xcd = 0;
-  int pipe_wgs = 0;  // > 0: persistent pipelined tile kernel with this many workgroups
+  int ntiles = 0;
+  int pipe_wgs = 0;  // persistent workgroups of the tile kernel (0: one per tile)
   // Kelvin-Voigt eta and 2.5D coefficient per element point, cell order [cell][25] (bulk
   // type), or null; either makes the tile kernel form d + eta v at the element points
   void *eta = nullptr, *b25 = nullptr;
-  int pipe_threads = 512;
   int4* tiles_dev = nullptr;
   int4* grids_dev = nullptr;
-  int* tlist_dev = nullptr;  // launch list of the pipelined kernel: full tiles, then the rest
-  int nfull = 0, npart = 0;
+  int* tlist_dev = nullptr;  // launch list of the adjoint tile kernels: full tiles, then the rest
+  int nfull = 0;
+  bool w32 = false;  // field, partial-force and per-cell arrays below 4 GiB per component
   // Stacey terms: boundary elements (storage-index edge nodes, K), per absorbing entry
   // of the deferred nodes the element points it subtracts, and their values per step
   int s_nbe = 0;
@@ -84,6 +84,8 @@ struct StructState {
   double *s_K = nullptr, *kxd = nullptr;
   int* spec_cnt = nullptr;
   int* spec_idx = nullptr;
+  int* mark_of = nullptr;  // recorded nodes inside tiles (TileArgs)
+  uint32_t* marks = nullptr;
   void* fpart = nullptr;
   size_t FPS = 0;
   DefTable defs;
@@ -158,6 +160,7 @@ struct sem2d_solver {
   bool src_dirty = false;
   // receivers
   int nrec = 0, isamp = 1, field = 1, nsamp = 0, taken = 0;
+  std::vector<int> rec_ref;      // reference nodes that are recorded (0-based)
   int* rec_node = nullptr;       // [nrec] node, or [nrec][25] element nodes when interpolated
   double* rec_w = nullptr;       // [nrec][25] interpolation weights (nullptr: receivers at nodes)
   double* seis = nullptr;
@@ -438,12 +441,15 @@ int sync_sources(sem2d_solver* h) {
   return 0;
 }
 
+// whether the state after step it is a receiver sample
+bool sampled(const sem2d_solver* h, int it) { return h->nrec && it % h->isamp == 0 && it / h->isamp < h->nsamp; }
+
+// marked: the recorded field is in the a array at the recorded nodes (StepOut::rec)
 template <typename R>
-int record_receivers(sem2d_solver* h) {
-  if (!h->nrec || h->it % h->isamp) return 0;
-  int s = h->it / h->isamp;
-  if (s >= h->nsamp) return 0;
-  const R* fld = (const R*)(h->field == 0 ? h->d : (h->field == 1 ? h->v : h->a));
+int record_receivers(sem2d_solver* h, bool marked = false) {
+  if (!sampled(h, h->it)) return 0;
+  const int s = h->it / h->isamp;
+  const R* fld = (const R*)(marked || h->field == 2 ? h->a : (h->field == 0 ? h->d : h->v));
   if (h->rec_w)
     k_receivers_interp<R><<<grid_for(h->nrec, 64), 64, 0, h->stream>>>(
         h->nrec, h->ndof, h->rec_node, h->rec_w, fld, h->fstride, h->seis + (size_t)s * h->ndof * h->nrec, h->np);
@@ -497,37 +503,38 @@ int potency_reserve(sem2d_solver* h, int rows) {
   return 0;
 }
 
+// sides: from FaultDev::side (the steps of a structured grid) instead of the fields
 template <typename R>
-void record_potency(sem2d_solver* h) {
+void record_potency(sem2d_solver* h, int sides) {
   FaultHost& F = h->flt;
   if (F.pot_rows >= F.pot_cap) return;  // reserved by the caller
   k_fault_potency<R><<<1, 256, 0, h->stream>>>(F.dev, (const R*)h->d, (const R*)h->v, h->fstride,
-                                               F.pot + (size_t)F.pot_rows * 2 * (h->ndof + 1));
+                                               F.pot + (size_t)F.pot_rows * 2 * (h->ndof + 1), sides);
   F.pot_rows++;
 }
 
 // per-side record (osides) of sample slot s from the current fields
-void record_sides(sem2d_solver* h, int s) {
+void record_sides(sem2d_solver* h, int s, int sides) {
   FaultHost& F = h->flt;
   double* out = F.srec + (size_t)s * 4 * h->ndof * F.nout;
   if (h->fp32)
     k_fault_sides<float><<<grid_for(F.nout, 64), 64, 0, h->stream>>>(F.dev, (const float*)h->d, (const float*)h->v,
-                                                                      h->fstride, F.oix1, F.oixd, F.nout, out);
+                                                                      h->fstride, F.oix1, F.oixd, F.nout, out, sides);
   else
     k_fault_sides<double><<<grid_for(F.nout, 64), 64, 0, h->stream>>>(
-        F.dev, (const double*)h->d, (const double*)h->v, h->fstride, F.oix1, F.oixd, F.nout, out);
+        F.dev, (const double*)h->d, (const double*)h->v, h->fstride, F.oix1, F.oixd, F.nout, out, sides);
 }
 
-int record_fault(sem2d_solver* h) {
+int record_fault(sem2d_solver* h, int sides = 0) {
   FaultHost& F = h->flt;
   if (!F.on) return 0;
-  if (h->fp32) record_potency<float>(h);
-  else record_potency<double>(h);
+  if (h->fp32) record_potency<float>(h, sides);
+  else record_potency<double>(h, sides);
   if (h->it < F.oit) return 0;
   if (F.taken < F.nsamp) {
     k_fault_record<<<grid_for(F.nout, 64), 64, 0, h->stream>>>(F.dev, F.oix1, F.oixd, F.nout,
                                                                F.rec + (size_t)F.taken * 6 * F.nout);
-    if (F.srec) record_sides(h, F.taken);
+    if (F.srec) record_sides(h, F.taken, sides);
     F.taken++;
   }
   F.oit += F.oitd;
@@ -553,6 +560,13 @@ static size_t storage_index(const StructState& S, int X, int Z) {
   if (k >= 0) return (size_t)S.ROW * S.NZ1 + (size_t)k * S.NZ1 + Z;
   return (size_t)Z * S.ROW + (size_t)(X / W) * W + (X % W) - 1;
 }
+
+// Workgroups of the tile kernel per CU.  Two by default: with six wavefronts each they keep
+// to 128 registers where the dispatcher packs four on a SIMD (P-SV, 1000 x 500 elements,
+// us per step with 1 / 2 / 3 / 4: FP64 225 / 182 / 198 / 210, FP32 176 / 117 / 137 / 118;
+// SH FP64, 600 x 300: 58 / 45 / 48 / 53).  The SH kernel with FP32 fields needs 62
+// registers and 25 KB of LDS at most: four (333 x 251: 30 / 24 / 22 / 21).
+static int tile_wgs_per_cu(bool fp32, int ndof) { return fp32 && ndof == 1 ? 4 : 2; }
 
 bool structured_map(sem2d_solver* h, const sem2d_desc* s) {
   StructState& S = h->st;
@@ -607,27 +621,18 @@ bool structured_map(sem2d_solver* h, const sem2d_desc* s) {
       }
   }
   S.ntiles = (int)S.tiles.size();
-  S.per_xcd = (S.ntiles + 7) / 8;
   {
     int dev = 0, ncu = 256;
     if (hipGetDevice(&dev) == hipSuccess) hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    // measured on MI355X (2000x1000-element P-SV, full-tile variant): 512 threads
-    // (20-element batches, one batch per colour) with 1 workgroup per CU for FP64 fields
-    // (VGPRs allow 8 waves per CU), 2 for FP32
-    int per_cu = h->fp32 ? 2 : 1;
+    int per_cu = tile_wgs_per_cu(h->fp32, h->ndof);
     const char* env = getenv("SEM2D_TILE_WG_PER_CU");
     if (env) per_cu = atoi(env);
-    S.pipe_threads = 512;
-    const char* envt = getenv("SEM2D_TILE_THREADS");
-    if (envt) S.pipe_threads = atoi(envt) == 256 ? 256 : 512;
-    // the persistent kernel pays off once there are several tiles per workgroup
-    S.pipe_wgs = per_cu > 0 && S.ntiles >= 4 * ncu * per_cu ? ncu * per_cu : 0;
-    S.pipe_wgs = ((S.pipe_wgs + 7) / 8) * 8;
+    S.pipe_wgs = std::max(0, (ncu * per_cu + 7) / 8 * 8);
   }
   return true;
 }
 
-// Launch list of the pipelined tile kernel: the full TX x TZ tiles (its constant-shape,
+// Launch list of the adjoint tile kernels: the full TX x TZ tiles (their constant-shape,
 // 32-bit-offset variant) first, then the others.  idx32: the field and partial-force
 // arrays are below 4 GiB per component, as that variant requires; otherwise every tile
 // goes to the general variant.
@@ -661,7 +666,8 @@ bool pack_defs(const std::vector<DefNode>& in, const std::vector<int>& part_off,
     DefDev e;
     e.g = n.g;
     e.pstart = n.pstart;
-    e.cnt = n.pcnt | (n.scnt << 8) | (n.acnt << 16) | ((n.fault ? 1 : 0) << 24) | ((n.dmask & 3) << 26);
+    e.cnt = n.pcnt | (n.scnt << 8) | (n.acnt << 16) | ((n.fault ? 1 : 0) << 24) | ((n.dmask & 3) << 26) |
+            ((n.rec ? 1 : 0) << 28);
     e.x = -1;
     if (n.scnt > 0 || n.acnt > 0) {
       e.x = (int)ext.size();
@@ -711,6 +717,10 @@ struct StructTables {
   std::vector<double> fault_rm;  // [ndof][nf]
   std::vector<unsigned char> fault_dmask;  // [npairs] Dirichlet after the fault: node 1 bits 0-1, node 2 bits 2-3
   std::vector<int> s_enode, ak_off, ak_idx;  // Stacey (see StructState)
+  // recorded nodes: inside tiles (TileArgs::mark_of, marks), of fault pairs (FaultDev::rmark)
+  std::vector<int> mark_of;
+  std::vector<uint32_t> marks;
+  std::vector<unsigned char> fault_rmark;
   std::vector<double> s_K;
 };
 
@@ -743,7 +753,7 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
       const int Xn = g % S.NX1 - X0, Zn = g / S.NX1 - Z0;
       if (Xn > 0 && Xn < PX - 1 && Zn > 0 && Zn < PZ - 1) {
         if (X.spec_cnt[t] >= MAXSPECIAL) return set_err(h, 5, "too many source nodes in one tile");
-        X.spec_idx[(size_t)t * MAXSPECIAL + X.spec_cnt[t]] = Zn * PX + Xn;
+        X.spec_idx[(size_t)t * MAXSPECIAL + X.spec_cnt[t]] = Zn * PXM + Xn;
         ents.push_back({(int)storage_index(S, X0 + Xn, Z0 + Zn), t, PERIM_MAX + X.spec_cnt[t]});
         X.spec_cnt[t]++;
       }
@@ -793,6 +803,8 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   }
   X.ak_off.assign(1, 0);
   X.ak_idx.clear();
+  std::vector<char> is_rec((size_t)h->npoin, 0);  // recorded reference nodes
+  for (int k : h->rec_ref) is_rec[k] = 1;
 
   X.defs.clear();
   X.part_off.clear();
@@ -829,6 +841,7 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
     n.acnt = (int)(X.dabso.size() / nd) - n.astart;
     n.fault = is_fault[ref];
     n.dmask = dmask_def[ref];
+    n.rec = is_rec[ref];
     X.defs.push_back(n);
     def_ref.push_back(ref);
     i = j;
@@ -845,6 +858,36 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   for (size_t k = 0; k < h->fault_n1.size(); ++k) {
     X.fault_dmask[k] = dmask_aft[h->fault_n1[k]];
     if (!h->fault_n2.empty()) X.fault_dmask[k] |= (unsigned char)(dmask_aft[h->fault_n2[k]] << 2);
+  }
+  X.fault_rmark.assign(h->fault_n1.size(), 0);
+  for (size_t k = 0; k < h->fault_n1.size(); ++k) {
+    X.fault_rmark[k] = is_rec[h->fault_n1[k]];
+    if (!h->fault_n2.empty()) X.fault_rmark[k] |= (unsigned char)(is_rec[h->fault_n2[k]] << 1);
+  }
+  // recorded nodes that are not deferred nodes: marks of the tile they lie in
+  X.mark_of.assign(S.ntiles, -1);
+  X.marks.clear();
+  {
+    std::vector<char> is_def((size_t)h->npoin, 0);
+    for (int ref : def_ref) is_def[ref] = 1;
+    const int ncx = (S.nx + TX - 1) / TX;
+    for (int ref : h->rec_ref) {
+      if (is_def[ref]) continue;
+      const int Xg = S.gridx[ref] % S.NX1, Zg = S.gridx[ref] / S.NX1;
+      const int band = S.ezflt > 0 && Zg > 4 * S.ezflt;
+      const int zl = band ? Zg - (4 * S.ezflt + 1) : Zg;
+      const int t = (band ? (S.ezflt + TZ - 1) / TZ * ncx : 0) + zl / (4 * TZ) * ncx + Xg / (4 * TX);
+      const int4 tg = S.tiles[t];
+      const int Xn = Xg - 4 * tg.x, Zn = Zg - tg.w;
+      if (Xn <= 0 || Zn <= 0 || Xn >= 4 * (tg.z & 0xff) || Zn >= 4 * ((tg.z >> 8) & 0xff))
+        return set_err(h, 5, "recorded node %d: not inside its tile", ref + 1);
+      if (X.mark_of[t] < 0) {
+        X.mark_of[t] = (int)(X.marks.size() / MARK_WORDS);
+        X.marks.resize(X.marks.size() + MARK_WORDS, 0u);
+      }
+      const int p = Zn * PXM + Xn;
+      X.marks[(size_t)X.mark_of[t] * MARK_WORDS + (p >> 5)] |= 1u << (p & 31);
+    }
   }
   // every split-fault node must be a deferred node: k_deferred leaves those nodes
   // uncorrected and k_fault finishes both nodes of each pair; a fault node inside a
@@ -911,6 +954,8 @@ int prepare_structured(sem2d_solver* h) {
   if ((rc = prep_upload(h, &S.grids_dev, X.grids.data(), X.grids.size()))) return rc;
   if ((rc = prep_upload(h, &S.spec_cnt, X.spec_cnt.data(), X.spec_cnt.size()))) return rc;
   if ((rc = prep_upload(h, &S.spec_idx, X.spec_idx.data(), X.spec_idx.size()))) return rc;
+  if ((rc = prep_upload(h, &S.mark_of, X.mark_of.data(), X.mark_of.size()))) return rc;
+  if ((rc = prep_upload(h, &S.marks, X.marks.data(), X.marks.size()))) return rc;
   {
     std::vector<DefDev> dn;
     std::vector<int2> dx;
@@ -934,8 +979,8 @@ int prepare_structured(sem2d_solver* h) {
     size_t ncell = h->coef_mode == COEF_SHARED ? (size_t)h->nelast * NP
                                                : (size_t)h->nelem * std::max(h->ndof, h->nelast) * NP;
     if (S.eta || S.b25) ncell = std::max(ncell, (size_t)h->nelem * NP);
-    const std::vector<int> list = tile_list(X.tiles, fits32(h->fstride, S.FPS, ncell, rsize(h)), S.nfull);
-    S.npart = S.ntiles - S.nfull;
+    S.w32 = fits32(h->fstride, S.FPS, ncell, rsize(h));
+    const std::vector<int> list = tile_list(X.tiles, S.w32, S.nfull);
     if ((rc = prep_upload(h, &S.tlist_dev, list.data(), list.size()))) return rc;
   }
   void* fp = nullptr;
@@ -962,6 +1007,17 @@ int prepare_structured(sem2d_solver* h) {
     HIPCHK(h, hipStreamSynchronize(h->stream));  // the vectors are local
     h->flt.dev.rmn1 = p1;
     h->flt.dev.rmn2 = p2;
+    const size_t nside = (size_t)4 * h->ndof * h->fault_n1.size() * rsize(h);
+    HIPCHK(h, hipMalloc(&h->flt.dev.side, nside));
+    S.prep_allocs.push_back(h->flt.dev.side);
+    HIPCHK(h, hipMemsetAsync(h->flt.dev.side, 0, nside, h->stream));
+    h->flt.dev.rmark = nullptr;
+    if (std::any_of(X.fault_rmark.begin(), X.fault_rmark.end(), [](unsigned char m) { return m != 0; })) {
+      unsigned char* pm = nullptr;
+      if ((rc = prep_upload(h, &pm, X.fault_rmark.data(), X.fault_rmark.size()))) return rc;
+      HIPCHK(h, hipStreamSynchronize(h->stream));
+      h->flt.dev.rmark = pm;
+    }
     h->flt.dev.dmask = nullptr;
     bool any = false;
     for (unsigned char m : X.fault_dmask) any |= m != 0;
@@ -984,13 +1040,12 @@ struct StepDev {
   size_t fstride = 0;
   void *d = nullptr, *v = nullptr, *a = nullptr;
   TileDev T{};
-  const int* tlist = nullptr;  // pipelined kernel: tlist[0 .. nfull) full tiles, then npart others
-  int nfull = 0, npart = 0;
+  bool w32 = false;  // field, partial-force and per-cell arrays below 4 GiB per component
   int s_nbe = 0;  // Stacey boundary elements (k_stacey_pre), their values passed to k_deferred
   const int* s_enode = nullptr;
   const double* s_K = nullptr;
   StaceyRefs SR{};
-  int pipe_wgs = 0, pipe_threads = 512;
+  int pipe_wgs = 0;  // persistent workgroups of the tile kernel (0: one per tile)
   const void *rmass0 = nullptr, *coefs = nullptr, *geom = nullptr;
   const void* nodemod = nullptr;  // per-node moduli (COEF_NODE), or null
   const void *eta = nullptr, *b25 = nullptr;  // element-point terms (Kelvin-Voigt, 2.5D), or null
@@ -1007,6 +1062,11 @@ struct StepDev {
   FaultDev F{};
   const int* itp = nullptr;  // device step counter (graph replay) or null: step index by value
   hipStream_t stream = nullptr;
+  bool pin = false;  // the state read is the predicted one (StepOut)
+  StepOut out;
+  void* rec = nullptr;  // where recorded nodes go (null: the a array)
+  const int* mark_of = nullptr;
+  const uint32_t* marks = nullptr;
   // out-of-place step (adjoint replay): read the state here, write it to d, v, a
   const void *din = nullptr, *vin = nullptr, *ain = nullptr;
 };
@@ -1022,22 +1082,20 @@ StepDev step_dev(sem2d_solver* h) {
   X.v = h->v;
   X.a = h->a;
   X.T.ntiles = S.ntiles;
-  X.T.per_xcd = S.per_xcd;
   X.T.tiles = S.tiles_dev;
   X.T.grids = S.grids_dev;
-  X.tlist = S.tlist_dev;
-  X.nfull = S.nfull;
-  X.npart = S.npart;
+  X.w32 = S.w32;
   X.s_nbe = S.s_nbe;
   X.s_enode = S.s_enode;
   X.s_K = S.s_K;
   if (S.s_nbe > 0) X.SR = StaceyRefs{S.ak_off, S.ak_idx, S.kxd};
   X.T.spec_cnt = S.spec_cnt;
   X.T.spec_idx = S.spec_idx;
+  X.mark_of = S.mark_of;
+  X.marks = S.marks;
   X.T.NGp = h->fstride;
   X.T.FPS = S.FPS;
   X.pipe_wgs = S.pipe_wgs;
-  X.pipe_threads = S.pipe_threads;
   X.rmass0 = S.rmass0;
   X.coefs = S.coefs;
   X.nodemod = S.nodemod;
@@ -1059,135 +1117,94 @@ StepDev step_dev(sem2d_solver* h) {
   return X;
 }
 
-// Pipelined tile kernel over n listed tiles (FULL: all of them full tiles; EP: with the
-// element-point terms, 512 threads)
-template <typename R, int NDOF, int NELAST, int MODE, bool OOP, bool FULL, bool EP = false>
-void launch_pipe(const StepDev& X, const int* list, int n, R dt, R c1, R c2, R c3, R c4, const R* di,
-                 const R* vi, const R* ai) {
-  if (n <= 0) return;
-  const int wgs = std::min(X.pipe_wgs, (n + 7) / 8 * 8);
-  const R* co = (const R*)(MODE == COEF_NODE ? X.nodemod : X.coefs);
-  if constexpr (EP) {
-    k_tile_pipe<R, NDOF, NELAST, MODE, 512, 20, OOP, FULL, true><<<wgs, 512, 0, X.stream>>>(
-        X.T, list, n, X.T.tiles, X.T.grids, X.T.spec_cnt, (R*)X.d, (R*)X.v, (R*)X.a, (const R*)X.rmass0, co,
-        (const R*)X.geom, (R*)X.fpart, dt, c1, c2, c3, c4, di, vi, ai, (const R*)X.eta, (const R*)X.b25);
-    return;
-  }
-  if (X.pipe_threads == 256)
-    k_tile_pipe<R, NDOF, NELAST, MODE, 256, 10, OOP, FULL><<<wgs, 256, 0, X.stream>>>(
-        X.T, list, n, X.T.tiles, X.T.grids, X.T.spec_cnt, (R*)X.d, (R*)X.v, (R*)X.a, (const R*)X.rmass0, co,
-        (const R*)X.geom, (R*)X.fpart, dt, c1, c2, c3, c4, di, vi, ai);
-  else
-    k_tile_pipe<R, NDOF, NELAST, MODE, 512, 20, OOP, FULL><<<wgs, 512, 0, X.stream>>>(
-        X.T, list, n, X.T.tiles, X.T.grids, X.T.spec_cnt, (R*)X.d, (R*)X.v, (R*)X.a, (const R*)X.rmass0, co,
-        (const R*)X.geom, (R*)X.fpart, dt, c1, c2, c3, c4, di, vi, ai);
+// Tile kernel over all tiles: pipe_wgs persistent workgroups, or one per tile where there
+// are fewer tiles (or pipe_wgs is 0).  Compact moduli are read once per node when the grid
+// has them in that form.
+template <typename R, int NDOF, int NELAST, int MODE, bool OOP, bool EP, bool PIN>
+void launch_tile_p(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
+  const int n = X.T.ntiles, per_tile = (n + 7) / 8 * 8;
+  const int wgs = X.pipe_wgs > 0 ? std::min(X.pipe_wgs, per_tile) : per_tile;
+  TileArgs<R> A;
+  A.d = (R*)X.d, A.v = (R*)X.v, A.a = (R*)X.a;
+  A.din = (const R*)X.din, A.vin = (const R*)X.vin, A.ain = (const R*)X.ain;
+  A.rmass0 = (const R*)X.rmass0;
+  A.coefs = (const R*)(MODE == COEF_NODE ? X.nodemod : X.coefs);
+  A.geom = (const R*)X.geom, A.eta = (const R*)X.eta, A.b25 = (const R*)X.b25;
+  A.fpart = (R*)X.fpart;
+  A.rec = (R*)(X.rec ? X.rec : X.a);
+  A.S = X.T.NGp, A.FPS = X.T.FPS;
+  A.tiles = X.T.tiles, A.grids = X.T.grids;
+  A.spec_cnt = X.T.spec_cnt, A.spec_idx = X.T.spec_idx;
+  A.mark_of = X.mark_of, A.marks = X.marks;
+  A.out = X.out;
+  A.ntiles = n;
+  A.dt = dt, A.c1 = c1, A.c2 = c2, A.c3 = c3, A.c4 = c4;
+  auto go = [&](auto w32) {
+    k_tile_step<R, NDOF, NELAST, MODE, OOP, decltype(w32)::value, EP, PIN><<<wgs, TS_NT, 0, X.stream>>>(A);
+  };
+  if (X.w32) go(std::true_type{});
+  else if constexpr (!PIN) go(std::false_type{});  // such grids keep to (d, v, a)
 }
 
-// both launches (full tiles, then edge tiles) of the pipelined kernel; compact moduli
-// are read once per node when the grid has them in that form
-template <typename R, int NDOF, int NELAST, int MODE, bool OOP, bool EP = false>
-void launch_pipe2(const StepDev& X, R dt, R c1, R c2, R c3, R c4, const R* di, const R* vi, const R* ai) {
-  // tiles that all fit in one wave of workgroups (small grids, e.g. 100 x 100 elements):
-  // a single launch of the general variant, whose duration is one tile's, instead of two
-  // launches in series
-  const bool one = X.nfull + X.npart <= X.pipe_wgs;
-  if constexpr (MODE == COEF_COMPACT && (NELAST == 6 || NELAST == 2)) {
-    if (X.nodemod) {
-      if (one) {
-        launch_pipe<R, NDOF, NELAST, COEF_NODE, OOP, false, EP>(X, X.tlist, X.nfull + X.npart, dt, c1, c2, c3, c4,
-                                                                di, vi, ai);
-        return;
-      }
-      launch_pipe<R, NDOF, NELAST, COEF_NODE, OOP, true, EP>(X, X.tlist, X.nfull, dt, c1, c2, c3, c4, di, vi, ai);
-      launch_pipe<R, NDOF, NELAST, COEF_NODE, OOP, false, EP>(X, X.tlist + X.nfull, X.npart, dt, c1, c2, c3, c4,
-                                                              di, vi, ai);
-      return;
-    }
-  }
-  if (one) {
-    launch_pipe<R, NDOF, NELAST, MODE, OOP, false, EP>(X, X.tlist, X.nfull + X.npart, dt, c1, c2, c3, c4, di, vi,
-                                                       ai);
-    return;
-  }
-  launch_pipe<R, NDOF, NELAST, MODE, OOP, true, EP>(X, X.tlist, X.nfull, dt, c1, c2, c3, c4, di, vi, ai);
-  launch_pipe<R, NDOF, NELAST, MODE, OOP, false, EP>(X, X.tlist + X.nfull, X.npart, dt, c1, c2, c3, c4, di, vi,
-                                                     ai);
+template <typename R, int NDOF, int NELAST, int MODE, bool OOP, bool EP>
+void launch_tile_k(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
+  if (X.pin) launch_tile_p<R, NDOF, NELAST, MODE, OOP, EP, true>(X, dt, c1, c2, c3, c4);
+  else launch_tile_p<R, NDOF, NELAST, MODE, OOP, EP, false>(X, dt, c1, c2, c3, c4);
 }
 
 template <typename R, int NDOF, int NELAST, int MODE>
 void launch_tile_t(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
-  if constexpr (MODE == COEF_COMPACT && NDOF == 2 && NELAST == 6) {
-    if (X.din) {  // out of place (only the adjoint replay, P-SV compact)
-      const R *di = (const R*)X.din, *vi = (const R*)X.vin, *ai = (const R*)X.ain;
-      if (X.pipe_wgs > 0) {
-        launch_pipe2<R, NDOF, NELAST, MODE, true>(X, dt, c1, c2, c3, c4, di, vi, ai);
-      } else {
-        k_tile<R, NDOF, NELAST, MODE, true><<<8 * X.T.per_xcd, TILE_THREADS, 0, X.stream>>>(
-            X.T, (R*)X.d, (R*)X.v, (R*)X.a, (const R*)X.rmass0, (const R*)X.coefs, (const R*)X.geom,
-            (R*)X.fpart, dt, c1, c2, c3, c4, di, vi, ai);
-      }
+  if constexpr (MODE == COEF_COMPACT) {
+    if (X.nodemod) {
+      launch_tile_t<R, NDOF, NELAST, COEF_NODE>(X, dt, c1, c2, c3, c4);
       return;
     }
   }
-  if constexpr ((NDOF == 2 && NELAST == 6) || (NDOF == 1 && NELAST == 2)) {
-    if (X.eta || X.b25) {  // Kelvin-Voigt or 2.5D: pipelined kernel with element-point terms
-      launch_pipe2<R, NDOF, NELAST, MODE, false, true>(X, dt, c1, c2, c3, c4, nullptr, nullptr, nullptr);
+  if constexpr ((MODE == COEF_COMPACT || MODE == COEF_NODE) && NDOF == 2) {
+    if (X.din) {  // out of place: the adjoint's forward and replay (P-SV, compact)
+      launch_tile_k<R, NDOF, NELAST, MODE, true, false>(X, dt, c1, c2, c3, c4);
       return;
     }
   }
-  if (X.pipe_wgs > 0) {
-    // persistent pipelined kernel: up to pipe_wgs workgroups, each on a run of tiles;
-    // the full tiles and the others (grid edges) in two launches
-    launch_pipe2<R, NDOF, NELAST, MODE, false>(X, dt, c1, c2, c3, c4, nullptr, nullptr, nullptr);
-  } else {
-    k_tile<R, NDOF, NELAST, MODE><<<8 * X.T.per_xcd, TILE_THREADS, 0, X.stream>>>(
-        X.T, (R*)X.d, (R*)X.v, (R*)X.a, (const R*)X.rmass0, (const R*)X.coefs, (const R*)X.geom, (R*)X.fpart,
-        dt, c1, c2, c3, c4);
-  }
+  if (X.eta || X.b25) launch_tile_k<R, NDOF, NELAST, MODE, false, true>(X, dt, c1, c2, c3, c4);
+  else launch_tile_k<R, NDOF, NELAST, MODE, false, false>(X, dt, c1, c2, c3, c4);
 }
 
 template <typename R, int NDOF, int NELAST>
 void launch_tile_m(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
   switch (X.coef_mode) {
     case COEF_SHARED: launch_tile_t<R, NDOF, NELAST, COEF_SHARED>(X, dt, c1, c2, c3, c4); break;
-    case COEF_COMPACT:
-      if constexpr (NELAST == 2 || NELAST == 6) launch_tile_t<R, NDOF, NELAST, COEF_COMPACT>(X, dt, c1, c2, c3, c4);
-      break;
+    case COEF_COMPACT: launch_tile_t<R, NDOF, NELAST, COEF_COMPACT>(X, dt, c1, c2, c3, c4); break;
     default: launch_tile_t<R, NDOF, NELAST, COEF_PER_ELEM>(X, dt, c1, c2, c3, c4);
   }
 }
 
 template <typename R>
 void launch_structured_step(const StepDev& X, int it, R dt, R c1, R c2, R c3, R c4) {
-  if (X.ndof == 2) {
-    if (X.nelast == 6) launch_tile_m<R, 2, 6>(X, dt, c1, c2, c3, c4);
-    else launch_tile_m<R, 2, 10>(X, dt, c1, c2, c3, c4);
-  } else {
-    if (X.nelast == 2) launch_tile_m<R, 1, 2>(X, dt, c1, c2, c3, c4);
-    else launch_tile_m<R, 1, 3>(X, dt, c1, c2, c3, c4);
-  }
-  const int gd = (X.ndef + 255) / 256;
+  if (X.ndof == 2) launch_tile_m<R, 2, 6>(X, dt, c1, c2, c3, c4);
+  else launch_tile_m<R, 1, 2>(X, dt, c1, c2, c3, c4);
   if (X.s_nbe > 0)  // Stacey terms from the previous step's state (boundary nodes are deferred)
     k_stacey_pre<R><<<(X.s_nbe * NG + 127) / 128, 128, 0, X.stream>>>(
         X.s_nbe, X.s_enode, X.s_K, (const R*)(X.din ? X.din : X.d), (const R*)(X.din && X.vin ? X.vin : X.v),
-        (const R*)(X.din && X.ain ? X.ain : X.a), X.fstride, dt, c1, (double*)X.SR.kxd);
-  if (X.ndof == 2 && X.din)
-    k_deferred<R, 2, true><<<gd, 256, 0, X.stream>>>(X.ndef, X.defs, X.part_off, (const R*)X.fpart, X.T.FPS,
-                                                      X.dsrc, X.ampl, X.ampl_nt, it, X.itp, X.dabso,
-                                                      (const R*)X.rmdef, (R*)X.d, (R*)X.v, (R*)X.a, X.fstride, dt,
-                                                      c1, c2, c3, c4, (const R*)X.din, (const R*)X.vin,
-                                                      (const R*)X.ain, X.SR);
-  else if (X.ndof == 2)
-    k_deferred<R, 2><<<gd, 256, 0, X.stream>>>(X.ndef, X.defs, X.part_off, (const R*)X.fpart, X.T.FPS, X.dsrc,
-                                                X.ampl, X.ampl_nt, it, X.itp, X.dabso, (const R*)X.rmdef, (R*)X.d,
-                                                (R*)X.v, (R*)X.a, X.fstride, dt, c1, c2, c3, c4, nullptr, nullptr,
-                                                nullptr, X.SR);
-  else
-    k_deferred<R, 1><<<gd, 256, 0, X.stream>>>(X.ndef, X.defs, X.part_off, (const R*)X.fpart, X.T.FPS, X.dsrc,
-                                                X.ampl, X.ampl_nt, it, X.itp, X.dabso, (const R*)X.rmdef, (R*)X.d,
-                                                (R*)X.v, (R*)X.a, X.fstride, dt, c1, c2, c3, c4);
+        (const R*)(X.din && X.ain ? X.ain : X.a), X.fstride, dt, c1, (double*)X.SR.kxd, X.pin);
+  auto deferred = [&](auto nd, auto oop, auto pin) {
+    k_deferred<R, decltype(nd)::value, decltype(oop)::value, decltype(pin)::value>
+        <<<(X.ndef + 255) / 256, 256, 0, X.stream>>>(
+            X.ndef, X.defs, X.part_off, (const R*)X.fpart, X.T.FPS, X.dsrc, X.ampl, X.ampl_nt, it, X.itp, X.dabso,
+            (const R*)X.rmdef, (R*)X.d, (R*)X.v, (R*)X.a, X.fstride, dt, c1, c2, c3, c4, X.out,
+            (R*)(X.rec ? X.rec : X.a), (const R*)X.din,
+            (const R*)X.vin, (const R*)X.ain, X.SR);
+  };
+  using N1 = std::integral_constant<int, 1>;
+  using N2 = std::integral_constant<int, 2>;
+  const std::true_type yes{};
+  const std::false_type no{};
+  if (X.ndof == 2 && X.din) X.pin ? deferred(N2{}, yes, yes) : deferred(N2{}, yes, no);
+  else if (X.ndof == 2) X.pin ? deferred(N2{}, no, yes) : deferred(N2{}, no, no);
+  else X.pin ? deferred(N1{}, no, yes) : deferred(N1{}, no, no);
   if (X.fault_on) {
-    k_fault<R, true><<<grid_for(X.F.np, 64), 64, 0, X.stream>>>(X.F, (R*)X.d, (R*)X.v, (R*)X.a, X.fstride, c3, c4,
+    k_fault<R, true><<<grid_for(X.F.np, 64), 64, 0, X.stream>>>(X.F, (R*)X.d, (R*)X.v, (R*)X.a, X.fstride, dt, c1,
+                                                                c2, c3, c4, X.out, (R*)(X.rec ? X.rec : X.a),
                                                                 (double)it * X.F.dt);
   }
 }
@@ -1243,10 +1260,15 @@ int do_steps(sem2d_solver* h, int nsteps) {
   for (int s = 0; s < nsteps; ++s) {
     const int it = h->it + 1;
     if (h->st.on) {
+      // the steps between hand the predicted state on (StepOut); the call's last step and
+      // those with a progress row store d, v and a
+      X.out.final = !X.w32 || s == nsteps - 1 || (h->itinfo > 0 && it % h->itinfo == 0);
+      X.out.rec = !X.out.final && sampled(h, it) ? h->field : -1;
       launch_structured_step<R>(X, it, dt, c1, c2, c3, c4);
+      X.pin = !X.out.final;
       h->it = it;
-      record_receivers<R>(h);
-      record_fault(h);
+      record_receivers<R>(h, !X.out.final);
+      record_fault(h, 1);
       record_info<R>(h, it);
       continue;
     }
@@ -1294,8 +1316,8 @@ int do_steps(sem2d_solver* h, int nsteps) {
                                                              h->lsf_B, h->lsf_W1, h->lsf_W2, h->lsf_kt, h->lsf_kn,
                                                              df, a, h->npoin);
     if (h->flt.on)
-      k_fault<R><<<grid_for(h->flt.dev.np, 64), 64, 0, h->stream>>>(h->flt.dev, d, v, a, h->npoin, R(0), R(0),
-                                                                    tbc);
+        k_fault<R><<<grid_for(h->flt.dev.np, 64), 64, 0, h->stream>>>(h->flt.dev, d, v, a, h->npoin, R(0), R(0), R(0),
+                                                                    R(0), R(0), StepOut{}, (R*)nullptr, tbc);
     for (auto& D : h->dirs)
       if (D.after_fault)
         k_dirichlet<R><<<grid_for(D.node.size(), 128), 128, 0, h->stream>>>((int)D.node.size(), D.node_dev, D.comp,
@@ -1371,7 +1393,11 @@ int sem2d_create(const sem2d_desc* s, sem2d_solver** out) {
   if (rc) return rc;
   // the NGLL = 5 kernels read H from constant memory (the same values for every problem)
   if (NG == sem2d::NG)
+  {
     HIPCHK(h, hipMemcpyToSymbol(HIP_SYMBOL(c_H), Hc.data(), NP * sizeof(double), 0, hipMemcpyHostToDevice));
+    const std::vector<float> Hf(Hc.begin(), Hc.end());
+    HIPCHK(h, hipMemcpyToSymbol(HIP_SYMBOL(c_Hf), Hf.data(), NP * sizeof(float), 0, hipMemcpyHostToDevice));
+  }
   if (s->coef_mode == COEF_COMPACT) {
     double W2[sem2d::NP];
     for (int j = 0; j < NG; ++j)
@@ -1635,15 +1661,17 @@ int sem2d_set_receivers(sem2d_solver* h, int nrec, const int* iglob, int isamp, 
   if (!h) return 1;
   if (nrec <= 0 || !iglob || isamp < 1 || field < 0 || field > 2 || nsamp < 1)
     return set_err(h, 3, "set_receivers: bad arguments");
-  std::vector<int> nd(nrec);
+  std::vector<int> nd(nrec), ref(nrec);
   for (int r = 0; r < nrec; ++r) {
     if (iglob[r] < 1 || iglob[r] > h->npoin) return set_err(h, 3, "set_receivers: node out of range");
-    nd[r] = iglob[r] - 1;
+    nd[r] = ref[r] = iglob[r] - 1;
     if (h->st.on) nd[r] = h->st.gmap[nd[r]];
   }
   int rc = upload(h, &h->rec_node, nd.data(), nd.size());
   if (rc) return rc;
   h->rec_w = nullptr;
+  h->rec_ref = std::move(ref);
+  h->st.ready = false;  // the tables mark the recorded nodes
   if ((rc = dev_alloc(h, &h->seis, (size_t)nsamp * h->ndof * nrec))) return rc;
   h->nrec = nrec;
   h->isamp = isamp;
@@ -1679,8 +1707,7 @@ static int upload_elem_points(sem2d_solver* h, void** dst, const double* src) {
   return upload_bulk(h, dst, e.data(), e.size());
 }
 
-// per-element-point array in cell order for the tile kernels of a structured grid; the
-// tile kernels then run pipelined (they hold these terms in that form only)
+// per-element-point array in cell order for the tile kernel of a structured grid
 static int upload_cell_points(sem2d_solver* h, void** dst, const double* src) {
   StructState& S = h->st;
   const int NP = h->np;
@@ -1689,11 +1716,10 @@ static int upload_cell_points(sem2d_solver* h, void** dst, const double* src) {
     std::memcpy(&c[(size_t)cell * NP], src + (size_t)S.cell_elem[cell] * NP, NP * sizeof(double));
   int rc = upload_bulk(h, dst, c.data(), c.size());
   if (rc) return rc;
-  // one 512-thread workgroup per CU: the variant's LDS and registers allow no more
+  // one workgroup per CU: the variant's LDS allows no more
   int dev = 0, ncu = 256;
   if (hipGetDevice(&dev) == hipSuccess) hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   S.pipe_wgs = ((ncu + 7) / 8) * 8;
-  S.pipe_threads = 512;
   S.ready = false;
   return 0;
 }
@@ -1755,14 +1781,17 @@ int sem2d_set_receivers_interp(sem2d_solver* h, int nrec, const int* elem, const
     return set_err(h, 3, "set_receivers_interp: bad arguments");
   if (h->elem_ibool.empty()) return set_err(h, 4, "set_receivers_interp: element table not kept");
   const int NP = h->np;
-  std::vector<int> nd((size_t)nrec * NP);
+  std::vector<int> nd((size_t)nrec * NP), ref((size_t)nrec * NP);
   for (int r = 0; r < nrec; ++r) {
     if (elem[r] < 1 || elem[r] > h->nelem) return set_err(h, 3, "set_receivers_interp: element out of range");
     for (int k = 0; k < NP; ++k) {
       int g = h->elem_ibool[(size_t)(elem[r] - 1) * NP + k];
       nd[(size_t)r * NP + k] = h->st.on ? h->st.gmap[g] : g;
+      ref[(size_t)r * NP + k] = g;
     }
   }
+  h->rec_ref = std::move(ref);
+  h->st.ready = false;  // the tables mark the recorded nodes
   int rc = upload(h, &h->rec_node, nd.data(), nd.size());
   if (rc) return rc;
   if ((rc = upload(h, &h->rec_w, interp, (size_t)nrec * NP))) return rc;
@@ -2113,7 +2142,7 @@ int sem2d_set_fault_sides(sem2d_solver* h, int on) {
   }
   int rc = dev_alloc(h, &F.srec, (size_t)F.nsamp * 4 * h->ndof * F.nout);
   if (rc) return rc;
-  if (F.taken) record_sides(h, 0);  // the record of step 0, taken by sem2d_set_fault
+  if (F.taken) record_sides(h, 0, 0);  // the record of step 0, taken by sem2d_set_fault
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return 0;
 }
@@ -2293,12 +2322,8 @@ int sem2d_set_tile_config(sem2d_solver* h, int threads, int wg_per_cu) {
   StructState& S = h->st;
   int dev = 0, ncu = 256;
   if (hipGetDevice(&dev) == hipSuccess) hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-  S.pipe_threads = threads;
-  if (wg_per_cu < 0) {  // automatic: the measured defaults
-    const int pc = h->fp32 ? 3 : 2;
-    S.pipe_wgs = S.ntiles >= 4 * ncu * pc ? ncu * pc : 0;
-  }
-  else S.pipe_wgs = ncu * wg_per_cu;
+  if (wg_per_cu < 0) wg_per_cu = tile_wgs_per_cu(h->fp32, h->ndof);  // automatic: the measured defaults
+  S.pipe_wgs = ncu * wg_per_cu;
   S.pipe_wgs = ((S.pipe_wgs + 7) / 8) * 8;
   return 0;
 }
@@ -2393,6 +2418,7 @@ struct sem2d_batch {
   std::vector<int> fault_base, rec_base, fout_base, src_base;
   StepDev X;
   int ncu = 256;
+  int threads = 512;  // as set by sem2d_batch_set_config (one kernel shape serves both values)
   // records
   int nrec = 0, isamp = 1, field = 1, nsamp = 0;
   int* rec_node = nullptr;
@@ -2624,18 +2650,24 @@ int gather_fault(sem2d_batch* b) {
 template <typename R>
 void launch_batch_record(sem2d_batch* b) {
   const int nq = std::max(std::max(b->nrec, b->fnout), 1);
-  const R* fld = (const R*)(b->field == 0 ? b->X.d : (b->field == 1 ? b->X.v : b->X.a));
+  const bool marked = !b->X.out.final;  // StepOut::rec
+  const R* fld = (const R*)(marked || b->field == 2 ? b->X.a : (b->field == 0 ? b->X.d : b->X.v));
   k_batch_record<R><<<grid_for(nq, 64), 64, 0, b->stream>>>(b->it_dev, b->nrec, b->ndof, b->rec_node, fld,
                                                             b->fstride, b->isamp, b->nsamp, b->seis, b->X.F,
                                                             b->fidx, b->fnout, b->oit0, b->oitd, b->fnsamp,
                                                             b->frec);
 }
 
+// nsteps steps that read the predicted state (pin) or (d, v, a); the last one stores the
+// latter (final), the others the former (StepOut)
 template <typename R>
-void launch_batch_steps(sem2d_batch* b, int nsteps) {
+void launch_batch_steps(sem2d_batch* b, int nsteps, bool pin, bool final) {
   const StepCoefs<R> K = step_coefs<R>(b->dt, b->beta, b->gamma, b->leapfrog);
   const R dt = K.dt, c1 = K.c1, c2 = K.c2, c3 = K.c3, c4 = K.c4;
   for (int s = 0; s < nsteps; ++s) {
+    b->X.pin = b->X.w32 && (pin || s > 0);
+    b->X.out.final = !b->X.w32 || (final && s == nsteps - 1);
+    b->X.out.rec = !b->X.out.final && b->nrec ? b->field : -1;
     launch_structured_step<R>(b->X, 0, dt, c1, c2, c3, c4);
     if (b->X.fault_on)
       k_batch_potency<R><<<b->n, 256, 0, b->stream>>>(b->X.F, b->fbase_dev, (const R*)b->X.d, (const R*)b->X.v,
@@ -2657,8 +2689,8 @@ int batch_graph(sem2d_batch* b, int chunk) {
   if (b->gexec && b->gsteps == chunk) return 0;
   batch_drop_graph(b);
   BHIPCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-  if (b->fp32) launch_batch_steps<float>(b, chunk);
-  else launch_batch_steps<double>(b, chunk);
+  if (b->fp32) launch_batch_steps<float>(b, chunk, true, false);
+  else launch_batch_steps<double>(b, chunk, true, false);
   BHIPCHK(b, hipStreamEndCapture(b->stream, &b->graph));
   BHIPCHK(b, hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
   b->gsteps = chunk;
@@ -2668,28 +2700,35 @@ int batch_graph(sem2d_batch* b, int chunk) {
 // launch configuration of the tile kernel: threads per workgroup (256: 10-element
 // batches, 512: 20-element batches) and workgroups per CU (0: one workgroup per tile)
 void batch_set_config(sem2d_batch* b, int threads, int per_cu) {
-  b->X.pipe_threads = threads;
+  b->threads = threads;
   b->X.pipe_wgs = per_cu > 0 ? ((b->ncu * per_cu + 7) / 8) * 8 : 0;
   batch_drop_graph(b);
 }
 
 int batch_run(sem2d_batch* b, int nsteps, bool use_graph) {
-  const int chunk = std::min(nsteps, 64);
+  // the first and the last step apart (they read and store d, v, a), the graph's steps in
+  // between hand the predicted state on
+  const int mid = nsteps - 2, chunk = std::min(mid, 64);
   if (b->X.fault_on) {
     int rc = batch_pot_reserve(b, b->pot_shift + 1 + b->it + nsteps);
     if (rc) return rc;
   }
-  BHIPCHK(b, hipEventRecord(b->ev0, b->stream));
-  int done = 0;
   if (use_graph && chunk > 0) {
     int rc = batch_graph(b, chunk);
     if (rc) return rc;
-    for (; done + chunk <= nsteps; done += chunk) BHIPCHK(b, hipGraphLaunch(b->gexec, b->stream));
   }
-  if (done < nsteps) {
-    if (b->fp32) launch_batch_steps<float>(b, nsteps - done);
-    else launch_batch_steps<double>(b, nsteps - done);
+  BHIPCHK(b, hipEventRecord(b->ev0, b->stream));
+  auto direct = [&](int n, bool pin, bool final) {
+    if (b->fp32) launch_batch_steps<float>(b, n, pin, final);
+    else launch_batch_steps<double>(b, n, pin, final);
+  };
+  int done = 0;
+  if (use_graph && chunk > 0) {
+    direct(1, false, false);
+    for (; done + chunk <= mid; done += chunk) BHIPCHK(b, hipGraphLaunch(b->gexec, b->stream));
+    ++done;
   }
+  if (done < nsteps) direct(nsteps - done, done > 0, true);
   BHIPCHK(b, hipEventRecord(b->ev1, b->stream));
   BHIPCHK(b, hipGetLastError());
   BHIPCHK(b, hipEventSynchronize(b->ev1));
@@ -2772,6 +2811,9 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
       A.grids.push_back(make_int4((int)nb, X.grids[t].y, X.grids[t].z, cellw));
     }
     A.spec_cnt.insert(A.spec_cnt.end(), X.spec_cnt.begin(), X.spec_cnt.end());
+    for (int r : X.mark_of) A.mark_of.push_back(r < 0 ? -1 : r + (int)(A.marks.size() / MARK_WORDS));
+    A.marks.insert(A.marks.end(), X.marks.begin(), X.marks.end());
+    A.fault_rmark.insert(A.fault_rmark.end(), X.fault_rmark.begin(), X.fault_rmark.end());
     A.spec_idx.insert(A.spec_idx.end(), X.spec_idx.begin(), X.spec_idx.end());
     for (DefNode d : X.defs) {
       d.g += (int)nb;
@@ -2833,6 +2875,12 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
   if ((rc = bupload(b, &grids, A.grids))) return rc;
   if ((rc = bupload(b, &sc, A.spec_cnt))) return rc;
   if ((rc = bupload(b, &si, A.spec_idx))) return rc;
+  int* mo;
+  uint32_t* mk;
+  if ((rc = bupload(b, &mo, A.mark_of))) return rc;
+  if ((rc = bupload(b, &mk, A.marks))) return rc;
+  X.mark_of = mo;
+  X.marks = mk;
   {
     std::vector<DefDev> dn;
     std::vector<int2> dx;
@@ -2848,20 +2896,10 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
   void* rmdef;
   if ((rc = bupload_bulk(b, &rmdef, A.rmdef))) return rc;
   {
-    int nfull = 0;
-    const std::vector<int> list = tile_list(A.tiles, fits32(nb, (size_t)ntiles * SLOTS,
-                                                      b->coef_mode == COEF_SHARED
-                                                          ? shared_off
-                                                          : cb * std::max(nd, b->nelast) * NP,
-                                                      rs), nfull);
-    int* tl = nullptr;
-    if ((rc = bupload(b, &tl, list))) return rc;
-    X.tlist = tl;
-    X.nfull = nfull;
-    X.npart = ntiles - nfull;
+    X.w32 = fits32(nb, (size_t)ntiles * SLOTS,
+                   b->coef_mode == COEF_SHARED ? shared_off : cb * std::max(nd, b->nelast) * NP, rs);
   }
   X.T.ntiles = ntiles;
-  X.T.per_xcd = (ntiles + 7) / 8;
   X.T.tiles = tiles;
   X.T.grids = grids;
   X.T.spec_cnt = sc;
@@ -2933,6 +2971,12 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
     if ((rc = bupload(b, &p2, r2))) return rc;
     b->X.F.rmn1 = p1;
     b->X.F.rmn2 = p2;
+    char* side;
+    unsigned char* rmk;
+    if ((rc = balloc(b, &side, (size_t)4 * nd * b->X.F.np * rs))) return rc;
+    b->X.F.side = side;
+    if ((rc = bupload(b, &rmk, A.fault_rmark))) return rc;
+    b->X.F.rmark = rmk;
   }
   // receivers: members with stations, member after member
   std::vector<int> rn;
@@ -2955,7 +2999,7 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
   if ((rc = bupload(b, &b->rec_node, rn))) return rc;
   if ((rc = balloc(b, &b->seis, (size_t)std::max(b->nsamp, 1) * nd * std::max(b->nrec, 1)))) return rc;
   // default launch configuration (sem2d_batch_tune measures the alternatives)
-  batch_set_config(b, 256, ntiles >= 8 * b->ncu ? (b->fp32 ? 3 : 2) : 0);
+  batch_set_config(b, 512, tile_wgs_per_cu(b->fp32, b->ndof));
   // records of step 0, then the counter moves to step 1
   if (b->fp32) launch_batch_record<float>(b);
   else launch_batch_record<double>(b);
@@ -3002,7 +3046,7 @@ int sem2d_batch_tune(sem2d_batch* b, int trial_steps, int* choice) {
   for (auto& k : blks)
     if ((rc = keep(k.p, k.bytes))) break;
   const int it0 = b->it;
-  const int cand[][2] = {{256, 3}, {512, 2}, {256, 2}, {512, 1}, {256, 1}, {256, 0}};
+  const int cand[][2] = {{512, 2}, {512, 3}, {512, 4}, {512, 1}, {512, 0}};
   const int ncand = sizeof(cand) / sizeof(cand[0]);
   double best = 1e30;
   int ibest = 0;
@@ -3038,8 +3082,8 @@ int sem2d_batch_set_config(sem2d_batch* b, int threads, int wg_per_cu) {
 
 int sem2d_batch_config(sem2d_batch* b, int* threads, int* wgs, int* ntiles) {
   if (!b) return 1;
-  if (threads) *threads = b->X.pipe_wgs > 0 ? b->X.pipe_threads : TILE_THREADS;
-  if (wgs) *wgs = b->X.pipe_wgs > 0 ? b->X.pipe_wgs : 8 * b->X.T.per_xcd;
+  if (threads) *threads = b->threads;
+  if (wgs) *wgs = b->X.pipe_wgs > 0 ? b->X.pipe_wgs : (b->X.T.ntiles + 7) / 8 * 8;
   if (ntiles) *ntiles = b->X.T.ntiles;
   return 0;
 }
@@ -3466,11 +3510,13 @@ int adj_backward(sem2d_solver* h, const double* gseis_host) {
   return 0;
 }
 
-// Forward sweep of the history mode.  Step n reads the displacement of history slot n-1
-// and writes it into slot n (out of place, with v, and a unless it has a history, in
-// place), so the history needs no copies; for FP32 fields the acceleration goes through
-// its own history the same way.  The receivers read the current slots; the solver's own
-// arrays receive the final state, and the acceleration after the last step is kept.
+// Forward sweep of the history mode.  With beta = 0 the displacement after a step is the
+// predicted one it started from, and the one the step hands on (StepOut) is that of the
+// next: step n reads history slot n and writes slot n+1 (out of place, with the predicted
+// velocity in place), so the history needs no copies; for FP32 fields the acceleration is
+// stored into its own history.  The recorded nodes go through the solver's a array; the
+// solver's own arrays receive the final state, and the acceleration after the last step
+// is kept.
 template <typename R>
 int adj_forward_hist(sem2d_solver* h) {
   AdjState& A = *h->adj;
@@ -3483,25 +3529,34 @@ int adj_forward_hist(sem2d_solver* h) {
   void *d0 = h->d, *a0 = h->a;
   auto Hn = [&](int n) { return (void*)(A.H + (size_t)n * nfb); };
   auto AHn = [&](int n) { return (void*)(A.AH + (size_t)n * nfb); };
-  HIPCHK(h, hipMemsetAsync(A.H, 0, nfb, h->stream));
+  // d_0 and, from the zero initial state, the first predicted displacement
+  HIPCHK(h, hipMemsetAsync(A.H, 0, 2 * nfb, h->stream));
   if (A.AH) HIPCHK(h, hipMemsetAsync(A.AH, 0, nfb, h->stream));
   HIPCHK(h, hipEventRecord(h->ev0, h->stream));
+  X.pin = X.w32;
+  X.out.accel = A.AH != nullptr;
   for (int n = 1; n <= A.nsteps; ++n) {
-    X.din = Hn(n - 1);
+    const bool last = n == A.nsteps;
+    X.din = Hn(X.pin ? n : n - 1);
     X.vin = nullptr;  // in place
     X.ain = A.AH ? AHn(n - 1) : nullptr;
-    X.d = Hn(n);
+    X.d = !X.pin ? Hn(n) : (last ? d0 : Hn(n + 1));
     X.a = A.AH ? AHn(n) : a0;
+    X.out.final = last || !X.pin;
+    X.rec = a0;
+    X.out.rec = !X.out.final && sampled(h, n) ? h->field : -1;
     launch_structured_step<R>(X, n, dt, c1, c2, c3, c4);
     h->it = n;
-    h->d = X.d;
-    h->a = X.a;
-    rc = record_receivers<R>(h);
+    if (X.out.final) {
+      h->d = X.d;
+      h->a = X.a;
+    }
+    rc = record_receivers<R>(h, !X.out.final);
     h->d = d0;
     h->a = a0;
     if (rc) return rc;
   }
-  HIPCHK(h, hipMemcpyAsync(d0, Hn(A.nsteps), nfb, hipMemcpyDeviceToDevice, h->stream));
+  if (!X.pin) HIPCHK(h, hipMemcpyAsync(d0, Hn(A.nsteps), nfb, hipMemcpyDeviceToDevice, h->stream));
   if (A.AH) HIPCHK(h, hipMemcpyAsync(a0, AHn(A.nsteps), nfb, hipMemcpyDeviceToDevice, h->stream));
   if (A.aN) HIPCHK(h, hipMemcpyAsync(A.aN, a0, nfb, hipMemcpyDeviceToDevice, h->stream));
   HIPCHK(h, hipEventRecord(h->ev1, h->stream));

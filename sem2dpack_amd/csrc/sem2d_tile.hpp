@@ -6,10 +6,9 @@
 // single pass over HBM, does for the tile's patch of (4*nxe+1) x (4*nze+1) nodes:
 //
 //   1. load d, v, a; Newmark predictor (SRC/solver.f90:59-60); predicted d in LDS;
-//   2. element forces f = -K d (ELAST_KD2_*, SRC/mat_elastic.f90:589-641,739-775)
-//      assembled into an LDS node array, colour by colour (2x2 checkerboard of the
-//      tile's elements: elements of one colour share no node, so the LDS updates
-//      need no atomics and the summation order is fixed);
+//   2. element forces f = -K d (ELAST_KD2_*, SRC/mat_elastic.f90:589-641,739-775),
+//      summed per node in the order of the 2x2 checkerboard colours of the tile's
+//      elements (no atomics, the summation order is fixed);
 //   3. interior patch nodes: a = f*rmass, corrector (SRC/solver.f90:78-82), store;
 //      patch-perimeter nodes and "special" nodes (point sources): store the
 //      partial force of this tile to fpart and leave the node untouched.
@@ -31,7 +30,7 @@ namespace sem2d {
 constexpr int TX = 8, TZ = 8;
 constexpr int PXM = 4 * TX + 1, PZM = 4 * TZ + 1;
 constexpr int PMAX = PXM * PZM;
-constexpr int TILE_THREADS = 256;
+constexpr int TILE_THREADS = 256;  // adjoint tile kernel
 constexpr int NODE_ITERS = (PMAX + TILE_THREADS - 1) / TILE_THREADS;
 constexpr int PERIM_MAX = 2 * PXM + 2 * (PZM - 2);
 constexpr int MAXSPECIAL = 16;
@@ -39,11 +38,10 @@ constexpr int SLOTS = PERIM_MAX + MAXSPECIAL;
 
 struct TileDev {
   int ntiles;
-  int per_xcd;        // tiles per XCD slice of the launch
   const int4* tiles;  // (tx0, tz0, nxe | nze << 8 | nx << 16, Z0), nx = elements per grid row
   const int4* grids;  // per tile: (node_base, ROW, NZ1, cell_base) of the grid the tile lies in
   const int* spec_cnt;
-  const int* spec_idx;  // [ntiles][MAXSPECIAL] local patch indices
+  const int* spec_idx;  // [ntiles][MAXSPECIAL] patch indices Z*PXM + X
   size_t NGp;           // component stride of the field arrays
   size_t FPS;           // component stride of fpart (ntiles*SLOTS)
 };
@@ -85,158 +83,6 @@ __device__ __forceinline__ int perim_slot(int X, int Z, int PX, int PZ) {
   s = Z == PZ - 1 ? PX + X : s;
   s = Z == 0 ? X : s;
   return s;
-}
-
-template <typename R, int NDOF, int NELAST, int MODE, bool OOP = false>
-__global__ __launch_bounds__(TILE_THREADS) void k_tile(TileDev T, R* __restrict__ d, R* __restrict__ v,
-                                                       R* __restrict__ a, const R* __restrict__ rmass0,
-                                                       const R* __restrict__ coefs, const R* __restrict__ geom,
-                                                       R* __restrict__ fpart, R dt, R c1, R c2, R c3, R c4,
-                                                       const R* __restrict__ din = nullptr,
-                                                       const R* __restrict__ vin = nullptr,
-                                                       const R* __restrict__ ain = nullptr) {
-  // out of place: a null vin / ain reads v / a (their step is then in place)
-  const R* __restrict__ dsrc = OOP ? din : d;
-  const R* vsrc = OOP && vin ? vin : v;
-  const R* asrc = OOP && ain ? ain : a;
-  __shared__ R Ud[NDOF][PMAX];
-  __shared__ R Fn[NDOF][PMAX];
-  __shared__ R T1[FE_EPB][NDOF][NP];
-  __shared__ R T2[FE_EPB][NDOF][NP];
-  __shared__ short sflag[PMAX];
-
-  // XCD-aware order: the 8 XCDs receive workgroups round-robin, so give each XCD a
-  // contiguous range of tiles (neighbouring tiles share patch rows in its L2).
-  const int bid = blockIdx.x;
-  const int t = (bid & 7) * T.per_xcd + (bid >> 3);
-  if (t >= T.ntiles) return;
-  const int tid = threadIdx.x;
-  const int4 tg = T.tiles[t];
-  const int4 gr = T.grids[t];
-  const int tx0 = tg.x, tz0 = tg.y, nxe = tg.z & 0xff, nze = (tg.z >> 8) & 0xff, Z0 = tg.w;
-  const int PX = 4 * nxe + 1, PZ = 4 * nze + 1, NPT = PX * PZ;
-  const int X0 = 4 * tx0;
-  const size_t S = T.NGp;
-  const int kL = tx0 / TX, kR = (tx0 + nxe + TX - 1) / TX;
-
-  R vp[NODE_ITERS][NDOF];
-#pragma unroll
-  for (int r = 0; r < NODE_ITERS; ++r) {
-    const int p = tid + TILE_THREADS * r;
-    if (p < NPT) {
-      const int Z = p / PX, X = p - Z * PX;
-      const size_t g = node_index(gr, X, Z, PX, X0, Z0, kL, kR);
-#pragma unroll
-      for (int c = 0; c < NDOF; ++c) {
-        const R dk = dsrc[c * S + g], vk = vsrc[c * S + g], ak = asrc[c * S + g];
-        Ud[c][p] = dk + dt * vk + c1 * ak;
-        vp[r][c] = vk + c2 * ak;
-        Fn[c][p] = 0;
-      }
-      sflag[p] = -1;
-    }
-  }
-  __syncthreads();
-  const int nspec = T.spec_cnt[t];
-  if (tid < nspec) sflag[T.spec_idx[t * MAXSPECIAL + tid]] = (short)tid;
-
-  // element forces, colour by colour
-  const int le = tid / NP;
-  const int pe = tid - le * NP;
-  const int ii = pe % NG, jj = pe / NG;
-#pragma unroll 1
-  for (int cc = 0; cc < 4; ++cc) {
-    const int cx = cc & 1, cz = cc >> 1;
-    const int ncx = (nxe - cx + 1) >> 1, ncz = (nze - cz + 1) >> 1;
-    const int nce = ncx * ncz;
-#pragma unroll 1
-    for (int b0 = 0; b0 < nce; b0 += FE_EPB) {
-      const int ce = b0 + le;
-      const bool active = (tid < FE_THREADS) && (ce < nce);
-      int base = 0;
-      if (active) {
-        const int lx = cx + 2 * (ce % ncx), lz = cz + 2 * (ce / ncx);
-        base = 4 * lz * PX + 4 * lx;
-        const size_t cell = cell_index(gr, tg.z >> 16, tx0, tz0, lx, lz);
-        R A[NELAST];
-        load_coefs<R, NDOF, NELAST, MODE>(grid_coefs<R, MODE>(coefs, gr), geom, cell, pe, A);
-        R dxi[NDOF], deta[NDOF];
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) {
-          R s1 = 0, s2 = 0;
-#pragma unroll
-          for (int k = 0; k < NG; ++k) {
-            s1 += Coef<R>::h(k, ii) * Ud[c][base + jj * PX + k];
-            s2 += Ud[c][base + k * PX + ii] * Coef<R>::h(k, jj);
-          }
-          dxi[c] = s1;
-          deta[c] = s2;
-        }
-        if constexpr (NDOF == 2) {
-          if constexpr (NELAST == 6) {
-            T1[le][0][pe] = A[0] * dxi[0] + A[1] * deta[1];
-            T2[le][0][pe] = A[3] * (deta[0] + dxi[1]);
-            T1[le][1][pe] = A[4] * deta[0] + A[5] * dxi[1];
-            T2[le][1][pe] = A[1] * dxi[0] + A[2] * deta[1];
-          } else {
-            T1[le][0][pe] = A[0] * dxi[0] + A[6] * deta[0] + A[7] * dxi[1] + A[1] * deta[1];
-            T2[le][0][pe] = A[6] * dxi[0] + A[3] * deta[0] + A[4] * dxi[1] + A[8] * deta[1];
-            T1[le][1][pe] = A[7] * dxi[0] + A[4] * deta[0] + A[5] * dxi[1] + A[9] * deta[1];
-            T2[le][1][pe] = A[1] * dxi[0] + A[8] * deta[0] + A[9] * dxi[1] + A[2] * deta[1];
-          }
-        } else {
-          if constexpr (NELAST == 2) {
-            T1[le][0][pe] = A[0] * dxi[0];
-            T2[le][0][pe] = A[1] * deta[0];
-          } else {
-            T1[le][0][pe] = A[0] * dxi[0] + A[2] * deta[0];
-            T2[le][0][pe] = A[2] * dxi[0] + A[1] * deta[0];
-          }
-        }
-      }
-      __syncthreads();
-      if (active) {
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) {
-          R s1 = 0, s2 = 0;
-#pragma unroll
-          for (int k = 0; k < NG; ++k) {
-            s1 += Coef<R>::h(ii, k) * T1[le][c][jj * NG + k];
-            s2 += T2[le][c][k * NG + ii] * Coef<R>::h(jj, k);
-          }
-          R* fp = &Fn[c][base + jj * PX + ii];
-          *fp = *fp + (s1 + s2);
-        }
-      }
-      __syncthreads();
-    }
-  }
-
-  // finish interior nodes, hand perimeter / special nodes over
-  const size_t fbase = (size_t)t * SLOTS;
-#pragma unroll
-  for (int r = 0; r < NODE_ITERS; ++r) {
-    const int p = tid + TILE_THREADS * r;
-    if (p < NPT) {
-      const int Z = p / PX, X = p - Z * PX;
-      int slot = perim_slot(X, Z, PX, PZ);
-      if (slot < 0 && sflag[p] >= 0) slot = PERIM_MAX + sflag[p];
-      if (slot >= 0) {
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) fpart[c * T.FPS + fbase + slot] = Fn[c][p];
-      } else {
-        const size_t g = node_index(gr, X, Z, PX, X0, Z0, kL, kR);
-        const R rm = rmass0[g];
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) {
-          const R ak = Fn[c][p] * rm;
-          a[c * S + g] = ak;
-          v[c * S + g] = vp[r][c] + c3 * ak;
-          d[c * S + g] = Ud[c][p] + c4 * ak;
-        }
-      }
-    }
-  }
 }
 
 // LDS node value of NDOF components stored together (one vector access for P-SV)
@@ -288,95 +134,143 @@ __device__ __forceinline__ uint32_t node_index_full(const int4 gr, int X, int Z,
   return (X == 0 || X == 4 * TX) ? edge : inner;
 }
 
-// Persistent, software-pipelined variant of k_tile.  Each workgroup walks a strided
-// sequence of tiles inside its XCD's share (see below).  No tile waits on a
-// global load issued during that tile: everything a tile reads comes from registers
-// filled while the previous tile was being processed.
-// Vector memory operations retire in issue order (loads and stores share one
-// counter), so a wait for a load also waits for every store issued before it, and the
-// compiler counts the stores issued after a load as the minimum over the branches.
-// Per tile, therefore:
-//   1. the predictor takes every wait, on loads issued a whole element phase earlier;
-//   2. the previous tile's results are stored from LDS (each thread stores the patch
-//      slots it overwrites next, so no barrier separates 2 and 3);
-//   3. the predicted values go to LDS;
-//   4. all loads of the next tile are issued in one group (d, v, a, inverse mass,
-//      moduli or point coefficients, geometric factors, special-node index);
-//   5. the element phase runs while they and the stores of 2 complete.
-// Tile descriptors are scalar loads, counted apart from vector memory.
-// Results are identical to k_tile: same predictor, same colour order and same
-// summation order.  NT threads per workgroup, EPB elements per element batch
-// (EPB*25 <= NT).  The launch covers the tiles tlist[0 .. nlist).  ttiles, tgrids and
-// tspc are T.tiles, T.grids and T.spec_cnt, passed as restricted arguments so that the
-// compiler may read them through the scalar cache.
+// Order of LDS accesses among the lanes of one wavefront (which the hardware executes in
+// program order): no access moves across it.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Persistent tile kernel.  Each workgroup walks a strided sequence of tiles inside its
+// XCD's share (see below); the state a tile reads is loaded into registers while the
+// previous tile is processed.
 //
-// FULL: every listed tile has TX x TZ elements, so patch and colour shapes are
-// compile-time constants (no run-time divisions in the index arithmetic), and the
-// field, inverse-mass, partial-force and per-cell arrays are addressed with 32-bit
-// offsets from per-component bases (the caller guarantees that every component of
-// these arrays is below 4 GiB).
+// Element phase: a lane per element row or column, 12 elements (60 lanes) per wavefront,
+// 6 wavefronts for the 64 elements of a tile.  Five points per lane make the entries of H
+// compile-time indices (scalar operands), and the two directions of an element are
+// exchanged through LDS between lanes of the same wavefront, without a barrier:
+//   A  column i:  deta(i, .) from the column's nodes, to the exchange array
+//   B  row j:     dxi(., j) from the row's nodes, stresses of the row's points, the row
+//                 part of the forces (kept in registers), the column fluxes to the array
+//   C  column i:  the column part of the forces
+//   D  row j:     both parts added: the element's forces
+//   E  (barrier)  every node adds the forces of its 1, 2 or 4 elements, in the order of
+//                 the 2x2 checkerboard of colours
+// An element costs 300 LDS accesses of a node value where a lane per point took 650
+// (10 + 2 + 10 + 4 per point), and a tile two barriers instead of five.
+//
+// Bound by HBM latency and bandwidth: P-SV with moduli per node, 1000 x 500 elements, moves
+// 0.70 GB (FP64) per step in 182 us and half of it (FP32) in 117 us with the deferred nodes'
+// kernel (3.9 and 3.0 TB/s; a large copy reaches 5.0); with a lane per point and (d, v, a)
+// handed on it was 283 and 140 us.  Two workgroups per CU overlap one's loads with the
+// other's phases; they fit only while a wavefront needs 128 registers at most, and a
+// spilled register costs more than it saves (the spill of a prefetched value waits for it):
+// FP64 with 34 registers spilled took 290 us.
+//
+// Per tile:
+//   1. the predicted displacement goes to LDS (the state read is the predicted one, PIN:
+//      nothing to compute), from loads issued an element phase earlier;
+//   2. the loads of this tile's predicted velocity (needed by its stores only), then of the
+//      next tile's displacement and moduli are issued;
+//   3. phases A and B; the inverse mass is loaded, which only the stores need; phases C, D
+//      and E;
+//   4. the tile's stores, which complete during the next tile's phases.
+// Vector memory operations retire in issue order, loads and stores in one counter, so
+// that a wait for a load also waits for what was issued before it: the order above has
+// each wait behind the longest stretch of work.
+// Tile descriptors are scalar loads, counted apart from vector memory.  The patch is laid
+// out with the row length of a full tile whatever the tile's size, so that the index
+// arithmetic has constant divisors; a smaller tile leaves slots and lanes idle.
+//
+// W32: the field, inverse-mass, partial-force and per-cell arrays are below 4 GiB per
+// component and are addressed with 32-bit offsets from per-component bases.
 //
 // EP: element-point terms, per element point in cell order [cell][25] (either may be
 // null): Kelvin-Voigt viscosity eta, the element displacement being d + eta v at each
 // point (MAT_KV_add_etav, SRC/mat_kelvin_voigt.f90:139-150), and the 2.5D coefficient
 // b25, the point force then losing b25 (d + eta v) (MAT_ELAST_add_25D_f,
 // SRC/mat_elastic.f90:447-459).  The predicted velocity then passes through LDS.
-template <typename R, int NDOF, int NELAST, int MODE, int NT, int EPB, bool OOP = false, bool FULL = false,
-          bool EP = false>
-// Register budget: FP32 fields at 512 threads run two workgroups per CU (4 waves per
-// SIMD, 128 VGPRs); every other shape (and the element-point variant, whose LDS allows
-// one workgroup per CU) runs at most 2 waves per SIMD of 512-thread workgroups or 3 of
-// 256-thread ones, so the kernel may use the registers of 2.
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 512 && sizeof(R) == 4 && !EP ? 4 : 2))) void k_tile_pipe(TileDev T, const int* __restrict__ tlist, int nlist,
-                                                            const int4* __restrict__ ttiles,
-                                                            const int4* __restrict__ tgrids,
-                                                            const int* __restrict__ tspc, R* __restrict__ d,
-                                                            R* __restrict__ v, R* __restrict__ a,
-                                                            const R* __restrict__ rmass0,
-                                                            const R* __restrict__ coefs, const R* __restrict__ geom,
-                                                            R* __restrict__ fpart, R dt, R c1, R c2, R c3, R c4,
-                                                            const R* __restrict__ din = nullptr,
-                                                            const R* __restrict__ vin = nullptr,
-                                                            const R* __restrict__ ain = nullptr,
-                                                            const R* __restrict__ eta = nullptr,
-                                                            const R* __restrict__ b25 = nullptr) {
-  // OOP: the step reads the state (din, vin, ain) and writes (d, v, a); otherwise in place
-  // out of place: a null vin / ain reads v / a (their step is then in place)
-  const R* __restrict__ dsrc = OOP ? din : d;
-  const R* vsrc = OOP && vin ? vin : v;
-  const R* asrc = OOP && ain ? ain : a;
+constexpr int TS_NT = 384;                  // threads per workgroup
+constexpr int TS_EPW = 12;                  // elements per wavefront (5 lanes each)
+constexpr int TS_ITER = (PMAX + TS_NT - 1) / TS_NT;  // patch nodes per thread
+static_assert(TS_EPW * (TS_NT / 64) >= TX * TZ, "not enough wavefronts for a tile's elements");
+static_assert(3 * TX * TZ <= TS_NT, "per-tile tables larger than the workgroup");
+
+constexpr int MARK_WORDS = (PMAX + 31) / 32;
+
+// Arguments of k_tile_step.  The kernel reads them from the argument segment where it uses
+// them (kernel_args): kept in scalar registers throughout, next to the 25 entries of H,
+// they would not fit, and the compiler spills scalars to vector registers.
+template <typename R>
+struct TileArgs {
+  R *d, *v, *a;
+  const R *din, *vin, *ain;  // state read by an out-of-place step; null vin / ain: v / a
+  const R *rmass0, *coefs, *geom, *eta, *b25;
+  R *fpart, *rec;  // rec: where recorded nodes go (StepOut::rec)
+  size_t S, FPS;  // component strides of the field arrays and of fpart
+  const int4 *tiles, *grids;
+  const int *spec_cnt, *spec_idx;
+  // recorded nodes inside tiles: per tile its row of marks (or -1), MARK_WORDS words each
+  const int* mark_of;
+  const uint32_t* marks;
+  int ntiles;
+  R dt, c1, c2, c3, c4;
+  StepOut out;
+};
+// entry i (uniform) of an array that no kernel writes: a scalar load
+__device__ __forceinline__ int sload(const int* p, int i) {
+  return ((const __attribute__((address_space(4))) int*)p)[i];
+}
+__device__ __forceinline__ int4 sload(const int4* p, int i) {
+  typedef int I4 __attribute__((ext_vector_type(4)));
+  const I4 x = ((const __attribute__((address_space(4))) I4*)p)[i];
+  return make_int4(x.x, x.y, x.z, x.w);
+}
+// the argument struct of a kernel whose only parameter it is, by a pointer the compiler
+// cannot look through (so that loads from it are not merged across uses)
+template <typename A>
+__device__ __forceinline__ const __attribute__((address_space(4))) A* kernel_args() {
+  auto p = (const __attribute__((address_space(4))) A*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// Launched with TS_NT threads.  The bound of 512 makes the compiler count two workgroups of
+// eight wavefronts per CU, that is 128 registers; two of six would seem to admit 168, but
+// the dispatcher may place four wavefronts of two workgroups on one SIMD.
+template <typename R, int NDOF, int NELAST, int MODE, bool OOP = false, bool W32 = true, bool EP = false,
+          bool PIN = false>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(EP || (!PIN && NDOF == 2 && sizeof(R) == 8) ? 2 : 4))) void
+k_tile_step(TileArgs<R> args) {
+  constexpr int PS = PXM;        // patch row length
+  constexpr int NEL = TX * TZ;   // element slots
+  constexpr bool NODEM = MODE == COEF_NODE;
+  constexpr bool COMP = MODE == COEF_COMPACT;
+  // FULLPF: the registers admit the prefetch of everything a tile reads but per-element
+  // moduli, and of a tile's forces until the next tile's loads have arrived.  Otherwise
+  // (FP64 P-SV) the predicted velocity and the inverse mass, which only the stores need,
+  // are loaded late (LATEV), and the stores follow the forces.
+  constexpr bool FULLPF = (sizeof(R) == 4 || NDOF == 1) && !EP;
+  constexpr bool LATEV = PIN && !EP && !FULLPF;
   // node values with both components side by side: one LDS access moves both
   using LV = typename LVec<R, NDOF>::T;
-  __shared__ LV Ud[PMAX];
-  __shared__ LV Fn[PMAX];
-  constexpr int NITER = (PMAX + NT - 1) / NT;                       // patch nodes per thread
-  constexpr int NBATCH = (TX * TZ / 4 + EPB - 1) / EPB;              // batches per colour
-  constexpr int PB_MAXB = 4 * NBATCH;                               // point tasks per thread
-  constexpr int ETHREADS = EPB * NP;
-  static_assert(ETHREADS <= NT, "element batch larger than the workgroup");
-  static_assert(3 * TX * TZ <= NT && MAXSPECIAL <= NT, "per-tile tables larger than the workgroup");
-  __shared__ LV Vp[PMAX];  // predicted velocity
-  __shared__ R Rm[PMAX];        // inverse mass of the patch nodes
-  __shared__ LV T1b[2][EPB][NP];  // double-buffered element stresses
-  __shared__ LV T2b[2][EPB][NP];
-  __shared__ short sflag[PMAX];
-  // H, GLL weight products and per-element geometric factors live in LDS (no global
-  // load inside the element phase).
-  __shared__ double sH[NP];
-  __shared__ double sW2[NP];
-  __shared__ R Gm[TX * TZ][3];
-  // moduli of each thread's point tasks (compact mode), staged from the prefetch
-  // registers by the predictor
-  __shared__ LV ML[MODE == COEF_COMPACT ? PB_MAXB : 1][MODE == COEF_COMPACT ? ETHREADS : 1];
-  // COEF_NODE: the moduli of the patch nodes (coefs is then a per-node array in the
-  // field layout, component stride T.NGp), loaded with the node values
-  constexpr bool NODEM = MODE == COEF_NODE;
-  __shared__ LV Mn[NODEM ? PMAX : 1];
-  // EP: eta and b25 of the tile's element points, [local element lz*nxe+lx][point]
-  constexpr int NEPT = EP ? TX * TZ * NP : 1;
+  __shared__ LV Ud[PMAX];               // predicted displacement
+  // exchange array: deta, column fluxes, forces; the last slot stays zero
+  __shared__ LV Ex[NEL * NP + 1];
+  // per patch node the exchange slots of its elements' forces, in the order of the
+  // colours; the zero slot stands for an element outside the patch
+  __shared__ ushort4 Eg[PMAX];
+  __shared__ LV Vp[EP ? PMAX : 1];      // predicted velocity
+  __shared__ LV Mn[NODEM ? PMAX : 1];   // moduli of the patch nodes
+  __shared__ R Sa[MODE == COEF_SHARED ? NELAST * NP : 1];  // the grid's point coefficients
+  __shared__ R Gm[NEL][3];              // geometric factors of the elements
+  __shared__ R sW2[NP];
+  constexpr int NEPT = EP ? NEL * NP : 1;  // eta and b25 of the tile's element points
   __shared__ R Eta[NEPT];
   __shared__ R Bet[NEPT];
 
+  const int nlist = args.ntiles;
   const int nwg = gridDim.x;
   const int bid = blockIdx.x;
   // Workgroups reach the 8 XCDs round-robin (XCD = bid & 7).  XCD x owns the x-th
@@ -391,345 +285,385 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 512 &&
   const int q0 = s0 + (bid >> 3);
   if (q0 >= s1) return;
   const int tid = threadIdx.x;
-  // lane index of the node loops, re-materialised per full tile (below) so that their
-  // per-lane index arithmetic is recomputed rather than held in registers across tiles
-  int tnode = tid;
-  const size_t S = T.NGp;
-  const int le = tid / NP;
-  const int pe = tid - le * NP;
-  const int ii = pe % NG, jj = pe / NG;
-  if (tid < NP) {
-    sH[tid] = c_H[tid];
-    sW2[tid] = c_W2[tid];
-  }
-  // this lane's element point (ii, jj) is the same for every tile: keep the H entries
-  // its contractions use in registers
-  const R w2 = (R)c_W2[pe];
-  R hA[NG], hB[NG], hC[NG], hD[NG];
+  if (tid < NP) sW2[tid] = (R)c_W2[tid];
+  if (tid == 0) Ex[NEL * NP] = LV{};
+  // this thread's patch nodes (X, Z), packed
+  int xz[TS_ITER];
 #pragma unroll
-  for (int k = 0; k < NG; ++k) {
-    hA[k] = (R)c_H[k * NG + ii];
-    hB[k] = (R)c_H[k * NG + jj];
-    hC[k] = (R)c_H[ii * NG + k];
-    hD[k] = (R)c_H[jj * NG + k];
+  for (int r = 0; r < TS_ITER; ++r) {
+    const int p = tid + TS_NT * r, Z = p / PS, X = p - Z * PS;
+    xz[r] = X | Z << 8;
+    // Of the two element columns (rows) that share a node the even one comes first,
+    // rows before columns: the order of the colours.
+    unsigned short sl[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int cx = q & 1, cz = q >> 1;
+      const int lx = ((X >> 2) & 1) == cx ? X >> 2 : (X >> 2) - 1;
+      const int lz = ((Z >> 2) & 1) == cz ? Z >> 2 : (Z >> 2) - 1;
+      const bool ok = lx >= 0 && lx < TX && (lx == X >> 2 || (X & 3) == 0) && lz >= 0 && lz < TZ &&
+                      (lz == Z >> 2 || (Z & 3) == 0);
+      sl[q] = (unsigned short)(ok ? (lz * TX + lx) * NP + (Z - 4 * lz) * NG + (X - 4 * lx) : NEL * NP);
+    }
+    if (p < PMAX) Eg[p] = make_ushort4(sl[0], sl[1], sl[2], sl[3]);
   }
-  // tile geometry: compile-time constants for full tiles
   struct Geo {
-    int tx0, tz0, nxe, nze, Z0, PX, PZ, NPT, X0, kL, kR;
+    int tx0, tz0, nxe, nze, Z0, PX, PZ, X0, kL, kR;
   };
   auto geo = [&](const int4 tg) {
     Geo g;
     g.tx0 = tg.x;
     g.tz0 = tg.y;
-    g.nxe = FULL ? TX : (tg.z & 0xff);
-    g.nze = FULL ? TZ : ((tg.z >> 8) & 0xff);
+    g.nxe = tg.z & 0xff;
+    g.nze = (tg.z >> 8) & 0xff;
     g.Z0 = tg.w;
     g.PX = 4 * g.nxe + 1;
     g.PZ = 4 * g.nze + 1;
-    g.NPT = g.PX * g.PZ;
     g.X0 = 4 * g.tx0;
     g.kL = g.tx0 / TX;
-    g.kR = FULL ? g.kL + 1 : (g.tx0 + g.nxe + TX - 1) / TX;
+    g.kR = (g.tx0 + g.nxe + TX - 1) / TX;
     return g;
   };
-  // storage index of patch node (X, Z) and field access (32-bit offsets for full tiles)
+  // storage index of patch node (X, Z), as node_index: a tile-edge column or a row segment
   auto nidx = [&](const int4 gr, const Geo& G, int X, int Z) {
-    if constexpr (FULL) return node_index_full(gr, X, Z, G.X0, G.Z0, G.kL);
-    else return node_index(gr, X, Z, G.PX, G.X0, G.Z0, G.kL, G.kR);
+    using I = std::conditional_t<W32, uint32_t, size_t>;
+    const I row = (I)gr.x + (I)G.Z0 * (I)gr.y + (I)(G.X0 - 1);            // uniform
+    const I edge = (I)gr.x + (I)gr.y * (I)gr.z + (I)G.Z0;                 // uniform
+    const I eL = edge + (I)G.kL * (I)gr.z, eR = edge + (I)G.kR * (I)gr.z;  // uniform
+    const I in = row + (I)((uint32_t)Z * (uint32_t)gr.y + (uint32_t)X);
+    const I ed = (X == 0 ? eL : eR) + (I)Z;
+    return X == 0 || X == G.PX - 1 ? ed : in;
   };
   auto fld = [&](auto* cbase, auto g) -> auto& {
-    if constexpr (FULL) return at32(cbase, (uint32_t)g);
+    if constexpr (W32) return at32(cbase, (uint32_t)g);
     else return cbase[g];
   };
   auto ubase = [&](auto* p) {
-    if constexpr (FULL) return sgpr_base(p);
+    if constexpr (W32) return sgpr_base(p);
     else return p;
   };
-  // per-component array bases, formed once
-  const R *bD[NDOF], *bV[NDOF], *bA[NDOF];
-  R *oD[NDOF], *oV[NDOF], *oA[NDOF], *bF[NDOF];
-#pragma unroll
-  for (int c = 0; c < NDOF; ++c) {
-    bD[c] = ubase(dsrc + c * S);
-    bV[c] = ubase(vsrc + c * S);
-    bA[c] = ubase(asrc + c * S);
-    if constexpr (OOP) {
-      oD[c] = ubase(d + c * S);
-      oV[c] = ubase(v + c * S);
-      oA[c] = ubase(a + c * S);
-    } else {
-      oD[c] = const_cast<R*>(bD[c]);
-      oV[c] = const_cast<R*>(bV[c]);
-      oA[c] = const_cast<R*>(bA[c]);
-    }
-    bF[c] = ubase(fpart + c * T.FPS);
-  }
-  const R* bRm = ubase(rmass0);
-  const R* bCo = ubase(coefs);
-  const R* bMo[NDOF];
-#pragma unroll
-  for (int c = 0; c < NDOF; ++c) bMo[c] = NODEM ? ubase(coefs + c * S) : bCo;
-  const R* bGe = ubase(geom);
-  const R* bEt = EP && eta ? ubase(eta) : nullptr;
-  const R* bBe = EP && b25 ? ubase(b25) : nullptr;
-  // cell index in the element arrays (32 bits for full tiles)
   auto cidx = [&](const int4 gr, int nx, const Geo& G, int lx, int lz) {
-    if constexpr (FULL) return (uint32_t)gr.w + (uint32_t)(G.tz0 + lz) * (uint32_t)nx + (uint32_t)(G.tx0 + lx);
+    if constexpr (W32) return (uint32_t)gr.w + (uint32_t)(G.tz0 + lz) * (uint32_t)nx + (uint32_t)(G.tx0 + lx);
     else return cell_index(gr, nx, G.tx0, G.tz0, lx, lz);
   };
 
-  // Registers of the next tile, all issued in one group at the start of the current
-  // tile's element phase: node values, inverse mass of the patch nodes, the moduli of
-  // this thread's point tasks (compact mode) or its point coefficients (shared mode: the
-  // same for every element of the tile's grid), one geometric factor and one
-  // special-node index.
-  R pd[NITER][NDOF], pv[NITER][NDOF], pa[NITER][NDOF];
-  R pm[NITER];
-  R pmod[NODEM ? NITER : 1][NDOF] = {};
-  R lm[PB_MAXB][NDOF] = {};
-  R sa[NELAST] = {}, sac[NELAST] = {};
-  R pg = 0;
-  int psp = -1;
-  constexpr int NEP = EP ? (TX * TZ * NP + NT - 1) / NT : 1;  // element points per thread
+  // lane index the compiler cannot look through: index arithmetic derived from it is
+  // recomputed where it is used rather than held in registers across tiles
+  auto lane_id = [&]() {
+    int q = tid;
+    asm volatile("" : "+v"(q));
+    __builtin_assume(q >= 0 && q < TS_NT);
+    return q;
+  };
+
+  // registers of the next tile, issued in one group at the start of the current tile's
+  // element phase.  Slots outside the patch load its nearest node: with loads under a
+  // condition the registers' old values would have to be kept for the other lanes.
+  constexpr int NEP = EP ? (NEL * NP + TS_NT - 1) / TS_NT : 1;
+  R pd[TS_ITER][NDOF] = {}, pv[LATEV ? 1 : TS_ITER][NDOF] = {}, pa[PIN ? 1 : TS_ITER][NDOF] = {};
+  R pmod[NODEM ? TS_ITER : 1][NDOF] = {}, pm[FULLPF ? TS_ITER : 1] = {};
   R peta[NEP] = {}, pbet[NEP] = {};
+  R psa = 0, pg = 0;
   auto issue = [&](int t) {
-    const int4 tg = ttiles[t];
-    const int4 gr = tgrids[t];
+    const auto* P = kernel_args<TileArgs<R>>();
+    const int4 tg = sload(P->tiles, t);
+    const int4 gr = sload(P->grids, t);
     const Geo G = geo(tg);
+    const R *bD[NDOF], *bV[NDOF], *bA[NDOF], *bMo[NDOF];
 #pragma unroll
-    for (int r = 0; r < NITER; ++r) {
-      const int p = tnode + NT * r;
-      if (p < G.NPT) {
-        const int Z = p / G.PX, X = p - Z * G.PX;
-        const auto g = nidx(gr, G, X, Z);
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) {
-          pd[r][c] = fld(bD[c], g);
-          pv[r][c] = fld(bV[c], g);
-          pa[r][c] = fld(bA[c], g);
-        }
-        pm[r] = fld(bRm, g);
-        if constexpr (NODEM) {
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) pmod[r][c] = fld(bMo[c], g);
-        }
-      }
+    for (int c = 0; c < NDOF; ++c) {
+      const size_t o = c * P->S;
+      bD[c] = ubase((OOP ? P->din : P->d) + o);
+      bV[c] = ubase((OOP && P->vin ? P->vin : P->v) + o);
+      bA[c] = ubase((OOP && P->ain ? P->ain : P->a) + o);
+      bMo[c] = NODEM ? ubase(P->coefs + o) : nullptr;
     }
-    if constexpr (MODE == COEF_COMPACT || NODEM) {
-      if (tid < G.nxe * G.nze * 3) {
-        const int e = tid / 3, k = tid - 3 * (tid / 3);
-        const int lx = e % G.nxe, lz = e / G.nxe;
-        pg = fld(bGe, cidx(gr, tg.z >> 16, G, lx, lz) * 3 + k);
+    const R* bRm = ubase(P->rmass0);
+    const R* bCo = ubase(P->coefs);
+    const R* bGe = ubase(P->geom);
+    const R* bEt = EP && P->eta ? ubase(P->eta) : nullptr;
+    const R* bBe = EP && P->b25 ? ubase(P->b25) : nullptr;
+    const int nx = tg.z >> 16;
+    const int tl = lane_id();
+#pragma unroll
+    for (int r = 0; r < TS_ITER; ++r) {
+      const auto g = nidx(gr, G, min(xz[r] & 0xff, G.PX - 1), min(xz[r] >> 8, G.PZ - 1));
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        pd[r][c] = fld(bD[c], g);
+        if constexpr (!LATEV) pv[r][c] = fld(bV[c], g);
+        if constexpr (!PIN) pa[r][c] = fld(bA[c], g);
+        if constexpr (NODEM) pmod[r][c] = fld(bMo[c], g);
       }
+      if constexpr (FULLPF) pm[r] = fld(bRm, g);
     }
-    if constexpr (MODE == COEF_COMPACT) {
-#pragma unroll
-      for (int q = 0; q < PB_MAXB; ++q) {
-        const int cc = q / NBATCH, b0 = (q % NBATCH) * EPB;
-        const int cx = cc & 1, cz = cc >> 1;
-        const int ncx = (G.nxe - cx + 1) >> 1, ncz = (G.nze - cz + 1) >> 1;
-        const int ce = b0 + le;
-        if (tid < ETHREADS && ce < ncx * ncz) {
-          const int lx = cx + 2 * (ce % ncx), lz = cz + 2 * (ce / ncx);
-          const auto cell = cidx(gr, tg.z >> 16, G, lx, lz);
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) lm[q][c] = fld(bCo, cell * NDOF * NP + c * NP + pe);
-        }
-      }
-    } else if constexpr (MODE == COEF_SHARED) {
-      if (tid < ETHREADS) load_coefs<R, NDOF, NELAST, MODE>(grid_coefs<R, MODE>(coefs, gr), geom, 0, pe, sa);
+    if constexpr (COMP || NODEM) {
+      const int e = tl / 3, k = tl - 3 * (tl / 3);
+      const int lx = min(e % TX, G.nxe - 1), lz = min(e / TX, G.nze - 1);
+      pg = fld(bGe, cidx(gr, nx, G, lx, lz) * 3 + k);
+    }
+    if constexpr (MODE == COEF_SHARED) {
+      psa = bCo[gr.w + min(tl, NELAST * NP - 1)];
     }
     if constexpr (EP) {
 #pragma unroll
       for (int j = 0; j < NEP; ++j) {
-        const int idx = tid + NT * j;
-        if (idx < G.nxe * G.nze * NP) {
-          const int e = idx / NP, p = idx - NP * (idx / NP);
-          const auto cell = cidx(gr, tg.z >> 16, G, e % G.nxe, e / G.nxe);
-          if (bEt) peta[j] = fld(bEt, cell * NP + p);
-          if (bBe) pbet[j] = fld(bBe, cell * NP + p);
-        }
+        const int q = tl + TS_NT * j;
+        const int e = q / NP, o = q - e * NP;
+        const auto cell = cidx(gr, nx, G, min(e % TX, G.nxe - 1), min(e / TX, G.nze - 1));
+        peta[j] = bEt ? fld(bEt, cell * NP + o) : R(0);
+        pbet[j] = bBe ? fld(bBe, cell * NP + o) : R(0);
       }
     }
-    if (tid < tspc[t]) psp = T.spec_idx[t * MAXSPECIAL + tid];
   };
 
-  // FP64 fields at 512 threads: a thread keeps the predicted velocity and inverse mass
-  // of its patch nodes in registers from its predictor to its stores (the registers are
-  // there at two waves per SIMD); other shapes pass them through LDS.
-  constexpr bool REGV = sizeof(R) == 8 && NT == 512 && !EP;
-  R vkeep[REGV ? NITER : 1][NDOF] = {}, rkeep[REGV ? NITER : 1] = {};
-  // likewise the moduli of the current tile's point tasks (compact mode): copied from
-  // the prefetch registers by the predictor instead of staged through LDS
-  constexpr bool REGM = REGV && MODE == COEF_COMPACT;
-  R lmc[REGM ? PB_MAXB : 1][NDOF] = {};
+  // predicted velocity and inverse mass of the tile's nodes, for its stores
+  R wk[EP ? 1 : TS_ITER][NDOF] = {}, rk[TS_ITER] = {};
 
-  // Stores of a finished tile (tile tp, descriptors tgp, grp) from LDS: a thread
-  // stores the patch nodes it owns in the node loops (p = tnode + NT r), so the next
-  // tile's predictor, run by the same thread on the same slots after this, needs no
-  // barrier in between.  Partial forces for perimeter and special nodes, new a, v, d
-  // for the others.
-  auto store_tile = [&](const int tp, const int4 tgp, const int4 grp) {
+  // Stores of a finished tile: partial forces for perimeter and special nodes, new a, v,
+  // d for the others.
+  auto store_tile = [&](const int tp, const int4 tgp, const int4 grp, const R (*fk)[NDOF]) {
+    const auto* P = kernel_args<TileArgs<R>>();
     const Geo G = geo(tgp);
-    const uint32_t fbase = (uint32_t)tp * SLOTS;
+    R *oD[NDOF], *oV[NDOF], *oA[NDOF], *bF[NDOF];
 #pragma unroll
-    for (int r = 0; r < NITER; ++r) {
-      const int p = tnode + NT * r;
-      if (p < G.NPT) {
-        const int Z = p / G.PX, X = p - Z * G.PX;
+    for (int c = 0; c < NDOF; ++c) {
+      const size_t o = c * P->S;
+      oD[c] = ubase(P->d + o);
+      oV[c] = ubase(P->v + o);
+      oA[c] = ubase(P->a + o);
+      bF[c] = ubase(P->fpart + c * P->FPS);
+    }
+    const R c3 = P->c3, c4 = P->c4, dt = P->dt, c1 = P->c1, c2 = P->c2;
+    const StepOut so = {P->out.final, P->out.accel, P->out.rec};
+    const int mrow = so.rec >= 0 ? sload(P->mark_of, tp) : -1;
+    const uint32_t fbase = (uint32_t)tp * SLOTS;
+    const int ns = sload(P->spec_cnt, tp);
+#pragma unroll
+    for (int r = 0; r < TS_ITER; ++r) {
+      const int X = xz[r] & 0xff, Z = xz[r] >> 8;
+      if (X < G.PX && Z < G.PZ) {
         int slot = perim_slot(X, Z, G.PX, G.PZ);
-        if (slot < 0 && sflag[p] >= 0) slot = PERIM_MAX + sflag[p];
+        for (int k = 0; k < ns; ++k)  // a handful of tiles have special nodes
+          if (sload(P->spec_idx, tp * MAXSPECIAL + k) == tid + TS_NT * r) slot = PERIM_MAX + k;
         if (slot >= 0) {
 #pragma unroll
-          for (int c = 0; c < NDOF; ++c) fld(bF[c], fbase + slot) = lv_get<R, NDOF>(Fn[p], c);
+          for (int c = 0; c < NDOF; ++c) fld(bF[c], fbase + slot) = fk[r][c];
         } else {
           const auto g = nidx(grp, G, X, Z);
-          const R rm = REGV ? rkeep[r] : Rm[p];
+          const LV u = Ud[tid + TS_NT * r];
 #pragma unroll
           for (int c = 0; c < NDOF; ++c) {
-            const R ak = lv_get<R, NDOF>(Fn[p], c) * rm;
-            fld(oA[c], g) = ak;
-            fld(oV[c], g) = (REGV ? vkeep[r][c] : lv_get<R, NDOF>(Vp[p], c)) + c3 * ak;
-            fld(oD[c], g) = lv_get<R, NDOF>(Ud[p], c) + c4 * ak;
+            const R ak = fk[r][c] * rk[r];
+            const R vn = (EP ? lv_get<R, NDOF>(Vp[EP ? tid + TS_NT * r : 0], c) : wk[EP ? 0 : r][c]) + c3 * ak;
+            const R dn = lv_get<R, NDOF>(u, c) + c4 * ak;
+            if (so.final) {
+              fld(oA[c], g) = ak;
+              fld(oV[c], g) = vn;
+              fld(oD[c], g) = dn;
+            } else {
+              fld(oV[c], g) = vn + c2 * ak;
+              fld(oD[c], g) = dn + dt * vn + c1 * ak;
+              if (so.accel) fld(oA[c], g) = ak;
+              if (mrow >= 0) {  // few tiles hold recorded nodes
+                const int p = tid + TS_NT * r;
+                if (P->marks[mrow * MARK_WORDS + (p >> 5)] >> (p & 31) & 1)
+                  fld(ubase(P->rec + c * P->S), g) = so.rec == 0 ? dn : (so.rec == 1 ? vn : ak);
+              }
+            }
           }
         }
       }
     }
   };
 
-  issue(tlist[q0]);
-  // the previous tile of this workgroup, whose results are still in LDS
-  int tp = -1;
+  issue(q0);
+  int tp = -1;  // FULLPF: the previous tile of this workgroup, not yet stored
   int4 tgp = {}, grp = {};
+  R fk[TS_ITER][NDOF] = {};
 
 #pragma unroll 1
-  for (int q0i = q0; q0i < s1; q0i += W) {
-    int lelem = le;  // likewise for the element-batch lane index (full tiles)
-    if constexpr (FULL) {
-      tnode = tid;
-      asm volatile("" : "+v"(tnode));
-      asm volatile("" : "+v"(lelem));
-      // keep the ranges known, so that loop bounds that hold for every lane fold away
-      __builtin_assume(tnode >= 0 && tnode < NT);
-      __builtin_assume(lelem >= 0 && lelem <= (NT - 1) / NP);
-    }
-    const int t = tlist[q0i];
-    const int tn = q0i + W < s1 ? tlist[q0i + W] : -1;  // next tile of this workgroup
-    const int4 tg = ttiles[t];
-    const int4 gr = tgrids[t];
+  for (int qi = q0; qi < s1; qi += W) {
+    const int t = qi;
+    const int tn = qi + W < s1 ? qi + W : -1;  // next tile of this workgroup
+    const auto* P = kernel_args<TileArgs<R>>();
+    const int4 tg = sload(P->tiles, t);
+    const int4 gr = sload(P->grids, t);
     const Geo G = geo(tg);
-    const int PX = G.PX, PZ = G.PZ, NPT = G.NPT;
+    const R dt = P->dt, c1 = P->c1, c2 = P->c2;
 
-    // predictor from the prefetched values (every wait on a global load of this tile
-    // is here, ahead of any store) ...
-    R u[NITER][NDOF], w[NITER][NDOF];
+    // predictor
+    R u[TS_ITER][NDOF], w[TS_ITER][NDOF];
 #pragma unroll
-    for (int r = 0; r < NITER; ++r) {
-      const int p = tnode + NT * r;
-      if (p < NPT) {
+    for (int r = 0; r < TS_ITER; ++r)
 #pragma unroll
-        for (int c = 0; c < NDOF; ++c) {
+      for (int c = 0; c < NDOF; ++c) {
+        if constexpr (PIN) {
+          u[r][c] = pd[r][c];
+          if constexpr (!LATEV) w[r][c] = pv[r][c];
+        } else {
           u[r][c] = pd[r][c] + dt * pv[r][c] + c1 * pa[r][c];
           w[r][c] = pv[r][c] + c2 * pa[r][c];
         }
       }
+    if constexpr (FULLPF) {
+      // the waits for this tile's loads stay ahead of the previous tile's stores
+#pragma unroll
+      for (int r = 0; r < TS_ITER; ++r) {
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) asm volatile("" : "+v"(u[r][c]), "+v"(w[r][c]));
+        asm volatile("" : "+v"(pm[r]));
+      }
+      if (tp >= 0) store_tile(tp, tgp, grp, fk);
     }
-    // ... then the previous tile's stores (this tile's element phase covers their
-    // completion, and the next wait on a load is for loads issued after them) ...
-    if (tp >= 0) store_tile(tp, tgp, grp);
-    // ... then this tile's node values into LDS (FP64: predicted velocity and inverse
-    // mass stay in this thread's registers until its stores)
 #pragma unroll
-    for (int r = 0; r < NITER; ++r) {
-      const int p = tnode + NT * r;
-      if (p < NPT) {
+    for (int r = 0; r < TS_ITER; ++r) {
+      const int p = tid + TS_NT * r;
+      if (p < PMAX) {
         Ud[p] = lv_make<R, NDOF>(u[r]);
-        if constexpr (REGV) {
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) vkeep[r][c] = w[r][c];
-          rkeep[r] = pm[r];
-        } else {
-          Vp[p] = lv_make<R, NDOF>(w[r]);
-          Rm[p] = pm[r];
-        }
-        Fn[p] = LV{};
-        sflag[p] = -1;
+        if constexpr (EP) Vp[p] = lv_make<R, NDOF>(w[r]);
         if constexpr (NODEM) Mn[p] = lv_make<R, NDOF>(pmod[r]);
       }
+      if constexpr (!LATEV && !EP) {
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) wk[r][c] = w[r][c];
+      }
+      if constexpr (FULLPF) rk[r] = pm[r];
     }
-    if constexpr (NODEM) {
-      if (tid < G.nxe * G.nze * 3) Gm[tid / 3][tid - 3 * (tid / 3)] = pg;
+    if constexpr (COMP || NODEM) {
+      if (tid < NEL * 3) Gm[tid / 3][tid - 3 * (tid / 3)] = pg;
+    }
+    if constexpr (MODE == COEF_SHARED) {
+      if (tid < NELAST * NP) Sa[tid] = psa;
     }
     if constexpr (EP) {
 #pragma unroll
-      for (int j = 0; j < NEP; ++j) {
-        const int idx = tid + NT * j;
-        if (idx < G.nxe * G.nze * NP) {
-          Eta[idx] = peta[j];
-          Bet[idx] = pbet[j];
+      for (int j = 0; j < NEP; ++j)
+        if (tid + TS_NT * j < NEPT) {
+          Eta[tid + TS_NT * j] = peta[j];
+          Bet[tid + TS_NT * j] = pbet[j];
         }
-      }
-    }
-    if constexpr (MODE == COEF_COMPACT) {
-      if (tid < G.nxe * G.nze * 3) Gm[tid / 3][tid - 3 * (tid / 3)] = pg;
-      if constexpr (REGM) {
-#pragma unroll
-        for (int q = 0; q < PB_MAXB; ++q)
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) lmc[q][c] = lm[q][c];
-      } else if (tid < ETHREADS) {
-#pragma unroll
-        for (int q = 0; q < PB_MAXB; ++q) ML[q][tid] = lv_make<R, NDOF>(lm[q]);
-      }
-    } else if constexpr (MODE == COEF_SHARED) {
-#pragma unroll
-      for (int k = 0; k < NELAST; ++k) sac[k] = sa[k];
     }
     __syncthreads();
-    if (psp >= 0) sflag[psp] = (short)tid;
-    psp = -1;
-    // overlap: all loads of the next tile fly during this tile's element phase
-    if (tn >= 0) issue(tn);
 
-    // Element batches, software-pipelined over one barrier per batch: in phase q the
-    // lanes compute the stresses of batch q (into T[q & 1]) and assemble batch q-1 (from
-    // T[(q-1) & 1]) into Fn.  Batch q-1's nodes belong to elements of one colour, and
-    // the elements of one colour share no node, so the per-node summation order is the
-    // colour order, as in the two-barrier form.
-    bool pv_valid = false, pv_active = false;
-    int pv_base = 0, pv_el = 0, nvb = 0;
+    // element phase: element e, row or column s
+    {
+      const int tl = lane_id(), lane = tl & 63;
+      const int e = (tl >> 6) * TS_EPW + lane / NG, s = lane % NG;
+      const int lx = e % TX, lz = e / TX;
+      const bool on = lane < TS_EPW * NG && e < NEL && lx < G.nxe && lz < G.nze;
+      const int base = 4 * lz * PS + 4 * lx;
+      LV* ex = Ex + e * NP;
+      // the moduli of the row's points, ahead of the next tile's loads (they would be
+      // waited for with those otherwise)
+      R m[COMP ? NG : 1][NDOF];
+      if constexpr (COMP) {
+        const R* bCo = ubase(P->coefs);
+        const auto cell = cidx(gr, tg.z >> 16, G, min(lx, G.nxe - 1), min(lz, G.nze - 1));
 #pragma unroll
-    for (int q = 0; q <= PB_MAXB; ++q) {
-      bool has = false, active = false;
-      int base = 0, elc = 0;
-      if (q < PB_MAXB) {
-        const int cc = q / NBATCH, b0 = (q % NBATCH) * EPB;
-        const int cx = cc & 1, cz = cc >> 1;
-        const int ncx = (G.nxe - cx + 1) >> 1, ncz = (G.nze - cz + 1) >> 1;
-        const int nce = ncx * ncz;
-        has = b0 < nce;  // uniform across the workgroup
-        const int ce = b0 + lelem;
-        active = has && (tid < ETHREADS) && (ce < nce);
-        if (active) {
-          const int lx = cx + 2 * (ce % ncx), lz = cz + 2 * (ce / ncx);
-          base = 4 * lz * PX + 4 * lx;
-          elc = lz * G.nxe + lx;
+        for (int i = 0; i < NG; ++i)
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) m[i][c] = fld(bCo, (cell * NDOF + c) * NP + s * NG + i);
+      }
+      if (tn >= 0) {
+        issue(tn);
+      } else {  // no old values to keep
+#pragma unroll
+        for (int r = 0; r < TS_ITER; ++r)
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) {
+            pd[r][c] = 0;
+            if constexpr (!LATEV) pv[r][c] = 0;
+            if constexpr (!PIN) pa[r][c] = 0;
+          }
+        if constexpr (NODEM) {
+#pragma unroll
+          for (int r = 0; r < TS_ITER; ++r)
+#pragma unroll
+            for (int c = 0; c < NDOF; ++c) pmod[r][c] = 0;
+        }
+        if constexpr (FULLPF) {
+#pragma unroll
+          for (int r = 0; r < TS_ITER; ++r) pm[r] = 0;
+        }
+        pg = psa = 0;
+      }
+
+      // H as scalar operands, read once per tile
+      const auto* hp = hconst<R>();
+      R H[NG][NG];
+#pragma unroll
+      for (int k = 0; k < NG; ++k)
+#pragma unroll
+        for (int i = 0; i < NG; ++i) H[k][i] = hp[k * NG + i];
+      // A: column s
+      if (on) {
+        R g[NG][NDOF];
+#pragma unroll
+        for (int j = 0; j < NG; ++j)
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
+#pragma unroll
+        for (int k = 0; k < NG; ++k) {
+          const LV x = Ud[base + k * PS + s];
+          LV y{};
+          R et = 0;
+          if constexpr (EP) {
+            y = Vp[base + k * PS + s];
+            et = Eta[e * NP + k * NG + s];
+          }
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) {
+            R xc = lv_get<R, NDOF>(x, c);
+            if constexpr (EP) xc = xc + et * lv_get<R, NDOF>(y, c);
+#pragma unroll
+            for (int j = 0; j < NG; ++j) g[j][c] += xc * H[k][j];
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
+      }
+      wave_order();
+      // B: row s
+      R s1r[NG][NDOF];
+      if (on) {
+        R x[NG][NDOF];
+#pragma unroll
+        for (int k = 0; k < NG; ++k) {
+          const LV xv = Ud[base + s * PS + k];
+          LV y{};
+          R et = 0;
+          if constexpr (EP) {
+            y = Vp[base + s * PS + k];
+            et = Eta[e * NP + s * NG + k];
+          }
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) {
+            x[k][c] = lv_get<R, NDOF>(xv, c);
+            if constexpr (EP) x[k][c] = x[k][c] + et * lv_get<R, NDOF>(y, c);
+            s1r[k][c] = 0;
+          }
+        }
+        R g0 = 0, g1 = 0, g2 = 0;
+        if constexpr (COMP || NODEM) {
+          g0 = Gm[e][0];
+          g1 = Gm[e][1];
+          g2 = Gm[e][2];
+        }
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+          const int pt = s * NG + i;
           R A[NELAST];
-          if constexpr (MODE == COEF_COMPACT || NODEM) {
-            const int el = lz * G.nxe + lx;
-            const R g0 = Gm[el][0], g1 = Gm[el][1], g2 = Gm[el][2];
+          if constexpr (COMP || NODEM) {
+            const R w2 = sW2[pt];
             R m0, m1;
             if constexpr (NODEM) {
-              const LV mm = Mn[base + jj * PX + ii];
+              const LV mm = Mn[base + s * PS + i];
               m0 = lv_get<R, NDOF>(mm, 0);
               m1 = lv_get<R, NDOF>(mm, NDOF - 1);
-            } else if constexpr (REGM) {
-              m0 = lmc[q][0];
-              m1 = lmc[q][NDOF - 1];
             } else {
-              const LV mm = ML[q][tid];
-              m0 = lv_get<R, NDOF>(mm, 0);
-              m1 = lv_get<R, NDOF>(mm, NDOF - 1);
+              m0 = m[i][0];
+              m1 = m[i][NDOF - 1];
             }
             if constexpr (NDOF == 2) {
               const R la = m0, mu = m1, kx = la + 2 * mu;
@@ -745,106 +679,132 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 512 &&
             }
           } else if constexpr (MODE == COEF_SHARED) {
 #pragma unroll
-            for (int k = 0; k < NELAST; ++k) A[k] = sac[k];
+            for (int k = 0; k < NELAST; ++k) A[k] = Sa[k * NP + pt];
           } else {
-            const size_t cell = cell_index(gr, tg.z >> 16, G.tx0, G.tz0, lx, lz);
-            load_coefs<R, NDOF, NELAST, MODE>(grid_coefs<R, MODE>(coefs, gr), geom, cell, pe, A);
+            const R* bCo = ubase(P->coefs);
+            const auto cell = cidx(gr, tg.z >> 16, G, lx, lz);
+#pragma unroll
+            for (int k = 0; k < NELAST; ++k) A[k] = fld(bCo, (cell * NELAST + k) * NP + pt);
           }
           R dxi[NDOF], deta[NDOF];
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) dxi[c] = deta[c] = 0;
-#pragma unroll
-          for (int k = 0; k < NG; ++k) {
-            const int n1 = base + jj * PX + k, n2 = base + k * PX + ii;
-            const LV u1 = Ud[n1], u2 = Ud[n2];
-            if constexpr (EP) {  // d + eta v at the element's points (k, jj) and (ii, k)
-              const LV w1 = Vp[n1], w2 = Vp[n2];
-              const R e1 = Eta[elc * NP + jj * NG + k], e2 = Eta[elc * NP + k * NG + ii];
-#pragma unroll
-              for (int c = 0; c < NDOF; ++c) {
-                dxi[c] += hA[k] * (lv_get<R, NDOF>(u1, c) + e1 * lv_get<R, NDOF>(w1, c));
-                deta[c] += (lv_get<R, NDOF>(u2, c) + e2 * lv_get<R, NDOF>(w2, c)) * hB[k];
-              }
-            } else {
-#pragma unroll
-              for (int c = 0; c < NDOF; ++c) {
-                dxi[c] += hA[k] * lv_get<R, NDOF>(u1, c);
-                deta[c] += lv_get<R, NDOF>(u2, c) * hB[k];
-              }
-            }
-          }
-          LV(*T1) = T1b[nvb & 1][le];
-          LV(*T2) = T2b[nvb & 1][le];
-          R t1[NDOF], t2[NDOF];
-          if constexpr (NDOF == 2) {
-            if constexpr (NELAST == 6) {
-              t1[0] = A[0] * dxi[0] + A[1] * deta[1];
-              t2[0] = A[3] * (deta[0] + dxi[1]);
-              t1[1] = A[4] * deta[0] + A[5] * dxi[1];
-              t2[1] = A[1] * dxi[0] + A[2] * deta[1];
-            } else {
-              t1[0] = A[0] * dxi[0] + A[6] * deta[0] + A[7] * dxi[1] + A[1] * deta[1];
-              t2[0] = A[6] * dxi[0] + A[3] * deta[0] + A[4] * dxi[1] + A[8] * deta[1];
-              t1[1] = A[7] * dxi[0] + A[4] * deta[0] + A[5] * dxi[1] + A[9] * deta[1];
-              t2[1] = A[1] * dxi[0] + A[8] * deta[0] + A[9] * dxi[1] + A[2] * deta[1];
-            }
-          } else {
-            if constexpr (NELAST == 2) {
-              t1[0] = A[0] * dxi[0];
-              t2[0] = A[1] * deta[0];
-            } else {
-              t1[0] = A[0] * dxi[0] + A[2] * deta[0];
-              t2[0] = A[2] * dxi[0] + A[1] * deta[0];
-            }
-          }
-          T1[pe] = lv_make<R, NDOF>(t1);
-          T2[pe] = lv_make<R, NDOF>(t2);
-        }
-      }
-      if (pv_active) {  // assemble the previous batch
-        const LV* T1 = T1b[(nvb - 1) & 1][le];
-        const LV* T2 = T2b[(nvb - 1) & 1][le];
-        R s1[NDOF], s2[NDOF], f[NDOF];
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) s1[c] = s2[c] = 0;
-#pragma unroll
-        for (int k = 0; k < NG; ++k) {
-          const LV a1 = T1[jj * NG + k], a2 = T2[k * NG + ii];
+          const LV gv = ex[pt];
 #pragma unroll
           for (int c = 0; c < NDOF; ++c) {
-            s1[c] += hC[k] * lv_get<R, NDOF>(a1, c);
-            s2[c] += lv_get<R, NDOF>(a2, c) * hD[k];
+            R sum = 0;
+#pragma unroll
+            for (int k = 0; k < NG; ++k) sum += H[k][i] * x[k][c];
+            dxi[c] = sum;
+            deta[c] = lv_get<R, NDOF>(gv, c);
+          }
+          R t1[NDOF], t2[NDOF];
+          if constexpr (NDOF == 2) {
+            t1[0] = A[0] * dxi[0] + A[1] * deta[1];
+            t2[0] = A[3] * (deta[0] + dxi[1]);
+            t1[1] = A[4] * deta[0] + A[5] * dxi[1];
+            t2[1] = A[1] * dxi[0] + A[2] * deta[1];
+          } else {
+            t1[0] = A[0] * dxi[0];
+            t2[0] = A[1] * deta[0];
+          }
+          ex[pt] = lv_make<R, NDOF>(t2);
+#pragma unroll
+          for (int q = 0; q < NG; ++q)
+#pragma unroll
+            for (int c = 0; c < NDOF; ++c) s1r[q][c] += H[q][i] * t1[c];
+          // one point at a time: hoisting the later points' LDS reads costs the registers
+          // of the next tile's loads
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      wave_order();
+      // what the stores need besides the forces, loaded when the registers of B are free
+      // and used after C, D and E
+      if constexpr (!FULLPF) {
+        const R* bRm = ubase(P->rmass0);
+        const R* bV[NDOF];
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) bV[c] = ubase((OOP && P->vin ? P->vin : P->v) + c * P->S);
+#pragma unroll
+        for (int r = 0; r < TS_ITER; ++r) {
+          const auto g = nidx(gr, G, min(xz[r] & 0xff, G.PX - 1), min(xz[r] >> 8, G.PZ - 1));
+          rk[r] = fld(bRm, g);
+          if constexpr (LATEV) {
+#pragma unroll
+            for (int c = 0; c < NDOF; ++c) wk[r][c] = fld(bV[c], g);
           }
         }
-        LV* fp = &Fn[pv_base + jj * PX + ii];
-        const LV f0 = *fp;
-        if (EP && bBe) {  // 2.5D: the point force loses b25 (d + eta v) of its own point
-          const int own = pv_base + jj * PX + ii;
-          const LV uo = Ud[own], wo = Vp[own];
-          const R eo = Eta[pv_el * NP + pe], bo = Bet[pv_el * NP + pe];
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c)
-            f[c] = lv_get<R, NDOF>(f0, c) +
-                   ((s1[c] + s2[c]) - bo * (lv_get<R, NDOF>(uo, c) + eo * lv_get<R, NDOF>(wo, c)));
-        } else {
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) f[c] = lv_get<R, NDOF>(f0, c) + (s1[c] + s2[c]);
-        }
-        *fp = lv_make<R, NDOF>(f);
       }
-      if (has || pv_valid) __syncthreads();
-      pv_valid = has;
-      pv_active = active;
-      pv_base = base;
-      pv_el = elc;
-      if (has) ++nvb;
+      // C: column s
+      if (on) {
+        R g[NG][NDOF];
+#pragma unroll
+        for (int j = 0; j < NG; ++j)
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
+#pragma unroll
+        for (int k = 0; k < NG; ++k) {
+          const LV tv = ex[k * NG + s];
+#pragma unroll
+          for (int j = 0; j < NG; ++j)
+#pragma unroll
+            for (int c = 0; c < NDOF; ++c) g[j][c] += lv_get<R, NDOF>(tv, c) * H[j][k];
+        }
+#pragma unroll
+        for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
+      }
+      wave_order();
+      // D: row s
+      if (on) {
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+          const LV c2v = ex[s * NG + i];
+          R f[NDOF];
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) f[c] = s1r[i][c] + lv_get<R, NDOF>(c2v, c);
+          if constexpr (EP) {
+            if (P->b25) {  // 2.5D: the point force loses b25 (d + eta v) of its own point
+              const int own = base + s * PS + i;
+              const LV uo = Ud[own], wo = Vp[own];
+              const R eo = Eta[e * NP + s * NG + i], bo = Bet[e * NP + s * NG + i];
+#pragma unroll
+              for (int c = 0; c < NDOF; ++c)
+                f[c] = f[c] - bo * (lv_get<R, NDOF>(uo, c) + eo * lv_get<R, NDOF>(wo, c));
+            }
+          }
+          ex[s * NG + i] = lv_make<R, NDOF>(f);
+        }
+      } else if (lane < TS_EPW * NG && e < NEL) {
+#pragma unroll
+        for (int i = 0; i < NG; ++i) ex[s * NG + i] = LV{};
+      }
     }
-    // the last element batch ended with a barrier: Fn is complete
-    tp = t;
-    tgp = tg;
-    grp = gr;
+    __syncthreads();
+    // E: nodes (elements outside the tile left zero)
+#pragma unroll
+    for (int r = 0; r < TS_ITER; ++r) {
+      const int p = tid + TS_NT * r;
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) fk[r][c] = 0;
+      if (p < PMAX) {
+        const ushort4 sl = Eg[p];
+        const LV f0 = Ex[sl.x], f1 = Ex[sl.y], f2 = Ex[sl.z], f3 = Ex[sl.w];
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c)
+          fk[r][c] = (((lv_get<R, NDOF>(f0, c)) + lv_get<R, NDOF>(f1, c)) + lv_get<R, NDOF>(f2, c)) +
+                     lv_get<R, NDOF>(f3, c);
+      }
+    }
+    if constexpr (FULLPF) {
+      tp = t;
+      tgp = tg;
+      grp = gr;
+    } else {
+      store_tile(t, tg, gr, fk);
+    }
   }
-  if (tp >= 0) store_tile(tp, tgp, grp);
+  if constexpr (FULLPF) {
+    if (tp >= 0) store_tile(tp, tgp, grp, fk);
+  }
 }
 
 // One deferred node: tile-perimeter, special or split-fault node.
@@ -860,14 +820,15 @@ struct DefNode {
   int dmask;    // Dirichlet components zeroed in the force (bit c: component c), after the
                 // absorbing terms; at a fault node, those of the Dirichlet boundaries that
                 // act before the fault
+  int rec;      // recorded node (StepOut::rec)
   int pinl;     // device form only: 1 when the two partial offsets are poff (pcnt == 2)
   int poff[2];
 };
 
 // Device form of a deferred-node list: 16 bytes per node (one vector load) plus a side
 // table for the few nodes with sources or absorbing terms.  cnt packs pcnt (bits 0-7),
-// scnt (bits 8-15), acnt (bits 16-23), fault (bit 24), "offsets inline" (bit 25) and
-// the Dirichlet mask (bits 26-27); x
+// scnt (bits 8-15), acnt (bits 16-23), fault (bit 24), "offsets inline" (bit 25), the
+// Dirichlet mask (bits 26-27) and "recorded" (bit 28); x
 // is the node's (sstart, astart) entry in ext, or -1 when it has neither.  A node with
 // two partial forces and no ext entry (a tile-edge node) holds its two partial offsets
 // in pstart and x instead (bit 25 set), so part_off is not read for it.
@@ -889,6 +850,7 @@ __device__ __forceinline__ DefNode def_unpack(const DefTable& D, int q) {
   n.fault = (e.cnt >> 24) & 1;
   n.pinl = (e.cnt >> 25) & 1;
   n.dmask = (e.cnt >> 26) & 3;
+  n.rec = (e.cnt >> 28) & 1;
   n.sstart = 0;
   n.astart = 0;
   n.poff[0] = n.poff[1] = 0;
@@ -916,11 +878,12 @@ struct StaceyRefs {
 // per boundary element e and edge point k: kxd[e][k][c] = K[e][k][c] * sum_j h'_j(x_k)
 // D_c(node[e][j]), D the predicted displacement d + dt v + c1 a.  The boundary nodes are
 // deferred nodes, which k_deferred predicts later in the step, so the prediction is formed
-// here from the state of the previous step (the same expression as in k_deferred).
+// here from the state of the previous step (the same expression as in k_deferred), or is
+// the d array itself (pin: the state is the predicted one).
 template <typename R>
 __global__ void k_stacey_pre(int nbe, const int* __restrict__ enode, const double* __restrict__ K,
                              const R* __restrict__ d, const R* __restrict__ v, const R* __restrict__ a, size_t GS,
-                             R dt, R c1, double* __restrict__ kxd) {
+                             R dt, R c1, double* __restrict__ kxd, int pin) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;  // e * NG + k
   if (q >= nbe * NG) return;
   const int e = q / NG, k = q - NG * e;
@@ -930,14 +893,35 @@ __global__ void k_stacey_pre(int nbe, const int* __restrict__ enode, const doubl
 #pragma unroll
     for (int j = 0; j < NG; ++j) {
       const size_t g = (size_t)c * GS + enode[e * NG + j];
-      const R dp = d[g] + dt * v[g] + c1 * a[g];
+      const R dp = pin ? d[g] : d[g] + dt * v[g] + c1 * a[g];
       s += c_H[j * NG + k] * (double)dp;
     }
     kxd[(size_t)q * 2 + c] = K[(size_t)q * 2 + c] * s;
   }
 }
 
-template <typename R, int NDOF, bool OOP = false>
+// Corrector and stores of one node component from its predicted displacement and
+// velocity and its new acceleration ak, as in the tile kernel (StepOut; recp: where a
+// recorded node goes, else null)
+template <typename R>
+__device__ __forceinline__ void store_node(R* d, R* v, R* a, size_t i, R dp, R vp, R ak, R dt, R c1, R c2, R c3,
+                                           R c4, const StepOut& so, R* recp) {
+  const R vn = vp + c3 * ak;
+  const R dn = dp + c4 * ak;
+  if (so.final) {
+    a[i] = ak;
+    v[i] = vn;
+    d[i] = dn;
+  } else {
+    v[i] = vn + c2 * ak;
+    d[i] = dn + dt * vn + c1 * ak;
+    if (so.accel) a[i] = ak;
+    if (recp && so.rec >= 0) recp[i] = so.rec == 0 ? dn : (so.rec == 1 ? vn : ak);
+  }
+}
+
+// PIN: the state read is the predicted one; so: what is stored (StepOut)
+template <typename R, int NDOF, bool OOP = false, bool PIN = false>
 __global__ __launch_bounds__(256) void k_deferred(int ndef, DefTable defs,
                                                   const int* __restrict__ part_off, const R* __restrict__ fpart,
                                                   size_t FPS, const SrcEntry* __restrict__ src,
@@ -945,7 +929,7 @@ __global__ __launch_bounds__(256) void k_deferred(int ndef, DefTable defs,
                                                   const int* __restrict__ itp,
                                                   const double* __restrict__ abso, const R* __restrict__ rmdef,
                                                   R* __restrict__ d, R* __restrict__ v, R* __restrict__ a, size_t GS,
-                                                  R dt, R c1, R c2, R c3, R c4,
+                                                  R dt, R c1, R c2, R c3, R c4, StepOut so, R* __restrict__ recp,
                                                   const R* __restrict__ din = nullptr,
                                                   const R* __restrict__ vin = nullptr,
                                                   const R* __restrict__ ain = nullptr, StaceyRefs SR = {}) {
@@ -961,9 +945,15 @@ __global__ __launch_bounds__(256) void k_deferred(int ndef, DefTable defs,
   R dp[NDOF], vpp[NDOF], f[NDOF];
 #pragma unroll
   for (int c = 0; c < NDOF; ++c) {
-    const R dk = dsrc[c * GS + g], vk = vsrc[c * GS + g], ak = asrc[c * GS + g];
-    dp[c] = dk + dt * vk + c1 * ak;
-    vpp[c] = vk + c2 * ak;
+    const R dk = dsrc[c * GS + g], vk = vsrc[c * GS + g];
+    if constexpr (PIN) {
+      dp[c] = dk;
+      vpp[c] = vk;
+    } else {
+      const R ak = asrc[c * GS + g];
+      dp[c] = dk + dt * vk + c1 * ak;
+      vpp[c] = vk + c2 * ak;
+    }
     R s = 0;
     if (n.pinl) {  // the loop below with pcnt = 2
       s = s + fpart[c * FPS + n.poff[0]];
@@ -1011,10 +1001,8 @@ __global__ __launch_bounds__(256) void k_deferred(int ndef, DefTable defs,
   }
 #pragma unroll
   for (int c = 0; c < NDOF; ++c) {
-    const R ak = f[c] * rmdef[(size_t)c * ndef + q];
-    a[c * GS + g] = ak;
-    v[c * GS + g] = vpp[c] + c3 * ak;
-    d[c * GS + g] = dp[c] + c4 * ak;
+    store_node<R>(d, v, a, c * GS + g, dp[c], vpp[c], f[c] * rmdef[(size_t)c * ndef + q], dt, c1, c2, c3, c4, so,
+                  n.rec ? recp : nullptr);
   }
 }
 
@@ -1206,7 +1194,10 @@ __global__ __launch_bounds__(TILE_THREADS) void k_adj_tile(
   }
   __syncthreads();
   const int nspec = T.spec_cnt[t];
-  if (tid < nspec) sflag[T.spec_idx[t * MAXSPECIAL + tid]] = (short)tid;
+  if (tid < nspec) {
+    const int q = T.spec_idx[t * MAXSPECIAL + tid];
+    sflag[(q / PXM) * PX + q % PXM] = (short)tid;
+  }
 
   // element batch q: colour cc = q / NBATCH, elements b0 .. b0+FE_EPB-1 of that colour
   constexpr int NBATCH = (TX * TZ / 4 + FE_EPB - 1) / FE_EPB;
@@ -1383,7 +1374,7 @@ __device__ __forceinline__ void inject_node(const InjectPlan& P, int u, R* __res
 // Persistent, pipelined form of k_adj_tile, with the same arithmetic and the same
 // summation orders (results equal bit for bit): AP_NT threads, one colour of a tile's
 // elements per batch (two barriers per batch), each workgroup on a run of tiles (the
-// XCD slices of k_tile_pipe).  While a tile's element batches run, the adjoint state,
+// XCD slices of k_tile_step).  While a tile's element batches run, the adjoint state,
 // inverse mass, forward displacements (or acceleration), mass sensitivity, moduli,
 // geometric factors and element sensitivities of the workgroup's next tile load into
 // registers; a finished tile is stored by the threads that own its patch slots, right
@@ -1670,7 +1661,7 @@ __global__ __launch_bounds__(AP_NT) __attribute__((amdgpu_waves_per_eu(2))) void
       for (int q = 0; q < NB; ++q) ML[q][tnode] = lv_make<R, NDOF>(plm[q]);
     }
     __syncthreads();
-    if (psp >= 0) sflag[psp] = (short)tid;
+    if (psp >= 0) sflag[(psp / PXM) * PX + psp % PXM] = (short)tid;
     psp = -1;
     if (tn >= 0) issue(tn);
 
