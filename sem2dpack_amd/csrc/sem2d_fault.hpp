@@ -36,18 +36,15 @@ struct FaultDev {
   double *T, *Tstick;                    // [2][np]
   double *MU, *sigma;                    // [np]
   int *nr_fail;                          // Newton iteration overflow flag
-  // structured grids: inverse mass of node 1 / node 2 of each pair [ndof][np], for the
-  // corrector that k_fault applies after the solve
-  const double *rmn1 = nullptr, *rmn2 = nullptr;
   // structured grids: Dirichlet components of the Dirichlet boundaries that act after
   // the fault, zeroed in the force of node 1 (bits 0-1) and node 2 (bits 2-3) before the
   // corrector (null: none)
   const unsigned char* dmask = nullptr;
   // structured grids: d and v after the step at both nodes of every pair, bulk type,
-  // [d, v][node 1, node 2][ndof][np] (k_fault; the field arrays hold the next step's
-  // predicted values), and the recorded nodes (bit 0: node 1, bit 1: node 2; null: none)
+  // [d, v][node 1, node 2][ndof][np] (the field arrays hold the next step's predicted
+  // values); the pairs' nodes in the deferred-node list (def2: -1 on one side)
   void* side = nullptr;
-  const unsigned char* rmark = nullptr;
+  const int *def1 = nullptr, *def2 = nullptr;
   // time-weakening friction (BC_DYNFLT_TWF): kind (0: none; law 3: time weakening alone),
   // parameters MuS, MuD, Mu0, X, Z, V, L, T, Dc and the fault node coordinates [2][np]
   int twf = 0;
@@ -69,29 +66,6 @@ __host__ __device__ inline double normal_sigma(int kind, double coef, double vc,
     case 2: return tn + coef * (sig_old - tn);
     case 3: return tn + exp(-(fabs(dv) + vc) * coef) * (sig_old - tn);
     default: return tn;
-  }
-}
-
-// Corrector of one split-fault node after the fault solve (a = f * rmass, then v and d;
-// SRC/solver.f90:78-82), in the bulk precision and outside the no-contraction region
-// below, like the corrector of every other node; sd, sv: where d and v after the step go
-// for the jumps the fault outputs are made of.
-template <typename R>
-__device__ __forceinline__ void fault_node_correct(R* d, R* v, R* a, size_t i, R rm, R dt, R c1, R c2, R c3, R c4,
-                                                   const StepOut& so, R* recp, R* sd, R* sv) {
-  const R ak = a[i] * rm;
-  const R vn = v[i] + c3 * ak;
-  const R dn = d[i] + c4 * ak;
-  *sd = dn;
-  *sv = vn;
-  if (so.final) {
-    a[i] = ak;
-    v[i] = vn;
-    d[i] = dn;
-  } else {
-    v[i] = vn + c2 * ak;
-    d[i] = dn + dt * vn + c1 * ak;
-    if (recp && so.rec >= 0) recp[i] = so.rec == 0 ? dn : (so.rec == 1 ? vn : ak);
   }
 }
 
@@ -250,29 +224,31 @@ __device__ inline double f_rsf_v(const FaultDev& F, int k, double tstick, double
   return f_nr_solver(F, k, fmin(0.0, tstick), fmax(0.0, tstick), tol, theta, tstick, sigma, Z, ok);
 }
 
-// CORR (structured grids): the pair's two nodes are finished here too (fault_node_correct
-// with the inverse masses rmn1, rmn2); the general path corrects every node afterwards.
-// launched with 64 lanes per workgroup: the Newton iteration's registers are then not
-// capped by the 1024-lane default (which spilled them to scratch).  time = it*dt of the
-// step (SRC/main.f90:53), read by time-weakening friction only.
-template <typename R, bool CORR = false>
-__global__ __launch_bounds__(64) void k_fault(FaultDev F, R* d, R* v, R* f, int npoin, R dt = 0, R c1 = 0, R c2 = 0, R c3 = 0, R c4 = 0,
-                                              StepOut so = {}, R* recp = nullptr, double time = 0.0) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= F.np) return;
-  const int np = F.np, nd = F.ndof;
-  const int i1 = F.n1[k], i2 = F.n2[k];
+// One node component by component: the predicted displacement and velocity and the force.
+template <typename R>
+struct NodeState {
+  R d[2] = {0, 0}, v[2] = {0, 0}, f[2] = {0, 0};
+};
+
+// Traction solve of pair k from the states of its nodes (n2 unused when two is false: a
+// fault with one side); the fault state of the pair is updated and its tractions added to
+// the nodes' forces.  time = it*dt of the step (SRC/main.f90:53), read by time-weakening
+// friction only.
+template <typename R, int nd>
+__device__ inline void fault_solve(const FaultDev& F, int k, double time, bool two, NodeState<R>& n1,
+                                   NodeState<R>& n2) {
+  const int np = F.np;
   double dD[2] = {0, 0}, dV[2] = {0, 0}, dA[2] = {0, 0}, T[2] = {0, 0}, Ts[2];
+#pragma unroll
   for (int c = 0; c < nd; ++c) {
-    const size_t o = (size_t)c * npoin;
-    if (i2 >= 0) {
-      dD[c] = (double)d[o + i2] - (double)d[o + i1];
-      dV[c] = (double)v[o + i2] - (double)v[o + i1];
-      dA[c] = F.invM2[c * np + k] * (double)f[o + i2] - F.invM1[c * np + k] * (double)f[o + i1];
+    if (two) {
+      dD[c] = (double)n2.d[c] - (double)n1.d[c];
+      dV[c] = (double)n2.v[c] - (double)n1.v[c];
+      dA[c] = F.invM2[c * np + k] * (double)n2.f[c] - F.invM1[c * np + k] * (double)n1.f[c];
     } else {  // one side: get_jump, get_weighted_jump (SRC/bc_dynflt.f90:692-719)
-      dD[c] = -2.0 * (double)d[o + i1];
-      dV[c] = -2.0 * (double)v[o + i1];
-      dA[c] = -2.0 * F.invM1[c * np + k] * (double)f[o + i1];
+      dD[c] = -2.0 * (double)n1.d[c];
+      dV[c] = -2.0 * (double)n1.v[c];
+      dA[c] = -2.0 * F.invM1[c * np + k] * (double)n1.f[c];
     }
     T[c] = F.Z[c * np + k] * (dV[c] + F.a2v * dA[c]);
   }
@@ -284,7 +260,7 @@ __global__ __launch_bounds__(64) void k_fault(FaultDev F, R* d, R* v, R* f, int 
     r0 = nz * dA[0] - nx * dA[1]; r1 = nx * dA[0] + nz * dA[1]; dA[0] = r0; dA[1] = r1;
     r0 = nz * T[0] - nx * T[1];   r1 = nx * T[0] + nz * T[1];   T[0] = r0;  T[1] = r1;
   }
-  if (nd == 1 || i2 < 0) T[1] = 0.0;  // SRC/bc_dynflt.f90:604
+  if (nd == 1 || !two) T[1] = 0.0;  // SRC/bc_dynflt.f90:604
   T[0] = T[0] + F.T0[k];
   T[1] = T[1] + F.T0[np + k];
   if (F.opening) T[1] = fmin(T[1], 0.0);
@@ -341,33 +317,48 @@ __global__ __launch_bounds__(64) void k_fault(FaultDev F, R* d, R* v, R* f, int 
     Tx[0] = nz * T[0] + nx * T[1];
     Tx[1] = -nx * T[0] + nz * T[1];
   }
+#pragma unroll
   for (int c = 0; c < nd; ++c) {
-    const size_t o = (size_t)c * npoin;
     const double bt = F.B[c * np + k] * Tx[c];
-    f[o + i1] = (R)((double)f[o + i1] + bt);
-    if (i2 >= 0) f[o + i2] = (R)((double)f[o + i2] - bt);
+    n1.f[c] = (R)((double)n1.f[c] + bt);
+    if (two) n2.f[c] = (R)((double)n2.f[c] - bt);
   }
+#pragma unroll
   for (int c = 0; c < nd; ++c) {
     const double tf = T[c];
     const double da = dA[c] - tf / (F.Z[c * np + k] * F.a2v);
     F.D[c * np + k] = dD[c] + F.a2d * da;
     F.V[c * np + k] = dV[c] + F.a2v * da;
   }
-  if constexpr (CORR) {
-    const int dm = F.dmask ? F.dmask[k] : 0;
-    for (int c = 0; c < nd; ++c) {
-      const size_t o = (size_t)c * npoin;
-      if (dm >> c & 1) f[o + i1] = 0;
-      if (i2 >= 0 && (dm >> (2 + c) & 1)) f[o + i2] = 0;
-      R* sd = (R*)F.side + (size_t)c * np + k;
-      R* sv = sd + (size_t)2 * nd * np;
-      const int rec = F.rmark ? F.rmark[k] : 0;
-      fault_node_correct<R>(d, v, f, o + i1, (R)F.rmn1[c * np + k], dt, c1, c2, c3, c4, so, rec & 1 ? recp : nullptr,
-                            sd, sv);
-      if (i2 >= 0)
-        fault_node_correct<R>(d, v, f, o + i2, (R)F.rmn2[c * np + k], dt, c1, c2, c3, c4, so, rec & 2 ? recp : nullptr,
-                              sd + (size_t)nd * np, sv + (size_t)nd * np);
+}
+
+// Fault of the general path: the pair's forces updated in place; every node is corrected
+// afterwards.  Launched with 64 lanes per workgroup: the Newton iteration's registers are
+// then not capped by the 1024-lane default (which spilled them to scratch).
+template <typename R, int nd>
+__global__ __launch_bounds__(64) void k_fault(FaultDev F, const R* d, const R* v, R* f, int npoin, double time) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= F.np) return;
+  const int i1 = F.n1[k], i2 = F.n2[k];
+  NodeState<R> n1, n2;
+#pragma unroll
+  for (int c = 0; c < nd; ++c) {
+    const size_t o = (size_t)c * npoin;
+    n1.d[c] = d[o + i1];
+    n1.v[c] = v[o + i1];
+    n1.f[c] = f[o + i1];
+    if (i2 >= 0) {
+      n2.d[c] = d[o + i2];
+      n2.v[c] = v[o + i2];
+      n2.f[c] = f[o + i2];
     }
+  }
+  fault_solve<R, nd>(F, k, time, i2 >= 0, n1, n2);
+#pragma unroll
+  for (int c = 0; c < nd; ++c) {
+    const size_t o = (size_t)c * npoin;
+    f[o + i1] = n1.f[c];
+    if (i2 >= 0) f[o + i2] = n2.f[c];
   }
 }
 
@@ -428,13 +419,12 @@ __global__ void k_fault_sides(FaultDev F, const R* __restrict__ d, const R* __re
 // SRC/bc_dynflt.f90:832-855): P-SV p11, p22, p12 of d then of v, SH p13, p23 of d
 // then of v, one row of 2*(ndof+1) values, over the fault pairs k0 .. k0+n-1.  One
 // workgroup of 256 lanes: lane t sums pairs k0+t, k0+t+256, ..., then a fixed-shape
-// tree, so the result is run-to-run identical and the same for a fault alone (k0 = 0)
-// and inside a batch (its pairs at k0 of the concatenated arrays).  side_arrays: the
-// jumps are taken from F.side instead of the fields.
+// tree, so the result is run-to-run identical.  The general path's rows and the row of
+// step 0; the steps of a structured grid make theirs in potency_wave.
 template <typename R>
 __device__ __forceinline__ void potency_row(const FaultDev& F, int k0, int n, const R* __restrict__ d,
                                             const R* __restrict__ v, size_t stride, double* __restrict__ out,
-                                            double (*red)[256], int side_arrays) {
+                                            double (*red)[256]) {
   const int t = threadIdx.x, np = F.np;
   double s[6] = {0, 0, 0, 0, 0, 0};
   for (int kl = t; kl < n; kl += 256) {
@@ -443,17 +433,8 @@ __device__ __forceinline__ void potency_row(const FaultDev& F, int k0, int n, co
     const double nx = F.nrm[k], nz = F.nrm[np + k], b = F.B[k];
     // get_jump (SRC/bc_dynflt.f90:692-704): x2 - x1, or -2 x1 on a one-sided fault
     auto jump = [&](int w, int c) {
-      double x1, x2 = 0.0;
-      if (side_arrays) {
-        const R* sc = (const R*)F.side + ((size_t)(w * 2) * F.ndof + c) * np + k;
-        x1 = (double)sc[0];
-        if (i2 >= 0) x2 = (double)sc[(size_t)F.ndof * np];
-      } else {
-        const R* x = (w == 0 ? d : v) + (size_t)c * stride;
-        x1 = (double)x[i1];
-        if (i2 >= 0) x2 = (double)x[i2];
-      }
-      return i2 >= 0 ? x2 - x1 : -2.0 * x1;
+      const R* x = (w == 0 ? d : v) + (size_t)c * stride;
+      return i2 >= 0 ? (double)x[i2] - (double)x[i1] : -2.0 * (double)x[i1];
     };
     const double jd0 = jump(0, 0), jv0 = jump(1, 0);
     if (F.ndof == 2) {
@@ -498,27 +479,101 @@ __device__ __forceinline__ void potency_row(const FaultDev& F, int k0, int n, co
 
 template <typename R>
 __global__ __launch_bounds__(256) void k_fault_potency(FaultDev F, const R* __restrict__ d, const R* __restrict__ v,
-                                                       size_t stride, double* __restrict__ out, int side_arrays) {
+                                                       size_t stride, double* __restrict__ out) {
   __shared__ double red[6][256];
-  potency_row<R>(F, 0, F.np, d, v, stride, out, red, side_arrays);
+  potency_row<R>(F, 0, F.np, d, v, stride, out, red);
 }
 
-// Batched potency: workgroup m writes member m's row for the state after the current
-// step, row row_shift + *itp of pot[m][cap][2*(ndof+1)] (itp: the batch's step counter
-// in device memory, which a replayed graph advances); fbase[m] .. fbase[m+1] are member
-// m's pairs in the concatenated fault arrays.
-template <typename R>
-__global__ __launch_bounds__(256) void k_batch_potency(FaultDev F, const int* __restrict__ fbase,
-                                                       const R* __restrict__ d, const R* __restrict__ v,
-                                                       size_t stride, const int* __restrict__ itp, int row_shift,
-                                                       int cap, double* __restrict__ pot) {
-  __shared__ double red[6][256];
-  const int m = blockIdx.x;
-  const int row = row_shift + *itp;
-  if (row < 0 || row >= cap) return;  // uniform over the workgroup; the host reserves the rows
-  const int k0 = fbase[m];
-  potency_row<R>(F, k0, fbase[m + 1] - k0, d, v, stride, pot + ((size_t)m * cap + row) * (2 * (F.ndof + 1)), red,
-                 1);
+// Per-step outputs of a fault on a structured grid, made where its pairs are finished.
+// A wavefront takes wave[w] = (first pair, pairs, member, -): 64 pairs of one member at
+// most, the member's wavefronts being member[m].x .. + member[m].y - 1 (a fault alone is
+// member 0).
+struct FaultOut {
+  int nwave = 0;
+  const int4* wave = nullptr;
+  const int2* member = nullptr;
+  // potency rows pot[member][pot_cap][2*(ndof+1)]: the row of this step is pot_row, or
+  // pot_row + the device step counter; part [nwave][6] and cnt [members] are scratch (cnt
+  // zero between launches)
+  double *pot = nullptr, *part = nullptr;
+  unsigned* cnt = nullptr;
+  int pot_cap = 0, pot_row = 0;
+  // fault records rec[sample][6][nout]: slot[k] is the output place of pair k or -1; the
+  // sample is rec_slot (-1: none), or, with the device step counter, that of the steps
+  // oit0, oit0 + oitd, ...
+  const int* slot = nullptr;
+  double* rec = nullptr;
+  int nout = 0, rec_slot = -1, oit0 = 0, oitd = 1, nsamp = 0;
+};
+
+// Potency of one step from the jumps of a wavefront's pairs (dj, vj: the displacement and
+// velocity jumps of this lane's pair, on: it has one): the wavefront's sums by a tree over
+// its lanes, then, by the last wavefront of the member, the sums of its wavefronts in a
+// fixed order.  The result does not depend on which wavefront is last and is the same for
+// a fault alone and inside a batch.  (One workgroup over all pairs took 12 us of a 79 us
+// step, 600 x 300 elements; this adds 1-2 us to the fault's.)
+template <int nd>
+__device__ inline void potency_wave(const FaultDev& F, const FaultOut& O, int w, int k, bool on, const double* dj,
+                                    const double* vj, int row) {
+  const int lane = threadIdx.x & 63, np = F.np;
+  double s[6] = {0, 0, 0, 0, 0, 0};
+  if (on) {
+    const double nx = F.nrm[k], nz = F.nrm[np + k], b = F.B[k];
+    if (nd == 2) {
+      s[0] = nx * dj[0] * b;
+      s[1] = nz * dj[1] * b;
+      s[2] = (nx * dj[1] + nz * dj[0]) * b;
+      s[3] = nx * vj[0] * b;
+      s[4] = nz * vj[1] * b;
+      s[5] = (nx * vj[1] + nz * vj[0]) * b;
+    } else {
+      s[0] = nx * dj[0] * b;
+      s[1] = nz * dj[0] * b;
+      s[2] = nx * vj[0] * b;
+      s[3] = nz * vj[0] * b;
+    }
+  }
+  auto tree = [&]() {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int q = 0; q < 6; ++q) s[q] = s[q] + __shfl_xor(s[q], o);
+  };
+  tree();
+  const int m = O.wave[w].z;
+  const int2 mw = O.member[m];
+  unsigned before = 0;
+  if (lane == 0) {
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+      __hip_atomic_store(&O.part[(size_t)w * 6 + q], s[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    before = __hip_atomic_fetch_add(&O.cnt[m], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  before = __shfl(before, 0);
+  if (before + 1 != (unsigned)mw.y) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll
+  for (int q = 0; q < 6; ++q) s[q] = 0;
+  for (int u = lane; u < mw.y; u += 64)
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+      s[q] = s[q] + __hip_atomic_load(&O.part[(size_t)(mw.x + u) * 6 + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  tree();
+  if (lane != 0) return;
+  __hip_atomic_store(&O.cnt[m], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (row < 0 || row >= O.pot_cap) return;  // the host reserves the rows
+  double* out = O.pot + ((size_t)m * O.pot_cap + row) * (2 * (nd + 1));
+  if (nd == 2) {
+    out[0] = s[0];
+    out[1] = s[1];
+    out[2] = 0.5 * s[2];
+    out[3] = s[3];
+    out[4] = s[4];
+    out[5] = 0.5 * s[5];
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) out[q] = 0.5 * s[q];
+  }
 }
 
 #pragma clang fp contract(on)

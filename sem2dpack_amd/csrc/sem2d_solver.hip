@@ -86,6 +86,8 @@ struct StructState {
   int* spec_idx = nullptr;
   int* mark_of = nullptr;  // recorded nodes inside tiles (TileArgs)
   uint32_t* marks = nullptr;
+  RecOut rec;   // receivers at nodes, recorded by k_deferred
+  FaultOut fo;  // fault outputs, made by k_deferred
   void* fpart = nullptr;
   size_t FPS = 0;
   DefTable defs;
@@ -503,17 +505,17 @@ int potency_reserve(sem2d_solver* h, int rows) {
   return 0;
 }
 
-// sides: from FaultDev::side (the steps of a structured grid) instead of the fields
 template <typename R>
-void record_potency(sem2d_solver* h, int sides) {
+void record_potency(sem2d_solver* h) {
   FaultHost& F = h->flt;
   if (F.pot_rows >= F.pot_cap) return;  // reserved by the caller
   k_fault_potency<R><<<1, 256, 0, h->stream>>>(F.dev, (const R*)h->d, (const R*)h->v, h->fstride,
-                                               F.pot + (size_t)F.pot_rows * 2 * (h->ndof + 1), sides);
+                                               F.pot + (size_t)F.pot_rows * 2 * (h->ndof + 1));
   F.pot_rows++;
 }
 
-// per-side record (osides) of sample slot s from the current fields
+// per-side record (osides) of sample slot s from the current fields, or from
+// FaultDev::side (sides: the steps of a structured grid)
 void record_sides(sem2d_solver* h, int s, int sides) {
   FaultHost& F = h->flt;
   double* out = F.srec + (size_t)s * 4 * h->ndof * F.nout;
@@ -525,20 +527,40 @@ void record_sides(sem2d_solver* h, int s, int sides) {
         F.dev, (const double*)h->d, (const double*)h->v, h->fstride, F.oix1, F.oixd, F.nout, out, sides);
 }
 
-int record_fault(sem2d_solver* h, int sides = 0) {
+int record_fault(sem2d_solver* h) {
   FaultHost& F = h->flt;
   if (!F.on) return 0;
-  if (h->fp32) record_potency<float>(h, sides);
-  else record_potency<double>(h, sides);
+  if (h->fp32) record_potency<float>(h);
+  else record_potency<double>(h);
   if (h->it < F.oit) return 0;
   if (F.taken < F.nsamp) {
     k_fault_record<<<grid_for(F.nout, 64), 64, 0, h->stream>>>(F.dev, F.oix1, F.oixd, F.nout,
                                                                F.rec + (size_t)F.taken * 6 * F.nout);
-    if (F.srec) record_sides(h, F.taken, sides);
+    if (F.srec) record_sides(h, F.taken, 0);
     F.taken++;
   }
   F.oit += F.oitd;
   return 0;
+}
+
+// structured grids: the fault outputs that k_deferred makes at step it ...
+void fault_out_step(sem2d_solver* h, int it, FaultOut& O) {
+  FaultHost& F = h->flt;
+  O.pot = F.pot;
+  O.pot_cap = F.pot_cap;
+  O.pot_row = F.pot_rows;
+  O.rec_slot = it >= F.oit && F.taken < F.nsamp ? F.taken : -1;
+}
+// ... and the bookkeeping after it, with the per-side record
+void fault_out_done(sem2d_solver* h, int it) {
+  FaultHost& F = h->flt;
+  if (F.pot_rows < F.pot_cap) F.pot_rows++;
+  if (it < F.oit) return;
+  if (F.taken < F.nsamp) {
+    if (F.srec) record_sides(h, F.taken, 1);
+    F.taken++;
+  }
+  F.oit += F.oitd;
 }
 
 // ---------------------------------------------------------------------------
@@ -713,14 +735,14 @@ struct StructTables {
   std::vector<SrcEntry> dsrc;
   std::vector<double> dabso;
   std::vector<double> rmdef;     // [ndof][ndef]
-  std::vector<int> fault_g;
-  std::vector<double> fault_rm;  // [ndof][nf]
   std::vector<unsigned char> fault_dmask;  // [npairs] Dirichlet after the fault: node 1 bits 0-1, node 2 bits 2-3
   std::vector<int> s_enode, ak_off, ak_idx;  // Stacey (see StructState)
-  // recorded nodes: inside tiles (TileArgs::mark_of, marks), of fault pairs (FaultDev::rmark)
+  // recorded nodes inside tiles (TileArgs::mark_of, marks)
   std::vector<int> mark_of;
   std::vector<uint32_t> marks;
-  std::vector<unsigned char> fault_rmark;
+  // receivers at nodes (RecOut): (storage index, or deferred node, or 2 * pair + side; receiver)
+  std::vector<std::pair<int, int>> rec_int, rec_def, rec_flt;
+  std::vector<int> fault_def1, fault_def2;  // the pairs' nodes in defs
   std::vector<double> s_K;
 };
 
@@ -859,20 +881,39 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
     X.fault_dmask[k] = dmask_aft[h->fault_n1[k]];
     if (!h->fault_n2.empty()) X.fault_dmask[k] |= (unsigned char)(dmask_aft[h->fault_n2[k]] << 2);
   }
-  X.fault_rmark.assign(h->fault_n1.size(), 0);
+  std::vector<int> def_of((size_t)h->npoin, -1);  // reference node -> deferred node
+  for (size_t q = 0; q < ndef; ++q) def_of[def_ref[q]] = (int)q;
+  X.fault_def1.clear();
+  X.fault_def2.clear();
+  std::unordered_map<int, int> flt_of;  // reference node -> 2 * pair + side
   for (size_t k = 0; k < h->fault_n1.size(); ++k) {
-    X.fault_rmark[k] = is_rec[h->fault_n1[k]];
-    if (!h->fault_n2.empty()) X.fault_rmark[k] |= (unsigned char)(is_rec[h->fault_n2[k]] << 1);
+    const int r1 = h->fault_n1[k], r2 = h->fault_n2.empty() ? -1 : h->fault_n2[k];
+    X.fault_def1.push_back(def_of[r1]);
+    X.fault_def2.push_back(r2 < 0 ? -1 : def_of[r2]);
+    flt_of[r1] = 2 * (int)k;
+    if (r2 >= 0) flt_of[r2] = 2 * (int)k + 1;
   }
+  X.rec_int.clear();
+  X.rec_def.clear();
+  X.rec_flt.clear();
+  if (h->nrec && !h->rec_w)
+    for (int r = 0; r < h->nrec; ++r) {
+      const int ref = h->rec_ref[r];
+      const auto f = flt_of.find(ref);
+      if (f != flt_of.end()) X.rec_flt.push_back({f->second, r});
+      else if (def_of[ref] >= 0) X.rec_def.push_back({def_of[ref], r});
+      else X.rec_int.push_back({S.gmap[ref], r});
+    }
+  std::sort(X.rec_int.begin(), X.rec_int.end());
+  std::sort(X.rec_def.begin(), X.rec_def.end());
+  std::sort(X.rec_flt.begin(), X.rec_flt.end());
   // recorded nodes that are not deferred nodes: marks of the tile they lie in
   X.mark_of.assign(S.ntiles, -1);
   X.marks.clear();
   {
-    std::vector<char> is_def((size_t)h->npoin, 0);
-    for (int ref : def_ref) is_def[ref] = 1;
     const int ncx = (S.nx + TX - 1) / TX;
     for (int ref : h->rec_ref) {
-      if (is_def[ref]) continue;
+      if (def_of[ref] >= 0) continue;
       const int Xg = S.gridx[ref] % S.NX1, Zg = S.gridx[ref] / S.NX1;
       const int band = S.ezflt > 0 && Zg > 4 * S.ezflt;
       const int zl = band ? Zg - (4 * S.ezflt + 1) : Zg;
@@ -903,32 +944,20 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   X.rmdef.assign((size_t)nd * ndef, 0.0);
   for (size_t q = 0; q < ndef; ++q)
     for (int c = 0; c < nd; ++c) X.rmdef[(size_t)c * ndef + q] = h->rmass_host[(size_t)c * h->npoin + def_ref[q]];
-  // split-fault nodes for the post-fault corrector
-  X.fault_g.clear();
-  for (int k : h->fault_n1) X.fault_g.push_back(S.gmap[k]);
-  for (int k : h->fault_n2) X.fault_g.push_back(S.gmap[k]);
-  const size_t nf = X.fault_g.size();
-  X.fault_rm.assign((size_t)nd * nf, 0.0);
-  for (size_t q = 0; q < nf; ++q) {
-    const int ref = q < h->fault_n1.size() ? h->fault_n1[q] : h->fault_n2[q - h->fault_n1.size()];
-    for (int c = 0; c < nd; ++c) X.fault_rm[(size_t)c * nf + q] = h->rmass_host[(size_t)c * h->npoin + ref];
-  }
   return 0;
 }
 
 // Upload the structured tables of the solver's own grid.
-// inverse masses of the split-fault nodes in pair order: r1 (node 1) and r2 (node 2),
-// [ndof][npairs] each, from the table's fault_rm ([ndof][node 1 of every pair, then node 2])
-// (np pairs; a one-sided fault has no node 2: r2 stays zero)
-void split_fault_rm(const StructTables& X, int nd, size_t np, std::vector<double>& r1, std::vector<double>& r2) {
-  const size_t nf = X.fault_g.size();
-  r1.assign((size_t)nd * np, 0.0);
-  r2.assign((size_t)nd * np, 0.0);
-  for (int c = 0; c < nd; ++c)
-    for (size_t k = 0; k < np; ++k) {
-      r1[(size_t)c * np + k] = X.fault_rm[(size_t)c * nf + k];
-      if (nf == 2 * np) r2[(size_t)c * np + k] = X.fault_rm[(size_t)c * nf + np + k];
-    }
+// Wavefronts of a fault's pairs (FaultOut): those of member m, whose pairs start at k0 and
+// whose record places start at o0
+void fault_waves(const FaultHost& F, int m, int k0, int o0, std::vector<int4>& wave, std::vector<int2>& member,
+                 std::vector<int>& slot) {
+  const int np = F.dev.np;
+  member.push_back(make_int2((int)wave.size(), (np + 63) / 64));
+  for (int k = 0; k < np; k += 64) wave.push_back(make_int4(k0 + k, std::min(64, np - k), m, 0));
+  const size_t s0 = slot.size();
+  slot.resize(s0 + np, -1);
+  for (int o = 0; o < F.nout; ++o) slot[s0 + F.oix1 - 1 + (size_t)o * F.oixd] = o0 + o;
 }
 
 int prepare_structured(sem2d_solver* h) {
@@ -998,26 +1027,56 @@ int prepare_structured(sem2d_solver* h) {
     S.prep_allocs.push_back(q);
     S.kxd = (double*)q;
   }
-  if (h->flt.on) {  // per-pair inverse masses for the corrector inside k_fault
-    std::vector<double> r1, r2;
-    split_fault_rm(X, h->ndof, h->fault_n1.size(), r1, r2);
-    double *p1 = nullptr, *p2 = nullptr;
-    if ((rc = prep_upload(h, &p1, r1.data(), r1.size()))) return rc;
-    if ((rc = prep_upload(h, &p2, r2.data(), r2.size()))) return rc;
-    HIPCHK(h, hipStreamSynchronize(h->stream));  // the vectors are local
-    h->flt.dev.rmn1 = p1;
-    h->flt.dev.rmn2 = p2;
+  auto up = [&](const int** p, const std::vector<int>& x) {
+    int* q = nullptr;
+    const int e = prep_upload(h, &q, x.data(), x.size());
+    if (!e) hipStreamSynchronize(h->stream);  // x may be a local copy
+    *p = q;
+    return e;
+  };
+  auto up2 = [&](const int** p, const int** r, int* n, const std::vector<std::pair<int, int>>& x) {
+    std::vector<int> a, b;
+    for (auto& e : x) a.push_back(e.first), b.push_back(e.second);
+    *n = (int)x.size();
+    const int e = up(p, a);
+    return e ? e : up(r, b);
+  };
+  S.rec = RecOut{};
+  if (h->nrec && !h->rec_w) {
+    S.rec.seis = h->seis;
+    S.rec.nrec = h->nrec, S.rec.isamp = h->isamp, S.rec.nsamp = h->nsamp, S.rec.field = h->field;
+    if ((rc = up2(&S.rec.int_g, &S.rec.int_r, &S.rec.nint, X.rec_int))) return rc;
+    if ((rc = up2(&S.rec.def_q, &S.rec.def_r, &S.rec.ndefr, X.rec_def))) return rc;
+    if ((rc = up2(&S.rec.flt_q, &S.rec.flt_r, &S.rec.nfltr, X.rec_flt))) return rc;
+  }
+  if (h->flt.on) {
+    if ((rc = up(&h->flt.dev.def1, X.fault_def1))) return rc;
+    if ((rc = up(&h->flt.dev.def2, X.fault_def2))) return rc;
+    S.fo = FaultOut{};
+    const FaultHost& FH = h->flt;
+    std::vector<int4> wave;
+    std::vector<int2> member;
+    std::vector<int> slot;
+    fault_waves(FH, 0, 0, 0, wave, member, slot);
+    int4* wv = nullptr;
+    int2* mb = nullptr;
+    int* sl = nullptr;
+    if ((rc = prep_upload(h, &wv, wave.data(), wave.size()))) return rc;
+    if ((rc = prep_upload(h, &mb, member.data(), member.size()))) return rc;
+    if ((rc = prep_upload(h, &sl, slot.data(), slot.size()))) return rc;
+    S.fo.nwave = (int)wave.size(), S.fo.wave = wv, S.fo.member = mb, S.fo.slot = sl;
+    void* q = nullptr;
+    HIPCHK(h, hipMalloc(&q, (wave.size() * 6 + 1) * sizeof(double)));
+    S.prep_allocs.push_back(q);
+    S.fo.part = (double*)q;
+    S.fo.cnt = (unsigned*)(S.fo.part + wave.size() * 6);
+    HIPCHK(h, hipMemsetAsync(S.fo.cnt, 0, sizeof(double), h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));  // the tables are local
+    S.fo.nout = FH.nout, S.fo.nsamp = FH.nsamp, S.fo.rec = FH.rec;
     const size_t nside = (size_t)4 * h->ndof * h->fault_n1.size() * rsize(h);
     HIPCHK(h, hipMalloc(&h->flt.dev.side, nside));
     S.prep_allocs.push_back(h->flt.dev.side);
     HIPCHK(h, hipMemsetAsync(h->flt.dev.side, 0, nside, h->stream));
-    h->flt.dev.rmark = nullptr;
-    if (std::any_of(X.fault_rmark.begin(), X.fault_rmark.end(), [](unsigned char m) { return m != 0; })) {
-      unsigned char* pm = nullptr;
-      if ((rc = prep_upload(h, &pm, X.fault_rmark.data(), X.fault_rmark.size()))) return rc;
-      HIPCHK(h, hipStreamSynchronize(h->stream));
-      h->flt.dev.rmark = pm;
-    }
     h->flt.dev.dmask = nullptr;
     bool any = false;
     for (unsigned char m : X.fault_dmask) any |= m != 0;
@@ -1060,6 +1119,9 @@ struct StepDev {
   int ampl_nt = 0;
   bool fault_on = false;
   FaultDev F{};
+  FaultOut fo;
+  RecOut recout;
+  int* tick = nullptr;      // device step counter that the tile kernel moves on, or null
   const int* itp = nullptr;  // device step counter (graph replay) or null: step index by value
   hipStream_t stream = nullptr;
   bool pin = false;  // the state read is the predicted one (StepOut)
@@ -1112,7 +1174,8 @@ StepDev step_dev(sem2d_solver* h) {
   X.ampl = h->ampl_dev;
   X.ampl_nt = h->ampl_nt;
   X.fault_on = h->flt.on;
-  if (h->flt.on) X.F = h->flt.dev;
+  if (h->flt.on) X.F = h->flt.dev, X.fo = S.fo;
+  X.recout = S.rec;
   X.stream = h->stream;
   return X;
 }
@@ -1136,6 +1199,7 @@ void launch_tile_p(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
   A.tiles = X.T.tiles, A.grids = X.T.grids;
   A.spec_cnt = X.T.spec_cnt, A.spec_idx = X.T.spec_idx;
   A.mark_of = X.mark_of, A.marks = X.marks;
+  A.tick = X.tick;
   A.out = X.out;
   A.ntiles = n;
   A.dt = dt, A.c1 = c1, A.c2 = c2, A.c3 = c3, A.c4 = c4;
@@ -1187,26 +1251,32 @@ void launch_structured_step(const StepDev& X, int it, R dt, R c1, R c2, R c3, R 
     k_stacey_pre<R><<<(X.s_nbe * NG + 127) / 128, 128, 0, X.stream>>>(
         X.s_nbe, X.s_enode, X.s_K, (const R*)(X.din ? X.din : X.d), (const R*)(X.din && X.vin ? X.vin : X.v),
         (const R*)(X.din && X.ain ? X.ain : X.a), X.fstride, dt, c1, (double*)X.SR.kxd, X.pin);
-  auto deferred = [&](auto nd, auto oop, auto pin) {
-    k_deferred<R, decltype(nd)::value, decltype(oop)::value, decltype(pin)::value>
-        <<<(X.ndef + 255) / 256, 256, 0, X.stream>>>(
-            X.ndef, X.defs, X.part_off, (const R*)X.fpart, X.T.FPS, X.dsrc, X.ampl, X.ampl_nt, it, X.itp, X.dabso,
-            (const R*)X.rmdef, (R*)X.d, (R*)X.v, (R*)X.a, X.fstride, dt, c1, c2, c3, c4, X.out,
-            (R*)(X.rec ? X.rec : X.a), (const R*)X.din,
-            (const R*)X.vin, (const R*)X.ain, X.SR);
+  DefArgs<R> A;
+  A.ndef = X.ndef, A.defs = X.defs, A.part_off = X.part_off;
+  A.fpart = (const R*)X.fpart, A.FPS = X.T.FPS;
+  A.src = X.dsrc, A.ampl = X.ampl, A.nt = X.ampl_nt, A.it = it, A.itp = X.itp;
+  A.abso = X.dabso, A.rmdef = (const R*)X.rmdef;
+  A.d = (R*)X.d, A.v = (R*)X.v, A.a = (R*)X.a, A.GS = X.fstride;
+  A.dt = dt, A.c1 = c1, A.c2 = c2, A.c3 = c3, A.c4 = c4;
+  A.so = X.out, A.recp = (R*)(X.rec ? X.rec : X.a);
+  A.din = (const R*)X.din, A.vin = (const R*)X.vin, A.ain = (const R*)X.ain;
+  A.SR = X.SR, A.rec = X.recout;
+  A.rec.src = !X.out.final ? (const void*)A.recp : (A.rec.field == 0 ? X.d : (A.rec.field == 1 ? X.v : X.a));
+  if (X.fault_on) A.F = X.F, A.fo = X.fo;
+  const int lanes = X.ndef + A.rec.nint + (X.fault_on ? A.fo.nwave * 64 : 0);
+  auto deferred = [&](auto nd, auto oop, auto pin, auto flt) {
+    k_deferred<R, decltype(nd)::value, decltype(oop)::value, decltype(pin)::value, decltype(flt)::value>
+        <<<(lanes + 255) / 256, 256, 0, X.stream>>>(A);
   };
   using N1 = std::integral_constant<int, 1>;
   using N2 = std::integral_constant<int, 2>;
   const std::true_type yes{};
   const std::false_type no{};
-  if (X.ndof == 2 && X.din) X.pin ? deferred(N2{}, yes, yes) : deferred(N2{}, yes, no);
-  else if (X.ndof == 2) X.pin ? deferred(N2{}, no, yes) : deferred(N2{}, no, no);
-  else X.pin ? deferred(N1{}, no, yes) : deferred(N1{}, no, no);
-  if (X.fault_on) {
-    k_fault<R, true><<<grid_for(X.F.np, 64), 64, 0, X.stream>>>(X.F, (R*)X.d, (R*)X.v, (R*)X.a, X.fstride, dt, c1,
-                                                                c2, c3, c4, X.out, (R*)(X.rec ? X.rec : X.a),
-                                                                (double)it * X.F.dt);
-  }
+  if (X.ndof == 2 && X.din) X.pin ? deferred(N2{}, yes, yes, no) : deferred(N2{}, yes, no, no);  // no faults
+  else if (X.ndof == 2 && X.fault_on) X.pin ? deferred(N2{}, no, yes, yes) : deferred(N2{}, no, no, yes);
+  else if (X.ndof == 2) X.pin ? deferred(N2{}, no, yes, no) : deferred(N2{}, no, no, no);
+  else if (X.fault_on) X.pin ? deferred(N1{}, no, yes, yes) : deferred(N1{}, no, no, yes);
+  else X.pin ? deferred(N1{}, no, yes, no) : deferred(N1{}, no, no, no);
 }
 
 // Predictor / corrector coefficients of one step: dp = d + dt v + c1 a, vp = v + c2 a,
@@ -1264,11 +1334,13 @@ int do_steps(sem2d_solver* h, int nsteps) {
       // those with a progress row store d, v and a
       X.out.final = !X.w32 || s == nsteps - 1 || (h->itinfo > 0 && it % h->itinfo == 0);
       X.out.rec = !X.out.final && sampled(h, it) ? h->field : -1;
+      if (h->flt.on) fault_out_step(h, it, X.fo);
       launch_structured_step<R>(X, it, dt, c1, c2, c3, c4);
       X.pin = !X.out.final;
       h->it = it;
-      record_receivers<R>(h, !X.out.final);
-      record_fault(h, 1);
+      if (h->flt.on) fault_out_done(h, it);
+      if (h->rec_w) record_receivers<R>(h, !X.out.final);
+      else if (sampled(h, it)) h->taken = std::max(h->taken, it / h->isamp + 1);
       record_info<R>(h, it);
       continue;
     }
@@ -1316,8 +1388,8 @@ int do_steps(sem2d_solver* h, int nsteps) {
                                                              h->lsf_B, h->lsf_W1, h->lsf_W2, h->lsf_kt, h->lsf_kn,
                                                              df, a, h->npoin);
     if (h->flt.on)
-        k_fault<R><<<grid_for(h->flt.dev.np, 64), 64, 0, h->stream>>>(h->flt.dev, d, v, a, h->npoin, R(0), R(0), R(0),
-                                                                    R(0), R(0), StepOut{}, (R*)nullptr, tbc);
+        h->ndof == 2 ? (k_fault<R, 2><<<grid_for(h->flt.dev.np, 64), 64, 0, h->stream>>>(h->flt.dev, d, v, a, h->npoin, tbc))
+                   : (k_fault<R, 1><<<grid_for(h->flt.dev.np, 64), 64, 0, h->stream>>>(h->flt.dev, d, v, a, h->npoin, tbc));
     for (auto& D : h->dirs)
       if (D.after_fault)
         k_dirichlet<R><<<grid_for(D.node.size(), 128), 128, 0, h->stream>>>((int)D.node.size(), D.node_dev, D.comp,
@@ -2399,10 +2471,6 @@ __global__ void k_batch_record(const int* __restrict__ itp, int nrec, int ndof, 
   }
 }
 
-__global__ void k_tick(int* itp) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *itp = *itp + 1;
-}
-
 }  // namespace
 
 struct sem2d_batch {
@@ -2431,7 +2499,6 @@ struct sem2d_batch {
   int it = 0;
   // potency rows: pot[member][pot_cap][2*(ndof+1)]; the row of the state after step s
   // is pot_shift + s (pot_shift + 1 rows precede the batch's first step)
-  int* fbase_dev = nullptr;  // [n+1] first fault pair of each member
   double* pot = nullptr;
   int pot_cap = 0, pot_shift = 0;
   // graph of a chunk of steps
@@ -2553,6 +2620,8 @@ int batch_pot_reserve(sem2d_batch* b, int rows) {
   if (b->pot) hipFree(b->pot);
   b->pot = p;
   b->pot_cap = cap;
+  b->X.fo.pot = p;
+  b->X.fo.pot_cap = cap;
   batch_drop_graph(b);
   return 0;
 }
@@ -2617,11 +2686,8 @@ int gather_fault(sem2d_batch* b) {
   F.nr_fail = b->flags;
   b->X.fault_on = true;
   b->X.F = F;
-  // potency: member pair ranges, and the rows recorded before the batch (one per member
-  // at fault set-up; equal for all members, none of which has been stepped)
-  std::vector<int> fb(b->fault_base);
-  fb.push_back(np);
-  if ((rc = bupload(b, &b->fbase_dev, fb))) return rc;
+  // potency: the rows recorded before the batch (one per member at fault set-up; equal for
+  // all members, none of which has been stepped)
   const int r0 = b->mem[0]->flt.pot_rows;
   for (int m = 0; m < b->n; ++m)
     if (b->mem[m]->flt.pot_rows != r0) return berr(b, 3, "member %d: potency rows differ from member 0's", m);
@@ -2647,11 +2713,11 @@ int gather_fault(sem2d_batch* b) {
   return 0;
 }
 
+// the records of step 0, from the members' state
 template <typename R>
 void launch_batch_record(sem2d_batch* b) {
   const int nq = std::max(std::max(b->nrec, b->fnout), 1);
-  const bool marked = !b->X.out.final;  // StepOut::rec
-  const R* fld = (const R*)(marked || b->field == 2 ? b->X.a : (b->field == 0 ? b->X.d : b->X.v));
+  const R* fld = (const R*)(b->field == 0 ? b->X.d : (b->field == 1 ? b->X.v : b->X.a));
   k_batch_record<R><<<grid_for(nq, 64), 64, 0, b->stream>>>(b->it_dev, b->nrec, b->ndof, b->rec_node, fld,
                                                             b->fstride, b->isamp, b->nsamp, b->seis, b->X.F,
                                                             b->fidx, b->fnout, b->oit0, b->oitd, b->fnsamp,
@@ -2669,11 +2735,6 @@ void launch_batch_steps(sem2d_batch* b, int nsteps, bool pin, bool final) {
     b->X.out.final = !b->X.w32 || (final && s == nsteps - 1);
     b->X.out.rec = !b->X.out.final && b->nrec ? b->field : -1;
     launch_structured_step<R>(b->X, 0, dt, c1, c2, c3, c4);
-    if (b->X.fault_on)
-      k_batch_potency<R><<<b->n, 256, 0, b->stream>>>(b->X.F, b->fbase_dev, (const R*)b->X.d, (const R*)b->X.v,
-                                                      b->fstride, b->it_dev, b->pot_shift, b->pot_cap, b->pot);
-    launch_batch_record<R>(b);
-    k_tick<<<1, 64, 0, b->stream>>>(b->it_dev);
   }
 }
 
@@ -2784,7 +2845,7 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
   }
   // member tables, concatenated
   StructTables A;
-  std::vector<double> rmdef_c[2], frm_c[2], frm2_c[2];  // fault: inverse mass of node 1 / 2
+  std::vector<double> rmdef_c[2];
   std::vector<SrcEntry> dsrc;
   std::vector<double> ampl;
   int ampl_nt = 0, nsrc = 0;
@@ -2797,6 +2858,7 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
   b->node_base.assign(n, 0);
   b->src_base.assign(n, 0);
   size_t nb = 0, cb = 0, shared_off = 0;
+  int nrec = 0;
   for (int m = 0; m < n; ++m) {
     sem2d_solver* h = b->mem[m];
     StructTables X;
@@ -2813,7 +2875,15 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
     A.spec_cnt.insert(A.spec_cnt.end(), X.spec_cnt.begin(), X.spec_cnt.end());
     for (int r : X.mark_of) A.mark_of.push_back(r < 0 ? -1 : r + (int)(A.marks.size() / MARK_WORDS));
     A.marks.insert(A.marks.end(), X.marks.begin(), X.marks.end());
-    A.fault_rmark.insert(A.fault_rmark.end(), X.fault_rmark.begin(), X.fault_rmark.end());
+    {  // the lists of k_deferred, with the member's offsets
+      const int db = (int)A.defs.size(), rb = nrec, fb = 2 * (int)A.fault_def1.size();
+      for (int q : X.fault_def1) A.fault_def1.push_back(q + db);
+      for (int q : X.fault_def2) A.fault_def2.push_back(q < 0 ? -1 : q + db);
+      for (auto& e : X.rec_int) A.rec_int.push_back({e.first + (int)nb, e.second + rb});
+      for (auto& e : X.rec_def) A.rec_def.push_back({e.first + db, e.second + rb});
+      for (auto& e : X.rec_flt) A.rec_flt.push_back({e.first + fb, e.second + rb});
+      nrec += h->nrec;
+    }
     A.spec_idx.insert(A.spec_idx.end(), X.spec_idx.begin(), X.spec_idx.end());
     for (DefNode d : X.defs) {
       d.g += (int)nb;
@@ -2828,20 +2898,9 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
       A.dsrc.push_back(e);
     }
     A.dabso.insert(A.dabso.end(), X.dabso.begin(), X.dabso.end());
-    const size_t ndef = X.defs.size(), nf = X.fault_g.size();
-    for (int c = 0; c < nd; ++c) {
+    const size_t ndef = X.defs.size();
+    for (int c = 0; c < nd; ++c)
       rmdef_c[c].insert(rmdef_c[c].end(), X.rmdef.begin() + c * ndef, X.rmdef.begin() + (c + 1) * ndef);
-    }
-    (void)nf;
-    if (h->flt.on) {  // per-pair inverse masses, in the batch's pair order
-      std::vector<double> r1, r2;
-      split_fault_rm(X, nd, h->fault_n1.size(), r1, r2);
-      const size_t npm = r1.size() / nd;
-      for (int c = 0; c < nd; ++c) {
-        frm_c[c].insert(frm_c[c].end(), r1.begin() + c * npm, r1.begin() + (c + 1) * npm);
-        frm2_c[c].insert(frm2_c[c].end(), r2.begin() + c * npm, r2.begin() + (c + 1) * npm);
-      }
-    }
     // source amplitude rows, padded to the common length
     b->src_base[m] = nsrc;
     for (int s = 0; s < h->nsrc; ++s) {
@@ -2958,25 +3017,32 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
   const int zero4[4] = {0, 0, 0, 0};
   BHIPCHK(b, hipMemcpy(b->flags, zero4, sizeof zero4, hipMemcpyHostToDevice));
   BHIPCHK(b, hipMemcpy(b->it_dev, zero4, sizeof(int), hipMemcpyHostToDevice));
-  X.itp = b->it_dev;
+  X.itp = X.tick = b->it_dev;
   if (h0->flt.on) {
     if ((rc = gather_fault(b))) return rc;
-    std::vector<double> r1, r2;
-    for (int c = 0; c < nd; ++c) {
-      r1.insert(r1.end(), frm_c[c].begin(), frm_c[c].end());
-      r2.insert(r2.end(), frm2_c[c].begin(), frm2_c[c].end());
-    }
-    double *p1, *p2;
-    if ((rc = bupload(b, &p1, r1))) return rc;
-    if ((rc = bupload(b, &p2, r2))) return rc;
-    b->X.F.rmn1 = p1;
-    b->X.F.rmn2 = p2;
+    std::vector<int4> wave;
+    std::vector<int2> member;
+    std::vector<int> slot;
+    for (int m = 0; m < n; ++m) fault_waves(b->mem[m]->flt, m, b->fault_base[m], b->fout_base[m], wave, member, slot);
+    int *d1, *d2, *sl;
+    int4* wv;
+    int2* mb;
+    if ((rc = bupload(b, &d1, A.fault_def1))) return rc;
+    if ((rc = bupload(b, &d2, A.fault_def2))) return rc;
+    if ((rc = bupload(b, &wv, wave))) return rc;
+    if ((rc = bupload(b, &mb, member))) return rc;
+    if ((rc = bupload(b, &sl, slot))) return rc;
     char* side;
-    unsigned char* rmk;
     if ((rc = balloc(b, &side, (size_t)4 * nd * b->X.F.np * rs))) return rc;
     b->X.F.side = side;
-    if ((rc = bupload(b, &rmk, A.fault_rmark))) return rc;
-    b->X.F.rmark = rmk;
+    b->X.F.def1 = d1;
+    b->X.F.def2 = d2;
+    FaultOut& O = b->X.fo;
+    O.nwave = (int)wave.size(), O.wave = wv, O.member = mb, O.slot = sl;
+    if ((rc = balloc(b, &O.part, wave.size() * 6))) return rc;
+    if ((rc = bupload(b, &O.cnt, std::vector<unsigned>(n, 0u)))) return rc;
+    O.pot = b->pot, O.pot_cap = b->pot_cap, O.pot_row = b->pot_shift;
+    O.rec = b->frec, O.nout = b->fnout, O.oit0 = b->oit0, O.oitd = b->oitd, O.nsamp = b->fnsamp;
   }
   // receivers: members with stations, member after member
   std::vector<int> rn;
@@ -2998,12 +3064,30 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
   b->nrec = (int)rn.size();
   if ((rc = bupload(b, &b->rec_node, rn))) return rc;
   if ((rc = balloc(b, &b->seis, (size_t)std::max(b->nsamp, 1) * nd * std::max(b->nrec, 1)))) return rc;
+  if (b->nrec) {
+    RecOut& P = X.recout;
+    P.seis = b->seis, P.nrec = b->nrec, P.isamp = b->isamp, P.nsamp = b->nsamp, P.field = b->field;
+    auto up2 = [&](const int** p, const int** r, int* cnt, const std::vector<std::pair<int, int>>& x) {
+      std::vector<int> k, v;
+      for (auto& e : x) k.push_back(e.first), v.push_back(e.second);
+      *cnt = (int)x.size();
+      int *pk = nullptr, *pv = nullptr;
+      int e = bupload(b, &pk, k);
+      if (!e) e = bupload(b, &pv, v);
+      *p = pk, *r = pv;
+      return e;
+    };
+    if ((rc = up2(&P.int_g, &P.int_r, &P.nint, A.rec_int))) return rc;
+    if ((rc = up2(&P.def_q, &P.def_r, &P.ndefr, A.rec_def))) return rc;
+    if ((rc = up2(&P.flt_q, &P.flt_r, &P.nfltr, A.rec_flt))) return rc;
+  }
   // default launch configuration (sem2d_batch_tune measures the alternatives)
   batch_set_config(b, 512, tile_wgs_per_cu(b->fp32, b->ndof));
-  // records of step 0, then the counter moves to step 1
-  if (b->fp32) launch_batch_record<float>(b);
-  else launch_batch_record<double>(b);
-  k_tick<<<1, 64, 0, b->stream>>>(b->it_dev);
+  // records of step 0
+  if (b->nrec || b->X.fault_on) {
+    if (b->fp32) launch_batch_record<float>(b);
+    else launch_batch_record<double>(b);
+  }
   BHIPCHK(b, hipGetLastError());
   BHIPCHK(b, hipStreamSynchronize(b->stream));
   return 0;
@@ -3426,6 +3510,7 @@ int adj_backward(sem2d_solver* h, const double* gseis_host) {
   HIPCHK(h, hipMemsetAsync(A.mbar, 0, GS * sizeof(double), h->stream));
   HIPCHK(h, hipMemsetAsync(A.gabs, 0, (size_t)h->ndof * std::max(S.ndef, 1) * sizeof(double), h->stream));
   StepDev X = step_dev(h);
+  X.recout = RecOut{};  // the replayed steps are not recorded again
   R* inj = (R*)(h->field == 0 ? A.ad : (h->field == 1 ? A.av : A.aa));
   auto sampled = [&](int n) { return h->nrec && n >= 1 && n % h->isamp == 0 && n / h->isamp < h->nsamp; };
   auto gs_of = [&](int n) { return A.gseis + (size_t)(n / h->isamp) * h->ndof * h->nrec; };
@@ -3547,6 +3632,10 @@ int adj_forward_hist(sem2d_solver* h) {
     X.out.rec = !X.out.final && sampled(h, n) ? h->field : -1;
     launch_structured_step<R>(X, n, dt, c1, c2, c3, c4);
     h->it = n;
+    if (!h->rec_w) {
+      if (sampled(h, n)) h->taken = std::max(h->taken, n / h->isamp + 1);
+      continue;
+    }
     if (X.out.final) {
       h->d = X.d;
       h->a = X.a;

@@ -15,14 +15,14 @@
 //
 // k_deferred then finishes every perimeter / special node: it sums the partial
 // forces of the tiles that share it (fixed tile order), adds sources and absorbing
-// boundaries (in BC order) and applies the corrector; split-fault nodes are handed
-// to the fault kernel instead (predicted d, v and the assembled force written to
-// d, v, a).
+// boundaries (in BC order) and applies the corrector; the nodes of a split fault get
+// there by pairs, with the traction solve in between.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
 
+#include "sem2d_fault.hpp"
 #include "sem2d_kernels.hpp"
 
 namespace sem2d {
@@ -214,6 +214,7 @@ struct TileArgs {
   // recorded nodes inside tiles: per tile its row of marks (or -1), MARK_WORDS words each
   const int* mark_of;
   const uint32_t* marks;
+  int* tick;  // device step counter moved to this step, or null
   int ntiles;
   R dt, c1, c2, c3, c4;
   StepOut out;
@@ -283,6 +284,7 @@ k_tile_step(TileArgs<R> args) {
   const int s0 = (bid & 7) * slice;
   const int s1 = min(s0 + slice, nlist);
   const int q0 = s0 + (bid >> 3);
+  if (args.tick && bid == 0 && threadIdx.x == 0) ++*args.tick;
   if (q0 >= s1) return;
   const int tid = threadIdx.x;
   if (tid < NP) sW2[tid] = (R)c_W2[tid];
@@ -816,7 +818,7 @@ struct DefNode {
   int scnt;
   int astart;   // absorbing coefficients abso[astart .. astart+acnt), [ndof] each
   int acnt;
-  int fault;    // 1: split-fault node (finished by the fault kernels)
+  int fault;    // 1: split-fault node (finished with its pair)
   int dmask;    // Dirichlet components zeroed in the force (bit c: component c), after the
                 // absorbing terms; at a fault node, those of the Dirichlet boundaries that
                 // act before the fault
@@ -900,87 +902,111 @@ __global__ void k_stacey_pre(int nbe, const int* __restrict__ enode, const doubl
   }
 }
 
-// Corrector and stores of one node component from its predicted displacement and
-// velocity and its new acceleration ak, as in the tile kernel (StepOut; recp: where a
-// recorded node goes, else null)
-template <typename R>
-__device__ __forceinline__ void store_node(R* d, R* v, R* a, size_t i, R dp, R vp, R ak, R dt, R c1, R c2, R c3,
-                                           R c4, const StepOut& so, R* recp) {
-  const R vn = vp + c3 * ak;
-  const R dn = dp + c4 * ak;
-  if (so.final) {
-    a[i] = ak;
-    v[i] = vn;
-    d[i] = dn;
-  } else {
-    v[i] = vn + c2 * ak;
-    d[i] = dn + dt * vn + c1 * ak;
-    if (so.accel) a[i] = ak;
-    if (recp && so.rec >= 0) recp[i] = so.rec == 0 ? dn : (so.rec == 1 ? vn : ak);
+// Receivers at nodes, recorded where the nodes are finished.  seis[sample][ndof][nrec]; a
+// sample is taken at the steps isamp, 2 isamp, ... below nsamp samples.  Receivers inside
+// tiles (int_g, int_r: storage index and receiver) read the recorded field from src, which
+// the tile kernel has stored; those on deferred nodes (def_q, def_r) and on fault nodes
+// (flt_q: 2 * pair + side, flt_r) take it from the node's lane.  Each list is sorted.
+struct RecOut {
+  double* seis = nullptr;  // null: no receivers, or receivers inside elements
+  int nrec = 0, isamp = 1, nsamp = 0, field = 0;
+  int nint = 0, ndefr = 0, nfltr = 0;
+  const int *int_g = nullptr, *int_r = nullptr, *def_q = nullptr, *def_r = nullptr;
+  const int *flt_q = nullptr, *flt_r = nullptr;
+  const void* src = nullptr;  // field array of the interior receivers (bulk type)
+};
+// the sample's rows of step it, or null
+__device__ __forceinline__ double* rec_rows(const RecOut& P, int ndof, int it) {
+  if (!P.seis || it % P.isamp || it / P.isamp >= P.nsamp) return nullptr;
+  return P.seis + (size_t)(it / P.isamp) * ndof * P.nrec;
+}
+// component c of the receivers listed under key in q[0 .. n)
+__device__ __forceinline__ void rec_put(double* rows, const RecOut& P, const int* __restrict__ q,
+                                        const int* __restrict__ r, int n, int key, int c, double x) {
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    const int m = (lo + hi) >> 1;
+    if (q[m] < key) lo = m + 1;
+    else hi = m;
   }
+  for (; lo < n && q[lo] == key; ++lo) rows[(size_t)c * P.nrec + r[lo]] = x;
 }
 
-// PIN: the state read is the predicted one; so: what is stored (StepOut)
-template <typename R, int NDOF, bool OOP = false, bool PIN = false>
-__global__ __launch_bounds__(256) void k_deferred(int ndef, DefTable defs,
-                                                  const int* __restrict__ part_off, const R* __restrict__ fpart,
-                                                  size_t FPS, const SrcEntry* __restrict__ src,
-                                                  const double* __restrict__ ampl, int nt, int it_arg,
-                                                  const int* __restrict__ itp,
-                                                  const double* __restrict__ abso, const R* __restrict__ rmdef,
-                                                  R* __restrict__ d, R* __restrict__ v, R* __restrict__ a, size_t GS,
-                                                  R dt, R c1, R c2, R c3, R c4, StepOut so, R* __restrict__ recp,
-                                                  const R* __restrict__ din = nullptr,
-                                                  const R* __restrict__ vin = nullptr,
-                                                  const R* __restrict__ ain = nullptr, StaceyRefs SR = {}) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= ndef) return;
-  const DefNode n = def_unpack(defs, q);
-  const size_t g = n.g;
-  const int it = itp ? *itp : it_arg;  // step index: device counter under graph replay
+// Arguments of k_deferred
+template <typename R>
+struct DefArgs {
+  int ndef;
+  DefTable defs;
+  const int* part_off;
+  const R* fpart;
+  size_t FPS;
+  const SrcEntry* src;
+  const double* ampl;
+  int nt, it;      // amplitude table length, step index
+  const int* itp;  // step index in device memory (graph replay), or null
+  const double* abso;
+  const R* rmdef;
+  R *d, *v, *a;
+  size_t GS;
+  R dt, c1, c2, c3, c4;
+  StepOut so;
+  R* recp;  // where recorded nodes go (StepOut::rec)
+  const R *din, *vin, *ain;
+  StaceyRefs SR;
+  RecOut rec;
+  FaultDev F;
+  FaultOut fo;
+};
+
+// Predicted state of deferred node n and its force: the partial forces of its tiles, the
+// sources, the absorbing terms and the Dirichlet components
+template <typename R, int NDOF, bool OOP, bool PIN>
+__device__ __forceinline__ NodeState<R> def_state(const DefArgs<R>& A, const DefNode& n, int it) {
+  const size_t g = n.g, GS = A.GS;
   // out of place: a null vin / ain reads v / a (their step is then in place)
-  const R* __restrict__ dsrc = OOP ? din : d;
-  const R* vsrc = OOP && vin ? vin : v;
-  const R* asrc = OOP && ain ? ain : a;
-  R dp[NDOF], vpp[NDOF], f[NDOF];
+  const R* dsrc = OOP ? A.din : A.d;
+  const R* vsrc = OOP && A.vin ? A.vin : A.v;
+  const R* asrc = OOP && A.ain ? A.ain : A.a;
+  NodeState<R> s;
 #pragma unroll
   for (int c = 0; c < NDOF; ++c) {
     const R dk = dsrc[c * GS + g], vk = vsrc[c * GS + g];
     if constexpr (PIN) {
-      dp[c] = dk;
-      vpp[c] = vk;
+      s.d[c] = dk;
+      s.v[c] = vk;
     } else {
       const R ak = asrc[c * GS + g];
-      dp[c] = dk + dt * vk + c1 * ak;
-      vpp[c] = vk + c2 * ak;
+      s.d[c] = dk + A.dt * vk + A.c1 * ak;
+      s.v[c] = vk + A.c2 * ak;
     }
-    R s = 0;
+    R f = 0;
     if (n.pinl) {  // the loop below with pcnt = 2
-      s = s + fpart[c * FPS + n.poff[0]];
-      s = s + fpart[c * FPS + n.poff[1]];
+      f = f + A.fpart[c * A.FPS + n.poff[0]];
+      f = f + A.fpart[c * A.FPS + n.poff[1]];
     } else {
-      for (int k = 0; k < n.pcnt; ++k) s = s + fpart[c * FPS + part_off[n.pstart + k]];
+      for (int k = 0; k < n.pcnt; ++k) f = f + A.fpart[c * A.FPS + A.part_off[n.pstart + k]];
     }
-    f[c] = s;
+    s.f[c] = f;
   }
   for (int k = 0; k < n.scnt; ++k) {
-    const SrcEntry e = src[n.sstart + k];
-    const double am = (it >= 1 && it <= nt) ? ampl[(size_t)e.src * nt + (it - 1)] : 0.0;
+    const SrcEntry e = A.src[n.sstart + k];
+    const double am = (it >= 1 && it <= A.nt) ? A.ampl[(size_t)e.src * A.nt + (it - 1)] : 0.0;
 #pragma unroll
     for (int c = 0; c < NDOF; ++c)
-      if (c == e.comp) f[c] = (R)((double)f[c] + e.coef * am);
+      if (c == e.comp) s.f[c] = (R)((double)s.f[c] + e.coef * am);
   }
   for (int k = 0; k < n.acnt; ++k) {
 #pragma unroll
-    for (int c = 0; c < NDOF; ++c) f[c] = (R)((double)f[c] - abso[(size_t)(n.astart + k) * NDOF + c] * (double)vpp[c]);
-    if (SR.off) {  // Stacey (P-SV)
-      const int t0 = SR.off[n.astart + k], t1 = SR.off[n.astart + k + 1];
+    for (int c = 0; c < NDOF; ++c)
+      s.f[c] = (R)((double)s.f[c] - A.abso[(size_t)(n.astart + k) * NDOF + c] * (double)s.v[c]);
+    if (A.SR.off) {  // Stacey (P-SV)
+      const int t0 = A.SR.off[n.astart + k], t1 = A.SR.off[n.astart + k + 1];
       if (t1 > t0) {
 #pragma unroll
         for (int c = 0; c < NDOF; ++c) {
-          double s = 0.0;
-          for (int t = t0; t < t1; ++t) s += SR.kxd[(size_t)SR.idx[t] * 2 + c];
-          f[c] = (R)((double)f[c] - s);
+          double x = 0.0;
+          for (int t = t0; t < t1; ++t) x += A.SR.kxd[(size_t)A.SR.idx[t] * 2 + c];
+          s.f[c] = (R)((double)s.f[c] - x);
         }
       }
     }
@@ -989,20 +1015,127 @@ __global__ __launch_bounds__(256) void k_deferred(int ndef, DefTable defs,
   // boundaries act first, then the others in their order
 #pragma unroll
   for (int c = 0; c < NDOF; ++c)
-    if (n.dmask >> c & 1) f[c] = 0;
-  if (n.fault) {
+    if (n.dmask >> c & 1) s.f[c] = 0;
+  return s;
+}
+
+// Corrector of component c of a deferred node from its predicted state and its new
+// acceleration ak, and the stores, as in the tile kernel (StepOut); the displacement and
+// velocity after the step are left in s.  rec: a recorded node
+template <typename R>
+__device__ __forceinline__ void def_store(const DefArgs<R>& A, NodeState<R>& s, int c, size_t i, R ak, bool rec) {
+  const R vn = s.v[c] + A.c3 * ak;
+  const R dn = s.d[c] + A.c4 * ak;
+  s.v[c] = vn;
+  s.d[c] = dn;
+  if (A.so.final) {
+    A.a[i] = ak;
+    A.v[i] = vn;
+    A.d[i] = dn;
+  } else {
+    A.v[i] = vn + A.c2 * ak;
+    A.d[i] = dn + A.dt * vn + A.c1 * ak;
+    if (A.so.accel) A.a[i] = ak;
+    if (rec && A.so.rec >= 0) A.recp[i] = A.so.rec == 0 ? dn : (A.so.rec == 1 ? vn : ak);
+  }
+}
+template <typename R>
+__device__ __forceinline__ double rec_value(const RecOut& P, const NodeState<R>& s, int c, R ak) {
+  const R dn = s.d[c], vn = s.v[c];
+  return (double)(P.field == 0 ? dn : (P.field == 1 ? vn : ak));
+}
+
+// Everything a step does after the tile kernel, in one launch: the deferred nodes (those
+// of the tile perimeters and the sources), the receivers, and, FLT, the fault: the first
+// FLT_WG * fo.nwave lanes' wavefronts take the fault pairs, each lane both nodes of a pair
+// from their partial forces to their stores, with the pair's traction solve, its record
+// and the step's potency row; the nodes' other lanes skip them.
+// PIN: the state read is the predicted one.
+template <typename R, int NDOF, bool OOP = false, bool PIN = false, bool FLT = false>
+__global__ __launch_bounds__(256) void k_deferred(DefArgs<R> A) {
+  const int it = A.itp ? *A.itp : A.it;
+  int q = blockIdx.x * blockDim.x + threadIdx.x;
+  double* const rows = rec_rows(A.rec, NDOF, it);
+  if constexpr (FLT) {
+    const int w = q >> 6;  // uniform in a wavefront
+    if (w < A.fo.nwave) {
+      const FaultDev& F = A.F;
+      const int4 wv = A.fo.wave[w];
+      const int lane = q & 63, k = wv.x + lane;
+      const bool on = lane < wv.y;
+      double dj[2] = {0, 0}, vj[2] = {0, 0};
+      if (on) {
+        const int np = F.np;
+        const int q1 = F.def1[k], q2 = F.def2[k];
+        const bool two = q2 >= 0;
+        const DefNode m1 = def_unpack(A.defs, q1);
+        DefNode m2 = m1;
+        NodeState<R> n1 = def_state<R, NDOF, OOP, PIN>(A, m1, it), n2;
+        if (two) {
+          m2 = def_unpack(A.defs, q2);
+          n2 = def_state<R, NDOF, OOP, PIN>(A, m2, it);
+        }
+        fault_solve<R, NDOF>(F, k, (double)it * F.dt, two, n1, n2);
+        const int dm = F.dmask ? F.dmask[k] : 0;
+        R* side = (R*)F.side + k;  // [d, v][node][ndof][np]
 #pragma unroll
-    for (int c = 0; c < NDOF; ++c) {
-      d[c * GS + g] = dp[c];
-      v[c * GS + g] = vpp[c];
-      a[c * GS + g] = f[c];
+        for (int c = 0; c < NDOF; ++c) {
+          if (dm >> c & 1) n1.f[c] = 0;
+          const R a1 = n1.f[c] * A.rmdef[(size_t)c * A.ndef + q1];
+          def_store<R>(A, n1, c, (size_t)c * A.GS + m1.g, a1, m1.rec);
+          side[(size_t)c * np] = n1.d[c];
+          side[(size_t)(2 * NDOF + c) * np] = n1.v[c];
+          if (rows && m1.rec)
+            rec_put(rows, A.rec, A.rec.flt_q, A.rec.flt_r, A.rec.nfltr, 2 * k, c, rec_value<R>(A.rec, n1, c, a1));
+          if (two) {
+            if (dm >> (2 + c) & 1) n2.f[c] = 0;
+            const R a2 = n2.f[c] * A.rmdef[(size_t)c * A.ndef + q2];
+            def_store<R>(A, n2, c, (size_t)c * A.GS + m2.g, a2, m2.rec);
+            side[(size_t)(NDOF + c) * np] = n2.d[c];
+            side[(size_t)(3 * NDOF + c) * np] = n2.v[c];
+            if (rows && m2.rec)
+              rec_put(rows, A.rec, A.rec.flt_q, A.rec.flt_r, A.rec.nfltr, 2 * k + 1, c,
+                      rec_value<R>(A.rec, n2, c, a2));
+          }
+          // get_jump (SRC/bc_dynflt.f90:692-704): x2 - x1, or -2 x1 on a one-sided fault
+          dj[c] = two ? (double)n2.d[c] - (double)n1.d[c] : -2.0 * (double)n1.d[c];
+          vj[c] = two ? (double)n2.v[c] - (double)n1.v[c] : -2.0 * (double)n1.v[c];
+        }
+        const FaultOut& O = A.fo;
+        int rs = O.rec_slot;
+        if (A.itp) rs = it >= O.oit0 && (it - O.oit0) % O.oitd == 0 ? (it - O.oit0) / O.oitd : -1;
+        if (rs >= 0 && rs < O.nsamp && O.slot[k] >= 0) {
+          double* out = O.rec + (size_t)rs * 6 * O.nout + O.slot[k];
+          out[0] = F.D[k];
+          out[(size_t)1 * O.nout] = F.V[k];
+          out[(size_t)2 * O.nout] = F.T[k];
+          out[(size_t)3 * O.nout] = F.T[np + k];
+          out[(size_t)4 * O.nout] = F.MU[k];
+          out[(size_t)5 * O.nout] = F.Tstick[k];
+        }
+      }
+      potency_wave<NDOF>(F, A.fo, w, k, on, dj, vj, A.fo.pot_row + (A.itp ? it : 0));
+      return;
     }
+    q -= A.fo.nwave * 64;
+  }
+  if (q >= A.ndef) {  // receivers inside tiles
+    const int r = q - A.ndef;
+    if (rows && r < A.rec.nint)
+      for (int c = 0; c < NDOF; ++c)
+        rows[(size_t)c * A.rec.nrec + A.rec.int_r[r]] =
+            (double)((const R*)A.rec.src)[(size_t)c * A.GS + A.rec.int_g[r]];
     return;
   }
+  const DefNode n = def_unpack(A.defs, q);
+  if (FLT && n.fault) return;
+  NodeState<R> s = def_state<R, NDOF, OOP, PIN>(A, n, it);
 #pragma unroll
   for (int c = 0; c < NDOF; ++c) {
-    store_node<R>(d, v, a, c * GS + g, dp[c], vpp[c], f[c] * rmdef[(size_t)c * ndef + q], dt, c1, c2, c3, c4, so,
-                  n.rec ? recp : nullptr);
+    const R ak = s.f[c] * A.rmdef[(size_t)c * A.ndef + q];
+    def_store<R>(A, s, c, (size_t)c * A.GS + n.g, ak, n.rec);
+    if (rows && n.rec)
+      rec_put(rows, A.rec, A.rec.def_q, A.rec.def_r, A.rec.ndefr, q, c, rec_value<R>(A.rec, s, c, ak));
   }
 }
 
