@@ -103,7 +103,23 @@ __device__ __forceinline__ void load_coefs(const R* __restrict__ coefs, const R*
   }
 }
 
-// Element forces of one colour.  With Kelvin-Voigt elements (kv != nullptr, [element
+// Element forces of a time step: every element at once, its forces stored by themselves
+// (fe[c*stride + element point], coalesced) instead of assembled colour by colour; the
+// node kernel adds a node's element forces in the order of the colours.  (A step by colours
+// was 5 to 15 launches that passed over the fields: 24,120 elements 52 us, 800 elements of
+// NGLL 9 37 us; now 30 and 12.  The larger is bound by its coefficients, 48 MB a step, and
+// the fields, at 4 TB/s; the smaller by the latency of two launches.)  pin: d and v are
+// the predicted fields (StepOut); otherwise they are formed here from d, v and a.
+template <typename R>
+struct ElemStep {
+  R* fe = nullptr;  // null: assembly into f (one colour)
+  size_t stride = 0;
+  const R* a = nullptr;
+  R dt = 0, c1 = 0, c2 = 0;
+  int pin = 1;
+};
+
+// Element forces of one colour, or of all elements (E.fe).  With Kelvin-Voigt elements (kv != nullptr, [element
 // in colour order][NGLL^2]) the element displacement is d + eta v (MAT_KV_add_etav,
 // SRC/mat_kelvin_voigt.f90:139-150, applied by MAT_Fint, SRC/mat_gen.f90:435).  NGL is
 // NGLL; for NGL != 5, hg holds h'_i(x_j) at hg[i*NGL+j] (for NGL = 5 it is c_H).
@@ -114,7 +130,8 @@ __global__ __launch_bounds__(256) void k_force_colour(int e0, int ne, const int*
                                                       int npoin, const R* __restrict__ v = nullptr,
                                                       const R* __restrict__ kv = nullptr,
                                                       const R* __restrict__ beta25 = nullptr,
-                                                      const double* __restrict__ hg = nullptr) {
+                                                      const double* __restrict__ hg = nullptr,
+                                                      ElemStep<R> E = {}) {
   constexpr int NPL = NGL * NGL;
   constexpr int EPB = fe_epb(NGL);
   // ELAST_KD1_PSV: the x force's second term is a4 dUx/deta + a5 dUz/dxi
@@ -140,7 +157,16 @@ __global__ __launch_bounds__(256) void k_force_colour(int e0, int ne, const int*
   int node = 0;
   if (active) {
     node = ibool[(size_t)e * NPL + p];
-    if (kv) {
+    if (!E.pin) {
+      const R eta = kv ? kv[(size_t)e * NPL + p] : R(0);
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        const size_t i = (size_t)c * npoin + node;
+        const R vk = v[i], ak = E.a[i];
+        const R dp = d[i] + E.dt * vk + E.c1 * ak;
+        U[le][c][p] = kv ? dp + eta * (vk + E.c2 * ak) : dp;
+      }
+    } else if (kv) {
       const R eta = kv[(size_t)e * NPL + p];
 #pragma unroll
       for (int c = 0; c < NDOF; ++c) U[le][c][p] = d[(size_t)c * npoin + node] + eta * v[(size_t)c * npoin + node];
@@ -200,11 +226,15 @@ __global__ __launch_bounds__(256) void k_force_colour(int e0, int ne, const int*
         s1 += H(i, k) * T1[le][c][j * NGL + k];
         s2 += T2[le][c][k * NGL + i] * H(j, k);
       }
-      R* fp = f + (size_t)c * npoin + node;
+      R fe = s1 + s2;
       if (beta25)  // 2.5D: MAT_ELAST_add_25D_f (SRC/mat_elastic.f90:447-459)
-        *fp = *fp + ((s1 + s2) - beta25[(size_t)e * NPL + p] * U[le][c][p]);
-      else
-        *fp = *fp + (s1 + s2);
+        fe = (s1 + s2) - beta25[(size_t)e * NPL + p] * U[le][c][p];
+      if (E.fe) {
+        E.fe[(size_t)c * E.stride + (size_t)e * NPL + p] = fe;
+      } else {
+        R* fp = f + (size_t)c * npoin + node;
+        *fp = *fp + fe;
+      }
     }
   }
 }

@@ -55,6 +55,7 @@ struct AbsoHost {
   std::vector<double> C;   // [ndof][n]
   std::vector<int> senode;  // Stacey: [nbe][NG] boundary-local node of each edge point
   std::vector<double> sK;   // [nbe][NG][2]
+  std::vector<double> nrm;  // [2][n] node normals of a boundary that is not flat
 };
 
 // Structured-mesh fast path (node-grid field order, fused tile kernel)
@@ -91,10 +92,11 @@ struct StructState {
   void* fpart = nullptr;
   size_t FPS = 0;
   DefTable defs;
+  DefDev* gen_def = nullptr;  // general path: the records of defs
   int ndef = 0;
   int* part_off = nullptr;
   SrcEntry* dsrc = nullptr;
-  double* dabso = nullptr;
+  double *dabso = nullptr, *dabson = nullptr;
   void* rmdef = nullptr;
   void* rmass0 = nullptr;
   void *coefs = nullptr, *geom = nullptr;  // cell-ordered per-element arrays
@@ -365,9 +367,15 @@ int build_colours(sem2d_solver* h, const sem2d_desc* s, std::vector<int>& colour
 }
 
 template <typename R, int NDOF, int NELAST, int MODE, int NGL>
-void launch_force_t(sem2d_solver* h, const R* d, R* f, const R* v) {
+void launch_force_t(sem2d_solver* h, const R* d, R* f, const R* v, const ElemStep<R>& E) {
   const R* kv = v ? (const R*)h->kv_eta : nullptr;
   constexpr int EPB = fe_epb(NGL);
+  if (E.fe) {
+    k_force_colour<R, NDOF, NELAST, MODE, NGL><<<(h->nelem + EPB - 1) / EPB, 256, 0, h->stream>>>(
+        0, h->nelem, h->ibool, (const R*)h->coefs, (const R*)h->geom, d, f, h->npoin, v, kv, (const R*)h->beta25,
+        h->hg, E);
+    return;
+  }
   for (size_t c = 0; c + 1 < h->colour_start.size(); ++c) {
     const int e0 = h->colour_start[c], ne = h->colour_start[c + 1] - e0;
     if (ne <= 0) continue;
@@ -378,40 +386,41 @@ void launch_force_t(sem2d_solver* h, const R* d, R* f, const R* v) {
 }
 
 template <typename R, int NDOF, int NELAST, int NGL>
-void launch_force_m(sem2d_solver* h, const R* d, R* f, const R* v) {
+void launch_force_m(sem2d_solver* h, const R* d, R* f, const R* v, const ElemStep<R>& E) {
   switch (h->coef_mode) {
-    case COEF_SHARED: launch_force_t<R, NDOF, NELAST, COEF_SHARED, NGL>(h, d, f, v); break;
+    case COEF_SHARED: launch_force_t<R, NDOF, NELAST, COEF_SHARED, NGL>(h, d, f, v, E); break;
     case COEF_COMPACT:  // built for NGLL = 5 only (checked at creation)
       if constexpr ((NELAST == 2 || NELAST == 6) && NGL == NG)
-        launch_force_t<R, NDOF, NELAST, COEF_COMPACT, NGL>(h, d, f, v);
+        launch_force_t<R, NDOF, NELAST, COEF_COMPACT, NGL>(h, d, f, v, E);
       break;
-    default: launch_force_t<R, NDOF, NELAST, COEF_PER_ELEM, NGL>(h, d, f, v);
+    default: launch_force_t<R, NDOF, NELAST, COEF_PER_ELEM, NGL>(h, d, f, v, E);
   }
 }
 
 template <typename R, int NGL>
-void launch_force_n(sem2d_solver* h, const R* d, R* f, const R* v) {
+void launch_force_n(sem2d_solver* h, const R* d, R* f, const R* v, const ElemStep<R>& E) {
   if (h->ndof == 2) {
-    if (h->nelast == 6) launch_force_m<R, 2, 6, NGL>(h, d, f, v);
-    else launch_force_m<R, 2, 10, NGL>(h, d, f, v);
+    if (h->nelast == 6) launch_force_m<R, 2, 6, NGL>(h, d, f, v, E);
+    else launch_force_m<R, 2, 10, NGL>(h, d, f, v, E);
   } else {
-    if (h->nelast == 2) launch_force_m<R, 1, 2, NGL>(h, d, f, v);
-    else launch_force_m<R, 1, 3, NGL>(h, d, f, v);
+    if (h->nelast == 2) launch_force_m<R, 1, 2, NGL>(h, d, f, v, E);
+    else launch_force_m<R, 1, 3, NGL>(h, d, f, v, E);
   }
 }
 
-// f = -K d, or -K (d + eta v) in Kelvin-Voigt elements when v is given
+// f = -K d, or -K (d + eta v) in Kelvin-Voigt elements when v is given; with E.fe the
+// element forces of a step instead (ElemStep)
 template <typename R>
-void launch_force(sem2d_solver* h, const R* d, R* f, const R* v = nullptr) {
+void launch_force(sem2d_solver* h, const R* d, R* f, const R* v = nullptr, const ElemStep<R>& E = {}) {
   switch (h->ng) {
-    case 3: launch_force_n<R, 3>(h, d, f, v); break;
-    case 4: launch_force_n<R, 4>(h, d, f, v); break;
-    case 6: launch_force_n<R, 6>(h, d, f, v); break;
-    case 7: launch_force_n<R, 7>(h, d, f, v); break;
-    case 8: launch_force_n<R, 8>(h, d, f, v); break;
-    case 9: launch_force_n<R, 9>(h, d, f, v); break;
-    case 10: launch_force_n<R, 10>(h, d, f, v); break;
-    default: launch_force_n<R, NG>(h, d, f, v);
+    case 3: launch_force_n<R, 3>(h, d, f, v, E); break;
+    case 4: launch_force_n<R, 4>(h, d, f, v, E); break;
+    case 6: launch_force_n<R, 6>(h, d, f, v, E); break;
+    case 7: launch_force_n<R, 7>(h, d, f, v, E); break;
+    case 8: launch_force_n<R, 8>(h, d, f, v, E); break;
+    case 9: launch_force_n<R, 9>(h, d, f, v, E); break;
+    case 10: launch_force_n<R, 10>(h, d, f, v, E); break;
+    default: launch_force_n<R, NG>(h, d, f, v, E);
   }
 }
 
@@ -694,10 +703,10 @@ bool pack_defs(const std::vector<DefNode>& in, const std::vector<int>& part_off,
     if (n.scnt > 0 || n.acnt > 0) {
       e.x = (int)ext.size();
       ext.push_back(make_int2(n.sstart, n.astart));
-    } else if (n.pcnt == 2) {  // offsets inline
+    } else if (!part_off.empty() && (n.pcnt == 1 || n.pcnt == 2)) {  // offsets inline
       e.cnt |= 1 << 25;
       e.pstart = part_off[n.pstart];
-      e.x = part_off[n.pstart + 1];
+      e.x = n.pcnt == 2 ? part_off[n.pstart + 1] : -1;
     }
     node[q] = e;
   }
@@ -733,7 +742,7 @@ struct StructTables {
   std::vector<DefNode> defs;
   std::vector<int> part_off;
   std::vector<SrcEntry> dsrc;
-  std::vector<double> dabso;
+  std::vector<double> dabso, dabson;
   std::vector<double> rmdef;     // [ndof][ndef]
   std::vector<unsigned char> fault_dmask;  // [npairs] Dirichlet after the fault: node 1 bits 0-1, node 2 bits 2-3
   std::vector<int> s_enode, ak_off, ak_idx;  // Stacey (see StructState)
@@ -746,9 +755,92 @@ struct StructTables {
   std::vector<double> s_K;
 };
 
-int struct_tables(sem2d_solver* h, StructTables& X) {
+// Partial forces of the deferred nodes: node g[i] (storage index, ascending) adds those at
+// off[start[i] .. start[i] + cnt[i]), in this order.
+struct Partials {
+  std::vector<int> g, start, cnt, off;
+};
+
+// General path: every node adds the forces of its element points, in the order of the
+// colours.  Their list is made on the device (on the host it took 20 ns per element point,
+// as much as 400 steps of a 24,120-element mesh gain): slot[i] is the place of element point
+// i among its node's, then each node's points are put in ascending order.
+__global__ void k_gen_count(size_t n, const int* __restrict__ ibool, int* __restrict__ cnt, int* __restrict__ slot) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) slot[i] = atomicAdd(&cnt[ibool[i]], 1);
+}
+__global__ void k_gen_place(size_t n, const int* __restrict__ ibool, const int* __restrict__ start,
+                            const int* __restrict__ slot, int* __restrict__ off) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) off[start[ibool[i]] + slot[i]] = (int)i;
+}
+__global__ void k_gen_defs(int n, const int* __restrict__ start, const int* __restrict__ cnt, int* __restrict__ off,
+                           DefDev* __restrict__ def) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= n) return;
+  const int c = cnt[g];
+  int* o = off + start[g];
+  for (int i = 1; i < c; ++i) {
+    const int x = o[i];
+    int j = i;
+    for (; j > 0 && o[j - 1] > x; --j) o[j] = o[j - 1];
+    o[j] = x;
+  }
+  DefDev e{g, start[g], c, -1};
+  if (c == 1 || c == 2) {  // offsets inline
+    e.cnt |= 1 << 25;
+    e.pstart = o[0];
+    e.x = c == 2 ? o[1] : -1;
+  }
+  def[g] = e;
+}
+// the records of the nodes that have more than partial forces
+__global__ void k_gen_put(int n, const DefDev* __restrict__ src, DefDev* __restrict__ def) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < n) def[src[q].g] = src[q];
+}
+
+template <typename T>
+int prep_alloc(sem2d_solver* h, T** p, size_t n) {
+  void* q = nullptr;
+  HIPCHK(h, hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)));
+  h->st.prep_allocs.push_back(q);
+  *p = (T*)q;
+  return 0;
+}
+
+// node records and point lists on the device; start and cnt of every node on the host
+int general_partials(sem2d_solver* h, std::vector<int>& start, std::vector<int>& cnt) {
   StructState& S = h->st;
-  const int nd = h->ndof;
+  const size_t n = (size_t)h->nelem * h->np;
+  const int nb = grid_for(n, 256), nn = h->npoin;
+  if (n > (size_t)65536 * 256) return set_err(h, 5, "general path: too many element points");
+  int *dcnt, *dstart, *slot;
+  int rc;
+  if ((rc = prep_alloc(h, &dcnt, nn)) || (rc = prep_alloc(h, &dstart, nn)) || (rc = prep_alloc(h, &slot, n))) return rc;
+  if ((rc = prep_alloc(h, &S.part_off, n)) || (rc = prep_alloc(h, &S.gen_def, nn))) return rc;
+  HIPCHK(h, hipMemsetAsync(dcnt, 0, (size_t)nn * sizeof(int), h->stream));
+  k_gen_count<<<nb, 256, 0, h->stream>>>(n, h->ibool, dcnt, slot);
+  start.resize(nn);
+  cnt.resize(nn);
+  HIPCHK(h, hipMemcpyAsync(cnt.data(), dcnt, (size_t)nn * sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  int at = 0;
+  for (int g = 0; g < nn; ++g) {
+    start[g] = at;
+    at += cnt[g];
+    if (cnt[g] > 255) return set_err(h, 5, "prepare: more than 255 elements at a node");
+  }
+  HIPCHK(h, hipMemcpyAsync(dstart, start.data(), (size_t)nn * sizeof(int), hipMemcpyHostToDevice, h->stream));
+  k_gen_place<<<nb, 256, 0, h->stream>>>(n, h->ibool, dstart, slot, S.part_off);
+  k_gen_defs<<<grid_for(nn, 256), 256, 0, h->stream>>>(nn, dstart, dcnt, S.part_off, S.gen_def);
+  HIPCHK(h, hipGetLastError());
+  return 0;
+}
+
+// structured grids: the nodes of the tile perimeters and the source nodes inside tiles
+int tile_partials(sem2d_solver* h, StructTables& X, Partials& P) {
+  StructState& S = h->st;
   X.tiles = S.tiles;
   X.grids.assign(S.ntiles, make_int4(0, S.ROW, S.NZ1, 0));
   // special nodes: point-source nodes inside a tile patch
@@ -784,9 +876,36 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   std::sort(ents.begin(), ents.end(), [](const Ent& a, const Ent& b) {
     return a.g != b.g ? a.g < b.g : a.t < b.t;
   });
+  for (size_t i = 0; i < ents.size(); ++i) {
+    if (i == 0 || ents[i].g != ents[i - 1].g) {
+      P.g.push_back(ents[i].g);
+      P.start.push_back((int)i);
+      P.cnt.push_back(0);
+    }
+    ++P.cnt.back();
+    P.off.push_back(ents[i].t * SLOTS + ents[i].slot);
+  }
+  return 0;
+}
+
+// Tables of the step kernels: of a structured grid, or of the general path, where every
+// node is a deferred node and the partial forces are the element forces.
+int struct_tables(sem2d_solver* h, StructTables& X) {
+  StructState& S = h->st;
+  const int nd = h->ndof;
+  const int NG = h->ng;
+  Partials P;
+  if (S.on)
+    if (int rc = tile_partials(h, X, P)) return rc;
+  auto stored = [&](int ref) { return S.on ? S.gmap[ref] : ref; };
   // inverse map storage -> reference node, for sources / ABC / fault lookups
-  std::vector<int> ginv(S.NS, -1);
-  for (int k = 0; k < h->npoin; ++k) ginv[S.gmap[k]] = k;
+  std::vector<int> ginv(S.on ? S.NS : 0, -1);
+  if (S.on)
+    for (int k = 0; k < h->npoin; ++k) ginv[S.gmap[k]] = k;
+  std::vector<char> extra((size_t)h->npoin, 0);  // nodes with sources (1) or absorbing terms (2)
+  for (const SrcEntry& e : h->src_host) extra[e.node] |= 1;
+  for (const AbsoHost& B : h->abso_host)
+    for (int k : B.node) extra[k] |= 2;
   std::unordered_map<int, std::vector<int>> src_of;  // ref node -> src_host indices
   for (size_t q = 0; q < h->src_host.size(); ++q) src_of[h->src_host[q].node].push_back((int)q);
   std::unordered_map<int, std::vector<std::pair<int, int>>> abso_of;  // ref node -> (bc, k)
@@ -818,7 +937,7 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
     for (int e = 0; e < nbe; ++e)
       for (int k = 0; k < NG; ++k) {
         const int bn = B.senode[(size_t)e * NG + k];
-        X.s_enode.push_back(S.gmap[B.node[bn]]);
+        X.s_enode.push_back(stored(B.node[bn]));
         scon[b][bn].push_back((base + e) * NG + k);
       }
     X.s_K.insert(X.s_K.end(), B.sK.begin(), B.sK.end());
@@ -827,35 +946,46 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   X.ak_idx.clear();
   std::vector<char> is_rec((size_t)h->npoin, 0);  // recorded reference nodes
   for (int k : h->rec_ref) is_rec[k] = 1;
+  if (!S.on) {
+    // the nodes that have more than partial forces; the records of the others are made on
+    // the device
+    std::vector<int> start, cnt;
+    if (int rc = general_partials(h, start, cnt)) return rc;
+    for (int g = 0; g < h->npoin; ++g)
+      if (extra[g] || is_fault[g] || dmask_def[g] || dmask_aft[g] || is_rec[g]) {
+        P.g.push_back(g);
+        P.start.push_back(start[g]);
+        P.cnt.push_back(cnt[g]);
+      }
+  }
 
   X.defs.clear();
-  X.part_off.clear();
   X.dsrc.clear();
   X.dabso.clear();
-  std::vector<int> def_ref;
-  for (size_t i = 0; i < ents.size();) {
-    size_t j = i;
+  X.dabson.clear();
+  bool skew = false;
+  for (const AbsoHost& B : h->abso_host) skew |= !B.nrm.empty();
+  X.part_off = std::move(P.off);
+  std::vector<int> def_ref(P.g.size());
+  X.defs.reserve(P.g.size());
+  for (size_t i = 0; i < P.g.size(); ++i) {
     DefNode n{};
-    n.g = ents[i].g;
-    n.pstart = (int)X.part_off.size();
-    while (j < ents.size() && ents[j].g == n.g) {
-      X.part_off.push_back(ents[j].t * SLOTS + ents[j].slot);
-      ++j;
-    }
-    n.pcnt = (int)X.part_off.size() - n.pstart;
-    const int ref = ginv[n.g];
+    n.g = P.g[i];
+    n.pstart = P.start[i];
+    n.pcnt = P.cnt[i];
+    const int ref = S.on ? ginv[n.g] : n.g;
     n.sstart = (int)X.dsrc.size();
-    auto its = src_of.find(ref);
-    if (its != src_of.end())
-      for (int q : its->second) X.dsrc.push_back(h->src_host[q]);
+    if (extra[ref] & 1)
+      for (int q : src_of[ref]) X.dsrc.push_back(h->src_host[q]);
     n.scnt = (int)X.dsrc.size() - n.sstart;
     n.astart = (int)(X.dabso.size() / nd);
-    auto ita = abso_of.find(ref);
-    if (ita != abso_of.end())
-      for (auto& bk : ita->second) {
+    if (extra[ref] & 2)
+      for (auto& bk : abso_of[ref]) {
         const AbsoHost& B = h->abso_host[bk.first];
         const size_t nb = B.node.size();
         for (int c = 0; c < nd; ++c) X.dabso.push_back(B.C[(size_t)c * nb + bk.second]);
+        if (skew)
+          for (int c = 0; c < 2; ++c) X.dabson.push_back(B.nrm.empty() ? 0.0 : B.nrm[c * nb + bk.second]);
         if (!scon[bk.first].empty())
           for (int t : scon[bk.first][bk.second]) X.ak_idx.push_back(t);
         X.ak_off.push_back((int)X.ak_idx.size());
@@ -865,8 +995,7 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
     n.dmask = dmask_def[ref];
     n.rec = is_rec[ref];
     X.defs.push_back(n);
-    def_ref.push_back(ref);
-    i = j;
+    def_ref[i] = ref;
   }
   const size_t ndef = X.defs.size();
   {  // every Dirichlet node is a deferred node (tile perimeters hold the box's sides)
@@ -882,7 +1011,7 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
     if (!h->fault_n2.empty()) X.fault_dmask[k] |= (unsigned char)(dmask_aft[h->fault_n2[k]] << 2);
   }
   std::vector<int> def_of((size_t)h->npoin, -1);  // reference node -> deferred node
-  for (size_t q = 0; q < ndef; ++q) def_of[def_ref[q]] = (int)q;
+  for (size_t q = 0; q < ndef; ++q) def_of[def_ref[q]] = S.on ? (int)q : def_ref[q];
   X.fault_def1.clear();
   X.fault_def2.clear();
   std::unordered_map<int, int> flt_of;  // reference node -> 2 * pair + side
@@ -908,9 +1037,9 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   std::sort(X.rec_def.begin(), X.rec_def.end());
   std::sort(X.rec_flt.begin(), X.rec_flt.end());
   // recorded nodes that are not deferred nodes: marks of the tile they lie in
-  X.mark_of.assign(S.ntiles, -1);
+  X.mark_of.assign(S.on ? S.ntiles : 0, -1);
   X.marks.clear();
-  {
+  if (S.on) {
     const int ncx = (S.nx + TX - 1) / TX;
     for (int ref : h->rec_ref) {
       if (def_of[ref] >= 0) continue;
@@ -941,8 +1070,8 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
                      "must follow a row of element edges (ezflt) for the structured path",
                      nfault_def, h->fault_n1.size() + h->fault_n2.size());
   }
-  X.rmdef.assign((size_t)nd * ndef, 0.0);
-  for (size_t q = 0; q < ndef; ++q)
+  X.rmdef.assign(S.on ? (size_t)nd * ndef : 0, 0.0);  // the general path has it: rmass
+  for (size_t q = 0; S.on && q < ndef; ++q)
     for (int c = 0; c < nd; ++c) X.rmdef[(size_t)c * ndef + q] = h->rmass_host[(size_t)c * h->npoin + def_ref[q]];
   return 0;
 }
@@ -968,23 +1097,19 @@ int prepare_structured(sem2d_solver* h) {
   StructTables X;
   int rc = struct_tables(h, X);
   if (rc) return rc;
-  S.ndef = (int)X.defs.size();
-  S.def_ref.resize(S.ndef);
-  for (int q = 0; q < S.ndef; ++q) {
-    // storage index -> reference node (inverse of gmap)
-    S.def_ref[q] = X.defs[q].g;
-  }
-  {
-    std::vector<int> ginv(S.NS, -1);
+  S.ndef = S.on ? (int)X.defs.size() : h->npoin;
+  if (S.on) {
+    S.def_ref.resize(S.ndef);
+    std::vector<int> ginv(S.NS, -1);  // storage index -> reference node (inverse of gmap)
     for (int k = 0; k < h->npoin; ++k) ginv[S.gmap[k]] = k;
-    for (int q = 0; q < S.ndef; ++q) S.def_ref[q] = ginv[S.def_ref[q]];
+    for (int q = 0; q < S.ndef; ++q) S.def_ref[q] = ginv[X.defs[q].g];
+    if ((rc = prep_upload(h, &S.tiles_dev, X.tiles.data(), X.tiles.size()))) return rc;
+    if ((rc = prep_upload(h, &S.grids_dev, X.grids.data(), X.grids.size()))) return rc;
+    if ((rc = prep_upload(h, &S.spec_cnt, X.spec_cnt.data(), X.spec_cnt.size()))) return rc;
+    if ((rc = prep_upload(h, &S.spec_idx, X.spec_idx.data(), X.spec_idx.size()))) return rc;
+    if ((rc = prep_upload(h, &S.mark_of, X.mark_of.data(), X.mark_of.size()))) return rc;
+    if ((rc = prep_upload(h, &S.marks, X.marks.data(), X.marks.size()))) return rc;
   }
-  if ((rc = prep_upload(h, &S.tiles_dev, X.tiles.data(), X.tiles.size()))) return rc;
-  if ((rc = prep_upload(h, &S.grids_dev, X.grids.data(), X.grids.size()))) return rc;
-  if ((rc = prep_upload(h, &S.spec_cnt, X.spec_cnt.data(), X.spec_cnt.size()))) return rc;
-  if ((rc = prep_upload(h, &S.spec_idx, X.spec_idx.data(), X.spec_idx.size()))) return rc;
-  if ((rc = prep_upload(h, &S.mark_of, X.mark_of.data(), X.mark_of.size()))) return rc;
-  if ((rc = prep_upload(h, &S.marks, X.marks.data(), X.marks.size()))) return rc;
   {
     std::vector<DefDev> dn;
     std::vector<int2> dx;
@@ -994,16 +1119,25 @@ int prepare_structured(sem2d_solver* h) {
     int2* px = nullptr;
     if ((rc = prep_upload(h, &pn, dn.data(), dn.size()))) return rc;
     if ((rc = prep_upload(h, &px, dx.data(), dx.size()))) return rc;
+    if (!S.on && !dn.empty())
+      k_gen_put<<<grid_for(dn.size(), 256), 256, 0, h->stream>>>((int)dn.size(), pn, S.gen_def);
     HIPCHK(h, hipStreamSynchronize(h->stream));  // the packed copies are local
-    S.defs.node = pn;
+    S.defs.node = S.on ? pn : S.gen_def;
     S.defs.ext = px;
   }
-  if ((rc = prep_upload(h, &S.part_off, X.part_off.data(), X.part_off.size()))) return rc;
+  if (S.on && (rc = prep_upload(h, &S.part_off, X.part_off.data(), X.part_off.size()))) return rc;
   if ((rc = prep_upload(h, &S.dsrc, X.dsrc.data(), X.dsrc.size()))) return rc;
   if ((rc = prep_upload(h, &S.dabso, X.dabso.data(), X.dabso.size()))) return rc;
-  if ((rc = prep_upload_bulk(h, &S.rmdef, X.rmdef))) return rc;
-  S.FPS = (size_t)S.ntiles * SLOTS;
-  {
+  S.dabson = nullptr;
+  if (!X.dabson.empty() && (rc = prep_upload(h, &S.dabson, X.dabson.data(), X.dabson.size()))) return rc;
+  if (S.on) {
+    if ((rc = prep_upload_bulk(h, &S.rmdef, X.rmdef))) return rc;
+  } else {
+    S.rmdef = h->rmass;
+  }
+  S.FPS = S.on ? (size_t)S.ntiles * SLOTS : (size_t)h->nelem * h->np;
+  S.w32 = true;
+  if (S.on) {
     // per-cell arrays: the element coefficients and the element-point terms (if any)
     size_t ncell = h->coef_mode == COEF_SHARED ? (size_t)h->nelast * NP
                                                : (size_t)h->nelem * std::max(h->ndof, h->nelast) * NP;
@@ -1016,7 +1150,7 @@ int prepare_structured(sem2d_solver* h) {
   HIPCHK(h, hipMalloc(&fp, std::max<size_t>(S.FPS * h->ndof, 1) * rsize(h)));
   S.prep_allocs.push_back(fp);
   S.fpart = fp;
-  S.s_nbe = (int)(X.s_enode.size() / NG);
+  S.s_nbe = (int)(X.s_enode.size() / h->ng);
   if (S.s_nbe > 0) {
     if ((rc = prep_upload(h, &S.s_enode, X.s_enode.data(), X.s_enode.size()))) return rc;
     if ((rc = prep_upload(h, &S.s_K, X.s_K.data(), X.s_K.size()))) return rc;
@@ -1113,7 +1247,9 @@ struct StepDev {
   DefTable defs;
   const int* part_off = nullptr;
   const SrcEntry* dsrc = nullptr;
-  const double* dabso = nullptr;
+  const double *dabso = nullptr, *dabson = nullptr;
+  int ng = NG;
+  const double* hg = nullptr;
   const void* rmdef = nullptr;
   const double* ampl = nullptr;
   int ampl_nt = 0;
@@ -1150,7 +1286,7 @@ StepDev step_dev(sem2d_solver* h) {
   X.s_nbe = S.s_nbe;
   X.s_enode = S.s_enode;
   X.s_K = S.s_K;
-  if (S.s_nbe > 0) X.SR = StaceyRefs{S.ak_off, S.ak_idx, S.kxd};
+  if (S.s_nbe > 0) X.SR = StaceyRefs{S.ak_off, S.ak_idx, S.kxd, S.on ? nullptr : S.s_K};
   X.T.spec_cnt = S.spec_cnt;
   X.T.spec_idx = S.spec_idx;
   X.mark_of = S.mark_of;
@@ -1170,6 +1306,9 @@ StepDev step_dev(sem2d_solver* h) {
   X.part_off = S.part_off;
   X.dsrc = S.dsrc;
   X.dabso = S.dabso;
+  X.dabson = S.dabson;
+  X.ng = h->ng;
+  X.hg = h->hg;
   X.rmdef = S.rmdef;
   X.ampl = h->ampl_dev;
   X.ampl_nt = h->ampl_nt;
@@ -1243,19 +1382,30 @@ void launch_tile_m(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
   }
 }
 
+// One step on the tables of a StepDev: the tiles, or (gen: the solver) the elements of the
+// general path, then everything else in k_deferred.
 template <typename R>
-void launch_structured_step(const StepDev& X, int it, R dt, R c1, R c2, R c3, R c4) {
-  if (X.ndof == 2) launch_tile_m<R, 2, 6>(X, dt, c1, c2, c3, c4);
+void launch_structured_step(const StepDev& X, int it, R dt, R c1, R c2, R c3, R c4, sem2d_solver* gen = nullptr) {
+  if (gen) {
+    ElemStep<R> E;
+    E.fe = (R*)X.fpart;
+    E.stride = X.T.FPS;
+    E.a = (const R*)X.a;
+    E.dt = dt, E.c1 = c1, E.c2 = c2;
+    E.pin = X.pin;
+    launch_force<R>(gen, (const R*)X.d, nullptr, (const R*)X.v, E);
+  } else if (X.ndof == 2) launch_tile_m<R, 2, 6>(X, dt, c1, c2, c3, c4);
   else launch_tile_m<R, 1, 2>(X, dt, c1, c2, c3, c4);
   if (X.s_nbe > 0)  // Stacey terms from the previous step's state (boundary nodes are deferred)
-    k_stacey_pre<R><<<(X.s_nbe * NG + 127) / 128, 128, 0, X.stream>>>(
-        X.s_nbe, X.s_enode, X.s_K, (const R*)(X.din ? X.din : X.d), (const R*)(X.din && X.vin ? X.vin : X.v),
-        (const R*)(X.din && X.ain ? X.ain : X.a), X.fstride, dt, c1, (double*)X.SR.kxd, X.pin);
+    k_stacey_pre<R><<<(X.s_nbe * X.ng + 127) / 128, 128, 0, X.stream>>>(
+        X.s_nbe, X.s_enode, X.SR.K ? nullptr : X.s_K, (const R*)(X.din ? X.din : X.d), (const R*)(X.din && X.vin ? X.vin : X.v),
+        (const R*)(X.din && X.ain ? X.ain : X.a), X.fstride, dt, c1, (double*)X.SR.kxd, X.pin, X.ng,
+        X.hg);
   DefArgs<R> A;
   A.ndef = X.ndef, A.defs = X.defs, A.part_off = X.part_off;
   A.fpart = (const R*)X.fpart, A.FPS = X.T.FPS;
   A.src = X.dsrc, A.ampl = X.ampl, A.nt = X.ampl_nt, A.it = it, A.itp = X.itp;
-  A.abso = X.dabso, A.rmdef = (const R*)X.rmdef;
+  A.abso = X.dabso, A.abson = X.dabson, A.rmdef = (const R*)X.rmdef;
   A.d = (R*)X.d, A.v = (R*)X.v, A.a = (R*)X.a, A.GS = X.fstride;
   A.dt = dt, A.c1 = c1, A.c2 = c2, A.c3 = c3, A.c4 = c4;
   A.so = X.out, A.recp = (R*)(X.rec ? X.rec : X.a);
@@ -1320,22 +1470,35 @@ int do_steps(sem2d_solver* h, int nsteps) {
   const StepCoefs<R> K = step_coefs<R>(h->dt, h->beta, h->gamma, h->leapfrog);
   const R dt = K.dt, c1 = K.c1, c2 = K.c2, c3 = K.c3, c4 = K.c4;
   const int gb = grid_for(n, 256);
-  if (h->st.on && !h->st.ready && (rc = prepare_structured(h))) return rc;
+  // The general path by elements and nodes (two launches a step) where its tables are there
+  // or the call is long enough to pay for them: 24,120 elements NGLL 5 with ten
+  // coefficients, 32 steps 2.2 ms against 1.7 by single launches, 64 steps 3.1 against 3.4,
+  // 1000 steps 30 against 52; 800 elements NGLL 9, 64 steps 1.1 against 1.8 ms, 1000 steps 12
+  // against 37.  Periodic boundaries, HHT-alpha, linear slip faults and incident waves keep
+  // the single launches.
+  bool tables = h->st.on || (!h->hht && !h->nper && !h->nlsf && (h->st.ready || nsteps >= 64));
+  for (auto& b : h->abso) tables = tables && !b.wxz;
+  if (tables && !h->st.on && !h->st.ready) {  // room for the element forces and the node records
+    const size_t pts = (size_t)h->nelem * h->np, need = pts * (h->ndof * rsize(h) + 8) + (size_t)h->npoin * 24;
+    size_t fr = 0, tot = 0;
+    tables = pts <= (size_t)65536 * 256 && hipMemGetInfo(&fr, &tot) == hipSuccess && need + need / 4 < fr;
+  }
+  if (tables && !h->st.ready && (rc = prepare_structured(h))) return rc;
   if (h->flt.on && (rc = potency_reserve(h, h->flt.pot_rows + nsteps))) return rc;
   if (h->itinfo > 0 && (rc = info_reserve(h, h->info_rows + (h->it + nsteps) / h->itinfo - h->it / h->itinfo)))
     return rc;
   StepDev X;
-  if (h->st.on) X = step_dev(h);
+  if (tables) X = step_dev(h);
   HIPCHK(h, hipEventRecord(h->ev0, h->stream));
   for (int s = 0; s < nsteps; ++s) {
     const int it = h->it + 1;
-    if (h->st.on) {
+    if (tables) {
       // the steps between hand the predicted state on (StepOut); the call's last step and
       // those with a progress row store d, v and a
       X.out.final = !X.w32 || s == nsteps - 1 || (h->itinfo > 0 && it % h->itinfo == 0);
       X.out.rec = !X.out.final && sampled(h, it) ? h->field : -1;
       if (h->flt.on) fault_out_step(h, it, X.fo);
-      launch_structured_step<R>(X, it, dt, c1, c2, c3, c4);
+      launch_structured_step<R>(X, it, dt, c1, c2, c3, c4, h->st.on ? nullptr : h);
       X.pin = !X.out.final;
       h->it = it;
       if (h->flt.on) fault_out_done(h, it);
@@ -1607,6 +1770,8 @@ int sem2d_set_abso_normals(sem2d_solver* h, int n, const double* nrm) {
     return set_err(h, 3, "set_abso_normals: a boundary that is not flat needs a solver on the general path");
   AbsoDev& ad = h->abso.back();
   if (!nrm || n != ad.n) return set_err(h, 3, "set_abso_normals: size differs from the boundary's");
+  h->abso_host.back().nrm.assign(nrm, nrm + (size_t)2 * n);
+  h->st.ready = false;
   return upload(h, &ad.nrm, nrm, (size_t)2 * n);
 }
 
@@ -1759,6 +1924,7 @@ int sem2d_set_receivers(sem2d_solver* h, int nrec, const int* iglob, int isamp, 
 // the fused tile kernels have neither the viscous nor the 2.5D term: a structured grid
 // with either uses the general element path, with the fields in the reference numbering
 static int use_general_path(sem2d_solver* h) {
+  h->st.ready = false;
   if (h->st.on) {
     h->st.on = false;
     h->fstride = (size_t)h->npoin;

@@ -824,7 +824,7 @@ struct DefNode {
                 // act before the fault
   int rec;      // recorded node (StepOut::rec)
   int pinl;     // device form only: 1 when the two partial offsets are poff (pcnt == 2)
-  int poff[2];
+  int poff[2];  // the second is -1 when pcnt == 1
 };
 
 // Device form of a deferred-node list: 16 bytes per node (one vector load) plus a side
@@ -832,8 +832,9 @@ struct DefNode {
 // scnt (bits 8-15), acnt (bits 16-23), fault (bit 24), "offsets inline" (bit 25), the
 // Dirichlet mask (bits 26-27) and "recorded" (bit 28); x
 // is the node's (sstart, astart) entry in ext, or -1 when it has neither.  A node with
-// two partial forces and no ext entry (a tile-edge node) holds its two partial offsets
-// in pstart and x instead (bit 25 set), so part_off is not read for it.
+// one or two partial forces and no ext entry (a tile-edge node, most nodes of the general
+// path) holds its partial offsets in pstart and x instead (bit 25 set), so part_off is not
+// read for it.
 struct alignas(16) DefDev {
   int g, pstart, cnt, x;
 };
@@ -874,6 +875,7 @@ struct StaceyRefs {
   const int* off = nullptr;
   const int* idx = nullptr;
   const double* kxd = nullptr;  // [boundary element][k][2], from k_stacey_pre
+  const double* K = nullptr;  // general path: kxd holds the derivatives, still without K
 };
 
 // Stacey term of flat P-SV absorbing boundaries (BC_ABSO_apply, SRC/bc_abso.f90:321-333)
@@ -881,24 +883,24 @@ struct StaceyRefs {
 // D_c(node[e][j]), D the predicted displacement d + dt v + c1 a.  The boundary nodes are
 // deferred nodes, which k_deferred predicts later in the step, so the prediction is formed
 // here from the state of the previous step (the same expression as in k_deferred), or is
-// the d array itself (pin: the state is the predicted one).
+// the d array itself (pin: the state is the predicted one).  K null: the sums without K.
 template <typename R>
 __global__ void k_stacey_pre(int nbe, const int* __restrict__ enode, const double* __restrict__ K,
                              const R* __restrict__ d, const R* __restrict__ v, const R* __restrict__ a, size_t GS,
-                             R dt, R c1, double* __restrict__ kxd, int pin) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;  // e * NG + k
-  if (q >= nbe * NG) return;
-  const int e = q / NG, k = q - NG * e;
+                             R dt, R c1, double* __restrict__ kxd, int pin, int ng,
+                             const double* __restrict__ hg) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;  // e * ng + k
+  if (q >= nbe * ng) return;
+  const int e = q / ng, k = q - ng * e;
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     double s = 0.0;
-#pragma unroll
-    for (int j = 0; j < NG; ++j) {
-      const size_t g = (size_t)c * GS + enode[e * NG + j];
+    for (int j = 0; j < ng; ++j) {
+      const size_t g = (size_t)c * GS + enode[e * ng + j];
       const R dp = pin ? d[g] : d[g] + dt * v[g] + c1 * a[g];
-      s += c_H[j * NG + k] * (double)dp;
+      s += hg[j * ng + k] * (double)dp;
     }
-    kxd[(size_t)q * 2 + c] = K[(size_t)q * 2 + c] * s;
+    kxd[(size_t)q * 2 + c] = K ? K[(size_t)q * 2 + c] * s : s;
   }
 }
 
@@ -944,7 +946,9 @@ struct DefArgs {
   const double* ampl;
   int nt, it;      // amplitude table length, step index
   const int* itp;  // step index in device memory (graph replay), or null
-  const double* abso;
+  const double* abso;   // [entry][NDOF]
+  const double* abson;  // [entry][2] normals of entries of boundaries that are not flat
+                        // (zero: flat), or null
   const R* rmdef;
   R *d, *v, *a;
   size_t GS;
@@ -980,9 +984,9 @@ __device__ __forceinline__ NodeState<R> def_state(const DefArgs<R>& A, const Def
       s.v[c] = vk + A.c2 * ak;
     }
     R f = 0;
-    if (n.pinl) {  // the loop below with pcnt = 2
+    if (n.pinl) {  // the loop below with pcnt = 1 or 2
       f = f + A.fpart[c * A.FPS + n.poff[0]];
-      f = f + A.fpart[c * A.FPS + n.poff[1]];
+      if (n.poff[1] >= 0) f = f + A.fpart[c * A.FPS + n.poff[1]];
     } else {
       for (int k = 0; k < n.pcnt; ++k) f = f + A.fpart[c * A.FPS + A.part_off[n.pstart + k]];
     }
@@ -996,16 +1000,36 @@ __device__ __forceinline__ NodeState<R> def_state(const DefArgs<R>& A, const Def
       if (c == e.comp) s.f[c] = (R)((double)s.f[c] + e.coef * am);
   }
   for (int k = 0; k < n.acnt; ++k) {
+    const double* C = A.abso + (size_t)(n.astart + k) * NDOF;
+    bool skew = false;
+    if constexpr (NDOF == 2) {
+      if (A.abson) {  // a boundary that is not flat (k_abso_normal)
+        const double nx = A.abson[(size_t)(n.astart + k) * 2], nz = A.abson[(size_t)(n.astart + k) * 2 + 1];
+        skew = nx != 0.0 || nz != 0.0;
+        if (skew) {
+          const double v1 = (double)s.v[0], v2 = (double)s.v[1];
+          const double dot = v1 * nx + v2 * nz;
+          const double vn1 = dot * nx, vn2 = dot * nz;
+          s.f[0] = (R)((double)s.f[0] - C[0] * vn1 - C[1] * (v1 - vn1));
+          s.f[1] = (R)((double)s.f[1] - C[0] * vn2 - C[1] * (v2 - vn2));
+        }
+      }
+    }
+    if (!skew) {
 #pragma unroll
-    for (int c = 0; c < NDOF; ++c)
-      s.f[c] = (R)((double)s.f[c] - A.abso[(size_t)(n.astart + k) * NDOF + c] * (double)s.v[c]);
+      for (int c = 0; c < NDOF; ++c) s.f[c] = (R)((double)s.f[c] - C[c] * (double)s.v[c]);
+    }
     if (A.SR.off) {  // Stacey (P-SV)
       const int t0 = A.SR.off[n.astart + k], t1 = A.SR.off[n.astart + k + 1];
       if (t1 > t0) {
 #pragma unroll
         for (int c = 0; c < NDOF; ++c) {
           double x = 0.0;
-          for (int t = t0; t < t1; ++t) x += A.SR.kxd[(size_t)A.SR.idx[t] * 2 + c];
+          for (int t = t0; t < t1; ++t) {
+            const size_t i = (size_t)A.SR.idx[t] * 2 + c;
+            if (A.SR.K) x += A.SR.K[i] * A.SR.kxd[i];
+            else x += A.SR.kxd[i];
+          }
           s.f[c] = (R)((double)s.f[c] - x);
         }
       }
@@ -1919,9 +1943,9 @@ __global__ __launch_bounds__(256) void k_adj_deferred(int ndef, DefTable defs,
     const R dk = ad[c * GS + g], vk = av[c * GS + g], ak = aa[c * GS + g];
     const R fb = (ak + c3 * vk) * rmdef[(size_t)c * ndef + q];
     R F = 0;
-    if (n.pinl) {  // the loop below with pcnt = 2
+    if (n.pinl) {  // the loop below with pcnt = 1 or 2
       F = F + fpart[c * FPS + n.poff[0]];
-      F = F + fpart[c * FPS + n.poff[1]];
+      if (n.poff[1] >= 0) F = F + fpart[c * FPS + n.poff[1]];
     } else {
       for (int k = 0; k < n.pcnt; ++k) F = F + fpart[c * FPS + part_off[n.pstart + k]];
     }
