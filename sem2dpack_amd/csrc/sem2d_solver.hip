@@ -75,8 +75,6 @@ struct StructState {
   void *eta = nullptr, *b25 = nullptr;
   int4* tiles_dev = nullptr;
   int4* grids_dev = nullptr;
-  int* tlist_dev = nullptr;  // launch list of the adjoint tile kernels: full tiles, then the rest
-  int nfull = 0;
   bool w32 = false;  // field, partial-force and per-cell arrays below 4 GiB per component
   // Stacey terms: boundary elements (storage-index edge nodes, K), per absorbing entry
   // of the deferred nodes the element points it subtracts, and their values per step
@@ -663,22 +661,6 @@ bool structured_map(sem2d_solver* h, const sem2d_desc* s) {
   return true;
 }
 
-// Launch list of the adjoint tile kernels: the full TX x TZ tiles (their constant-shape,
-// 32-bit-offset variant) first, then the others.  idx32: the field and partial-force
-// arrays are below 4 GiB per component, as that variant requires; otherwise every tile
-// goes to the general variant.
-static std::vector<int> tile_list(const std::vector<int4>& tiles, bool idx32, int& nfull) {
-  std::vector<int> list;
-  list.reserve(tiles.size());
-  auto full = [&](const int4& tg) { return idx32 && (tg.z & 0xffff) == (TX | (TZ << 8)); };
-  for (int t = 0; t < (int)tiles.size(); ++t)
-    if (full(tiles[t])) list.push_back(t);
-  nfull = (int)list.size();
-  for (int t = 0; t < (int)tiles.size(); ++t)
-    if (!full(tiles[t])) list.push_back(t);
-  return list;
-}
-
 // ngp, fps: field and partial-force component strides; ncoef: entries of the per-cell
 // coefficient array
 static bool fits32(size_t ngp, size_t fps, size_t ncoef, size_t rs) {
@@ -1143,8 +1125,6 @@ int prepare_structured(sem2d_solver* h) {
                                                : (size_t)h->nelem * std::max(h->ndof, h->nelast) * NP;
     if (S.eta || S.b25) ncell = std::max(ncell, (size_t)h->nelem * NP);
     S.w32 = fits32(h->fstride, S.FPS, ncell, rsize(h));
-    const std::vector<int> list = tile_list(X.tiles, S.w32, S.nfull);
-    if ((rc = prep_upload(h, &S.tlist_dev, list.data(), list.size()))) return rc;
   }
   void* fp = nullptr;
   HIPCHK(h, hipMalloc(&fp, std::max<size_t>(S.FPS * h->ndof, 1) * rsize(h)));
@@ -3481,7 +3461,6 @@ void sem2d_batch_destroy(sem2d_batch* b) {
 // ===========================================================================
 struct AdjState {
   int nsteps = 0, seg = 0, nck = 0;
-  int wgs = 256;  // workgroups of the adjoint tile kernel: one per CU, a multiple of 8
   // history mode: the displacement after every step (FP32 bulk: and the acceleration)
   // kept in device memory, so that the backward sweep needs no replay
   bool hist = false;
@@ -3492,13 +3471,11 @@ struct AdjState {
   int nu = 0;
   int *unode = nullptr, *uoff = nullptr, *urec = nullptr;
   double* uw = nullptr;
-  // the injection of step n-1 done by the deferred kernel of step n: per deferred node the
-  // injection node it finishes (or -1), and the injection nodes that are not deferred
-  int *udef = nullptr, *uext = nullptr;
-  int next = 0;
+  int* udef = nullptr;             // injection node of each deferred node, or -1
+  unsigned char* utile = nullptr;  // tiles with an injection node in their patch
   size_t state_bytes = 0;  // d, v, a of one state
   std::vector<char*> ck, slot;
-  char *ad = nullptr, *av = nullptr, *aa = nullptr, *rmass = nullptr;
+  char *ad = nullptr, *av = nullptr, *rmass = nullptr;  // av: the w of AdjNode
   double *glam = nullptr, *gmu = nullptr, *mbar = nullptr, *gabs = nullptr, *gseis = nullptr;
   std::vector<void*> allocs;
   double fwd_ms = 0, bwd_ms = 0;
@@ -3619,43 +3596,33 @@ inline char* st_d(sem2d_solver* h, char* s) { (void)h; return s; }
 inline char* st_v(sem2d_solver* h, char* s) { return s + (size_t)h->ndof * h->fstride * rsize(h); }
 inline char* st_a(sem2d_solver* h, char* s) { return s + 2 * (size_t)h->ndof * h->fstride * rsize(h); }
 
-// One adjoint tile step: the full tiles of the launch list with the constant-shape
-// variant (every array it addresses with 32-bit offsets below 4 GiB, the double
-// mass-sensitivity array included), the others with the general one.  FP64 fields with
-// a displacement history (the acceleration formed from d_{n-1}, d_n, d_{n+1}):
-// persistent pipelined kernels of one 512-thread workgroup per CU (their LDS allows no
-// more; 162 against 182 us per 400x400-element step).  Otherwise one 256-thread
-// workgroup per tile (stored acceleration, FP64: 139 against 156 us; FP32 fields, four
-// workgroups per CU: 91 against 114 us).
+// One adjoint tile step (dp, dn: d_{n-1}, d_{n+1} where the acceleration afw is not stored)
 template <typename R>
 void launch_adj_tile(sem2d_solver* h, const StepDev& X, const R* dfw, const R* afw, const R* dp, const R* dn,
-                     R dt, R c1, R c2, R c3, double idt2) {
+                     R dt, R c1, R c2, R c3, double idt2, const InjectPlan& inj) {
   AdjState& A = *h->adj;
   StructState& S = h->st;
-  const int nf = (h->fstride * sizeof(double) < (size_t(1) << 32)) ? S.nfull : 0;
-  const int np = S.ntiles - nf;
-  if (sizeof(R) == 4 || afw) {
-    if (nf > 0)
-      k_adj_tile<R, true><<<8 * ((nf + 7) / 8), TILE_THREADS, 0, h->stream>>>(
-          X.T, S.tlist_dev, nf, (R*)A.ad, (R*)A.av, (R*)A.aa, (const R*)A.rmass, dfw, afw, (const R*)S.coefs,
-          (const R*)S.geom, (R*)S.fpart, A.glam, A.gmu, A.mbar, dt, c1, c2, c3, dp, dn, idt2);
-    if (np > 0)
-      k_adj_tile<R, false><<<8 * ((np + 7) / 8), TILE_THREADS, 0, h->stream>>>(
-          X.T, S.tlist_dev + nf, np, (R*)A.ad, (R*)A.av, (R*)A.aa, (const R*)A.rmass, dfw, afw,
-          (const R*)S.coefs, (const R*)S.geom, (R*)S.fpart, A.glam, A.gmu, A.mbar, dt, c1, c2, c3, dp, dn, idt2);
-  } else if constexpr (sizeof(R) == 8) {
-    auto wgs = [&](int n) { return std::min(A.wgs, (n + 7) / 8 * 8); };
-    if (nf > 0)
-      k_adj_pipe<R, true><<<wgs(nf), AP_NT, 0, h->stream>>>(
-          X.T, S.tlist_dev, nf, X.T.tiles, X.T.grids, X.T.spec_cnt, (R*)A.ad, (R*)A.av, (R*)A.aa,
-          (const R*)A.rmass, dfw, afw, (const R*)S.coefs, (const R*)S.geom, (R*)S.fpart, A.glam, A.gmu, A.mbar,
-          dt, c1, c2, c3, dp, dn, idt2);
-    if (np > 0)
-      k_adj_pipe<R, false><<<wgs(np), AP_NT, 0, h->stream>>>(
-          X.T, S.tlist_dev + nf, np, X.T.tiles, X.T.grids, X.T.spec_cnt, (R*)A.ad, (R*)A.av, (R*)A.aa,
-          (const R*)A.rmass, dfw, afw, (const R*)S.coefs, (const R*)S.geom, (R*)S.fpart, A.glam, A.gmu, A.mbar,
-          dt, c1, c2, c3, dp, dn, idt2);
-  }
+  AdjArgs<R> G;
+  G.ad = (R*)A.ad, G.w = (R*)A.av;
+  G.rmass = (const R*)A.rmass, G.dfw = dfw;
+  G.x1 = afw ? afw : dp, G.x2 = afw ? nullptr : dn;
+  G.coefs = (const R*)S.coefs, G.geom = (const R*)S.geom, G.fpart = (R*)S.fpart;
+  G.glam = A.glam, G.gmu = A.gmu, G.mbar = A.mbar;
+  G.S = h->fstride, G.FPS = S.FPS;
+  G.tiles = X.T.tiles, G.grids = X.T.grids, G.spec_cnt = X.T.spec_cnt, G.spec_idx = X.T.spec_idx;
+  G.ntiles = S.ntiles;
+  G.dt = dt, G.c1 = c1, G.c2 = c2, G.c3 = c3, G.idt2 = idt2;
+  G.inj = inj;
+  // 32-bit offsets: the double mass-sensitivity array below 4 GiB too
+  const bool w32 = S.w32 && h->fstride * sizeof(double) < (size_t(1) << 32);
+  const int wgs = (S.ntiles + 7) / 8 * 8;
+  auto go = [&](auto hist, auto w) {
+    k_adj_step<R, decltype(hist)::value, decltype(w)::value><<<wgs, TS_NT, 0, h->stream>>>(G);
+  };
+  const std::true_type yes{};
+  const std::false_type no{};
+  if (afw) w32 ? go(no, yes) : go(no, no);
+  else w32 ? go(yes, yes) : go(yes, no);
 }
 
 template <typename R>
@@ -3670,40 +3637,30 @@ int adj_backward(sem2d_solver* h, const double* gseis_host) {
     HIPCHK(h, hipMemcpyAsync(A.gseis, gseis_host, ns * sizeof(double), hipMemcpyHostToDevice, h->stream));
   HIPCHK(h, hipMemsetAsync(A.ad, 0, nf * sizeof(R), h->stream));
   HIPCHK(h, hipMemsetAsync(A.av, 0, nf * sizeof(R), h->stream));
-  HIPCHK(h, hipMemsetAsync(A.aa, 0, nf * sizeof(R), h->stream));
   HIPCHK(h, hipMemsetAsync(A.glam, 0, (size_t)h->nelem * sizeof(double), h->stream));
   HIPCHK(h, hipMemsetAsync(A.gmu, 0, (size_t)h->nelem * sizeof(double), h->stream));
   HIPCHK(h, hipMemsetAsync(A.mbar, 0, GS * sizeof(double), h->stream));
   HIPCHK(h, hipMemsetAsync(A.gabs, 0, (size_t)h->ndof * std::max(S.ndef, 1) * sizeof(double), h->stream));
   StepDev X = step_dev(h);
   X.recout = RecOut{};  // the replayed steps are not recorded again
-  R* inj = (R*)(h->field == 0 ? A.ad : (h->field == 1 ? A.av : A.aa));
-  auto sampled = [&](int n) { return h->nrec && n >= 1 && n % h->isamp == 0 && n / h->isamp < h->nsamp; };
-  auto gs_of = [&](int n) { return A.gseis + (size_t)(n / h->isamp) * h->ndof * h->nrec; };
-  // the deferred kernel of step n also adds the sample of step n-1 (after its own
-  // updates, before the tile kernel of step n-1 reads the field); the first step's
-  // sample gets its own launch
+  // the sample of step n, added to the state the step starts from
   auto plan_for = [&](int n) {
     InjectPlan P;
-    if (!sampled(n - 1)) return P;
+    if (!(h->nrec && n >= 1 && sampled(h, n))) return P;
     P.nu = A.nu;
     P.nrec = h->nrec;
+    P.field = h->field;
     P.unode = A.unode;
     P.off = A.uoff;
     P.rec = A.urec;
     P.w = A.uw;
-    P.g = gs_of(n - 1);
-    P.fld = inj;
+    P.g = A.gseis + (size_t)(n / h->isamp) * h->ndof * h->nrec;
     P.udef = A.udef;
-    P.uext = A.uext;
-    P.next = A.next;
+    P.tile = A.utile;
     return P;
   };
-  auto deferred_grid = [&](const InjectPlan& P) { return (S.ndef + (P.g ? P.next : 0) + 255) / 256; };
+  const int gd = (S.ndef + 255) / 256;
   HIPCHK(h, hipEventRecord(h->ev0, h->stream));
-  if (sampled(A.nsteps))
-    k_adj_inject<R><<<grid_for(A.nu, 64), 64, 0, h->stream>>>(A.nu, A.unode, A.uoff, A.urec, A.uw, h->nrec,
-                                                             gs_of(A.nsteps), inj, GS);
   if (A.hist) {
     // no replay: the forward displacements are all in memory
     const size_t nfb = nf * sizeof(R);
@@ -3714,11 +3671,11 @@ int adj_backward(sem2d_solver* h, const double* gseis_host) {
       const R* dp = (const R*)(A.H + (size_t)(n - 1) * nfb);
       const R* dn = n < N ? (const R*)(A.H + (size_t)(n + 1) * nfb) : nullptr;
       const R* af = A.AH ? (const R*)(A.AH + (size_t)n * nfb) : (n == N ? (const R*)A.aN : nullptr);
-      launch_adj_tile<R>(h, X, dc, af, dp, dn, dt, c1, c2, c3, idt2);
       const InjectPlan P = plan_for(n);
-      k_adj_deferred<R><<<deferred_grid(P), 256, 0, h->stream>>>(
+      launch_adj_tile<R>(h, X, dc, af, dp, dn, dt, c1, c2, c3, idt2, P);
+      k_adj_deferred<R><<<gd, 256, 0, h->stream>>>(
           S.ndef, S.defs, S.part_off, (const R*)S.fpart, S.FPS, S.dabso, (const R*)S.rmdef, (R*)A.ad, (R*)A.av,
-          (R*)A.aa, GS, af, nullptr, nullptr, A.mbar, A.gabs, dt, c1, c2, c3, dc, dp, dn, idt, idt2, P);
+          GS, af, nullptr, nullptr, A.mbar, A.gabs, dt, c1, c2, c3, dc, dp, dn, idt, idt2, P);
     }
   }
   for (int k = A.hist ? -1 : A.nck - 1; k >= 0; --k) {
@@ -3744,11 +3701,11 @@ int adj_backward(sem2d_solver* h, const double* gseis_host) {
       const int j = n - s0;
       const R* dfw = (const R*)st_d(h, A.slot[j]);
       const R* afw = (const R*)st_a(h, A.slot[j]);
-      launch_adj_tile<R>(h, X, dfw, afw, nullptr, nullptr, dt, c1, c2, c3, 0.0);
-      const InjectPlan P = plan_for(n);  // the sample of step n-1 (the replay leaves the adjoint alone)
-      k_adj_deferred<R><<<deferred_grid(P), 256, 0, h->stream>>>(
+      const InjectPlan P = plan_for(n);
+      launch_adj_tile<R>(h, X, dfw, afw, nullptr, nullptr, dt, c1, c2, c3, 0.0, P);
+      k_adj_deferred<R><<<gd, 256, 0, h->stream>>>(
           S.ndef, S.defs, S.part_off, (const R*)S.fpart, S.FPS, S.dabso, (const R*)S.rmdef, (R*)A.ad, (R*)A.av,
-          (R*)A.aa, GS, afw, (const R*)st_v(h, A.slot[j - 1]), (const R*)st_a(h, A.slot[j - 1]), A.mbar, A.gabs,
+          GS, afw, (const R*)st_v(h, A.slot[j - 1]), (const R*)st_a(h, A.slot[j - 1]), A.mbar, A.gabs,
           dt, c1, c2, c3, nullptr, nullptr, nullptr, 0.0, 0.0, P);
     }
   }
@@ -3847,11 +3804,6 @@ int sem2d_adjoint_init(sem2d_solver* h, int nsteps, int seg) {
   if (h->flt.pot) hipFree(h->flt.pot);
   h->adj = new AdjState();
   AdjState& A = *h->adj;
-  {
-    int dev = 0, ncu = 256;
-    if (hipGetDevice(&dev) == hipSuccess) hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    A.wgs = std::max(8, (ncu + 7) / 8 * 8);
-  }
   A.nsteps = nsteps;
   A.seg = std::min(seg, nsteps);
   A.nck = (nsteps + A.seg - 1) / A.seg;
@@ -3898,8 +3850,6 @@ int sem2d_adjoint_init(sem2d_solver* h, int nsteps, int seg) {
   A.ad = (char*)p;
   if ((rc = adj_alloc(h, &p, nf))) return rc;
   A.av = (char*)p;
-  if ((rc = adj_alloc(h, &p, nf))) return rc;
-  A.aa = (char*)p;
   if ((rc = adj_alloc(h, &p, (size_t)h->nelem * sizeof(double)))) return rc;
   A.glam = (double*)p;
   if ((rc = adj_alloc(h, &p, (size_t)h->nelem * sizeof(double)))) return rc;
@@ -3947,29 +3897,28 @@ int sem2d_adjoint_init(sem2d_solver* h, int nsteps, int seg) {
     HIPCHK(h, hipMemcpy(A.urec, rec.data(), rec.size() * sizeof(int), hipMemcpyHostToDevice));
     HIPCHK(h, hipMemcpy(A.uw, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
     // injection nodes that are deferred nodes (storage index of deferred node q:
-    // gmap[def_ref[q]]) are finished by that deferred lane, the others by extra lanes
+    // gmap[def_ref[q]]), and the tiles with an injection node in their patch
     const StructState& S = h->st;
     std::unordered_map<int, int> u_at;  // injection node -> u (a few entries)
     for (int u = 0; u < (int)un.size(); ++u) u_at[un[u]] = u;
-    std::vector<int> udef(std::max(S.ndef, 1), -1), uext;
-    std::vector<char> taken(un.size(), 0);
+    std::vector<int> udef(std::max(S.ndef, 1), -1);
     for (int q = 0; q < S.ndef; ++q) {
       auto it = u_at.find(S.gmap[S.def_ref[q]]);
-      if (it != u_at.end()) {
-        udef[q] = it->second;
-        taken[it->second] = 1;
-      }
+      if (it != u_at.end()) udef[q] = it->second;
     }
-    for (int u = 0; u < (int)un.size(); ++u)
-      if (!taken[u]) uext.push_back(u);
-    A.next = (int)uext.size();
+    std::vector<unsigned char> utile(S.ntiles, 0);
+    const int ncx = (S.nx + TX - 1) / TX, ncz = (S.nz + TZ - 1) / TZ;
+    for (int ref : h->rec_ref) {
+      const int Xg = S.gridx[ref] % S.NX1, Zg = S.gridx[ref] / S.NX1, W = 4 * TX;
+      for (int tz = (Zg > 0 ? (Zg - 1) / W : 0); tz <= Zg / W && tz < ncz; ++tz)
+        for (int tx = (Xg > 0 ? (Xg - 1) / W : 0); tx <= Xg / W && tx < ncx; ++tx) utile[(size_t)tz * ncx + tx] = 1;
+    }
     if ((rc = adj_alloc(h, &q, udef.size() * sizeof(int)))) return rc;
     A.udef = (int*)q;
-    if ((rc = adj_alloc(h, &q, std::max<size_t>(uext.size(), 1) * sizeof(int)))) return rc;
-    A.uext = (int*)q;
+    if ((rc = adj_alloc(h, &q, utile.size()))) return rc;
+    A.utile = (unsigned char*)q;
     HIPCHK(h, hipMemcpy(A.udef, udef.data(), udef.size() * sizeof(int), hipMemcpyHostToDevice));
-    if (!uext.empty())
-      HIPCHK(h, hipMemcpy(A.uext, uext.data(), uext.size() * sizeof(int), hipMemcpyHostToDevice));
+    HIPCHK(h, hipMemcpy(A.utile, utile.data(), utile.size(), hipMemcpyHostToDevice));
   }
   // inverse mass of both components in storage order.  The tile kernels' single-
   // component array holds it at every node whose components are equal; the deferred

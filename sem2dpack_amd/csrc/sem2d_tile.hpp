@@ -30,8 +30,6 @@ namespace sem2d {
 constexpr int TX = 8, TZ = 8;
 constexpr int PXM = 4 * TX + 1, PZM = 4 * TZ + 1;
 constexpr int PMAX = PXM * PZM;
-constexpr int TILE_THREADS = 256;  // adjoint tile kernel
-constexpr int NODE_ITERS = (PMAX + TILE_THREADS - 1) / TILE_THREADS;
 constexpr int PERIM_MAX = 2 * PXM + 2 * (PZM - 2);
 constexpr int MAXSPECIAL = 16;
 constexpr int SLOTS = PERIM_MAX + MAXSPECIAL;
@@ -125,21 +123,32 @@ __device__ __forceinline__ T* sgpr_base(T* p) {
   return (T*)g;
 }
 
-// node_index for a full tile (PX = 4*TX+1, right edge on line kL+1), in 32 bits and
-// branch-free (both forms computed, one selected)
-__device__ __forceinline__ uint32_t node_index_full(const int4 gr, int X, int Z, int X0, int Z0, int kL) {
-  const uint32_t edge = (uint32_t)gr.x + (uint32_t)gr.y * (uint32_t)gr.z + (uint32_t)(Z0 + Z) +
-                        (uint32_t)(X == 0 ? kL : kL + 1) * (uint32_t)gr.z;
-  const uint32_t inner = (uint32_t)gr.x + (uint32_t)(Z0 + Z) * (uint32_t)gr.y + (uint32_t)(X0 + X - 1);
-  return (X == 0 || X == 4 * TX) ? edge : inner;
-}
-
 // Order of LDS accesses among the lanes of one wavefront (which the hardware executes in
 // program order): no access moves across it.
 __device__ __forceinline__ void wave_order() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Exchange slots of the forces of the elements at patch node (X, Z) (slot = element * NP +
+// point, elements row by row of a full tile; the slot after the last stands for an element
+// outside the patch)
+__device__ __forceinline__ ushort4 node_slots(int X, int Z) {
+  constexpr int NEL = TX * TZ;
+      // Of the two element columns (rows) that share a node the even one comes first,
+      // rows before columns: the order of the colours.
+      unsigned short sl[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int cx = q & 1, cz = q >> 1;
+        const int lx = ((X >> 2) & 1) == cx ? X >> 2 : (X >> 2) - 1;
+        const int lz = ((Z >> 2) & 1) == cz ? Z >> 2 : (Z >> 2) - 1;
+        const bool ok = lx >= 0 && lx < TX && (lx == X >> 2 || (X & 3) == 0) && lz >= 0 && lz < TZ &&
+                        (lz == Z >> 2 || (Z & 3) == 0);
+        sl[q] = (unsigned short)(ok ? (lz * TX + lx) * NP + (Z - 4 * lz) * NG + (X - 4 * lx) : NEL * NP);
+      }
+  return make_ushort4(sl[0], sl[1], sl[2], sl[3]);
 }
 
 // Persistent tile kernel.  Each workgroup walks a strided sequence of tiles inside its
@@ -295,19 +304,7 @@ k_tile_step(TileArgs<R> args) {
   for (int r = 0; r < TS_ITER; ++r) {
     const int p = tid + TS_NT * r, Z = p / PS, X = p - Z * PS;
     xz[r] = X | Z << 8;
-    // Of the two element columns (rows) that share a node the even one comes first,
-    // rows before columns: the order of the colours.
-    unsigned short sl[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int cx = q & 1, cz = q >> 1;
-      const int lx = ((X >> 2) & 1) == cx ? X >> 2 : (X >> 2) - 1;
-      const int lz = ((Z >> 2) & 1) == cz ? Z >> 2 : (Z >> 2) - 1;
-      const bool ok = lx >= 0 && lx < TX && (lx == X >> 2 || (X & 3) == 0) && lz >= 0 && lz < TZ &&
-                      (lz == Z >> 2 || (Z & 3) == 0);
-      sl[q] = (unsigned short)(ok ? (lz * TX + lx) * NP + (Z - 4 * lz) * NG + (X - 4 * lx) : NEL * NP);
-    }
-    if (p < PMAX) Eg[p] = make_ushort4(sl[0], sl[1], sl[2], sl[3]);
+    if (p < PMAX) Eg[p] = node_slots(X, Z);
   }
   struct Geo {
     int tx0, tz0, nxe, nze, Z0, PX, PZ, X0, kL, kR;
@@ -1199,301 +1196,419 @@ __device__ __forceinline__ double fwd_accel(const R* __restrict__ a, const R* __
   return (((double)dnext[i] - dc) - (dc - (double)dprev[i])) * idt2;
 }
 
-template <typename R, bool FULL = false>
-__global__ __launch_bounds__(TILE_THREADS) void k_adj_tile(
-    TileDev T, const int* __restrict__ tlist, int nlist, R* __restrict__ ad, R* __restrict__ av,
-    R* __restrict__ aa, const R* __restrict__ rmass,
-    const R* __restrict__ dfw, const R* __restrict__ afw, const R* __restrict__ coefs, const R* __restrict__ geom,
-    R* __restrict__ fpart, double* __restrict__ glam, double* __restrict__ gmu, double* __restrict__ mbar,
-    R dt, R c1, R c2, R c3, const R* __restrict__ dprev = nullptr, const R* __restrict__ dnext = nullptr,
-    double idt2 = 0.0) {
-  constexpr int NDOF = 2;
-  using LV = typename LVec<R, NDOF>::T;  // both components of a node side by side
+// Injection of dJ/d(recorded field): the sample of step n is added to the adjoint state
+// that step n starts from, at the injection nodes unode[0 .. nu) (ascending storage
+// indices), node u with the contributions (receiver rec[k], weight w[k], k in [off[u],
+// off[u+1])) in receiver order.
+struct InjectPlan {
+  int nu = 0, nrec = 0, field = 1;
+  const int *unode = nullptr, *off = nullptr, *rec = nullptr;
+  const double* w = nullptr;
+  const double* g = nullptr;  // the sample, [ndof][nrec]; null: no injection
+  const int* udef = nullptr;  // injection node of deferred node q, or -1
+  const unsigned char* tile = nullptr;  // tiles with an injection node in their patch
+};
+template <typename R>
+__device__ __forceinline__ R inject_at(const InjectPlan& P, int u, int c, R x) {
+  for (int k = P.off[u]; k < P.off[u + 1]; ++k) x = (R)((double)x + P.w[k] * P.g[(size_t)c * P.nrec + P.rec[k]]);
+  return x;
+}
+__device__ __forceinline__ int inject_find(const InjectPlan& P, int node) {
+  int lo = 0, hi = P.nu;
+  while (lo < hi) {
+    const int m = (lo + hi) >> 1;
+    if (P.unode[m] < node) lo = m + 1;
+    else hi = m;
+  }
+  return lo < P.nu && P.unode[lo] == node ? lo : -1;
+}
+
+// The adjoint state is kept as the pair (ad, w) that the last update formed it from,
+// av = w + dt ad and aa = c2 w + c1 ad; the injected values come on top where the state is
+// read.  (Two field arrays each way instead of three.)
+template <typename R>
+struct AdjNode {
+  R d, v, a;
+};
+template <typename R>
+__device__ __forceinline__ AdjNode<R> adj_node(R dn, R w, R dt, R c1, R c2) {
+  return {dn, w + dt * dn, c2 * w + c1 * dn};
+}
+
+template <typename R>
+struct AdjArgs {
+  R *ad, *w;
+  const R *rmass, *dfw, *x1, *x2;  // x1, x2: forward acceleration and null, or d_{n-1} and d_{n+1}
+  const R *coefs, *geom;
+  R* fpart;
+  double *glam, *gmu, *mbar;
+  size_t S, FPS;
+  const int4 *tiles, *grids;
+  const int *spec_cnt, *spec_idx;
+  int ntiles;
+  R dt, c1, c2, c3;
+  double idt2;
+  InjectPlan inj;
+};
+
+// Adjoint tile step, one tile per workgroup, with the element phase of k_tile_step (a lane
+// per element row or column, exchanges inside a wavefront): the gradient of the forward
+// displacement first, kept for the row's five points in registers, then that of fb, the
+// transposed fluxes and the sensitivities, whose sums over an element are the rows' sums
+// added in row order.  HIST: the forward acceleration is the second difference of the
+// displacement history (fwd_accel).  The adjoint state of the interior nodes is read again
+// for the stores (a register each through the element phase would halve the wavefronts).
+template <typename R, bool HIST, bool W32>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_step(AdjArgs<R> args) {
+  constexpr int NDOF = 2, PS = PXM, NEL = TX * TZ;
+  using LV = typename LVec<R, NDOF>::T;
   __shared__ LV Uf[PMAX];  // fb
   __shared__ LV Ud[PMAX];  // forward d_n
-  __shared__ LV Fn[PMAX];
-  __shared__ LV T1[FE_EPB][NP];
-  __shared__ LV T2[FE_EPB][NP];
-  __shared__ double Gr[FE_EPB][NP][2];
-  __shared__ double Gs[FE_EPB][NG][2];  // row sums of Gr
-  __shared__ double Ge[TX * TZ][2];     // dJ/dlambda, dJ/dmu of the tile's elements, accumulated
-  __shared__ R Gm[TX * TZ][3];          // geometric factors of the tile's elements
-  __shared__ short sflag[PMAX];
-
-  // workgroup -> listed tile: each XCD (bid & 7) takes a contiguous eighth of the list
-  const int bid = blockIdx.x;
-  const int per = (nlist + 7) >> 3;
-  const int qt = (bid & 7) * per + (bid >> 3);
-  if (qt >= nlist) return;
-  const int t = tlist[qt];
+  __shared__ LV Ex[NEL * NP + 1];
+  __shared__ ushort4 Eg[PMAX];
+  __shared__ R Gm[NEL][3];
+  __shared__ R sW2[NP];
+  // each XCD (bid & 7) takes a contiguous eighth of the tiles
+  const int per = (args.ntiles + 7) >> 3, bid = blockIdx.x;
+  const int t = (bid & 7) * per + (bid >> 3);
+  if ((bid >> 3) >= per || t >= args.ntiles) return;
   const int tid = threadIdx.x;
-  const int4 tg = T.tiles[t];
-  const int4 gr = T.grids[t];
-  const int tx0 = tg.x, tz0 = tg.y, Z0 = tg.w;
-  const int nxe = FULL ? TX : (tg.z & 0xff), nze = FULL ? TZ : ((tg.z >> 8) & 0xff);
-  const int PX = 4 * nxe + 1, PZ = 4 * nze + 1, NPT = PX * PZ;
-  const int X0 = 4 * tx0;
-  const size_t S = T.NGp;
-  const int kL = tx0 / TX, kR = FULL ? kL + 1 : (tx0 + nxe + TX - 1) / TX;
-  // full tiles: compile-time shapes, 32-bit offsets from per-component bases held in
-  // scalar registers (every array below 4 GiB, checked by the caller)
+  if (tid < NP) sW2[tid] = (R)c_W2[tid];
+  if (tid == 0) Ex[NEL * NP] = LV{};
+  const auto* P = kernel_args<AdjArgs<R>>();
+  const int4 tg = sload(P->tiles, t), gr = sload(P->grids, t);
+  const int nxe = tg.z & 0xff, nze = (tg.z >> 8) & 0xff, nx = tg.z >> 16;
+  const int PX = 4 * nxe + 1, PZ = 4 * nze + 1, X0 = 4 * tg.x, Z0 = tg.w;
+  const int kL = tg.x / TX, kR = (tg.x + nxe + TX - 1) / TX;
+  using I = std::conditional_t<W32, uint32_t, size_t>;
   auto nidx = [&](int X, int Z) {
-    if constexpr (FULL) return node_index_full(gr, X, Z, X0, Z0, kL);
-    else return node_index(gr, X, Z, PX, X0, Z0, kL, kR);
+    const I row = (I)gr.x + (I)Z0 * (I)gr.y + (I)(X0 - 1);
+    const I edge = (I)gr.x + (I)gr.y * (I)gr.z + (I)Z0;
+    const I eL = edge + (I)kL * (I)gr.z, eR = edge + (I)kR * (I)gr.z;
+    const I in = row + (I)((uint32_t)Z * (uint32_t)gr.y + (uint32_t)X);
+    return X == 0 || X == PX - 1 ? (X == 0 ? eL : eR) + (I)Z : in;
   };
-  auto cidx = [&](int lx, int lz) {
-    if constexpr (FULL)
-      return (uint32_t)gr.w + (uint32_t)(tz0 + lz) * (uint32_t)(tg.z >> 16) + (uint32_t)(tx0 + lx);
-    else return cell_index(gr, tg.z >> 16, tx0, tz0, lx, lz);
-  };
+  auto cidx = [&](int lx, int lz) { return (I)gr.w + (I)(tg.y + lz) * (I)nx + (I)(tg.x + lx); };
   auto ub = [&](auto* p) {
-    if constexpr (FULL) return sgpr_base(p);
+    if constexpr (W32) return sgpr_base(p);
     else return p;
   };
   auto at = [&](auto* base, auto g) -> auto& {
-    if constexpr (FULL) return at32(base, (uint32_t)g);
+    if constexpr (W32) return at32(base, (uint32_t)g);
     else return base[g];
   };
-  R *bad[NDOF], *bav[NDOF], *baa[NDOF], *bfp[NDOF];
-  const R *brm[NDOF], *bdf[NDOF], *baf[NDOF], *bdp[NDOF], *bdn[NDOF];
-#pragma unroll
-  for (int c = 0; c < NDOF; ++c) {
-    bad[c] = ub(ad + c * S);
-    bav[c] = ub(av + c * S);
-    baa[c] = ub(aa + c * S);
-    brm[c] = ub(rmass + c * S);
-    bdf[c] = ub(dfw + c * S);
-    baf[c] = afw ? ub(afw + c * S) : nullptr;
-    bdp[c] = dprev ? ub(dprev + c * S) : nullptr;
-    bdn[c] = dnext ? ub(dnext + c * S) : nullptr;
-    bfp[c] = ub(fpart + c * T.FPS);
-  }
-  double* bmb = ub(mbar);
-  double* bgl = ub(glam);
-  double* bgm = ub(gmu);
-  const R* bco = ub(coefs);
-  const R* bge = ub(geom);
-  // forward acceleration at node g (as fwd_accel)
-  auto accel = [&](int c, auto g, R dcur) -> double {
-    if (afw) return (double)at(baf[c], g);
-    const double dc = (double)dcur;
-    return (((double)at(bdn[c], g) - dc) - (dc - (double)at(bdp[c], g))) * idt2;
+  const size_t S = P->S;
+  // lane index the compiler cannot look through (as in k_tile_step)
+  auto lane_id = [&]() {
+    int q = tid;
+    asm volatile("" : "+v"(q));
+    __builtin_assume(q >= 0 && q < TS_NT);
+    return q;
   };
-  const int le = tid / NP;
-  const int pe = tid - le * NP;
-  const int ii = pe % NG, jj = pe / NG;
-  // the H entries and GLL weight of this lane's element point
-  const R w = (R)c_W2[pe];
-  R hA[NG], hB[NG], hC[NG], hD[NG];
+  const int ns = sload(P->spec_cnt, t);
+  auto special = [&](int p) {
+    int k = -1;
+    for (int q = 0; q < ns; ++q)
+      if (sload(P->spec_idx, t * MAXSPECIAL + q) == p) k = q;
+    return k;
+  };
+  const bool inj = P->inj.g && P->inj.tile[t];
+  const int field = P->inj.field;
+  const R dt = P->dt, c1 = P->c1, c2 = P->c2, c3 = P->c3;
+  // adds the injected values of node g to the arrays f of its components
+  auto inject = [&](I g, auto&&... f) {
+    const InjectPlan J = args.inj;
+    const int u = inject_find(J, (int)g);
+    if (u >= 0) {
+      int c = 0;
+      ((f = inject_at<R>(J, u, c++, f)), ...);
+    }
+  };
+  {
+    const int tl = lane_id();
+    I g[TS_ITER];
+    R u[TS_ITER][NDOF], v[TS_ITER][NDOF], a[TS_ITER][NDOF], rm[TS_ITER][NDOF];
+    R x1[TS_ITER][NDOF], x2[TS_ITER][NDOF];
+    double mb[TS_ITER];
+    double* const bmb = ub(P->mbar);
+    // all loads first
 #pragma unroll
-  for (int k = 0; k < NG; ++k) {
-    hA[k] = (R)c_H[k * NG + ii];
-    hB[k] = (R)c_H[k * NG + jj];
-    hC[k] = (R)c_H[ii * NG + k];
-    hD[k] = (R)c_H[jj * NG + k];
-  }
-
-  R adr[NODE_ITERS][NDOF], avr[NODE_ITERS][NDOF];
-  double mbr[NODE_ITERS];  // mass sensitivity of the node, -fb . a_n (used at interior nodes)
+    for (int r = 0; r < TS_ITER; ++r) {
+      const int p = tl + TS_NT * r, Z = p / PS, X = p - Z * PS;
+      g[r] = nidx(min(X, PX - 1), min(Z, PZ - 1));
+    }
 #pragma unroll
-  for (int r = 0; r < NODE_ITERS; ++r) {
-    const int p = tid + TILE_THREADS * r;
-    if (p < NPT) {
-      const int Z = p / PX, X = p - Z * PX;
-      const auto g = nidx(X, Z);
-      R f[NDOF], u[NDOF];
-      double mb = 0;
+    for (int r = 0; r < TS_ITER; ++r) {
 #pragma unroll
       for (int c = 0; c < NDOF; ++c) {
-        const R dk = at(bad[c], g), vk = at(bav[c], g), ak = at(baa[c], g);
-        f[c] = (ak + c3 * vk) * at(brm[c], g);
-        u[c] = at(bdf[c], g);
-        adr[r][c] = dk;
-        avr[r][c] = vk;
-        mb -= (double)f[c] * accel(c, g, u[c]);
+        v[r][c] = at(ub(P->w + c * S), g[r]);
+        a[r][c] = at(ub(P->ad + c * S), g[r]);
+        rm[r][c] = at(ub(P->rmass + c * S), g[r]);
+        u[r][c] = at(ub(P->dfw + c * S), g[r]);
+        x1[r][c] = at(ub(P->x1 + c * S), g[r]);
+        if constexpr (HIST) x2[r][c] = at(ub(P->x2 + c * S), g[r]);
       }
-      // interior nodes: the running sum is read here, with the other loads, and written
-      // back in the store phase (perimeter and special nodes are the deferred kernel's)
-      mbr[r] = perim_slot(X, Z, PX, PZ) < 0 ? at(bmb, g) + mb : 0.0;
-      Uf[p] = lv_make<R, NDOF>(f);
-      Ud[p] = lv_make<R, NDOF>(u);
-      Fn[p] = LV{};
-      sflag[p] = -1;
+      mb[r] = at(bmb, g[r]);
     }
-  }
-  // FP64 fields: moduli of this lane's point in each batch loaded with the node values
-  // (no global load inside the element batches; with FP32 fields the registers are
-  // better spent on occupancy, and the batches load their own); geometric factors of the
-  // elements in LDS
-  constexpr bool PREF = sizeof(R) == 8;
-  R lm[4 * ((TX * TZ / 4 + FE_EPB - 1) / FE_EPB)][2];
 #pragma unroll
-  for (int q = 0; q < (PREF ? 4 * ((TX * TZ / 4 + FE_EPB - 1) / FE_EPB) : 0); ++q) {
-    constexpr int NB = (TX * TZ / 4 + FE_EPB - 1) / FE_EPB;
-    const int cc = q / NB, b0 = (q % NB) * FE_EPB;
-    const int cx = cc & 1, cz = cc >> 1;
-    const int ncx = (nxe - cx + 1) >> 1, ncz = (nze - cz + 1) >> 1;
-    const int ce = b0 + le;
-    if (tid < FE_THREADS && ce < ncx * ncz) {
-      const auto cell = cidx(cx + 2 * (ce % ncx), cz + 2 * (ce / ncx));
-      lm[q][0] = at(bco, cell * 2 * NP + pe);
-      lm[q][1] = at(bco, cell * 2 * NP + NP + pe);
+    for (int r = 0; r < TS_ITER; ++r)
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        const AdjNode<R> s = adj_node<R>(a[r][c], v[r][c], dt, c1, c2);
+        v[r][c] = s.v;
+        a[r][c] = s.a;
+      }
+    if (inj && field) {
+#pragma unroll
+      for (int r = 0; r < TS_ITER; ++r) {
+        if (field == 1) inject(g[r], v[r][0], v[r][1]);
+        else inject(g[r], a[r][0], a[r][1]);
+      }
+    }
+    const double idt2 = P->idt2;
+#pragma unroll
+    for (int r = 0; r < TS_ITER; ++r) {
+      R f[NDOF];
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        f[c] = (a[r][c] + c3 * v[r][c]) * rm[r][c];
+        double acc = (double)x1[r][c];
+        if constexpr (HIST) {
+          const double dc = (double)u[r][c];
+          acc = (((double)x2[r][c] - dc) - (dc - (double)x1[r][c])) * idt2;
+        }
+        mb[r] -= (double)f[c] * acc;
+      }
+      const int p = tl + TS_NT * r, Z = p / PS, X = p - Z * PS;
+      if (p < PMAX) {
+        Uf[p] = lv_make<R, NDOF>(f);
+        Ud[p] = lv_make<R, NDOF>(u[r]);
+        Eg[p] = node_slots(X, Z);
+      }
+      // the mass sensitivity of interior nodes (perimeter and special nodes: k_adj_deferred)
+      if (X < PX && Z < PZ && perim_slot(X, Z, PX, PZ) < 0 && special(p) < 0) at(bmb, g[r]) = mb[r];
     }
   }
-  if (tid < nxe * nze * 3) {
+  if (tid < NEL * 3) {
     const int e = tid / 3, k = tid - 3 * (tid / 3);
-    Gm[e][k] = at(bge, cidx(e % nxe, e / nxe) * 3 + k);
-  }
-  if (tid < nxe * nze) {  // the elements' running sensitivities (local index lz*nxe + lx)
-    const auto cell = cidx(tid % nxe, tid / nxe);
-    Ge[tid][0] = at(bgl, cell);
-    Ge[tid][1] = at(bgm, cell);
+    Gm[e][k] = at(ub(P->geom), cidx(min(e % TX, nxe - 1), min(e / TX, nze - 1)) * 3 + k);
   }
   __syncthreads();
-  const int nspec = T.spec_cnt[t];
-  if (tid < nspec) {
-    const int q = T.spec_idx[t * MAXSPECIAL + tid];
-    sflag[(q / PXM) * PX + q % PXM] = (short)tid;
-  }
 
-  // element batch q: colour cc = q / NBATCH, elements b0 .. b0+FE_EPB-1 of that colour
-  constexpr int NBATCH = (TX * TZ / 4 + FE_EPB - 1) / FE_EPB;
-  auto batch = [&](const int q) {
-    const int cc = q / NBATCH, b0 = (q % NBATCH) * FE_EPB;
-    const int cx = cc & 1, cz = cc >> 1;
-    const int ncx = (nxe - cx + 1) >> 1, ncz = (nze - cz + 1) >> 1;
-    const int nce = ncx * ncz;
-    if (b0 < nce) {  // uniform
-      const int ce = b0 + le;
-      const bool active = (tid < FE_THREADS) && (ce < nce);
-      int base = 0, el = 0;
-      if (active) {
-        const int lx = cx + 2 * (ce % ncx), lz = cz + 2 * (ce / ncx);
-        base = 4 * lz * PX + 4 * lx;
-        el = lz * nxe + lx;
-        const R g0 = Gm[el][0], g1 = Gm[el][1], g2 = Gm[el][2];
-        R la, mu;
-        if constexpr (PREF) {
-          la = lm[q][0];
-          mu = lm[q][1];
-        } else {
-          const auto cell = cidx(lx, lz);
-          la = at(bco, cell * 2 * NP + pe);
-          mu = at(bco, cell * 2 * NP + NP + pe);
-        }
-        const R kx = la + 2 * mu;
-        const R A0 = w * kx * g0, A1 = w * la * g2, A2 = w * kx * g1;
-        const R A3 = w * mu * g1, A4 = w * mu * g2, A5 = w * mu * g0;
-        R pxi[NDOF] = {0, 0}, peta[NDOF] = {0, 0}, gxi[NDOF] = {0, 0}, geta[NDOF] = {0, 0};
+  {
+    const int te = lane_id(), lane = te & 63;
+    const int e = (te >> 6) * TS_EPW + lane / NG, s = lane % NG;
+    const int lx = e % TX, lz = e / TX;
+    const bool on = lane < TS_EPW * NG && e < NEL && lx < nxe && lz < nze;
+    const int base = 4 * lz * PS + 4 * lx;
+    const I cell = cidx(min(lx, nxe - 1), min(lz, nze - 1));
+    LV* ex = Ex + min(e, NEL - 1) * NP;
+    const auto* hp = hconst<R>();
+    R H[NG][NG];
+#pragma unroll
+    for (int k = 0; k < NG; ++k)
+#pragma unroll
+      for (int i = 0; i < NG; ++i) H[k][i] = hp[k * NG + i];
+    // column derivatives of a patch array into the exchange array
+    auto column = [&](const LV* U) {
+      if (on) {
+        R g[NG][NDOF];
+#pragma unroll
+        for (int j = 0; j < NG; ++j)
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
 #pragma unroll
         for (int k = 0; k < NG; ++k) {
-          const LV f1 = Uf[base + jj * PX + k], f2 = Uf[base + k * PX + ii];
-          const LV u1 = Ud[base + jj * PX + k], u2 = Ud[base + k * PX + ii];
+          const LV x = U[base + k * PS + s];
 #pragma unroll
-          for (int c = 0; c < NDOF; ++c) {
-            pxi[c] += hA[k] * lv_get<R, NDOF>(f1, c);
-            peta[c] += lv_get<R, NDOF>(f2, c) * hB[k];
-            gxi[c] += hA[k] * lv_get<R, NDOF>(u1, c);
-            geta[c] += lv_get<R, NDOF>(u2, c) * hB[k];
-          }
+          for (int c = 0; c < NDOF; ++c)
+#pragma unroll
+            for (int j = 0; j < NG; ++j) g[j][c] += lv_get<R, NDOF>(x, c) * H[k][j];
         }
-        const R pxx = pxi[0], pex = peta[0], pxz = pxi[1], pez = peta[1];
-        const R gxx = gxi[0], gex = geta[0], gxz = gxi[1], gez = geta[1];
-        T1[le][pe] = LV{A0 * pxx + A1 * pez, A3 * pex + A5 * pxz};
-        T2[le][pe] = LV{A3 * pex + A4 * pxz, A1 * pxx + A2 * pez};
-        const double wd = (double)w;
-        Gr[le][pe][0] = wd * ((double)g0 * pxx * gxx + (double)g2 * (pxx * gez + pez * gxx) + (double)g1 * pez * gez);
-        Gr[le][pe][1] = wd * (2.0 * g0 * pxx * gxx + 2.0 * g1 * pez * gez + (double)g1 * pex * (gex + gxz) +
-                              (double)g2 * pxz * gex + (double)g0 * pxz * gxz);
+#pragma unroll
+        for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
       }
-      __syncthreads();
-      if (active) {
-        R s1[NDOF] = {0, 0}, s2[NDOF] = {0, 0}, f[NDOF];
+      wave_order();
+    };
+    column(Ud);
+    R gxi[NG][NDOF], get[NG][NDOF];  // gradient of d_n at the row's points
+    {
+      R x[NG][NDOF];
 #pragma unroll
-        for (int k = 0; k < NG; ++k) {
-          const LV a1 = T1[le][jj * NG + k], a2 = T2[le][k * NG + ii];
+      for (int k = 0; k < NG; ++k) {
+        const LV xv = Ud[min(base + s * PS + k, PMAX - 1)];
 #pragma unroll
-          for (int c = 0; c < NDOF; ++c) {
-            s1[c] += hC[k] * lv_get<R, NDOF>(a1, c);
-            s2[c] += lv_get<R, NDOF>(a2, c) * hD[k];
-          }
-        }
-        LV* fp = &Fn[base + jj * PX + ii];
-        const LV f0 = *fp;
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) f[c] = lv_get<R, NDOF>(f0, c) + (s1[c] + s2[c]);
-        *fp = lv_make<R, NDOF>(f);
+        for (int c = 0; c < NDOF; ++c) x[k][c] = lv_get<R, NDOF>(xv, c);
       }
-      // fixed-order sum over the element's points in two levels: lanes pe < 5 sum the
-      // rows jj = pe into Gs, then (after the barrier) lane pe = 0 sums the five row
-      // sums.  Gs is written again only after the next batch's first barrier, which
-      // lane pe = 0 reaches after its reads; the barrier also orders this batch's Fn
-      // updates and Gr, T1, T2 reads before the next batch's writes.
-      if (active && pe < NG) {
-        double rl = 0, rm = 0;
 #pragma unroll
-        for (int q = 0; q < NG; ++q) {
-          rl += Gr[le][pe * NG + q][0];
-          rm += Gr[le][pe * NG + q][1];
-        }
-        Gs[le][pe][0] = rl;
-        Gs[le][pe][1] = rm;
-      }
-      __syncthreads();
-      if (active && pe == 0) {
-        double sl = 0, sm = 0;
-#pragma unroll
-        for (int q = 0; q < NG; ++q) {
-          sl += Gs[le][q][0];
-          sm += Gs[le][q][1];
-        }
-        Ge[el][0] += sl;
-        Ge[el][1] += sm;
-      }
-    }
-  };
-  if constexpr (PREF) {  // moduli in registers: batches unrolled
-#pragma unroll
-    for (int q = 0; q < 4 * NBATCH; ++q) batch(q);
-  } else {
-#pragma unroll 1
-    for (int q = 0; q < 4 * NBATCH; ++q) batch(q);
-  }
-  __syncthreads();  // every batch's element sums are in Ge
-  if (tid < nxe * nze) {
-    const auto cell = cidx(tid % nxe, tid / nxe);
-    at(bgl, cell) = Ge[tid][0];
-    at(bgm, cell) = Ge[tid][1];
-  }
-  const uint32_t fbase = (uint32_t)t * SLOTS;
-  // lane index re-materialised for the store loop, so that the node-index arithmetic of
-  // the load loop is recomputed here instead of being held in registers through the
-  // element batches
-  int tst = tid;
-  asm volatile("" : "+v"(tst));
-  __builtin_assume(tst >= 0 && tst < TILE_THREADS);
-#pragma unroll
-  for (int r = 0; r < NODE_ITERS; ++r) {
-    const int p = tst + TILE_THREADS * r;
-    if (p < NPT) {
-      const int Z = p / PX, X = p - Z * PX;
-      int slot = perim_slot(X, Z, PX, PZ);
-      if (slot < 0 && sflag[p] >= 0) slot = PERIM_MAX + sflag[p];
-      const LV fn = Fn[p];
-      if (slot >= 0) {
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) at(bfp[c], fbase + slot) = lv_get<R, NDOF>(fn, c);
-      } else {
-        const auto g = nidx(X, Z);
+      for (int i = 0; i < NG; ++i) {
+        const LV gv = ex[s * NG + i];
 #pragma unroll
         for (int c = 0; c < NDOF; ++c) {
-          const R dn = adr[r][c] + lv_get<R, NDOF>(fn, c);
-          const R vbp = avr[r][c];
-          at(bad[c], g) = dn;
-          at(bav[c], g) = vbp + dt * dn;
-          at(baa[c], g) = c2 * vbp + c1 * dn;
+          R sum = 0;
+#pragma unroll
+          for (int k = 0; k < NG; ++k) sum += H[k][i] * x[k][c];
+          gxi[i][c] = sum;
+          get[i][c] = lv_get<R, NDOF>(gv, c);
         }
-        at(bmb, g) = mbr[r];
+      }
+    }
+    wave_order();
+    // moduli of the row's points, the element's running sensitivities
+    R m[NG][NDOF];
+    {
+      const R* bco = ub(P->coefs);
+#pragma unroll
+      for (int i = 0; i < NG; ++i)
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) m[i][c] = at(bco, (cell * NDOF + c) * NP + s * NG + i);
+    }
+    column(Uf);
+    // the sensitivities first, then the fluxes: the gradient of d_n and the transposed
+    // sums are not in registers together (FP64: 128 of them, without spills)
+    R x[NG][NDOF];
+    double rl = 0, rmu = 0;
+    const int em = min(e, NEL - 1);
+    const R g0 = Gm[em][0], g1 = Gm[em][1], g2 = Gm[em][2];
+    auto pgrad = [&](int i, R (&pxi)[NDOF]) {
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        R sum = 0;
+#pragma unroll
+        for (int k = 0; k < NG; ++k) sum += H[k][i] * x[k][c];
+        pxi[c] = sum;
+      }
+    };
+    if (on) {
+#pragma unroll
+      for (int k = 0; k < NG; ++k) {
+        const LV xv = Uf[base + s * PS + k];
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) x[k][c] = lv_get<R, NDOF>(xv, c);
+      }
+#pragma unroll
+      for (int i = 0; i < NG; ++i) {
+        R pxi[NDOF];
+        pgrad(i, pxi);
+        const LV pv = ex[s * NG + i];
+        const double wd = (double)(R)sW2[s * NG + i];
+        const R pxx = pxi[0], pxz = pxi[1], pex = lv_get<R, NDOF>(pv, 0), pez = lv_get<R, NDOF>(pv, 1);
+        const R gxx = gxi[i][0], gxz = gxi[i][1], gex = get[i][0], gez = get[i][1];
+        rl += wd * ((double)g0 * pxx * gxx + (double)g2 * (pxx * gez + pez * gxx) + (double)g1 * pez * gez);
+        rmu += wd * (2.0 * g0 * pxx * gxx + 2.0 * g1 * pez * gez + (double)g1 * pex * (gex + gxz) +
+                     (double)g2 * pxz * gex + (double)g0 * pxz * gxz);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    R s1r[NG][NDOF] = {};
+    if (on) {
+#pragma unroll
+      for (int i = 0; i < NG; ++i) {
+        const int pt = s * NG + i;
+        const R w = sW2[pt];
+        const R la = m[i][0], mu = m[i][1], kx = la + 2 * mu;
+        const R A0 = w * kx * g0, A1 = w * la * g2, A2 = w * kx * g1;
+        const R A3 = w * mu * g1, A4 = w * mu * g2, A5 = w * mu * g0;
+        R pxi[NDOF];
+        pgrad(i, pxi);
+        const LV pv = ex[pt];
+        const R pxx = pxi[0], pxz = pxi[1], pex = lv_get<R, NDOF>(pv, 0), pez = lv_get<R, NDOF>(pv, 1);
+        const R t1[NDOF] = {A0 * pxx + A1 * pez, A3 * pex + A5 * pxz};
+        const R t2[NDOF] = {A3 * pex + A4 * pxz, A1 * pxx + A2 * pez};
+        ex[pt] = lv_make<R, NDOF>(t2);
+#pragma unroll
+        for (int q = 0; q < NG; ++q)
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) s1r[q][c] += H[q][i] * t1[c];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    {  // rows of the element in order, by its first lane
+      double sl = 0, sm = 0;
+#pragma unroll
+      for (int q = 0; q < NG; ++q) {
+        const int from = min(lane - s + q, 63);
+        sl += __shfl(rl, from);
+        sm += __shfl(rmu, from);
+      }
+      if (on && s == 0) {
+        at(ub(P->glam), cell) = at(ub(P->glam), cell) + sl;
+        at(ub(P->gmu), cell) = at(ub(P->gmu), cell) + sm;
+      }
+    }
+    wave_order();
+    if (on) {
+      R g[NG][NDOF];
+#pragma unroll
+      for (int j = 0; j < NG; ++j)
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
+#pragma unroll
+      for (int k = 0; k < NG; ++k) {
+        const LV tv = ex[k * NG + s];
+#pragma unroll
+        for (int j = 0; j < NG; ++j)
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c) g[j][c] += lv_get<R, NDOF>(tv, c) * H[j][k];
+      }
+#pragma unroll
+      for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
+    }
+    wave_order();
+    if (on) {
+#pragma unroll
+      for (int i = 0; i < NG; ++i) {
+        const LV cv = ex[s * NG + i];
+        R f[NDOF];
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) f[c] = s1r[i][c] + lv_get<R, NDOF>(cv, c);
+        ex[s * NG + i] = lv_make<R, NDOF>(f);
+      }
+    } else if (lane < TS_EPW * NG && e < NEL) {
+#pragma unroll
+      for (int i = 0; i < NG; ++i) ex[s * NG + i] = LV{};
+    }
+  }
+  // the adjoint state again, for the stores
+  const int ts = lane_id();
+  R ad[TS_ITER][NDOF], av[TS_ITER][NDOF];
+#pragma unroll
+  for (int r = 0; r < TS_ITER; ++r) {
+    const int p = ts + TS_NT * r, Z = p / PS, X = p - Z * PS;
+    const I g = nidx(min(X, PX - 1), min(Z, PZ - 1));
+#pragma unroll
+    for (int c = 0; c < NDOF; ++c) {
+      ad[r][c] = at(ub(P->ad + c * S), g);
+      av[r][c] = at(ub(P->w + c * S), g);
+    }
+  }
+  __syncthreads();
+  const uint32_t fbase = (uint32_t)t * SLOTS;
+#pragma unroll
+  for (int r = 0; r < TS_ITER; ++r) {
+    const int p = ts + TS_NT * r, Z = p / PS, X = p - Z * PS;
+    if (X < PX && Z < PZ) {
+      const ushort4 sl = Eg[p];
+      const LV f0 = Ex[sl.x], f1 = Ex[sl.y], f2 = Ex[sl.z], f3 = Ex[sl.w];
+      const I g = nidx(X, Z);
+      int slot = perim_slot(X, Z, PX, PZ);
+      if (const int k = special(p); k >= 0) slot = PERIM_MAX + k;
+      R F[NDOF];
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        F[c] = ((lv_get<R, NDOF>(f0, c) + lv_get<R, NDOF>(f1, c)) + lv_get<R, NDOF>(f2, c)) + lv_get<R, NDOF>(f3, c);
+        av[r][c] = av[r][c] + dt * ad[r][c];
+      }
+      if (inj && field == 0) inject(g, ad[r][0], ad[r][1]);
+      if (inj && field == 1) inject(g, av[r][0], av[r][1]);
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        if (slot >= 0) {
+          at(ub(P->fpart + c * P->FPS), fbase + slot) = F[c];
+        } else {
+          at(ub(P->ad + c * S), g) = ad[r][c] + F[c];
+          at(ub(P->w + c * S), g) = av[r][c];
+        }
       }
     }
   }
@@ -1503,425 +1618,12 @@ __global__ __launch_bounds__(TILE_THREADS) void k_adj_tile(
 // forces -K^T fb of the tiles, the absorbing term, the mass and ABC sensitivities.
 // gabs[c][q] accumulates dJ/dC_c of the node (for nodes with absorbing entries):
 // -fb_c (vp_c + c3 a_c), vp = v_{n-1} + c2 a_{n-1} the forward predicted velocity.
-// dJ/d(recorded field) of one sample at the receiver nodes (see k_adj_inject); the
-// injection of step n-1 can ride on the deferred kernel of step n: udef[q] is the
-// injection node handled by deferred node q after its own update (or -1), uext the
-// injection nodes that are not deferred nodes, done by extra lanes.
-struct InjectPlan {
-  int nu = 0, nrec = 0;
-  const int *unode = nullptr, *off = nullptr, *rec = nullptr;
-  const double* w = nullptr;
-  const double* g = nullptr;  // the sample, [ndof][nrec]; null: no injection
-  void* fld = nullptr;        // the adjoint field it is added to (bulk type)
-  const int* udef = nullptr;
-  const int* uext = nullptr;
-  int next = 0;
-};
-
-template <typename R>
-__device__ __forceinline__ void inject_node(const InjectPlan& P, int u, R* __restrict__ fld, size_t GS) {
-  for (int c = 0; c < 2; ++c) {
-    const size_t i = c * GS + P.unode[u];
-    R x = fld[i];
-    for (int k = P.off[u]; k < P.off[u + 1]; ++k) x = (R)((double)x + P.w[k] * P.g[(size_t)c * P.nrec + P.rec[k]]);
-    fld[i] = x;
-  }
-}
-
-// Persistent, pipelined form of k_adj_tile, with the same arithmetic and the same
-// summation orders (results equal bit for bit): AP_NT threads, one colour of a tile's
-// elements per batch (two barriers per batch), each workgroup on a run of tiles (the
-// XCD slices of k_tile_step).  While a tile's element batches run, the adjoint state,
-// inverse mass, forward displacements (or acceleration), mass sensitivity, moduli,
-// geometric factors and element sensitivities of the workgroup's next tile load into
-// registers; a finished tile is stored by the threads that own its patch slots, right
-// before they overwrite those slots with the next tile's values.  The adjoint state of
-// the patch and the running mass sensitivity wait in LDS for the store (the registers
-// hold the prefetch).  The launch covers tlist[0 .. nlist); the grid is a multiple of 8.
-constexpr int AP_NT = 512;
-constexpr int AP_EPB = 20;  // elements per batch: a whole colour of a full tile (16)
-template <typename R, bool FULL = false>
-__global__ __launch_bounds__(AP_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_pipe(
-    TileDev T, const int* __restrict__ tlist, int nlist, const int4* __restrict__ ttiles,
-    const int4* __restrict__ tgrids, const int* __restrict__ tspc, R* __restrict__ ad, R* __restrict__ av,
-    R* __restrict__ aa, const R* __restrict__ rmass, const R* __restrict__ dfw, const R* __restrict__ afw,
-    const R* __restrict__ coefs, const R* __restrict__ geom, R* __restrict__ fpart, double* __restrict__ glam,
-    double* __restrict__ gmu, double* __restrict__ mbar, R dt, R c1, R c2, R c3,
-    const R* __restrict__ dprev = nullptr, const R* __restrict__ dnext = nullptr, double idt2 = 0.0) {
-  constexpr int NDOF = 2;
-  using LV = typename LVec<R, NDOF>::T;
-  constexpr int NITER = (PMAX + AP_NT - 1) / AP_NT;        // patch nodes per thread
-  constexpr int NBC = (TX * TZ / 4 + AP_EPB - 1) / AP_EPB;  // batches per colour
-  constexpr int NB = 4 * NBC;                               // batches per tile
-  constexpr int ETH = AP_EPB * NP;
-  static_assert(ETH <= AP_NT && 3 * TX * TZ <= AP_NT && MAXSPECIAL <= AP_NT, "tables larger than the workgroup");
-  __shared__ LV Uf[PMAX];  // fb
-  __shared__ LV Ud[PMAX];  // forward d_n
-  __shared__ LV Fn[PMAX];  // -K^T fb, assembled
-  __shared__ LV Ad[PMAX];  // adjoint displacement and velocity, kept for the store
-  __shared__ LV Av[PMAX];
-  __shared__ double Mb[PMAX];  // running mass sensitivity of the interior nodes
-  __shared__ LV T1[AP_EPB][NP];
-  __shared__ LV T2[AP_EPB][NP];
-  __shared__ double Gr[AP_EPB][NP][2];
-  __shared__ double Gs[AP_EPB][NG][2];
-  __shared__ double Ge[TX * TZ][2];
-  __shared__ R Gm[TX * TZ][3];
-  __shared__ short sflag[PMAX];
-  __shared__ LV ML[NB][ETH];  // this tile's moduli (lambda, mu) of each lane's point, per batch
-  __shared__ double sH[NP];
-
-  const int nwg = gridDim.x;
-  const int bid = blockIdx.x;
-  const int W = nwg >> 3;
-  const int slice = (nlist + 7) >> 3;
-  const int s0 = (bid & 7) * slice;
-  const int s1 = min(s0 + slice, nlist);
-  const int q0 = s0 + (bid >> 3);
-  if (q0 >= s1) return;
-  const int tid = threadIdx.x;
-  const size_t S = T.NGp;
-  // lane indices of the node loops and of the element batches, re-materialised per
-  // tile (below) so that the index arithmetic derived from them is recomputed in each
-  // tile rather than held in registers through the loop
-  int tnode = tid, lel = tid / NP;
-  // H entries from LDS (the registers hold the prefetch)
-  if (tid < NP) sH[tid] = c_H[tid];
-  struct Geo {
-    int tx0, tz0, nxe, nze, Z0, PX, PZ, NPT, X0, kL, kR;
-  };
-  auto geo = [&](const int4 tg) {
-    Geo g;
-    g.tx0 = tg.x;
-    g.tz0 = tg.y;
-    g.nxe = FULL ? TX : (tg.z & 0xff);
-    g.nze = FULL ? TZ : ((tg.z >> 8) & 0xff);
-    g.Z0 = tg.w;
-    g.PX = 4 * g.nxe + 1;
-    g.PZ = 4 * g.nze + 1;
-    g.NPT = g.PX * g.PZ;
-    g.X0 = 4 * g.tx0;
-    g.kL = g.tx0 / TX;
-    g.kR = FULL ? g.kL + 1 : (g.tx0 + g.nxe + TX - 1) / TX;
-    return g;
-  };
-  auto nidx = [&](const int4 gr, const Geo& G, int X, int Z) {
-    if constexpr (FULL) return node_index_full(gr, X, Z, G.X0, G.Z0, G.kL);
-    else return node_index(gr, X, Z, G.PX, G.X0, G.Z0, G.kL, G.kR);
-  };
-  auto cidx = [&](const int4 gr, const int4 tg, const Geo& G, int lx, int lz) {
-    if constexpr (FULL)
-      return (uint32_t)gr.w + (uint32_t)(G.tz0 + lz) * (uint32_t)(tg.z >> 16) + (uint32_t)(G.tx0 + lx);
-    else return cell_index(gr, tg.z >> 16, G.tx0, G.tz0, lx, lz);
-  };
-  auto ub = [&](auto* p) {
-    if constexpr (FULL) return sgpr_base(p);
-    else return p;
-  };
-  auto at = [&](auto* base, auto g) -> auto& {
-    if constexpr (FULL) return at32(base, (uint32_t)g);
-    else return base[g];
-  };
-  R *bad[NDOF], *bav[NDOF], *baa[NDOF], *bfp[NDOF];
-  const R *brm[NDOF], *bdf[NDOF], *baf[NDOF], *bdp[NDOF], *bdn[NDOF];
-#pragma unroll
-  for (int c = 0; c < NDOF; ++c) {
-    bad[c] = ub(ad + c * S);
-    bav[c] = ub(av + c * S);
-    baa[c] = ub(aa + c * S);
-    brm[c] = ub(rmass + c * S);
-    bdf[c] = ub(dfw + c * S);
-    baf[c] = afw ? ub(afw + c * S) : nullptr;
-    bdp[c] = dprev ? ub(dprev + c * S) : nullptr;
-    bdn[c] = dnext ? ub(dnext + c * S) : nullptr;
-    bfp[c] = ub(fpart + c * T.FPS);
-  }
-  // x1: the forward acceleration (stored) or d_{n-1}; x2: d_{n+1} (history of d only)
-  const R *bx1[NDOF], *bx2[NDOF];
-#pragma unroll
-  for (int c = 0; c < NDOF; ++c) {
-    bx1[c] = afw ? baf[c] : bdp[c];
-    bx2[c] = bdn[c];
-  }
-  double* bmb = ub(mbar);
-  double* bgl = ub(glam);
-  double* bgm = ub(gmu);
-  const R* bco = ub(coefs);
-  const R* bge = ub(geom);
-
-  // next tile's registers: node values (x1, x2: the forward acceleration, or d_{n-1}
-  // and d_{n+1}), the mass sensitivity of interior nodes, this lane's moduli in each
-  // batch, one geometric factor, one element's two sensitivities, one special node
-  R pad[NITER][NDOF] = {}, pav[NITER][NDOF] = {}, paa[NITER][NDOF] = {}, prm[NITER][NDOF] = {};
-  R pdf[NITER][NDOF] = {}, px1[NITER][NDOF] = {}, px2[NITER][NDOF] = {};
-  double pmb[NITER] = {};
-  R plm[NB][2] = {};
-  R pg = 0;
-  double pge0 = 0, pge1 = 0;
-  int psp = -1;
-  auto issue = [&](int t) {
-    const int4 tg = ttiles[t];
-    const int4 gr = tgrids[t];
-    const Geo G = geo(tg);
-#pragma unroll
-    for (int r = 0; r < NITER; ++r) {
-      const int p = tnode + AP_NT * r;
-      if (p < G.NPT) {
-        const int Z = p / G.PX, X = p - Z * G.PX;
-        const auto g = nidx(gr, G, X, Z);
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) {
-          pad[r][c] = at(bad[c], g);
-          pav[r][c] = at(bav[c], g);
-          paa[r][c] = at(baa[c], g);
-          prm[r][c] = at(brm[c], g);
-          pdf[r][c] = at(bdf[c], g);
-          px1[r][c] = at(bx1[c], g);
-          if (!afw) px2[r][c] = at(bx2[c], g);
-        }
-        pmb[r] = perim_slot(X, Z, G.PX, G.PZ) < 0 ? at(bmb, g) : 0.0;
-      }
-    }
-    const int pl = tnode - lel * NP;
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int cc = q / NBC, b0 = (q % NBC) * AP_EPB;
-      const int cx = cc & 1, cz = cc >> 1;
-      const int ncx = (G.nxe - cx + 1) >> 1, ncz = (G.nze - cz + 1) >> 1;
-      const int ce = b0 + lel;
-      if (tnode < ETH && ce < ncx * ncz) {
-        const auto cell = cidx(gr, tg, G, cx + 2 * (ce % ncx), cz + 2 * (ce / ncx));
-        plm[q][0] = at(bco, cell * 2 * NP + pl);
-        plm[q][1] = at(bco, cell * 2 * NP + NP + pl);
-      }
-    }
-    if (tid < G.nxe * G.nze * 3) {
-      const int e = tid / 3, k = tid - 3 * (tid / 3);
-      pg = at(bge, cidx(gr, tg, G, e % G.nxe, e / G.nxe) * 3 + k);
-    }
-    if (tid < G.nxe * G.nze) {
-      const auto cell = cidx(gr, tg, G, tid % G.nxe, tid / G.nxe);
-      pge0 = at(bgl, cell);
-      pge1 = at(bgm, cell);
-    }
-    if (tid < tspc[t]) psp = T.spec_idx[t * MAXSPECIAL + tid];
-  };
-
-  // Stores of a finished tile from LDS (the element sensitivities, the partial forces
-  // of perimeter and special nodes, the new adjoint state and mass sensitivity of the
-  // others), by the threads that own the slots
-  auto store_tile = [&](const int tp, const int4 tgp, const int4 grp) {
-    const Geo G = geo(tgp);
-    if (tid < G.nxe * G.nze) {
-      const auto cell = cidx(grp, tgp, G, tid % G.nxe, tid / G.nxe);
-      at(bgl, cell) = Ge[tid][0];
-      at(bgm, cell) = Ge[tid][1];
-    }
-    const uint32_t fbase = (uint32_t)tp * SLOTS;
-#pragma unroll
-    for (int r = 0; r < NITER; ++r) {
-      const int p = tnode + AP_NT * r;
-      if (p < G.NPT) {
-        const int Z = p / G.PX, X = p - Z * G.PX;
-        int slot = perim_slot(X, Z, G.PX, G.PZ);
-        if (slot < 0 && sflag[p] >= 0) slot = PERIM_MAX + sflag[p];
-        const LV fn = Fn[p];
-        if (slot >= 0) {
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) at(bfp[c], fbase + slot) = lv_get<R, NDOF>(fn, c);
-        } else {
-          const auto g = nidx(grp, G, X, Z);
-          const LV a0 = Ad[p], v0 = Av[p];
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) {
-            const R dn = lv_get<R, NDOF>(a0, c) + lv_get<R, NDOF>(fn, c);
-            const R vbp = lv_get<R, NDOF>(v0, c);
-            at(bad[c], g) = dn;
-            at(bav[c], g) = vbp + dt * dn;
-            at(baa[c], g) = c2 * vbp + c1 * dn;
-          }
-          at(bmb, g) = Mb[p];
-        }
-      }
-    }
-  };
-
-  issue(tlist[q0]);
-  int tp = -1;
-  int4 tgp = {}, grp = {};
-#pragma unroll 1
-  for (int qi = q0; qi < s1; qi += W) {
-    tnode = tid;
-    lel = tid / NP;
-    asm volatile("" : "+v"(tnode));
-    asm volatile("" : "+v"(lel));
-    __builtin_assume(tnode >= 0 && tnode < AP_NT);
-    __builtin_assume(lel >= 0 && lel <= (AP_NT - 1) / NP);
-    const int pe = tnode - lel * NP;
-    const int ii = pe % NG, jj = pe / NG;
-    const R w = (R)c_W2[pe];
-    const int t = tlist[qi];
-    const int tn = qi + W < s1 ? tlist[qi + W] : -1;
-    const int4 tg = ttiles[t];
-    const int4 gr = tgrids[t];
-    const Geo G = geo(tg);
-    const int PX = G.PX, NPT = G.NPT;
-    // this tile's fb, forward displacement and mass-sensitivity increment from the
-    // prefetched values ...
-    R f[NITER][NDOF], u[NITER][NDOF];
-    double mb[NITER];
-#pragma unroll
-    for (int r = 0; r < NITER; ++r) {
-      const int p = tnode + AP_NT * r;
-      if (p < NPT) {
-        double m = 0;
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) {
-          f[r][c] = (paa[r][c] + c3 * pav[r][c]) * prm[r][c];
-          u[r][c] = pdf[r][c];
-          double acc;
-          if (afw) {
-            acc = (double)px1[r][c];
-          } else {
-            const double dc = (double)u[r][c];
-            acc = (((double)px2[r][c] - dc) - (dc - (double)px1[r][c])) * idt2;
-          }
-          m -= (double)f[r][c] * acc;
-        }
-        mb[r] = m;
-      }
-    }
-    // ... then the previous tile's stores ...
-    if (tp >= 0) store_tile(tp, tgp, grp);
-    // ... then this tile's values into the slots just stored
-#pragma unroll
-    for (int r = 0; r < NITER; ++r) {
-      const int p = tnode + AP_NT * r;
-      if (p < NPT) {
-        const int Z = p / PX, X = p - Z * PX;
-        Uf[p] = lv_make<R, NDOF>(f[r]);
-        Ud[p] = lv_make<R, NDOF>(u[r]);
-        Fn[p] = LV{};
-        Ad[p] = lv_make<R, NDOF>(pad[r]);
-        Av[p] = lv_make<R, NDOF>(pav[r]);
-        Mb[p] = perim_slot(X, Z, PX, G.PZ) < 0 ? pmb[r] + mb[r] : 0.0;
-        sflag[p] = -1;
-      }
-    }
-    if (tid < G.nxe * G.nze * 3) Gm[tid / 3][tid - 3 * (tid / 3)] = pg;
-    if (tid < G.nxe * G.nze) {
-      Ge[tid][0] = pge0;
-      Ge[tid][1] = pge1;
-    }
-    if (tnode < ETH) {
-#pragma unroll
-      for (int q = 0; q < NB; ++q) ML[q][tnode] = lv_make<R, NDOF>(plm[q]);
-    }
-    __syncthreads();
-    if (psp >= 0) sflag[(psp / PXM) * PX + psp % PXM] = (short)tid;
-    psp = -1;
-    if (tn >= 0) issue(tn);
-
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int cc = q / NBC, b0 = (q % NBC) * AP_EPB;
-      const int cx = cc & 1, cz = cc >> 1;
-      const int ncx = (G.nxe - cx + 1) >> 1, ncz = (G.nze - cz + 1) >> 1;
-      const int nce = ncx * ncz;
-      if (b0 < nce) {  // uniform
-        const int ce = b0 + lel;
-        const bool active = (tnode < ETH) && (ce < nce);
-        int base = 0, el = 0;
-        if (active) {
-          const int lx = cx + 2 * (ce % ncx), lz = cz + 2 * (ce / ncx);
-          base = 4 * lz * PX + 4 * lx;
-          el = lz * G.nxe + lx;
-          const R g0 = Gm[el][0], g1 = Gm[el][1], g2 = Gm[el][2];
-          const LV mm = ML[q][tnode];
-          const R la = lv_get<R, NDOF>(mm, 0), mu = lv_get<R, NDOF>(mm, 1);
-          const R kx = la + 2 * mu;
-          const R A0 = w * kx * g0, A1 = w * la * g2, A2 = w * kx * g1;
-          const R A3 = w * mu * g1, A4 = w * mu * g2, A5 = w * mu * g0;
-          R pxi[NDOF] = {0, 0}, peta[NDOF] = {0, 0}, gxi[NDOF] = {0, 0}, geta[NDOF] = {0, 0};
-#pragma unroll
-          for (int k = 0; k < NG; ++k) {
-            const LV f1 = Uf[base + jj * PX + k], f2 = Uf[base + k * PX + ii];
-            const LV u1 = Ud[base + jj * PX + k], u2 = Ud[base + k * PX + ii];
-            const R ha = (R)sH[k * NG + ii], hb = (R)sH[k * NG + jj];
-#pragma unroll
-            for (int c = 0; c < NDOF; ++c) {
-              pxi[c] += ha * lv_get<R, NDOF>(f1, c);
-              peta[c] += lv_get<R, NDOF>(f2, c) * hb;
-              gxi[c] += ha * lv_get<R, NDOF>(u1, c);
-              geta[c] += lv_get<R, NDOF>(u2, c) * hb;
-            }
-          }
-          const R pxx = pxi[0], pex = peta[0], pxz = pxi[1], pez = peta[1];
-          const R gxx = gxi[0], gex = geta[0], gxz = gxi[1], gez = geta[1];
-          T1[lel][pe] = LV{A0 * pxx + A1 * pez, A3 * pex + A5 * pxz};
-          T2[lel][pe] = LV{A3 * pex + A4 * pxz, A1 * pxx + A2 * pez};
-          const double wd = (double)w;
-          Gr[lel][pe][0] =
-              wd * ((double)g0 * pxx * gxx + (double)g2 * (pxx * gez + pez * gxx) + (double)g1 * pez * gez);
-          Gr[lel][pe][1] = wd * (2.0 * g0 * pxx * gxx + 2.0 * g1 * pez * gez + (double)g1 * pex * (gex + gxz) +
-                                (double)g2 * pxz * gex + (double)g0 * pxz * gxz);
-        }
-        __syncthreads();
-        if (active) {
-          R s1[NDOF] = {0, 0}, s2[NDOF] = {0, 0}, fo[NDOF];
-#pragma unroll
-          for (int k = 0; k < NG; ++k) {
-            const LV a1 = T1[lel][jj * NG + k], a2 = T2[lel][k * NG + ii];
-            const R hc = (R)sH[ii * NG + k], hd = (R)sH[jj * NG + k];
-#pragma unroll
-            for (int c = 0; c < NDOF; ++c) {
-              s1[c] += hc * lv_get<R, NDOF>(a1, c);
-              s2[c] += lv_get<R, NDOF>(a2, c) * hd;
-            }
-          }
-          LV* fp = &Fn[base + jj * PX + ii];
-          const LV f0 = *fp;
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) fo[c] = lv_get<R, NDOF>(f0, c) + (s1[c] + s2[c]);
-          *fp = lv_make<R, NDOF>(fo);
-        }
-        if (active && pe < NG) {
-          double rl = 0, rm = 0;
-#pragma unroll
-          for (int q2 = 0; q2 < NG; ++q2) {
-            rl += Gr[lel][pe * NG + q2][0];
-            rm += Gr[lel][pe * NG + q2][1];
-          }
-          Gs[lel][pe][0] = rl;
-          Gs[lel][pe][1] = rm;
-        }
-        __syncthreads();
-        if (active && pe == 0) {
-          double sl = 0, sm = 0;
-#pragma unroll
-          for (int q2 = 0; q2 < NG; ++q2) {
-            sl += Gs[lel][q2][0];
-            sm += Gs[lel][q2][1];
-          }
-          Ge[el][0] += sl;
-          Ge[el][1] += sm;
-        }
-      }
-    }
-    __syncthreads();  // the last batch's element sums are in Ge
-    tp = t;
-    tgp = tg;
-    grp = gr;
-  }
-  if (tp >= 0) store_tile(tp, tgp, grp);
-}
-
 template <typename R>
 __global__ __launch_bounds__(256) void k_adj_deferred(int ndef, DefTable defs,
                                                       const int* __restrict__ part_off, const R* __restrict__ fpart,
                                                       size_t FPS, const double* __restrict__ abso,
                                                       const R* __restrict__ rmdef, R* __restrict__ ad,
-                                                      R* __restrict__ av, R* __restrict__ aa, size_t GS,
+                                                      R* __restrict__ aw, size_t GS,
                                                       const R* __restrict__ afw, const R* __restrict__ vprev,
                                                       const R* __restrict__ aprev, double* __restrict__ mbar,
                                                       double* __restrict__ gabs, R dt, R c1, R c2, R c3,
@@ -1931,17 +1633,19 @@ __global__ __launch_bounds__(256) void k_adj_deferred(int ndef, DefTable defs,
                                                       double idt2 = 0.0, InjectPlan IP = {}) {
   constexpr int NDOF = 2;
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= ndef) {  // injection lanes (nodes that are not deferred)
-    if (IP.g && q < ndef + IP.next) inject_node<R>(IP, IP.uext[q - ndef], (R*)IP.fld, GS);
-    return;
-  }
+  if (q >= ndef) return;
   const DefNode n = def_unpack(defs, q);
   const size_t g = n.g;
+  const int u = IP.g ? IP.udef[q] : -1;
   double mb = 0;
 #pragma unroll
   for (int c = 0; c < NDOF; ++c) {
-    const R dk = ad[c * GS + g], vk = av[c * GS + g], ak = aa[c * GS + g];
-    const R fb = (ak + c3 * vk) * rmdef[(size_t)c * ndef + q];
+    AdjNode<R> s = adj_node<R>(ad[c * GS + g], aw[c * GS + g], dt, c1, c2);
+    if (u >= 0) {
+      R& x = IP.field == 0 ? s.d : (IP.field == 1 ? s.v : s.a);
+      x = inject_at<R>(IP, u, c, x);
+    }
+    const R fb = (s.a + c3 * s.v) * rmdef[(size_t)c * ndef + q];
     R F = 0;
     if (n.pinl) {  // the loop below with pcnt = 1 or 2
       F = F + fpart[c * FPS + n.poff[0]];
@@ -1951,11 +1655,8 @@ __global__ __launch_bounds__(256) void k_adj_deferred(int ndef, DefTable defs,
     }
     double Cc = 0;
     for (int k = 0; k < n.acnt; ++k) Cc += abso[(size_t)(n.astart + k) * NDOF + c];
-    const R vbp = (R)((double)vk - Cc * (double)fb);
-    const R dn = dk + F;
-    ad[c * GS + g] = dn;
-    av[c * GS + g] = vbp + dt * dn;
-    aa[c * GS + g] = c2 * vbp + c1 * dn;
+    ad[c * GS + g] = s.d + F;
+    aw[c * GS + g] = (R)((double)s.v - Cc * (double)fb);
     // with a displacement history (dcur set): a_n as in fwd_accel, and the predicted
     // velocity v_{n-1} + dt/2 a_{n-1} = (d_n - d_{n-1}) / dt
     const double an = dcur ? fwd_accel(afw, dprev, dnext, c * GS + g, dcur[c * GS + g], idt2)
@@ -1968,28 +1669,6 @@ __global__ __launch_bounds__(256) void k_adj_deferred(int ndef, DefTable defs,
     }
   }
   mbar[g] += mb;
-  if (IP.g && IP.udef[q] >= 0) inject_node<R>(IP, IP.udef[q], (R*)IP.fld, GS);  // after the update
-}
-
-// dJ/d(recorded field) of one sample added at the receiver nodes, or spread over the
-// element nodes with the interpolation weights (the transpose of the interpolation).
-// One lane per distinct node u: its contributions (receiver rec[k], weight w[k], k in
-// [off[u], off[u+1]), in receiver order) are added one after the other, which is the
-// order a receiver-by-receiver loop would use.
-template <typename R>
-__global__ void k_adj_inject(int nu, const int* __restrict__ unode, const int* __restrict__ off,
-                             const int* __restrict__ rec, const double* __restrict__ w, int nrec,
-                             const double* __restrict__ g, R* __restrict__ fld, size_t GS) {
-  const int u = blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= nu) return;
-  InjectPlan P;
-  P.nrec = nrec;
-  P.unode = unode;
-  P.off = off;
-  P.rec = rec;
-  P.w = w;
-  P.g = g;
-  inject_node<R>(P, u, fld, GS);
 }
 
 }  // namespace sem2d
