@@ -69,15 +69,57 @@ __host__ __device__ inline double normal_sigma(int kind, double coef, double vc,
   }
 }
 
+// What the traction solve of a pair reads, loaded in one group: with the loads where the
+// values are used, each behind the stores of the state before it (which may alias), a step
+// waited for memory about ten times one after the other (600 x 300 SH elements, FP64: the
+// launch after the tile kernel 13.9 us, with the pair's and the nodes' values in groups 9.4 us).
+struct PairData {
+  double B[2], iM1[2], iM2[2], Z[2], nx, nz, T0[2], sigma;
+  double theta = 0, D = 0, V = 0, coh = 0, p0 = 0, p1 = 0, p2 = 0, p3 = 0, p4 = 0, p5 = 0, Tc = 0, coeft = 0;
+};
+template <int nd>
+__device__ __forceinline__ PairData pair_load(const FaultDev& F, int k, bool two) {
+  PairData P;
+  const int np = F.np;
+#pragma unroll
+  for (int c = 0; c < nd; ++c) {
+    P.B[c] = F.B[c * np + k];
+    P.iM1[c] = F.invM1[c * np + k];
+    P.iM2[c] = two ? F.invM2[c * np + k] : 0.0;
+    P.Z[c] = F.Z[c * np + k];
+  }
+  P.nx = F.nrm[k], P.nz = F.nrm[np + k];
+  P.T0[0] = F.T0[k], P.T0[1] = F.T0[np + k];
+  P.sigma = F.sigma[k];
+  P.D = F.D[k];
+  if (F.law != 2) P.coh = F.coh[k];
+  if (F.law != 3) {
+    P.theta = F.theta[k];
+    P.p0 = F.p0[k], P.p1 = F.p1[k], P.p2 = F.p2[k], P.p3 = F.p3[k];
+    if (F.law == 2 || F.kind > 2) P.p4 = F.p4[k];
+  }
+  if (F.law == 2) {
+    P.V = F.V[k];
+    if (F.kind == 4) P.p5 = F.p5[k];
+    if (F.kind == 1) P.Tc = F.Tc[k], P.coeft = F.coeft[k];
+  }
+  return P;
+}
+
+// the pair's state after the step
+struct PairOut {
+  double D0, V0, T[2], Ts0, mu;
+};
+
 #pragma clang fp contract(off)
 
-__device__ inline double f_swf_mu(const FaultDev& F, int k) {
-  const double th = F.theta[k], dc = F.p0[k], mus = F.p1[k], mud = F.p2[k];
+__device__ inline double f_swf_mu(const FaultDev& F, const PairData& P, double th) {
+  const double dc = P.p0, mus = P.p1, mud = P.p2;
   double mu;
   if (F.kind == 1) mu = mus - (mus - mud) * fmin(th / dc, 1.0);
   else if (F.kind == 2) mu = mud - (mud - mus) * exp(-th / dc);
-  else mu = mud + (mus - mud) / pow(1.0 + th / dc, F.p4[k]);
-  return mu + F.p3[k] * th;
+  else mu = mud + (mus - mud) / pow(1.0 + th / dc, P.p4);
+  return mu + P.p3 * th;
 }
 
 // twf_mu (SRC/bc_dynflt_twf.f90:129-183) of kind 1..3 with tw = MuS, MuD, Mu0, X, Z, V, L,
@@ -116,21 +158,21 @@ __device__ inline double f_twf_mu(const FaultDev& F, int k, double time, double 
   return twf_mu(F.twf, F.tw, F.xz[k], F.xz[F.np + k], time, d);
 }
 
-__device__ inline double f_rsf_mu(const FaultDev& F, int k, double v) {
-  const double dc = F.p0[k], mus = F.p1[k], a = F.p2[k], b = F.p3[k], vs = F.p4[k], th = F.theta[k];
+__device__ inline double f_rsf_mu(const FaultDev& F, const PairData& P, double th, double v) {
+  const double dc = P.p0, mus = P.p1, a = P.p2, b = P.p3, vs = P.p4;
   switch (F.kind) {
     case 1: return mus + a * fabs(v) / (fabs(v) + vs) - b * th / (th + dc);
     case 2:
     case 3: return a * libm::asinh(fabs(v) / (2.0 * vs) * exp((mus + b * log(vs * th / dc)) / a));
-    default: return a * libm::asinh(fabs(v) / (2.0 * vs) * exp((mus + b * log(F.p5[k] * th / dc + 1)) / a));
+    default: return a * libm::asinh(fabs(v) / (2.0 * vs) * exp((mus + b * log(P.p5 * th / dc + 1)) / a));
   }
 }
 
-__device__ inline double f_rsf_theta(const FaultDev& F, int k, double theta, double v) {
-  const double dc = F.p0[k], dt = F.dt;
+__device__ inline double f_rsf_theta(const FaultDev& F, const PairData& P, double theta, double v) {
+  const double dc = P.p0, dt = F.dt;
   switch (F.kind) {
     case 1: {
-      double tn = theta * F.coeft[k] + F.Tc[k] * fabs(v) * (1.0 - F.coeft[k]);
+      double tn = theta * P.coeft + P.Tc * fabs(v) * (1.0 - P.coeft);
       return tn < 1.0e-12 ? 0.0 : tn;
     }
     case 2:
@@ -147,10 +189,10 @@ __device__ inline double f_rsf_theta(const FaultDev& F, int k, double theta, dou
   }
 }
 
-__device__ inline void f_fric(const FaultDev& F, int k, double theta, double tau, double tstick,
+__device__ inline void f_fric(const FaultDev& F, const PairData& P, double theta, double tau, double tstick,
                               double sigma, double Z, double& fv, double& dfv, double& v) {
-  const double dc = F.p0[k], mus = F.p1[k], a = F.p2[k], b = F.p3[k], vs = F.p4[k];
-  double tmp = (F.kind == 4) ? mus + b * log(F.p5[k] * theta / dc + 1.0) : mus + b * log(vs * theta / dc);
+  const double dc = P.p0, mus = P.p1, a = P.p2, b = P.p3, vs = P.p4;
+  double tmp = (F.kind == 4) ? mus + b * log(P.p5 * theta / dc + 1.0) : mus + b * log(vs * theta / dc);
   tmp = 2.0 * vs * exp(-tmp / a);
   v = libm::sinh(tau / (-sigma * a)) * tmp;
   fv = tstick - Z * v - tau;
@@ -158,19 +200,19 @@ __device__ inline void f_fric(const FaultDev& F, int k, double theta, double tau
   dfv = -Z * dv - 1.0;
 }
 
-__device__ inline double f_nr_solver(const FaultDev& F, int k, double xL, double xR, double xacc,
+__device__ inline double f_nr_solver(const FaultDev& F, const PairData& P, double xL, double xR, double xacc,
                                      double theta, double tstick, double sigma, double Z, bool& ok) {
   double flow, fhigh, dfdx, v, xlow, xhigh, dx, dxold, fx;
   ok = true;
-  f_fric(F, k, theta, xL, tstick, sigma, Z, flow, dfdx, v);
-  f_fric(F, k, theta, xR, tstick, sigma, Z, fhigh, dfdx, v);
+  f_fric(F, P, theta, xL, tstick, sigma, Z, flow, dfdx, v);
+  f_fric(F, P, theta, xR, tstick, sigma, Z, fhigh, dfdx, v);
   double xl = xL, xr = xR;
   int guard = 0;
   while (flow * fhigh > 0 && guard++ < 2100) {
     xl = xl / 2.0;
     xr = xr * 2.0;
-    f_fric(F, k, theta, xl, tstick, sigma, Z, flow, dfdx, v);
-    f_fric(F, k, theta, xr, tstick, sigma, Z, fhigh, dfdx, v);
+    f_fric(F, P, theta, xl, tstick, sigma, Z, flow, dfdx, v);
+    f_fric(F, P, theta, xr, tstick, sigma, Z, fhigh, dfdx, v);
   }
   if (flow * fhigh > 0) { ok = false; return v; }
   if (flow == 0) return v;
@@ -179,7 +221,7 @@ __device__ inline double f_nr_solver(const FaultDev& F, int k, double xL, double
   double xest = 0.5 * (xl + xr);
   dxold = fabs(xr - xl);
   dx = dxold;
-  f_fric(F, k, theta, xest, tstick, sigma, Z, fx, dfdx, v);
+  f_fric(F, P, theta, xest, tstick, sigma, Z, fx, dfdx, v);
   for (int is = 1; is <= 200; ++is) {
     if (((xest - xhigh) * dfdx - fx) * ((xest - xlow) * dfdx - fx) > 0 ||
         fabs(2 * fx) > fabs(dxold * dfdx)) {
@@ -195,24 +237,24 @@ __device__ inline double f_nr_solver(const FaultDev& F, int k, double xL, double
       if (tmp == xest) return v;
     }
     if (fabs(dx) < fabs(xacc)) {
-      f_fric(F, k, theta, xest, tstick, sigma, Z, fx, dfdx, v);
+      f_fric(F, P, theta, xest, tstick, sigma, Z, fx, dfdx, v);
       return v;
     }
-    f_fric(F, k, theta, xest, tstick, sigma, Z, fx, dfdx, v);
+    f_fric(F, P, theta, xest, tstick, sigma, Z, fx, dfdx, v);
     if (fx < 0) xlow = xest; else xhigh = xest;
   }
   ok = false;
   return v;
 }
 
-__device__ inline double f_rsf_v(const FaultDev& F, int k, double tstick, double sigma, double theta,
+__device__ inline double f_rsf_v(const FaultDev& F, const PairData& P, double tstick, double sigma, double theta,
                                  double Z, bool& ok) {
   ok = true;
   if (F.kind == 1) {
-    const double dc = F.p0[k], mus = F.p1[k], a = F.p2[k], b = F.p3[k], vs = F.p4[k];
+    const double dc = P.p0, mus = P.p1, a = P.p2, b = P.p3, vs = P.p4;
     // rsf_mu_no_direct reads the stored state (the state before this step), not the
     // updated estimate: SRC/bc_dynflt_rsf.f90:189-196,338
-    const double th0 = F.theta[k];
+    const double th0 = P.theta;
     const double mnd = mus - b * th0 / (th0 + dc);
     double v = (tstick + sigma * mnd) / Z;
     const double tmp = v - vs + sigma * a / Z;
@@ -220,8 +262,8 @@ __device__ inline double f_rsf_v(const FaultDev& F, int k, double tstick, double
     v = fmax(0.0, v);
     return v < 1.0e-12 ? 0.0 : v;
   }
-  const double tol = -0.001 * F.p2[k] * sigma;
-  return f_nr_solver(F, k, fmin(0.0, tstick), fmax(0.0, tstick), tol, theta, tstick, sigma, Z, ok);
+  const double tol = -0.001 * P.p2 * sigma;
+  return f_nr_solver(F, P, fmin(0.0, tstick), fmax(0.0, tstick), tol, theta, tstick, sigma, Z, ok);
 }
 
 // One node component by component: the predicted displacement and velocity and the force.
@@ -235,8 +277,8 @@ struct NodeState {
 // the nodes' forces.  time = it*dt of the step (SRC/main.f90:53), read by time-weakening
 // friction only.
 template <typename R, int nd>
-__device__ inline void fault_solve(const FaultDev& F, int k, double time, bool two, NodeState<R>& n1,
-                                   NodeState<R>& n2) {
+__device__ inline PairOut fault_solve(const FaultDev& F, const PairData& P, int k, double time, bool two,
+                                      NodeState<R>& n1, NodeState<R>& n2) {
   const int np = F.np;
   double dD[2] = {0, 0}, dV[2] = {0, 0}, dA[2] = {0, 0}, T[2] = {0, 0}, Ts[2];
 #pragma unroll
@@ -244,15 +286,15 @@ __device__ inline void fault_solve(const FaultDev& F, int k, double time, bool t
     if (two) {
       dD[c] = (double)n2.d[c] - (double)n1.d[c];
       dV[c] = (double)n2.v[c] - (double)n1.v[c];
-      dA[c] = F.invM2[c * np + k] * (double)n2.f[c] - F.invM1[c * np + k] * (double)n1.f[c];
+      dA[c] = P.iM2[c] * (double)n2.f[c] - P.iM1[c] * (double)n1.f[c];
     } else {  // one side: get_jump, get_weighted_jump (SRC/bc_dynflt.f90:692-719)
       dD[c] = -2.0 * (double)n1.d[c];
       dV[c] = -2.0 * (double)n1.v[c];
-      dA[c] = -2.0 * F.invM1[c * np + k] * (double)n1.f[c];
+      dA[c] = -2.0 * P.iM1[c] * (double)n1.f[c];
     }
-    T[c] = F.Z[c * np + k] * (dV[c] + F.a2v * dA[c]);
+    T[c] = P.Z[c] * (dV[c] + F.a2v * dA[c]);
   }
-  const double nx = F.nrm[k], nz = F.nrm[np + k];
+  const double nx = P.nx, nz = P.nz;
   if (nd == 2) {
     double r0, r1;
     r0 = nz * dD[0] - nx * dD[1]; r1 = nx * dD[0] + nz * dD[1]; dD[0] = r0; dD[1] = r1;
@@ -261,57 +303,50 @@ __device__ inline void fault_solve(const FaultDev& F, int k, double time, bool t
     r0 = nz * T[0] - nx * T[1];   r1 = nx * T[0] + nz * T[1];   T[0] = r0;  T[1] = r1;
   }
   if (nd == 1 || !two) T[1] = 0.0;  // SRC/bc_dynflt.f90:604
-  T[0] = T[0] + F.T0[k];
-  T[1] = T[1] + F.T0[np + k];
+  T[0] = T[0] + P.T0[0];
+  T[1] = T[1] + P.T0[1];
   if (F.opening) T[1] = fmin(T[1], 0.0);
-  const double sigma = normal_sigma(F.nor_kind, F.nor_coef, F.nor_v, F.sigma[k], T[1], dV[0]);
-  F.sigma[k] = sigma;
+  const double sigma = normal_sigma(F.nor_kind, F.nor_coef, F.nor_v, P.sigma, T[1], dV[0]);
   Ts[0] = T[0];
   Ts[1] = T[1];
+  double th = P.theta, mu;  // friction state and coefficient
   if (F.law == 2) {
-    const double vold = F.V[k], Z1 = F.Z[k];
+    const double vold = P.V, Z1 = P.Z[0];
     bool ok1, ok2;
-    double th = f_rsf_theta(F, k, F.theta[k], vold);
-    double vn = f_rsf_v(F, k, T[0], sigma, th, Z1, ok1);
-    th = f_rsf_theta(F, k, F.theta[k], 0.5 * (vold + vn));
-    vn = f_rsf_v(F, k, T[0], sigma, th, Z1, ok2);
+    th = f_rsf_theta(F, P, P.theta, vold);
+    double vst = f_rsf_v(F, P, T[0], sigma, th, Z1, ok1);
+    th = f_rsf_theta(F, P, P.theta, 0.5 * (vold + vst));
+    vst = f_rsf_v(F, P, T[0], sigma, th, Z1, ok2);
     if (!(ok1 && ok2)) atomicOr(F.nr_fail, 1);
-    F.theta[k] = th;
-    F.V[k] = vn;
-    F.MU[k] = f_rsf_mu(F, k, vn);
+    mu = f_rsf_mu(F, P, th, vst);
     // superimposed time weakening (SRC/bc_dynflt.f90:632)
-    if (F.twf) F.MU[k] = fmin(F.MU[k], f_twf_mu(F, k, time, F.D[k]));
-    const double strength = -F.MU[k] * sigma;
+    if (F.twf) mu = fmin(mu, f_twf_mu(F, k, time, P.D));
+    const double strength = -mu * sigma;
     T[0] = copysign(fabs(strength), T[0]);
   } else if (F.law == 3) {  // time weakening alone (SRC/bc_dynflt.f90:656-657)
-    F.MU[k] = f_twf_mu(F, k, time, F.D[k]);
-    const double strength = F.coh[k] - F.MU[k] * sigma;
+    mu = f_twf_mu(F, k, time, P.D);
+    const double strength = P.coh - mu * sigma;
     T[0] = copysign(fmin(fabs(T[0]), strength), T[0]);
   } else {
     if (F.a2d == 0.0) {
       if (F.healing) {
-        double th = F.theta[k] + fabs(dV[0]) * F.dt;
+        th = P.theta + fabs(dV[0]) * F.dt;
         if (fabs(dV[0]) < 1e-14) th = 0.0;
-        F.theta[k] = th;
       } else {
-        F.theta[k] = fabs(dD[0]);
+        th = fabs(dD[0]);
       }
     } else {
-      F.theta[k] = fabs(F.D[k]);
+      th = fabs(P.D);
     }
-    F.MU[k] = f_swf_mu(F, k);
-    if (F.twf) F.MU[k] = fmin(F.MU[k], f_twf_mu(F, k, time, F.D[k]));  // :653
-    const double strength = F.coh[k] - F.MU[k] * sigma;
+    mu = f_swf_mu(F, P, th);
+    if (F.twf) mu = fmin(mu, f_twf_mu(F, k, time, P.D));  // :653
+    const double strength = P.coh - mu * sigma;
     T[0] = copysign(fmin(fabs(T[0]), strength), T[0]);
   }
-  T[0] = T[0] - F.T0[k];
-  T[1] = T[1] - F.T0[np + k];
-  Ts[0] = Ts[0] - F.T0[k];
-  Ts[1] = Ts[1] - F.T0[np + k];
-  F.T[k] = T[0];
-  F.T[np + k] = T[1];
-  F.Tstick[k] = Ts[0];
-  F.Tstick[np + k] = Ts[1];
+  T[0] = T[0] - P.T0[0];
+  T[1] = T[1] - P.T0[1];
+  Ts[0] = Ts[0] - P.T0[0];
+  Ts[1] = Ts[1] - P.T0[1];
   double Tx[2] = {T[0], T[1]};
   if (nd == 2) {
     Tx[0] = nz * T[0] + nx * T[1];
@@ -319,17 +354,29 @@ __device__ inline void fault_solve(const FaultDev& F, int k, double time, bool t
   }
 #pragma unroll
   for (int c = 0; c < nd; ++c) {
-    const double bt = F.B[c * np + k] * Tx[c];
+    const double bt = P.B[c] * Tx[c];
     n1.f[c] = (R)((double)n1.f[c] + bt);
     if (two) n2.f[c] = (R)((double)n2.f[c] - bt);
   }
+  F.sigma[k] = sigma;
+  if (F.law != 3) F.theta[k] = th;
+  F.MU[k] = mu;
+  F.T[k] = T[0];
+  F.T[np + k] = T[1];
+  F.Tstick[k] = Ts[0];
+  F.Tstick[np + k] = Ts[1];
+  PairOut out;
+  out.T[0] = T[0], out.T[1] = T[1], out.Ts0 = Ts[0], out.mu = mu;
 #pragma unroll
   for (int c = 0; c < nd; ++c) {
     const double tf = T[c];
-    const double da = dA[c] - tf / (F.Z[c * np + k] * F.a2v);
-    F.D[c * np + k] = dD[c] + F.a2d * da;
-    F.V[c * np + k] = dV[c] + F.a2v * da;
+    const double da = dA[c] - tf / (P.Z[c] * F.a2v);
+    const double D = dD[c] + F.a2d * da, V = dV[c] + F.a2v * da;
+    F.D[c * np + k] = D;
+    F.V[c * np + k] = V;
+    if (c == 0) out.D0 = D, out.V0 = V;
   }
+  return out;
 }
 
 // Fault of the general path: the pair's forces updated in place; every node is corrected
@@ -353,7 +400,7 @@ __global__ __launch_bounds__(64) void k_fault(FaultDev F, const R* d, const R* v
       n2.f[c] = f[o + i2];
     }
   }
-  fault_solve<R, nd>(F, k, time, i2 >= 0, n1, n2);
+  fault_solve<R, nd>(F, pair_load<nd>(F, k, i2 >= 0), k, time, i2 >= 0, n1, n2);
 #pragma unroll
   for (int c = 0; c < nd; ++c) {
     const size_t o = (size_t)c * npoin;
@@ -513,12 +560,12 @@ struct FaultOut {
 // a fault alone and inside a batch.  (One workgroup over all pairs took 12 us of a 79 us
 // step, 600 x 300 elements; this adds 1-2 us to the fault's.)
 template <int nd>
-__device__ inline void potency_wave(const FaultDev& F, const FaultOut& O, int w, int k, bool on, const double* dj,
-                                    const double* vj, int row) {
-  const int lane = threadIdx.x & 63, np = F.np;
+__device__ inline void potency_wave(const PairData& P, const FaultOut& O, int w, int m, int2 mw, bool on,
+                                    const double* dj, const double* vj, int row) {
+  const int lane = threadIdx.x & 63;
   double s[6] = {0, 0, 0, 0, 0, 0};
   if (on) {
-    const double nx = F.nrm[k], nz = F.nrm[np + k], b = F.B[k];
+    const double nx = P.nx, nz = P.nz, b = P.B[0];
     if (nd == 2) {
       s[0] = nx * dj[0] * b;
       s[1] = nz * dj[1] * b;
@@ -540,18 +587,20 @@ __device__ inline void potency_wave(const FaultDev& F, const FaultOut& O, int w,
       for (int q = 0; q < 6; ++q) s[q] = s[q] + __shfl_xor(s[q], o);
   };
   tree();
-  const int m = O.wave[w].z;
-  const int2 mw = O.member[m];
   unsigned before = 0;
   if (lane == 0) {
 #pragma unroll
     for (int q = 0; q < 6; ++q)
       __hip_atomic_store(&O.part[(size_t)w * 6 + q], s[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    before = __hip_atomic_fetch_add(&O.cnt[m], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    // the sums have to be in device memory before the count; they are stored past the L2
+    // (agent scope), so waiting for the stores is enough, and the write-back of the whole L2
+    // that a release at agent scope makes is not needed
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    before = __hip_atomic_fetch_add(&O.cnt[m], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   before = __shfl(before, 0);
   if (before + 1 != (unsigned)mw.y) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  asm volatile("" ::: "memory");  // the sums are read (past the L2 too) after the count
 #pragma unroll
   for (int q = 0; q < 6; ++q) s[q] = 0;
   for (int u = lane; u < mw.y; u += 64)

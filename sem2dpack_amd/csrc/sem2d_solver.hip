@@ -90,6 +90,7 @@ struct StructState {
   void* fpart = nullptr;
   size_t FPS = 0;
   DefTable defs;
+  const DefDev* fdef = nullptr;  // entries of the fault pairs' nodes, [side][pair]
   DefDev* gen_def = nullptr;  // general path: the records of defs
   int ndef = 0;
   int* part_off = nullptr;
@@ -670,7 +671,7 @@ static bool fits32(size_t ngp, size_t fps, size_t ncoef, size_t rs) {
 // device form of a deferred-node list (DefDev records and their side table); false when
 // a count does not fit its 8 bits
 bool pack_defs(const std::vector<DefNode>& in, const std::vector<int>& part_off, std::vector<DefDev>& node,
-               std::vector<int2>& ext) {
+               std::vector<int4>& ext) {
   node.resize(in.size());
   ext.clear();
   for (size_t q = 0; q < in.size(); ++q) {
@@ -682,9 +683,9 @@ bool pack_defs(const std::vector<DefNode>& in, const std::vector<int>& part_off,
     e.cnt = n.pcnt | (n.scnt << 8) | (n.acnt << 16) | ((n.fault ? 1 : 0) << 24) | ((n.dmask & 3) << 26) |
             ((n.rec ? 1 : 0) << 28);
     e.x = -1;
-    if (n.scnt > 0 || n.acnt > 0) {
+    if (n.scnt > 0 || n.acnt > 0 || n.rec_at >= 0) {
       e.x = (int)ext.size();
-      ext.push_back(make_int2(n.sstart, n.astart));
+      ext.push_back(make_int4(n.sstart, n.astart, n.rec_at, 0));
     } else if (!part_off.empty() && (n.pcnt == 1 || n.pcnt == 2)) {  // offsets inline
       e.cnt |= 1 << 25;
       e.pstart = part_off[n.pstart];
@@ -733,7 +734,8 @@ struct StructTables {
   std::vector<uint32_t> marks;
   // receivers at nodes (RecOut): (storage index, or deferred node, or 2 * pair + side; receiver)
   std::vector<std::pair<int, int>> rec_int, rec_def, rec_flt;
-  std::vector<int> fault_def1, fault_def2;  // the pairs' nodes in defs
+  std::vector<int> fault_def1, fault_def2;  // the pairs' nodes as k_deferred counts them (-1: one side)
+  std::vector<int> fault_at;                // [side][pair]: their places in defs (one side: side 1 twice)
   std::vector<double> s_K;
 };
 
@@ -976,6 +978,7 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
     n.fault = is_fault[ref];
     n.dmask = dmask_def[ref];
     n.rec = is_rec[ref];
+    n.rec_at = -1;
     X.defs.push_back(n);
     def_ref[i] = ref;
   }
@@ -1018,6 +1021,14 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   std::sort(X.rec_int.begin(), X.rec_int.end());
   std::sort(X.rec_def.begin(), X.rec_def.end());
   std::sort(X.rec_flt.begin(), X.rec_flt.end());
+  std::vector<int> at((size_t)h->npoin, -1);  // reference node -> its place in defs
+  for (size_t q = 0; q < ndef; ++q) at[def_ref[q]] = (int)q;
+  for (int k = (int)X.rec_def.size() - 1; k >= 0; --k) X.defs[at[h->rec_ref[X.rec_def[k].second]]].rec_at = k;
+  for (int k = (int)X.rec_flt.size() - 1; k >= 0; --k) X.defs[at[h->rec_ref[X.rec_flt[k].second]]].rec_at = k;
+  X.fault_at.clear();
+  for (int side = 0; side < 2; ++side)
+    for (size_t k = 0; k < h->fault_n1.size(); ++k)
+      X.fault_at.push_back(at[side && !h->fault_n2.empty() ? h->fault_n2[k] : h->fault_n1[k]]);
   // recorded nodes that are not deferred nodes: marks of the tile they lie in
   X.mark_of.assign(S.on ? S.ntiles : 0, -1);
   X.marks.clear();
@@ -1094,13 +1105,18 @@ int prepare_structured(sem2d_solver* h) {
   }
   {
     std::vector<DefDev> dn;
-    std::vector<int2> dx;
+    std::vector<int4> dx;
     if (!pack_defs(X.defs, X.part_off, dn, dx))
       return set_err(h, 5, "prepare: more than 255 entries at a deferred node");
     DefDev* pn = nullptr;
-    int2* px = nullptr;
+    int4* px = nullptr;
     if ((rc = prep_upload(h, &pn, dn.data(), dn.size()))) return rc;
     if ((rc = prep_upload(h, &px, dx.data(), dx.size()))) return rc;
+    std::vector<DefDev> fd;
+    for (int i : X.fault_at) fd.push_back(dn[i]);
+    DefDev* pf = nullptr;
+    if ((rc = prep_upload(h, &pf, fd.data(), fd.size()))) return rc;
+    S.fdef = pf;
     if (!S.on && !dn.empty())
       k_gen_put<<<grid_for(dn.size(), 256), 256, 0, h->stream>>>((int)dn.size(), pn, S.gen_def);
     HIPCHK(h, hipStreamSynchronize(h->stream));  // the packed copies are local
@@ -1225,6 +1241,7 @@ struct StepDev {
   void* fpart = nullptr;
   int ndef = 0;
   DefTable defs;
+  const DefDev* fdef = nullptr;
   const int* part_off = nullptr;
   const SrcEntry* dsrc = nullptr;
   const double *dabso = nullptr, *dabson = nullptr;
@@ -1282,7 +1299,7 @@ StepDev step_dev(sem2d_solver* h) {
   X.geom = S.geom;
   X.fpart = S.fpart;
   X.ndef = S.ndef;
-  X.defs = S.defs;
+  X.defs = S.defs, X.fdef = S.fdef;
   X.part_off = S.part_off;
   X.dsrc = S.dsrc;
   X.dabso = S.dabso;
@@ -1392,6 +1409,7 @@ void launch_structured_step(const StepDev& X, int it, R dt, R c1, R c2, R c3, R 
   A.din = (const R*)X.din, A.vin = (const R*)X.vin, A.ain = (const R*)X.ain;
   A.SR = X.SR, A.rec = X.recout;
   A.rec.src = !X.out.final ? (const void*)A.recp : (A.rec.field == 0 ? X.d : (A.rec.field == 1 ? X.v : X.a));
+  A.fdef = X.fdef;
   if (X.fault_on) A.F = X.F, A.fo = X.fo;
   const int lanes = X.ndef + A.rec.nint + (X.fault_on ? A.fo.nwave * 64 : 0);
   auto deferred = [&](auto nd, auto oop, auto pin, auto flt) {
@@ -3023,6 +3041,9 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
     A.marks.insert(A.marks.end(), X.marks.begin(), X.marks.end());
     {  // the lists of k_deferred, with the member's offsets
       const int db = (int)A.defs.size(), rb = nrec, fb = 2 * (int)A.fault_def1.size();
+      const int rd = (int)A.rec_def.size(), rf = (int)A.rec_flt.size();
+      for (DefNode& d : X.defs)
+        if (d.rec_at >= 0) d.rec_at += d.fault ? rf : rd;
       for (int q : X.fault_def1) A.fault_def1.push_back(q + db);
       for (int q : X.fault_def2) A.fault_def2.push_back(q < 0 ? -1 : q + db);
       for (auto& e : X.rec_int) A.rec_int.push_back({e.first + (int)nb, e.second + rb});
@@ -3073,7 +3094,7 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
   int4 *tiles, *grids;
   int *sc, *si, *po;
   DefDev* defs;
-  int2* defx;
+  int4* defx;
   SrcEntry* ds;
   double *dab, *amp;
   if ((rc = bupload(b, &tiles, A.tiles))) return rc;
@@ -3088,10 +3109,16 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
   X.marks = mk;
   {
     std::vector<DefDev> dn;
-    std::vector<int2> dx;
+    std::vector<int4> dx;
     if (!pack_defs(A.defs, A.part_off, dn, dx)) return berr(b, 5, "batch: more than 255 entries at a deferred node");
     if ((rc = bupload(b, &defs, dn))) return rc;
     if ((rc = bupload(b, &defx, dx))) return rc;
+    std::vector<DefDev> fd;
+    for (int q : A.fault_def1) fd.push_back(dn[q]);
+    for (size_t k = 0; k < A.fault_def2.size(); ++k) fd.push_back(dn[A.fault_def2[k] < 0 ? A.fault_def1[k] : A.fault_def2[k]]);
+    DefDev* pf = nullptr;
+    if ((rc = bupload(b, &pf, fd))) return rc;
+    X.fdef = pf;
   }
   if ((rc = bupload(b, &po, A.part_off))) return rc;
   if ((rc = bupload(b, &ds, A.dsrc))) return rc;

@@ -820,15 +820,16 @@ struct DefNode {
                 // absorbing terms; at a fault node, those of the Dirichlet boundaries that
                 // act before the fault
   int rec;      // recorded node (StepOut::rec)
+  int rec_at;   // its first entry in the receiver list (RecOut), or -1
   int pinl;     // device form only: 1 when the two partial offsets are poff (pcnt == 2)
   int poff[2];  // the second is -1 when pcnt == 1
 };
 
 // Device form of a deferred-node list: 16 bytes per node (one vector load) plus a side
-// table for the few nodes with sources or absorbing terms.  cnt packs pcnt (bits 0-7),
+// table for the few nodes with sources, absorbing terms or receivers.  cnt packs pcnt (bits 0-7),
 // scnt (bits 8-15), acnt (bits 16-23), fault (bit 24), "offsets inline" (bit 25), the
 // Dirichlet mask (bits 26-27) and "recorded" (bit 28); x
-// is the node's (sstart, astart) entry in ext, or -1 when it has neither.  A node with
+// is the node's (sstart, astart, rec_at, -) entry in ext, or -1 when it has none of them.  A node with
 // one or two partial forces and no ext entry (a tile-edge node, most nodes of the general
 // path) holds its partial offsets in pstart and x instead (bit 25 set), so part_off is not
 // read for it.
@@ -837,10 +838,9 @@ struct alignas(16) DefDev {
 };
 struct DefTable {
   const DefDev* node = nullptr;
-  const int2* ext = nullptr;
+  const int4* ext = nullptr;
 };
-__device__ __forceinline__ DefNode def_unpack(const DefTable& D, int q) {
-  const DefDev e = D.node[q];
+__device__ __forceinline__ DefNode def_unpack(const DefTable& D, const DefDev e) {
   DefNode n;
   n.g = e.g;
   n.pstart = e.pstart;
@@ -853,17 +853,20 @@ __device__ __forceinline__ DefNode def_unpack(const DefTable& D, int q) {
   n.rec = (e.cnt >> 28) & 1;
   n.sstart = 0;
   n.astart = 0;
+  n.rec_at = -1;
   n.poff[0] = n.poff[1] = 0;
   if (n.pinl) {
     n.poff[0] = e.pstart;
     n.poff[1] = e.x;
   } else if (e.x >= 0) {
-    const int2 x = D.ext[e.x];
+    const int4 x = D.ext[e.x];
     n.sstart = x.x;
     n.astart = x.y;
+    n.rec_at = x.z;
   }
   return n;
 }
+__device__ __forceinline__ DefNode def_unpack(const DefTable& D, int q) { return def_unpack(D, D.node[q]); }
 
 // Stacey terms of the absorbing entries of the deferred nodes: entry q (the q-th
 // absorbing coefficient set of the step, in boundary order) subtracts kxd[idx[t]],
@@ -919,16 +922,26 @@ __device__ __forceinline__ double* rec_rows(const RecOut& P, int ndof, int it) {
   if (!P.seis || it % P.isamp || it / P.isamp >= P.nsamp) return nullptr;
   return P.seis + (size_t)(it / P.isamp) * ndof * P.nrec;
 }
-// component c of the receivers listed under key in q[0 .. n)
-__device__ __forceinline__ void rec_put(double* rows, const RecOut& P, const int* __restrict__ q,
-                                        const int* __restrict__ r, int n, int key, int c, double x) {
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    const int m = (lo + hi) >> 1;
-    if (q[m] < key) lo = m + 1;
-    else hi = m;
+// The receivers of one node: entries at, at + 1, ... of the list with the same key.  The
+// first one and the key after it are loaded ahead of the node's stores, not searched for in
+// the list after them (log2(n) loads one after the other).
+struct RecRef {
+  int at = -1, r = 0, next = -1;
+};
+__device__ __forceinline__ RecRef rec_ref(const int* __restrict__ q, const int* __restrict__ r, int n, int at) {
+  RecRef p;
+  p.at = at;
+  if (at >= 0) {
+    p.r = r[at];
+    p.next = q[min(at + 1, n - 1)];
   }
-  for (; lo < n && q[lo] == key; ++lo) rows[(size_t)c * P.nrec + r[lo]] = x;
+  return p;
+}
+__device__ __forceinline__ void rec_put(double* rows, const RecOut& P, const int* __restrict__ q,
+                                        const int* __restrict__ r, int n, const RecRef& p, int key, int c, double x) {
+  rows[(size_t)c * P.nrec + p.r] = x;
+  if (p.next != key) return;
+  for (int l = p.at + 1; l < n && q[l] == key; ++l) rows[(size_t)c * P.nrec + r[l]] = x;
 }
 
 // Arguments of k_deferred
@@ -957,47 +970,104 @@ struct DefArgs {
   RecOut rec;
   FaultDev F;
   FaultOut fo;
+  const DefDev* fdef;  // [side][np]: the list entries of the pairs' nodes
 };
 
-// Predicted state of deferred node n and its force: the partial forces of its tiles, the
-// sources, the absorbing terms and the Dirichlet components
+// What a deferred node reads, loaded in one group before anything is stored: its state,
+// inverse mass, up to four partial forces, its first source and absorbing entry.  The launch
+// is bound by the chain list entry -> values -> stores, a round trip to memory each: with
+// loads behind the first stores (which may alias them) and the partial forces one by one it
+// took 7.8 us on 100 x 100 P-SV elements and 14.7 us on the 386 000 nodes of a 201 x 120
+// layered mesh, now 4.0 and 11.0.
+template <typename R, int NDOF>
+struct DefVals {
+  R d[NDOF], v[NDOF], a[NDOF], rm[NDOF], f[4][NDOF];
+  double C[NDOF], am;
+  SrcEntry e;
+};
 template <typename R, int NDOF, bool OOP, bool PIN>
-__device__ __forceinline__ NodeState<R> def_state(const DefArgs<R>& A, const DefNode& n, int it) {
+__device__ __forceinline__ DefVals<R, NDOF> def_load(const DefArgs<R>& A, const DefNode& n, int q, int it) {
   const size_t g = n.g, GS = A.GS;
+  DefVals<R, NDOF> s;
   // out of place: a null vin / ain reads v / a (their step is then in place)
   const R* dsrc = OOP ? A.din : A.d;
   const R* vsrc = OOP && A.vin ? A.vin : A.v;
   const R* asrc = OOP && A.ain ? A.ain : A.a;
+  int o[4] = {0, 0, 0, 0};
+  if (n.pinl) {
+    o[0] = n.poff[0];
+    o[1] = n.poff[1] >= 0 ? n.poff[1] : o[0];
+  } else if (n.pcnt > 0) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = A.part_off[n.pstart + min(k, n.pcnt - 1)];
+  }
+#pragma unroll
+  for (int c = 0; c < NDOF; ++c) {
+    s.d[c] = dsrc[c * GS + g];
+    s.v[c] = vsrc[c * GS + g];
+    if constexpr (!PIN) s.a[c] = asrc[c * GS + g];
+    s.rm[c] = A.rmdef[(size_t)c * A.ndef + q];
+  }
+#pragma unroll
+  for (int c = 0; c < NDOF; ++c) {
+    s.f[0][c] = A.fpart[c * A.FPS + o[0]];
+    s.f[1][c] = A.fpart[c * A.FPS + o[1]];
+  }
+  if (!n.pinl) {
+#pragma unroll
+    for (int c = 0; c < NDOF; ++c) {
+      s.f[2][c] = A.fpart[c * A.FPS + o[2]];
+      s.f[3][c] = A.fpart[c * A.FPS + o[3]];
+    }
+  }
+  if (n.acnt > 0) {
+#pragma unroll
+    for (int c = 0; c < NDOF; ++c) s.C[c] = A.abso[(size_t)n.astart * NDOF + c];
+  }
+  if (n.scnt > 0) {
+    s.e = A.src[n.sstart];
+    s.am = (it >= 1 && it <= A.nt) ? A.ampl[(size_t)s.e.src * A.nt + (it - 1)] : 0.0;
+  }
+  return s;
+}
+
+// Predicted state of deferred node n and its force: the partial forces of its tiles, the
+// sources, the absorbing terms and the Dirichlet components
+template <typename R, int NDOF, bool PIN>
+__device__ __forceinline__ NodeState<R> def_state(const DefArgs<R>& A, const DefNode& n,
+                                                  const DefVals<R, NDOF>& x, int it) {
   NodeState<R> s;
 #pragma unroll
   for (int c = 0; c < NDOF; ++c) {
-    const R dk = dsrc[c * GS + g], vk = vsrc[c * GS + g];
     if constexpr (PIN) {
-      s.d[c] = dk;
-      s.v[c] = vk;
+      s.d[c] = x.d[c];
+      s.v[c] = x.v[c];
     } else {
-      const R ak = asrc[c * GS + g];
-      s.d[c] = dk + A.dt * vk + A.c1 * ak;
-      s.v[c] = vk + A.c2 * ak;
+      s.d[c] = x.d[c] + A.dt * x.v[c] + A.c1 * x.a[c];
+      s.v[c] = x.v[c] + A.c2 * x.a[c];
     }
     R f = 0;
-    if (n.pinl) {  // the loop below with pcnt = 1 or 2
-      f = f + A.fpart[c * A.FPS + n.poff[0]];
-      if (n.poff[1] >= 0) f = f + A.fpart[c * A.FPS + n.poff[1]];
-    } else {
-      for (int k = 0; k < n.pcnt; ++k) f = f + A.fpart[c * A.FPS + A.part_off[n.pstart + k]];
+    if (n.pcnt > 0) f = f + x.f[0][c];
+    if (n.pcnt > 1) f = f + x.f[1][c];
+    if (!n.pinl) {
+      if (n.pcnt > 2) f = f + x.f[2][c];
+      if (n.pcnt > 3) f = f + x.f[3][c];
+      for (int k = 4; k < n.pcnt; ++k) f = f + A.fpart[c * A.FPS + A.part_off[n.pstart + k]];
     }
     s.f[c] = f;
   }
   for (int k = 0; k < n.scnt; ++k) {
-    const SrcEntry e = A.src[n.sstart + k];
-    const double am = (it >= 1 && it <= A.nt) ? A.ampl[(size_t)e.src * A.nt + (it - 1)] : 0.0;
+    const SrcEntry e = k == 0 ? x.e : A.src[n.sstart + k];
+    double am = x.am;
+    if (k) am = (it >= 1 && it <= A.nt) ? A.ampl[(size_t)e.src * A.nt + (it - 1)] : 0.0;
 #pragma unroll
     for (int c = 0; c < NDOF; ++c)
       if (c == e.comp) s.f[c] = (R)((double)s.f[c] + e.coef * am);
   }
   for (int k = 0; k < n.acnt; ++k) {
-    const double* C = A.abso + (size_t)(n.astart + k) * NDOF;
+    double C[NDOF];
+#pragma unroll
+    for (int c = 0; c < NDOF; ++c) C[c] = k == 0 ? x.C[c] : A.abso[(size_t)(n.astart + k) * NDOF + c];
     bool skew = false;
     if constexpr (NDOF == 2) {
       if (A.abson) {  // a boundary that is not flat (k_abso_normal)
@@ -1081,61 +1151,71 @@ __global__ __launch_bounds__(256) void k_deferred(DefArgs<R> A) {
     const int w = q >> 6;  // uniform in a wavefront
     if (w < A.fo.nwave) {
       const FaultDev& F = A.F;
-      const int4 wv = A.fo.wave[w];
+      const FaultOut& O = A.fo;
+      const int4 wv = O.wave[w];
+      const int2 mw = O.member[wv.z];
       const int lane = q & 63, k = wv.x + lane;
       const bool on = lane < wv.y;
+      PairData P;
       double dj[2] = {0, 0}, vj[2] = {0, 0};
       if (on) {
         const int np = F.np;
         const int q1 = F.def1[k], q2 = F.def2[k];
+        const DefDev e1 = A.fdef[k], e2 = A.fdef[np + k];
         const bool two = q2 >= 0;
-        const DefNode m1 = def_unpack(A.defs, q1);
-        DefNode m2 = m1;
-        NodeState<R> n1 = def_state<R, NDOF, OOP, PIN>(A, m1, it), n2;
-        if (two) {
-          m2 = def_unpack(A.defs, q2);
-          n2 = def_state<R, NDOF, OOP, PIN>(A, m2, it);
-        }
-        fault_solve<R, NDOF>(F, k, (double)it * F.dt, two, n1, n2);
+        int rs = O.rec_slot;
+        if (A.itp) rs = it >= O.oit0 && (it - O.oit0) % O.oitd == 0 ? (it - O.oit0) / O.oitd : -1;
+        const int slot = rs >= 0 && rs < O.nsamp ? O.slot[k] : -1;
         const int dm = F.dmask ? F.dmask[k] : 0;
+        P = pair_load<NDOF>(F, k, two);
+        const DefNode m1 = def_unpack(A.defs, e1), m2 = def_unpack(A.defs, e2);
+        const DefVals<R, NDOF> x1 = def_load<R, NDOF, OOP, PIN>(A, m1, q1, it);
+        DefVals<R, NDOF> x2;
+        if (two) x2 = def_load<R, NDOF, OOP, PIN>(A, m2, q2, it);
+        RecRef r1, r2;
+        if (rows) {
+          r1 = rec_ref(A.rec.flt_q, A.rec.flt_r, A.rec.nfltr, m1.rec_at);
+          if (two) r2 = rec_ref(A.rec.flt_q, A.rec.flt_r, A.rec.nfltr, m2.rec_at);
+        }
+        NodeState<R> n1 = def_state<R, NDOF, PIN>(A, m1, x1, it), n2;
+        if (two) n2 = def_state<R, NDOF, PIN>(A, m2, x2, it);
+        const PairOut po = fault_solve<R, NDOF>(F, P, k, (double)it * F.dt, two, n1, n2);
         R* side = (R*)F.side + k;  // [d, v][node][ndof][np]
 #pragma unroll
         for (int c = 0; c < NDOF; ++c) {
           if (dm >> c & 1) n1.f[c] = 0;
-          const R a1 = n1.f[c] * A.rmdef[(size_t)c * A.ndef + q1];
+          const R a1 = n1.f[c] * x1.rm[c];
           def_store<R>(A, n1, c, (size_t)c * A.GS + m1.g, a1, m1.rec);
           side[(size_t)c * np] = n1.d[c];
           side[(size_t)(2 * NDOF + c) * np] = n1.v[c];
-          if (rows && m1.rec)
-            rec_put(rows, A.rec, A.rec.flt_q, A.rec.flt_r, A.rec.nfltr, 2 * k, c, rec_value<R>(A.rec, n1, c, a1));
+          if (r1.at >= 0)
+            rec_put(rows, A.rec, A.rec.flt_q, A.rec.flt_r, A.rec.nfltr, r1, 2 * k, c,
+                    rec_value<R>(A.rec, n1, c, a1));
           if (two) {
             if (dm >> (2 + c) & 1) n2.f[c] = 0;
-            const R a2 = n2.f[c] * A.rmdef[(size_t)c * A.ndef + q2];
+            const R a2 = n2.f[c] * x2.rm[c];
             def_store<R>(A, n2, c, (size_t)c * A.GS + m2.g, a2, m2.rec);
             side[(size_t)(NDOF + c) * np] = n2.d[c];
             side[(size_t)(3 * NDOF + c) * np] = n2.v[c];
-            if (rows && m2.rec)
-              rec_put(rows, A.rec, A.rec.flt_q, A.rec.flt_r, A.rec.nfltr, 2 * k + 1, c,
+            if (r2.at >= 0)
+              rec_put(rows, A.rec, A.rec.flt_q, A.rec.flt_r, A.rec.nfltr, r2, 2 * k + 1, c,
                       rec_value<R>(A.rec, n2, c, a2));
           }
           // get_jump (SRC/bc_dynflt.f90:692-704): x2 - x1, or -2 x1 on a one-sided fault
           dj[c] = two ? (double)n2.d[c] - (double)n1.d[c] : -2.0 * (double)n1.d[c];
           vj[c] = two ? (double)n2.v[c] - (double)n1.v[c] : -2.0 * (double)n1.v[c];
         }
-        const FaultOut& O = A.fo;
-        int rs = O.rec_slot;
-        if (A.itp) rs = it >= O.oit0 && (it - O.oit0) % O.oitd == 0 ? (it - O.oit0) / O.oitd : -1;
-        if (rs >= 0 && rs < O.nsamp && O.slot[k] >= 0) {
-          double* out = O.rec + (size_t)rs * 6 * O.nout + O.slot[k];
-          out[0] = F.D[k];
-          out[(size_t)1 * O.nout] = F.V[k];
-          out[(size_t)2 * O.nout] = F.T[k];
-          out[(size_t)3 * O.nout] = F.T[np + k];
-          out[(size_t)4 * O.nout] = F.MU[k];
-          out[(size_t)5 * O.nout] = F.Tstick[k];
+        if (slot >= 0) {
+          double* out = O.rec + (size_t)rs * 6 * O.nout + slot;
+          out[0] = po.D0;
+          out[(size_t)1 * O.nout] = po.V0;
+          out[(size_t)2 * O.nout] = po.T[0];
+          out[(size_t)3 * O.nout] = po.T[1];
+          out[(size_t)4 * O.nout] = po.mu;
+          out[(size_t)5 * O.nout] = po.Ts0;
         }
       }
-      potency_wave<NDOF>(F, A.fo, w, k, on, dj, vj, A.fo.pot_row + (A.itp ? it : 0));
+      potency_wave<NDOF>(P, O, w, wv.z, mw, on, dj, vj, O.pot_row + (A.itp ? it : 0));
       return;
     }
     q -= A.fo.nwave * 64;
@@ -1150,13 +1230,16 @@ __global__ __launch_bounds__(256) void k_deferred(DefArgs<R> A) {
   }
   const DefNode n = def_unpack(A.defs, q);
   if (FLT && n.fault) return;
-  NodeState<R> s = def_state<R, NDOF, OOP, PIN>(A, n, it);
+  const DefVals<R, NDOF> x = def_load<R, NDOF, OOP, PIN>(A, n, q, it);
+  RecRef rr;
+  if (rows) rr = rec_ref(A.rec.def_q, A.rec.def_r, A.rec.ndefr, n.rec_at);
+  NodeState<R> s = def_state<R, NDOF, PIN>(A, n, x, it);
 #pragma unroll
   for (int c = 0; c < NDOF; ++c) {
-    const R ak = s.f[c] * A.rmdef[(size_t)c * A.ndef + q];
+    const R ak = s.f[c] * x.rm[c];
     def_store<R>(A, s, c, (size_t)c * A.GS + n.g, ak, n.rec);
-    if (rows && n.rec)
-      rec_put(rows, A.rec, A.rec.def_q, A.rec.def_r, A.rec.ndefr, q, c, rec_value<R>(A.rec, s, c, ak));
+    if (rr.at >= 0)
+      rec_put(rows, A.rec, A.rec.def_q, A.rec.def_r, A.rec.ndefr, rr, q, c, rec_value<R>(A.rec, s, c, ak));
   }
 }
 
@@ -1184,16 +1267,12 @@ __global__ __launch_bounds__(256) void k_deferred(DefArgs<R> A) {
 // (p.. the derivatives of fb, g.. those of d_n), summed over the element's points.
 // One workgroup per tile; interior nodes finish here, perimeter nodes in k_adj_deferred.
 // ===========================================================================
-// Forward acceleration a_n at field index i: stored (a != nullptr), or, from a history
-// of displacements, the second difference (d_{n+1} - 2 d_n + d_{n-1}) / dt^2, which equals
-// a_n for the explicit Newmark scheme (beta = 0, gamma = 1/2): d_{n+1} - d_n = dt v_n +
-// dt^2/2 a_n and v_n - v_{n-1} = dt/2 (a_{n-1} + a_n).
-template <typename R>
-__device__ __forceinline__ double fwd_accel(const R* __restrict__ a, const R* __restrict__ dprev,
-                                            const R* __restrict__ dnext, size_t i, R dcur, double idt2) {
-  if (a) return (double)a[i];
-  const double dc = (double)dcur;
-  return (((double)dnext[i] - dc) - (dc - (double)dprev[i])) * idt2;
+// Forward acceleration a_n from a history of displacements: the second difference
+// (d_{n+1} - 2 d_n + d_{n-1}) / dt^2, which equals a_n for the explicit Newmark scheme
+// (beta = 0, gamma = 1/2): d_{n+1} - d_n = dt v_n + dt^2/2 a_n and v_n - v_{n-1} =
+// dt/2 (a_{n-1} + a_n).
+__device__ __forceinline__ double fwd_accel(double dprev, double dcur, double dnext, double idt2) {
+  return ((dnext - dcur) - (dcur - dprev)) * idt2;
 }
 
 // Injection of dJ/d(recorded field): the sample of step n is added to the adjoint state
@@ -1373,10 +1452,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
       for (int c = 0; c < NDOF; ++c) {
         f[c] = (a[r][c] + c3 * v[r][c]) * rm[r][c];
         double acc = (double)x1[r][c];
-        if constexpr (HIST) {
-          const double dc = (double)u[r][c];
-          acc = (((double)x2[r][c] - dc) - (dc - (double)x1[r][c])) * idt2;
-        }
+        if constexpr (HIST) acc = fwd_accel((double)x1[r][c], (double)u[r][c], (double)x2[r][c], idt2);
         mb[r] -= (double)f[c] * acc;
       }
       const int p = tl + TS_NT * r, Z = p / PS, X = p - Z * PS;
@@ -1637,38 +1713,69 @@ __global__ __launch_bounds__(256) void k_adj_deferred(int ndef, DefTable defs,
   const DefNode n = def_unpack(defs, q);
   const size_t g = n.g;
   const int u = IP.g ? IP.udef[q] : -1;
-  double mb = 0;
+  // all loads first
+  R xd[NDOF], xw[NDOF], rm[NDOF], u0[NDOF], u1[NDOF], u2[NDOF], F[NDOF];
+  double C[NDOF] = {}, gb[NDOF] = {};
+  const bool two = n.pinl && n.poff[1] >= 0;
+  const int o0 = n.pinl ? n.poff[0] : 0, o1 = two ? n.poff[1] : o0;
+  R p0[NDOF], p1[NDOF];
+  double mb = mbar[g];
 #pragma unroll
   for (int c = 0; c < NDOF; ++c) {
-    AdjNode<R> s = adj_node<R>(ad[c * GS + g], aw[c * GS + g], dt, c1, c2);
+    const size_t i = c * GS + g;
+    xd[c] = ad[i];
+    xw[c] = aw[i];
+    rm[c] = rmdef[(size_t)c * ndef + q];
+    p0[c] = fpart[c * FPS + o0];
+    p1[c] = fpart[c * FPS + o1];
+    if (dcur) {
+      u0[c] = dcur[i];
+      u1[c] = dprev[i];
+      u2[c] = afw ? afw[i] : dnext[i];
+    } else {
+      u0[c] = afw[i];
+      u1[c] = 0, u2[c] = 0;
+      if (n.acnt > 0) u1[c] = vprev[i], u2[c] = aprev[i];
+    }
+    if (n.acnt > 0) {
+      C[c] = abso[(size_t)n.astart * NDOF + c];
+      gb[c] = gabs[(size_t)c * ndef + q];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NDOF; ++c) {
+    F[c] = 0;
+    if (n.pinl) {  // the loop below with pcnt = 1 or 2
+      F[c] = F[c] + p0[c];
+      if (two) F[c] = F[c] + p1[c];
+    } else {
+      for (int k = 0; k < n.pcnt; ++k) F[c] = F[c] + fpart[c * FPS + part_off[n.pstart + k]];
+    }
+  }
+  double sum = 0;
+#pragma unroll
+  for (int c = 0; c < NDOF; ++c) {
+    AdjNode<R> s = adj_node<R>(xd[c], xw[c], dt, c1, c2);
     if (u >= 0) {
       R& x = IP.field == 0 ? s.d : (IP.field == 1 ? s.v : s.a);
       x = inject_at<R>(IP, u, c, x);
     }
-    const R fb = (s.a + c3 * s.v) * rmdef[(size_t)c * ndef + q];
-    R F = 0;
-    if (n.pinl) {  // the loop below with pcnt = 1 or 2
-      F = F + fpart[c * FPS + n.poff[0]];
-      if (n.poff[1] >= 0) F = F + fpart[c * FPS + n.poff[1]];
-    } else {
-      for (int k = 0; k < n.pcnt; ++k) F = F + fpart[c * FPS + part_off[n.pstart + k]];
-    }
+    const R fb = (s.a + c3 * s.v) * rm[c];
     double Cc = 0;
-    for (int k = 0; k < n.acnt; ++k) Cc += abso[(size_t)(n.astart + k) * NDOF + c];
-    ad[c * GS + g] = s.d + F;
+    for (int k = 0; k < n.acnt; ++k) Cc += k == 0 ? C[c] : abso[(size_t)(n.astart + k) * NDOF + c];
+    ad[c * GS + g] = s.d + F[c];
     aw[c * GS + g] = (R)((double)s.v - Cc * (double)fb);
-    // with a displacement history (dcur set): a_n as in fwd_accel, and the predicted
+    // with a displacement history (dcur set) the predicted velocity is
     // velocity v_{n-1} + dt/2 a_{n-1} = (d_n - d_{n-1}) / dt
-    const double an = dcur ? fwd_accel(afw, dprev, dnext, c * GS + g, dcur[c * GS + g], idt2)
-                           : (double)afw[c * GS + g];
-    mb -= (double)fb * an;
+    double an = (double)u0[c];
+    if (dcur) an = afw ? (double)u2[c] : fwd_accel((double)u1[c], (double)u0[c], (double)u2[c], idt2);
+    sum -= (double)fb * an;
     if (n.acnt > 0) {
-      const double vp = dcur ? ((double)dcur[c * GS + g] - (double)dprev[c * GS + g]) * idt
-                             : (double)vprev[c * GS + g] + (double)c2 * (double)aprev[c * GS + g];
-      gabs[(size_t)c * ndef + q] -= (double)fb * (vp + (double)c3 * an);
+      const double vp = dcur ? ((double)u0[c] - (double)u1[c]) * idt : (double)u1[c] + (double)c2 * (double)u2[c];
+      gabs[(size_t)c * ndef + q] = gb[c] - (double)fb * (vp + (double)c3 * an);
     }
   }
-  mbar[g] += mb;
+  mbar[g] = mb + sum;
 }
 
 }  // namespace sem2d
