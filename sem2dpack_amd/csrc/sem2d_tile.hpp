@@ -131,24 +131,222 @@ __device__ __forceinline__ void wave_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Exchange slots of the forces of the elements at patch node (X, Z) (slot = element * NP +
-// point, elements row by row of a full tile; the slot after the last stands for an element
-// outside the patch)
-__device__ __forceinline__ ushort4 node_slots(int X, int Z) {
-  constexpr int NEL = TX * TZ;
-      // Of the two element columns (rows) that share a node the even one comes first,
-      // rows before columns: the order of the colours.
-      unsigned short sl[4];
-#pragma unroll
+// Exchange slots of the forces of the elements at a patch node (X, Z), node Z * PXM + X of
+// the table (slot = element * NP + point, elements row by row of a full tile; slot NEL * NP
+// stands for an element outside the patch).  Of the two element columns (rows) that share a
+// node the even one comes first, rows before columns: the order of the colours.  A table
+// that the kernels copy to LDS behind their first loads: computed there it was some 600
+// instructions of a lane before the tile's first load.
+struct alignas(8) NodeSlots {
+  unsigned short q[4];
+};
+struct SlotTable {
+  NodeSlots node[PMAX];
+};
+constexpr SlotTable make_slot_table() {
+  SlotTable T{};
+  for (int Z = 0; Z < PMAX / PXM; ++Z)
+    for (int X = 0; X < PXM; ++X)
       for (int q = 0; q < 4; ++q) {
         const int cx = q & 1, cz = q >> 1;
         const int lx = ((X >> 2) & 1) == cx ? X >> 2 : (X >> 2) - 1;
         const int lz = ((Z >> 2) & 1) == cz ? Z >> 2 : (Z >> 2) - 1;
         const bool ok = lx >= 0 && lx < TX && (lx == X >> 2 || (X & 3) == 0) && lz >= 0 && lz < TZ &&
                         (lz == Z >> 2 || (Z & 3) == 0);
-        sl[q] = (unsigned short)(ok ? (lz * TX + lx) * NP + (Z - 4 * lz) * NG + (X - 4 * lx) : NEL * NP);
+        T.node[Z * PXM + X].q[q] =
+            (unsigned short)(ok ? (lz * TX + lx) * NP + (Z - 4 * lz) * NG + (X - 4 * lx) : TX * TZ * NP);
       }
-  return make_ushort4(sl[0], sl[1], sl[2], sl[3]);
+  return T;
+}
+__device__ const SlotTable c_slots = make_slot_table();
+
+// Element phase of the tile kernels: element e, its lane s (row or column s), base the patch
+// index of its first node, ex its part of the exchange array; on: the element is inside the
+// grid.  Between the four steps the lanes of an element exchange through ex (wave_order).
+// A: column s, d/deta of its nodes' displacement (EP: of d + eta v)
+template <typename R, int NDOF, bool EP, typename LV>
+__device__ __forceinline__ void el_gradient(bool on, int base, int s, int e, LV* ex, const LV* Ud, const LV* Vp,
+                                            const R* Eta, const R (&H)[NG][NG]) {
+  constexpr int PS = PXM;
+  if (on) {
+    R g[NG][NDOF];
+#pragma unroll
+    for (int j = 0; j < NG; ++j)
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
+#pragma unroll
+    for (int k = 0; k < NG; ++k) {
+      const LV x = Ud[base + k * PS + s];
+      LV y{};
+      R et = 0;
+      if constexpr (EP) {
+        y = Vp[base + k * PS + s];
+        et = Eta[e * NP + k * NG + s];
+      }
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        R xc = lv_get<R, NDOF>(x, c);
+        if constexpr (EP) xc = xc + et * lv_get<R, NDOF>(y, c);
+#pragma unroll
+        for (int j = 0; j < NG; ++j) g[j][c] += xc * H[k][j];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
+  }
+}
+// B: row s, the fluxes at its points: the eta fluxes into ex, the row's xi sums into s1r
+template <typename R, int NDOF, int NELAST, int MODE, bool EP, typename LV, typename M, typename F>
+__device__ __forceinline__ void el_flux(bool on, int base, int s, int e, LV* ex, const LV* Ud, const LV* Vp,
+                                        const R* Eta, const R (&H)[NG][NG], const R (*Gm)[3], const R* sW2,
+                                        const R* Sa, const LV* Mn, const M& m, F coef, R (&s1r)[NG][NDOF]) {
+  constexpr int PS = PXM;
+  if (on) {
+    R x[NG][NDOF];
+#pragma unroll
+    for (int k = 0; k < NG; ++k) {
+      const LV xv = Ud[base + s * PS + k];
+      LV y{};
+      R et = 0;
+      if constexpr (EP) {
+        y = Vp[base + s * PS + k];
+        et = Eta[e * NP + s * NG + k];
+      }
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        x[k][c] = lv_get<R, NDOF>(xv, c);
+        if constexpr (EP) x[k][c] = x[k][c] + et * lv_get<R, NDOF>(y, c);
+        s1r[k][c] = 0;
+      }
+    }
+    R g0 = 0, g1 = 0, g2 = 0;
+    if constexpr (MODE == COEF_COMPACT || MODE == COEF_NODE) {
+      g0 = Gm[e][0];
+      g1 = Gm[e][1];
+      g2 = Gm[e][2];
+    }
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      const int pt = s * NG + i;
+      R A[NELAST];
+      if constexpr (MODE == COEF_COMPACT || MODE == COEF_NODE) {
+        const R w2 = sW2[pt];
+        R m0, m1;
+        if constexpr (MODE == COEF_NODE) {
+          const LV mm = Mn[base + s * PS + i];
+          m0 = lv_get<R, NDOF>(mm, 0);
+          m1 = lv_get<R, NDOF>(mm, NDOF - 1);
+        } else {
+          m0 = m[i][0];
+          m1 = m[i][NDOF - 1];
+        }
+        if constexpr (NDOF == 2) {
+          const R la = m0, mu = m1, kx = la + 2 * mu;
+          A[0] = w2 * kx * g0;
+          A[1] = w2 * la * g2;
+          A[2] = w2 * kx * g1;
+          A[3] = w2 * mu * g1;
+          A[4] = w2 * mu * g2;
+          A[5] = w2 * mu * g0;
+        } else {
+          A[0] = w2 * m0 * g0;
+          A[1] = w2 * m0 * g1;
+        }
+      } else if constexpr (MODE == COEF_SHARED) {
+#pragma unroll
+        for (int k = 0; k < NELAST; ++k) A[k] = Sa[k * NP + pt];
+      } else {
+#pragma unroll
+        for (int k = 0; k < NELAST; ++k) A[k] = coef(k, pt);
+      }
+      R dxi[NDOF], deta[NDOF];
+      const LV gv = ex[pt];
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        R sum = 0;
+#pragma unroll
+        for (int k = 0; k < NG; ++k) sum += H[k][i] * x[k][c];
+        dxi[c] = sum;
+        deta[c] = lv_get<R, NDOF>(gv, c);
+      }
+      R t1[NDOF], t2[NDOF];
+      if constexpr (NDOF == 2) {
+        t1[0] = A[0] * dxi[0] + A[1] * deta[1];
+        t2[0] = A[3] * (deta[0] + dxi[1]);
+        t1[1] = A[4] * deta[0] + A[5] * dxi[1];
+        t2[1] = A[1] * dxi[0] + A[2] * deta[1];
+      } else {
+        t1[0] = A[0] * dxi[0];
+        t2[0] = A[1] * deta[0];
+      }
+      ex[pt] = lv_make<R, NDOF>(t2);
+#pragma unroll
+      for (int q = 0; q < NG; ++q)
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) s1r[q][c] += H[q][i] * t1[c];
+      // one point at a time: hoisting the later points' LDS reads costs the registers
+      // of the next tile's loads
+      if constexpr (MODE != COEF_SHARED) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+// C: column s, the eta sums of the fluxes
+template <typename R, int NDOF, typename LV>
+__device__ __forceinline__ void el_divergence(bool on, int s, LV* ex, const R (&H)[NG][NG]) {
+  if (on) {
+    R g[NG][NDOF];
+#pragma unroll
+    for (int j = 0; j < NG; ++j)
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
+#pragma unroll
+    for (int k = 0; k < NG; ++k) {
+      const LV tv = ex[k * NG + s];
+#pragma unroll
+      for (int j = 0; j < NG; ++j)
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) g[j][c] += lv_get<R, NDOF>(tv, c) * H[j][k];
+    }
+#pragma unroll
+    for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
+  }
+}
+// D: row s, the forces of its points (slot: an element outside the grid, zero)
+template <typename R, int NDOF, bool EP, typename LV>
+__device__ __forceinline__ void el_force(bool on, bool slot, bool b25, int base, int s, int e, LV* ex, const LV* Ud,
+                                         const LV* Vp, const R* Eta, const R* Bet, const R (&s1r)[NG][NDOF]) {
+  constexpr int PS = PXM;
+  if (on) {
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      const LV c2v = ex[s * NG + i];
+      R f[NDOF];
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) f[c] = s1r[i][c] + lv_get<R, NDOF>(c2v, c);
+      if constexpr (EP) {
+        if (b25) {  // 2.5D: the point force loses b25 (d + eta v) of its own point
+          const int own = base + s * PS + i;
+          const LV uo = Ud[own], wo = Vp[own];
+          const R eo = Eta[e * NP + s * NG + i], bo = Bet[e * NP + s * NG + i];
+#pragma unroll
+          for (int c = 0; c < NDOF; ++c)
+            f[c] = f[c] - bo * (lv_get<R, NDOF>(uo, c) + eo * lv_get<R, NDOF>(wo, c));
+        }
+      }
+      ex[s * NG + i] = lv_make<R, NDOF>(f);
+    }
+  } else if (slot) {
+#pragma unroll
+    for (int i = 0; i < NG; ++i) ex[s * NG + i] = LV{};
+  }
+}
+
+// Touches the cache lines of H that hconst reads as scalars.
+template <typename R>
+__device__ __forceinline__ void warm_h() {
+  const auto* hp = hconst<R>();
+  const R a = hp[0], b = hp[8], c = hp[16], d = hp[24];
+  asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
 }
 
 // Persistent tile kernel.  Each workgroup walks a strided sequence of tiles inside its
@@ -270,7 +468,7 @@ k_tile_step(TileArgs<R> args) {
   __shared__ LV Ex[NEL * NP + 1];
   // per patch node the exchange slots of its elements' forces, in the order of the
   // colours; the zero slot stands for an element outside the patch
-  __shared__ ushort4 Eg[PMAX];
+  __shared__ NodeSlots Eg[PMAX];
   __shared__ LV Vp[EP ? PMAX : 1];      // predicted velocity
   __shared__ LV Mn[NODEM ? PMAX : 1];   // moduli of the patch nodes
   __shared__ R Sa[MODE == COEF_SHARED ? NELAST * NP : 1];  // the grid's point coefficients
@@ -296,15 +494,12 @@ k_tile_step(TileArgs<R> args) {
   if (args.tick && bid == 0 && threadIdx.x == 0) ++*args.tick;
   if (q0 >= s1) return;
   const int tid = threadIdx.x;
-  if (tid < NP) sW2[tid] = (R)c_W2[tid];
-  if (tid == 0) Ex[NEL * NP] = LV{};
   // this thread's patch nodes (X, Z), packed
   int xz[TS_ITER];
 #pragma unroll
   for (int r = 0; r < TS_ITER; ++r) {
     const int p = tid + TS_NT * r, Z = p / PS, X = p - Z * PS;
     xz[r] = X | Z << 8;
-    if (p < PMAX) Eg[p] = node_slots(X, Z);
   }
   struct Geo {
     int tx0, tz0, nxe, nze, Z0, PX, PZ, X0, kL, kR;
@@ -421,7 +616,8 @@ k_tile_step(TileArgs<R> args) {
 
   // Stores of a finished tile: partial forces for perimeter and special nodes, new a, v,
   // d for the others.
-  auto store_tile = [&](const int tp, const int4 tgp, const int4 grp, const R (*fk)[NDOF]) {
+  auto store_tile = [&](const int tp, const int4 tgp, const int4 grp, const int ns, const int mark,
+                        const R (*fk)[NDOF]) {
     const auto* P = kernel_args<TileArgs<R>>();
     const Geo G = geo(tgp);
     R *oD[NDOF], *oV[NDOF], *oA[NDOF], *bF[NDOF];
@@ -435,9 +631,8 @@ k_tile_step(TileArgs<R> args) {
     }
     const R c3 = P->c3, c4 = P->c4, dt = P->dt, c1 = P->c1, c2 = P->c2;
     const StepOut so = {P->out.final, P->out.accel, P->out.rec};
-    const int mrow = so.rec >= 0 ? sload(P->mark_of, tp) : -1;
+    const int mrow = so.rec >= 0 ? mark : -1;
     const uint32_t fbase = (uint32_t)tp * SLOTS;
-    const int ns = sload(P->spec_cnt, tp);
 #pragma unroll
     for (int r = 0; r < TS_ITER; ++r) {
       const int X = xz[r] & 0xff, Z = xz[r] >> 8;
@@ -477,8 +672,17 @@ k_tile_step(TileArgs<R> args) {
   };
 
   issue(q0);
+  // behind the first tile's loads: the exchange slots, the GLL weights, and the lines of H,
+  // which the element phase reads as scalars, into the scalar cache
+#pragma unroll
+  for (int r = 0; r < TS_ITER; ++r)
+    if (const int p = tid + TS_NT * r; p < PMAX) Eg[p] = c_slots.node[p];
+  if (tid < NP) sW2[tid] = (R)c_W2[tid];
+  if (tid == 0) Ex[NEL * NP] = LV{};
+  warm_h<R>();
   int tp = -1;  // FULLPF: the previous tile of this workgroup, not yet stored
   int4 tgp = {}, grp = {};
+  int nsp = 0, markp = -1;
   R fk[TS_ITER][NDOF] = {};
 
 #pragma unroll 1
@@ -488,8 +692,24 @@ k_tile_step(TileArgs<R> args) {
     const auto* P = kernel_args<TileArgs<R>>();
     const int4 tg = sload(P->tiles, t);
     const int4 gr = sload(P->grids, t);
+    // for the stores (there the loads would be waited for: they are the tile's first)
+    const int ns = sload(P->spec_cnt, t), mark = sload(P->mark_of, t);
     const Geo G = geo(tg);
     const R dt = P->dt, c1 = P->c1, c2 = P->c2;
+
+    // the moduli of the points of this lane's row (element phase below), ahead of the waits
+    // for the tile's node values
+    R m[COMP ? NG : 1][NDOF];
+    if constexpr (COMP) {
+      const int tl = lane_id(), lane = tl & 63;
+      const int e = min((tl >> 6) * TS_EPW + lane / NG, NEL - 1), s = lane % NG;
+      const R* bCo = ubase(P->coefs);
+      const auto cell = cidx(gr, tg.z >> 16, G, min(e % TX, G.nxe - 1), min(e / TX, G.nze - 1));
+#pragma unroll
+      for (int i = 0; i < NG; ++i)
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) m[i][c] = fld(bCo, (cell * NDOF + c) * NP + s * NG + i);
+    }
 
     // predictor
     R u[TS_ITER][NDOF], w[TS_ITER][NDOF];
@@ -513,7 +733,7 @@ k_tile_step(TileArgs<R> args) {
         for (int c = 0; c < NDOF; ++c) asm volatile("" : "+v"(u[r][c]), "+v"(w[r][c]));
         asm volatile("" : "+v"(pm[r]));
       }
-      if (tp >= 0) store_tile(tp, tgp, grp, fk);
+      if (tp >= 0) store_tile(tp, tgp, grp, nsp, markp, fk);
     }
 #pragma unroll
     for (int r = 0; r < TS_ITER; ++r) {
@@ -553,17 +773,6 @@ k_tile_step(TileArgs<R> args) {
       const bool on = lane < TS_EPW * NG && e < NEL && lx < G.nxe && lz < G.nze;
       const int base = 4 * lz * PS + 4 * lx;
       LV* ex = Ex + e * NP;
-      // the moduli of the row's points, ahead of the next tile's loads (they would be
-      // waited for with those otherwise)
-      R m[COMP ? NG : 1][NDOF];
-      if constexpr (COMP) {
-        const R* bCo = ubase(P->coefs);
-        const auto cell = cidx(gr, tg.z >> 16, G, min(lx, G.nxe - 1), min(lz, G.nze - 1));
-#pragma unroll
-        for (int i = 0; i < NG; ++i)
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) m[i][c] = fld(bCo, (cell * NDOF + c) * NP + s * NG + i);
-      }
       if (tn >= 0) {
         issue(tn);
       } else {  // no old values to keep
@@ -595,126 +804,15 @@ k_tile_step(TileArgs<R> args) {
       for (int k = 0; k < NG; ++k)
 #pragma unroll
         for (int i = 0; i < NG; ++i) H[k][i] = hp[k * NG + i];
-      // A: column s
-      if (on) {
-        R g[NG][NDOF];
-#pragma unroll
-        for (int j = 0; j < NG; ++j)
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
-#pragma unroll
-        for (int k = 0; k < NG; ++k) {
-          const LV x = Ud[base + k * PS + s];
-          LV y{};
-          R et = 0;
-          if constexpr (EP) {
-            y = Vp[base + k * PS + s];
-            et = Eta[e * NP + k * NG + s];
-          }
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) {
-            R xc = lv_get<R, NDOF>(x, c);
-            if constexpr (EP) xc = xc + et * lv_get<R, NDOF>(y, c);
-#pragma unroll
-            for (int j = 0; j < NG; ++j) g[j][c] += xc * H[k][j];
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
-      }
+      el_gradient<R, NDOF, EP>(on, base, s, e, ex, Ud, Vp, Eta, H);
       wave_order();
-      // B: row s
       R s1r[NG][NDOF];
-      if (on) {
-        R x[NG][NDOF];
-#pragma unroll
-        for (int k = 0; k < NG; ++k) {
-          const LV xv = Ud[base + s * PS + k];
-          LV y{};
-          R et = 0;
-          if constexpr (EP) {
-            y = Vp[base + s * PS + k];
-            et = Eta[e * NP + s * NG + k];
-          }
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) {
-            x[k][c] = lv_get<R, NDOF>(xv, c);
-            if constexpr (EP) x[k][c] = x[k][c] + et * lv_get<R, NDOF>(y, c);
-            s1r[k][c] = 0;
-          }
-        }
-        R g0 = 0, g1 = 0, g2 = 0;
-        if constexpr (COMP || NODEM) {
-          g0 = Gm[e][0];
-          g1 = Gm[e][1];
-          g2 = Gm[e][2];
-        }
-#pragma unroll
-        for (int i = 0; i < NG; ++i) {
-          const int pt = s * NG + i;
-          R A[NELAST];
-          if constexpr (COMP || NODEM) {
-            const R w2 = sW2[pt];
-            R m0, m1;
-            if constexpr (NODEM) {
-              const LV mm = Mn[base + s * PS + i];
-              m0 = lv_get<R, NDOF>(mm, 0);
-              m1 = lv_get<R, NDOF>(mm, NDOF - 1);
-            } else {
-              m0 = m[i][0];
-              m1 = m[i][NDOF - 1];
-            }
-            if constexpr (NDOF == 2) {
-              const R la = m0, mu = m1, kx = la + 2 * mu;
-              A[0] = w2 * kx * g0;
-              A[1] = w2 * la * g2;
-              A[2] = w2 * kx * g1;
-              A[3] = w2 * mu * g1;
-              A[4] = w2 * mu * g2;
-              A[5] = w2 * mu * g0;
-            } else {
-              A[0] = w2 * m0 * g0;
-              A[1] = w2 * m0 * g1;
-            }
-          } else if constexpr (MODE == COEF_SHARED) {
-#pragma unroll
-            for (int k = 0; k < NELAST; ++k) A[k] = Sa[k * NP + pt];
-          } else {
-            const R* bCo = ubase(P->coefs);
-            const auto cell = cidx(gr, tg.z >> 16, G, lx, lz);
-#pragma unroll
-            for (int k = 0; k < NELAST; ++k) A[k] = fld(bCo, (cell * NELAST + k) * NP + pt);
-          }
-          R dxi[NDOF], deta[NDOF];
-          const LV gv = ex[pt];
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) {
-            R sum = 0;
-#pragma unroll
-            for (int k = 0; k < NG; ++k) sum += H[k][i] * x[k][c];
-            dxi[c] = sum;
-            deta[c] = lv_get<R, NDOF>(gv, c);
-          }
-          R t1[NDOF], t2[NDOF];
-          if constexpr (NDOF == 2) {
-            t1[0] = A[0] * dxi[0] + A[1] * deta[1];
-            t2[0] = A[3] * (deta[0] + dxi[1]);
-            t1[1] = A[4] * deta[0] + A[5] * dxi[1];
-            t2[1] = A[1] * dxi[0] + A[2] * deta[1];
-          } else {
-            t1[0] = A[0] * dxi[0];
-            t2[0] = A[1] * deta[0];
-          }
-          ex[pt] = lv_make<R, NDOF>(t2);
-#pragma unroll
-          for (int q = 0; q < NG; ++q)
-#pragma unroll
-            for (int c = 0; c < NDOF; ++c) s1r[q][c] += H[q][i] * t1[c];
-          // one point at a time: hoisting the later points' LDS reads costs the registers
-          // of the next tile's loads
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
+      el_flux<R, NDOF, NELAST, MODE, EP>(on, base, s, e, ex, Ud, Vp, Eta, H, Gm, sW2, Sa, Mn, m,
+                                         [&](int k, int pt) {
+                                           return fld(ubase(P->coefs),
+                                                      (cidx(gr, tg.z >> 16, G, lx, lz) * NELAST + k) * NP + pt);
+                                         },
+                                         s1r);
       wave_order();
       // what the stores need besides the forces, loaded when the registers of B are free
       // and used after C, D and E
@@ -733,49 +831,9 @@ k_tile_step(TileArgs<R> args) {
           }
         }
       }
-      // C: column s
-      if (on) {
-        R g[NG][NDOF];
-#pragma unroll
-        for (int j = 0; j < NG; ++j)
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
-#pragma unroll
-        for (int k = 0; k < NG; ++k) {
-          const LV tv = ex[k * NG + s];
-#pragma unroll
-          for (int j = 0; j < NG; ++j)
-#pragma unroll
-            for (int c = 0; c < NDOF; ++c) g[j][c] += lv_get<R, NDOF>(tv, c) * H[j][k];
-        }
-#pragma unroll
-        for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
-      }
+      el_divergence<R, NDOF>(on, s, ex, H);
       wave_order();
-      // D: row s
-      if (on) {
-#pragma unroll
-        for (int i = 0; i < NG; ++i) {
-          const LV c2v = ex[s * NG + i];
-          R f[NDOF];
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) f[c] = s1r[i][c] + lv_get<R, NDOF>(c2v, c);
-          if constexpr (EP) {
-            if (P->b25) {  // 2.5D: the point force loses b25 (d + eta v) of its own point
-              const int own = base + s * PS + i;
-              const LV uo = Ud[own], wo = Vp[own];
-              const R eo = Eta[e * NP + s * NG + i], bo = Bet[e * NP + s * NG + i];
-#pragma unroll
-              for (int c = 0; c < NDOF; ++c)
-                f[c] = f[c] - bo * (lv_get<R, NDOF>(uo, c) + eo * lv_get<R, NDOF>(wo, c));
-            }
-          }
-          ex[s * NG + i] = lv_make<R, NDOF>(f);
-        }
-      } else if (lane < TS_EPW * NG && e < NEL) {
-#pragma unroll
-        for (int i = 0; i < NG; ++i) ex[s * NG + i] = LV{};
-      }
+      el_force<R, NDOF, EP>(on, lane < TS_EPW * NG && e < NEL, EP && P->b25, base, s, e, ex, Ud, Vp, Eta, Bet, s1r);
     }
     __syncthreads();
     // E: nodes (elements outside the tile left zero)
@@ -785,8 +843,8 @@ k_tile_step(TileArgs<R> args) {
 #pragma unroll
       for (int c = 0; c < NDOF; ++c) fk[r][c] = 0;
       if (p < PMAX) {
-        const ushort4 sl = Eg[p];
-        const LV f0 = Ex[sl.x], f1 = Ex[sl.y], f2 = Ex[sl.z], f3 = Ex[sl.w];
+        const NodeSlots sl = Eg[p];
+        const LV f0 = Ex[sl.q[0]], f1 = Ex[sl.q[1]], f2 = Ex[sl.q[2]], f3 = Ex[sl.q[3]];
 #pragma unroll
         for (int c = 0; c < NDOF; ++c)
           fk[r][c] = (((lv_get<R, NDOF>(f0, c)) + lv_get<R, NDOF>(f1, c)) + lv_get<R, NDOF>(f2, c)) +
@@ -797,12 +855,14 @@ k_tile_step(TileArgs<R> args) {
       tp = t;
       tgp = tg;
       grp = gr;
+      nsp = ns;
+      markp = mark;
     } else {
-      store_tile(t, tg, gr, fk);
+      store_tile(t, tg, gr, ns, mark, fk);
     }
   }
   if constexpr (FULLPF) {
-    if (tp >= 0) store_tile(tp, tgp, grp, fk);
+    if (tp >= 0) store_tile(tp, tgp, grp, nsp, markp, fk);
   }
 }
 
@@ -1344,7 +1404,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
   __shared__ LV Uf[PMAX];  // fb
   __shared__ LV Ud[PMAX];  // forward d_n
   __shared__ LV Ex[NEL * NP + 1];
-  __shared__ ushort4 Eg[PMAX];
+  __shared__ NodeSlots Eg[PMAX];
   __shared__ R Gm[NEL][3];
   __shared__ R sW2[NP];
   // each XCD (bid & 7) takes a contiguous eighth of the tiles
@@ -1352,8 +1412,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
   const int t = (bid & 7) * per + (bid >> 3);
   if ((bid >> 3) >= per || t >= args.ntiles) return;
   const int tid = threadIdx.x;
-  if (tid < NP) sW2[tid] = (R)c_W2[tid];
-  if (tid == 0) Ex[NEL * NP] = LV{};
   const auto* P = kernel_args<AdjArgs<R>>();
   const int4 tg = sload(P->tiles, t), gr = sload(P->grids, t);
   const int nxe = tg.z & 0xff, nze = (tg.z >> 8) & 0xff, nx = tg.z >> 16;
@@ -1429,6 +1487,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
       }
       mb[r] = at(bmb, g[r]);
     }
+    // behind these loads, as in k_tile_step
+#pragma unroll
+    for (int r = 0; r < TS_ITER; ++r)
+      if (const int p = tl + TS_NT * r; p < PMAX) Eg[p] = c_slots.node[p];
+    if (tl < NP) sW2[tl] = (R)c_W2[tl];
+    if (tl == 0) Ex[NEL * NP] = LV{};
+    if (tl < NEL * 3) {
+      const int e = tl / 3, k = tl - 3 * (tl / 3);
+      Gm[e][k] = at(ub(P->geom), cidx(min(e % TX, nxe - 1), min(e / TX, nze - 1)) * 3 + k);
+    }
+    warm_h<R>();
 #pragma unroll
     for (int r = 0; r < TS_ITER; ++r)
 #pragma unroll
@@ -1459,18 +1528,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
       if (p < PMAX) {
         Uf[p] = lv_make<R, NDOF>(f);
         Ud[p] = lv_make<R, NDOF>(u[r]);
-        Eg[p] = node_slots(X, Z);
       }
       // the mass sensitivity of interior nodes (perimeter and special nodes: k_adj_deferred)
       if (X < PX && Z < PZ && perim_slot(X, Z, PX, PZ) < 0 && special(p) < 0) at(bmb, g[r]) = mb[r];
     }
   }
-  if (tid < NEL * 3) {
-    const int e = tid / 3, k = tid - 3 * (tid / 3);
-    Gm[e][k] = at(ub(P->geom), cidx(min(e % TX, nxe - 1), min(e / TX, nze - 1)) * 3 + k);
-  }
   __syncthreads();
 
+  const int ts = lane_id();
+  R ad[TS_ITER][NDOF], av[TS_ITER][NDOF];  // the adjoint state again, for the stores
   {
     const int te = lane_id(), lane = te & 63;
     const int e = (te >> 6) * TS_EPW + lane / NG, s = lane % NG;
@@ -1487,23 +1553,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
       for (int i = 0; i < NG; ++i) H[k][i] = hp[k * NG + i];
     // column derivatives of a patch array into the exchange array
     auto column = [&](const LV* U) {
-      if (on) {
-        R g[NG][NDOF];
-#pragma unroll
-        for (int j = 0; j < NG; ++j)
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
-#pragma unroll
-        for (int k = 0; k < NG; ++k) {
-          const LV x = U[base + k * PS + s];
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c)
-#pragma unroll
-            for (int j = 0; j < NG; ++j) g[j][c] += lv_get<R, NDOF>(x, c) * H[k][j];
-        }
-#pragma unroll
-        for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
-      }
+      el_gradient<R, NDOF, false>(on, base, s, e, ex, U, U, (const R*)nullptr, H);
       wave_order();
     };
     column(Ud);
@@ -1576,6 +1626,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    // the element's running sensitivities, for the sums below
+    const double gl0 = at(ub(P->glam), cell), gm0 = at(ub(P->gmu), cell);
     R s1r[NG][NDOF] = {};
     if (on) {
 #pragma unroll
@@ -1608,55 +1660,25 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         sm += __shfl(rmu, from);
       }
       if (on && s == 0) {
-        at(ub(P->glam), cell) = at(ub(P->glam), cell) + sl;
-        at(ub(P->gmu), cell) = at(ub(P->gmu), cell) + sm;
+        at(ub(P->glam), cell) = gl0 + sl;
+        at(ub(P->gmu), cell) = gm0 + sm;
       }
     }
     wave_order();
-    if (on) {
-      R g[NG][NDOF];
 #pragma unroll
-      for (int j = 0; j < NG; ++j)
+    for (int r = 0; r < TS_ITER; ++r) {
+      const int p = ts + TS_NT * r, Z = p / PS, X = p - Z * PS;
+      const I g = nidx(min(X, PX - 1), min(Z, PZ - 1));
 #pragma unroll
-        for (int c = 0; c < NDOF; ++c) g[j][c] = 0;
-#pragma unroll
-      for (int k = 0; k < NG; ++k) {
-        const LV tv = ex[k * NG + s];
-#pragma unroll
-        for (int j = 0; j < NG; ++j)
-#pragma unroll
-          for (int c = 0; c < NDOF; ++c) g[j][c] += lv_get<R, NDOF>(tv, c) * H[j][k];
+      for (int c = 0; c < NDOF; ++c) {
+        ad[r][c] = at(ub(P->ad + c * S), g);
+        av[r][c] = at(ub(P->w + c * S), g);
       }
-#pragma unroll
-      for (int j = 0; j < NG; ++j) ex[j * NG + s] = lv_make<R, NDOF>(g[j]);
     }
+    el_divergence<R, NDOF>(on, s, ex, H);
     wave_order();
-    if (on) {
-#pragma unroll
-      for (int i = 0; i < NG; ++i) {
-        const LV cv = ex[s * NG + i];
-        R f[NDOF];
-#pragma unroll
-        for (int c = 0; c < NDOF; ++c) f[c] = s1r[i][c] + lv_get<R, NDOF>(cv, c);
-        ex[s * NG + i] = lv_make<R, NDOF>(f);
-      }
-    } else if (lane < TS_EPW * NG && e < NEL) {
-#pragma unroll
-      for (int i = 0; i < NG; ++i) ex[s * NG + i] = LV{};
-    }
-  }
-  // the adjoint state again, for the stores
-  const int ts = lane_id();
-  R ad[TS_ITER][NDOF], av[TS_ITER][NDOF];
-#pragma unroll
-  for (int r = 0; r < TS_ITER; ++r) {
-    const int p = ts + TS_NT * r, Z = p / PS, X = p - Z * PS;
-    const I g = nidx(min(X, PX - 1), min(Z, PZ - 1));
-#pragma unroll
-    for (int c = 0; c < NDOF; ++c) {
-      ad[r][c] = at(ub(P->ad + c * S), g);
-      av[r][c] = at(ub(P->w + c * S), g);
-    }
+    el_force<R, NDOF, false>(on, lane < TS_EPW * NG && e < NEL, false, base, s, e, ex, Uf, Uf, (const R*)nullptr,
+                             (const R*)nullptr, s1r);
   }
   __syncthreads();
   const uint32_t fbase = (uint32_t)t * SLOTS;
@@ -1664,8 +1686,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
   for (int r = 0; r < TS_ITER; ++r) {
     const int p = ts + TS_NT * r, Z = p / PS, X = p - Z * PS;
     if (X < PX && Z < PZ) {
-      const ushort4 sl = Eg[p];
-      const LV f0 = Ex[sl.x], f1 = Ex[sl.y], f2 = Ex[sl.z], f3 = Ex[sl.w];
+      const NodeSlots sl = Eg[p];
+      const LV f0 = Ex[sl.q[0]], f1 = Ex[sl.q[1]], f2 = Ex[sl.q[2]], f3 = Ex[sl.q[3]];
       const I g = nidx(X, Z);
       int slot = perim_slot(X, Z, PX, PZ);
       if (const int k = special(p); k >= 0) slot = PERIM_MAX + k;
