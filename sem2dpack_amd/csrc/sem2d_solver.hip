@@ -102,6 +102,14 @@ struct StructState {
   // compact moduli once per node in the field layout ([ndof][NS], bulk type), when every
   // element sharing a node holds the same values there (COEF_NODE tile kernel)
   void* nodemod = nullptr;
+  // k_run_steps: neighbours of the tiles, deferred node of each partial force, the second
+  // array of partial forces, flags and count, whether a launch has given up; run_ok: 0 not
+  // asked yet, 1 the grid's tiles are resident together, -1 not so or not a run's grid
+  int *nbr = nullptr, *slot_def = nullptr, *run_fail = nullptr;
+  unsigned *run_flag = nullptr, *run_count = nullptr;
+  void* fpart2 = nullptr;
+  unsigned epoch = 0;
+  int run_ok = -1;
   std::vector<void*> prep_allocs;  // freed when the deferred tables are rebuilt
   std::vector<int> cell_elem;      // cell (iz*nx + ix) -> element (0-based)
   std::vector<int> def_ref;        // deferred node -> reference node (0-based)
@@ -1082,6 +1090,54 @@ void fault_waves(const FaultHost& F, int m, int k0, int o0, std::vector<int4>& w
   for (int o = 0; o < F.nout; ++o) slot[s0 + F.oix1 - 1 + (size_t)o * F.oixd] = o0 + o;
 }
 
+// Tiles a grid may have for its tiles to be asked whether they are resident together
+// (k_run_steps): one or two workgroups on each of the 256 compute units.  In larger grids a
+// workgroup has more than one tile, and two launches a step are no longer most of its time.
+constexpr int RUN_MAX_TILES = 512;
+
+// Tables of k_run_steps for a grid without faults, element-point terms, Stacey terms,
+// receivers inside elements and boundaries that are not flat (other grids: nbr stays null)
+int run_tables(sem2d_solver* h, const StructTables& X) {
+  StructState& S = h->st;
+  S.run_ok = -1;
+  if (!S.on || S.ntiles > RUN_MAX_TILES || h->flt.on || S.eta || S.b25 || S.s_nbe > 0 || S.dabson || h->rec_w ||
+      h->coef_mode == COEF_PER_ELEM)
+    return 0;
+  // [ntiles][8] neighbours, [ntiles][SLOTS] deferred nodes, flags, count, fail
+  const size_t at_slot = (size_t)S.ntiles * 8, at_flag = at_slot + (size_t)S.ntiles * SLOTS;
+  const size_t at_count = at_flag + (size_t)S.ntiles * FLAG_STRIDE;
+  std::vector<int> tab(at_count + 2, 0);
+  std::fill(tab.begin(), tab.begin() + at_flag, -1);
+  for (size_t q = 0; q < X.defs.size(); ++q) {
+    const DefNode& n = X.defs[q];
+    if (n.pcnt < 1 || n.pcnt > 4) return 0;
+    for (int k = 0; k < n.pcnt; ++k) {
+      const int o = X.part_off[n.pstart + k];
+      tab[at_slot + o] = (int)q;
+      int* nb = tab.data() + (size_t)(o / SLOTS) * 8;
+      for (int l = 0; l < n.pcnt; ++l) {
+        const int u = X.part_off[n.pstart + l] / SLOTS;
+        int j = 0;
+        while (j < 8 && nb[j] >= 0 && nb[j] != u) ++j;
+        if (u == o / SLOTS) continue;
+        if (j == 8) return 0;
+        nb[j] = u;
+      }
+    }
+  }
+  int* p = nullptr;
+  int rc = prep_upload(h, &p, tab.data(), tab.size());
+  if (rc) return rc;
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  S.nbr = p, S.slot_def = p + at_slot;
+  S.run_flag = (unsigned*)p + at_flag, S.run_count = (unsigned*)p + at_count;
+  S.run_fail = p + at_count + 1;
+  S.fpart2 = (char*)S.fpart + S.FPS * h->ndof * rsize(h);
+  S.epoch = 0;
+  S.run_ok = 0;
+  return 0;
+}
+
 int prepare_structured(sem2d_solver* h) {
   StructState& S = h->st;
   HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -1143,7 +1199,8 @@ int prepare_structured(sem2d_solver* h) {
     S.w32 = fits32(h->fstride, S.FPS, ncell, rsize(h));
   }
   void* fp = nullptr;
-  HIPCHK(h, hipMalloc(&fp, std::max<size_t>(S.FPS * h->ndof, 1) * rsize(h)));
+  // two arrays for the runs of steps of small grids (k_run_steps)
+  HIPCHK(h, hipMalloc(&fp, std::max<size_t>(S.FPS * h->ndof, 1) * rsize(h) * (S.on && S.ntiles <= RUN_MAX_TILES ? 2 : 1)));
   S.prep_allocs.push_back(fp);
   S.fpart = fp;
   S.s_nbe = (int)(X.s_enode.size() / h->ng);
@@ -1218,6 +1275,7 @@ int prepare_structured(sem2d_solver* h) {
     }
   }
   HIPCHK(h, hipStreamSynchronize(h->stream));
+  if ((rc = run_tables(h, X))) return rc;
   S.ready = true;
   return 0;
 }
@@ -1319,10 +1377,8 @@ StepDev step_dev(sem2d_solver* h) {
 // Tile kernel over all tiles: pipe_wgs persistent workgroups, or one per tile where there
 // are fewer tiles (or pipe_wgs is 0).  Compact moduli are read once per node when the grid
 // has them in that form.
-template <typename R, int NDOF, int NELAST, int MODE, bool OOP, bool EP, bool PIN>
-void launch_tile_p(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
-  const int n = X.T.ntiles, per_tile = (n + 7) / 8 * 8;
-  const int wgs = X.pipe_wgs > 0 ? std::min(X.pipe_wgs, per_tile) : per_tile;
+template <typename R, int MODE>
+TileArgs<R> tile_args(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
   TileArgs<R> A;
   A.d = (R*)X.d, A.v = (R*)X.v, A.a = (R*)X.a;
   A.din = (const R*)X.din, A.vin = (const R*)X.vin, A.ain = (const R*)X.ain;
@@ -1337,8 +1393,15 @@ void launch_tile_p(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
   A.mark_of = X.mark_of, A.marks = X.marks;
   A.tick = X.tick;
   A.out = X.out;
-  A.ntiles = n;
+  A.ntiles = X.T.ntiles;
   A.dt = dt, A.c1 = c1, A.c2 = c2, A.c3 = c3, A.c4 = c4;
+  return A;
+}
+template <typename R, int NDOF, int NELAST, int MODE, bool OOP, bool EP, bool PIN>
+void launch_tile_p(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
+  const int per_tile = (X.T.ntiles + 7) / 8 * 8;
+  const int wgs = X.pipe_wgs > 0 ? std::min(X.pipe_wgs, per_tile) : per_tile;
+  const TileArgs<R> A = tile_args<R, MODE>(X, dt, c1, c2, c3, c4);
   auto go = [&](auto w32) {
     k_tile_step<R, NDOF, NELAST, MODE, OOP, decltype(w32)::value, EP, PIN><<<wgs, TS_NT, 0, X.stream>>>(A);
   };
@@ -1378,6 +1441,24 @@ void launch_tile_m(const StepDev& X, R dt, R c1, R c2, R c3, R c4) {
     default: launch_tile_t<R, NDOF, NELAST, COEF_PER_ELEM>(X, dt, c1, c2, c3, c4);
   }
 }
+template <typename R>
+DefArgs<R> def_args(const StepDev& X, int it, R dt, R c1, R c2, R c3, R c4) {
+  DefArgs<R> A;
+  A.ndef = X.ndef, A.defs = X.defs, A.part_off = X.part_off;
+  A.fpart = (const R*)X.fpart, A.FPS = X.T.FPS;
+  A.src = X.dsrc, A.ampl = X.ampl, A.nt = X.ampl_nt, A.it = it, A.itp = X.itp;
+  A.abso = X.dabso, A.abson = X.dabson, A.rmdef = (const R*)X.rmdef;
+  A.d = (R*)X.d, A.v = (R*)X.v, A.a = (R*)X.a, A.GS = X.fstride;
+  A.dt = dt, A.c1 = c1, A.c2 = c2, A.c3 = c3, A.c4 = c4;
+  A.so = X.out, A.recp = (R*)(X.rec ? X.rec : X.a);
+  A.din = (const R*)X.din, A.vin = (const R*)X.vin, A.ain = (const R*)X.ain;
+  A.SR = X.SR, A.rec = X.recout;
+  A.rec.src = !X.out.final ? (const void*)A.recp : (A.rec.field == 0 ? X.d : (A.rec.field == 1 ? X.v : X.a));
+  A.fdef = X.fdef;
+  if (X.fault_on) A.F = X.F, A.fo = X.fo;
+  return A;
+}
+
 
 // One step on the tables of a StepDev: the tiles, or (gen: the solver) the elements of the
 // general path, then everything else in k_deferred.
@@ -1398,19 +1479,7 @@ void launch_structured_step(const StepDev& X, int it, R dt, R c1, R c2, R c3, R 
         X.s_nbe, X.s_enode, X.SR.K ? nullptr : X.s_K, (const R*)(X.din ? X.din : X.d), (const R*)(X.din && X.vin ? X.vin : X.v),
         (const R*)(X.din && X.ain ? X.ain : X.a), X.fstride, dt, c1, (double*)X.SR.kxd, X.pin, X.ng,
         X.hg);
-  DefArgs<R> A;
-  A.ndef = X.ndef, A.defs = X.defs, A.part_off = X.part_off;
-  A.fpart = (const R*)X.fpart, A.FPS = X.T.FPS;
-  A.src = X.dsrc, A.ampl = X.ampl, A.nt = X.ampl_nt, A.it = it, A.itp = X.itp;
-  A.abso = X.dabso, A.abson = X.dabson, A.rmdef = (const R*)X.rmdef;
-  A.d = (R*)X.d, A.v = (R*)X.v, A.a = (R*)X.a, A.GS = X.fstride;
-  A.dt = dt, A.c1 = c1, A.c2 = c2, A.c3 = c3, A.c4 = c4;
-  A.so = X.out, A.recp = (R*)(X.rec ? X.rec : X.a);
-  A.din = (const R*)X.din, A.vin = (const R*)X.vin, A.ain = (const R*)X.ain;
-  A.SR = X.SR, A.rec = X.recout;
-  A.rec.src = !X.out.final ? (const void*)A.recp : (A.rec.field == 0 ? X.d : (A.rec.field == 1 ? X.v : X.a));
-  A.fdef = X.fdef;
-  if (X.fault_on) A.F = X.F, A.fo = X.fo;
+  const DefArgs<R> A = def_args<R>(X, it, dt, c1, c2, c3, c4);
   const int lanes = X.ndef + A.rec.nint + (X.fault_on ? A.fo.nwave * 64 : 0);
   auto deferred = [&](auto nd, auto oop, auto pin, auto flt) {
     k_deferred<R, decltype(nd)::value, decltype(oop)::value, decltype(pin)::value, decltype(flt)::value>
@@ -1457,6 +1526,69 @@ __global__ void k_periodic(int n, const int* __restrict__ m, const int* __restri
   }
 }
 
+// Polls of one wait of k_run_steps before it gives up (0.5 us or more each); SEM2D_RUN_SPINS
+// sets it, 0 makes a launch give up where a neighbour is not there yet.
+int run_spins() {
+  const char* env = getenv("SEM2D_RUN_SPINS");
+  return env ? std::max(0, atoi(env)) : 1 << 20;
+}
+
+// Steps from which a run of them is one launch of k_run_steps: the launch, its start and
+// end and the check that it went through cost some 30 us more than two launches, and a step
+// saves 8 (100 x 100 P-SV elements, FP64: 14.2 -> 6.0 us).
+constexpr int RUN_MIN = 16;
+// Steps h->it + 1 .. h->it + n from the predicted state to the final one in one launch;
+// *done: whether they were taken (the state is unchanged otherwise)
+template <typename R, int NDOF, int NELAST, int MODE>
+int launch_run_k(sem2d_solver* h, const StepDev& X, int n, const StepCoefs<R>& K, bool* done) {
+  StructState& S = h->st;
+  *done = false;
+  const void* kern = (const void*)k_run_steps<R, NDOF, NELAST, MODE>;
+  if (S.run_ok == 0) {
+    int dev = 0, ncu = 0, coop = 0, per = 0;
+    HIPCHK(h, hipGetDevice(&dev));
+    HIPCHK(h, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    HIPCHK(h, hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+    HIPCHK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, TS_NT, 0));
+    S.run_ok = coop && S.ntiles <= ncu * per ? 1 : -1;
+    if (S.run_ok < 0) return 0;
+  }
+  HIPCHK(h, hipMemsetAsync(S.run_count, 0, sizeof(unsigned), h->stream));
+  RunArgs<R> A;
+  A.T = tile_args<R, MODE>(X, K.dt, K.c1, K.c2, K.c3, K.c4);
+  A.D = def_args<R>(X, h->it + 1, K.dt, K.c1, K.c2, K.c3, K.c4);
+  A.fpart2 = (R*)S.fpart2;
+  A.nbr = S.nbr, A.slot_def = S.slot_def;
+  A.flag = S.run_flag, A.arrived = S.run_count, A.fail = S.run_fail;
+  A.epoch = S.epoch;
+  A.nsteps = n;
+  A.spins = run_spins();
+  void* args[] = {&A};
+  if (hipLaunchCooperativeKernel(kern, dim3(S.ntiles), dim3(TS_NT), args, 0, h->stream) != hipSuccess) {
+    (void)hipGetLastError();  // one process at a time has the device's cooperative queue
+    S.run_ok = -1;
+    return 0;
+  }
+  S.epoch += n;
+  int fail = 0;
+  HIPCHK(h, hipMemcpyAsync(&fail, S.run_fail, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  if (fail) S.run_ok = -1;  // the device is shared with something that keeps tiles waiting
+  *done = !fail;
+  return 0;
+}
+template <typename R>
+int launch_run(sem2d_solver* h, const StepDev& X, int n, const StepCoefs<R>& K, bool* done) {
+  if (X.ndof == 2) {
+    if (X.coef_mode == COEF_SHARED) return launch_run_k<R, 2, 6, COEF_SHARED>(h, X, n, K, done);
+    if (X.nodemod) return launch_run_k<R, 2, 6, COEF_NODE>(h, X, n, K, done);
+    return launch_run_k<R, 2, 6, COEF_COMPACT>(h, X, n, K, done);
+  }
+  if (X.coef_mode == COEF_SHARED) return launch_run_k<R, 1, 2, COEF_SHARED>(h, X, n, K, done);
+  if (X.nodemod) return launch_run_k<R, 1, 2, COEF_NODE>(h, X, n, K, done);
+  return launch_run_k<R, 1, 2, COEF_COMPACT>(h, X, n, K, done);
+}
+
 template <typename R>
 int do_steps(sem2d_solver* h, int nsteps) {
   int rc = sync_sources(h);
@@ -1490,6 +1622,22 @@ int do_steps(sem2d_solver* h, int nsteps) {
   HIPCHK(h, hipEventRecord(h->ev0, h->stream));
   for (int s = 0; s < nsteps; ++s) {
     const int it = h->it + 1;
+    if (tables && X.pin && h->st.run_ok >= 0) {
+      // up to the call's last step or the next progress row
+      int n = nsteps - s;
+      if (h->itinfo > 0) n = std::min(n, h->itinfo - h->it % h->itinfo);
+      bool done = false;
+      if (n >= RUN_MIN && (rc = launch_run<R>(h, X, n, K, &done))) return rc;
+      if (done) {
+        for (int k = 1; k <= n; ++k)
+          if (sampled(h, h->it + k)) h->taken = std::max(h->taken, (h->it + k) / h->isamp + 1);
+        h->it += n;
+        X.pin = false;
+        record_info<R>(h, h->it);
+        s += n - 1;
+        continue;
+      }
+    }
     if (tables) {
       // the steps between hand the predicted state on (StepOut); the call's last step and
       // those with a progress row store d, v and a

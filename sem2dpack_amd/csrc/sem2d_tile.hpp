@@ -1045,6 +1045,19 @@ struct DefVals {
   double C[NDOF], am;
   SrcEntry e;
 };
+// places of the first four partial forces (the last one again past their number)
+template <typename R>
+__device__ __forceinline__ void def_offsets(const DefArgs<R>& A, const DefNode& n, int (&o)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = 0;
+  if (n.pinl) {
+    o[0] = n.poff[0];
+    o[1] = n.poff[1] >= 0 ? n.poff[1] : o[0];
+  } else if (n.pcnt > 0) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = A.part_off[n.pstart + min(k, n.pcnt - 1)];
+  }
+}
 template <typename R, int NDOF, bool OOP, bool PIN>
 __device__ __forceinline__ DefVals<R, NDOF> def_load(const DefArgs<R>& A, const DefNode& n, int q, int it) {
   const size_t g = n.g, GS = A.GS;
@@ -1053,14 +1066,8 @@ __device__ __forceinline__ DefVals<R, NDOF> def_load(const DefArgs<R>& A, const 
   const R* dsrc = OOP ? A.din : A.d;
   const R* vsrc = OOP && A.vin ? A.vin : A.v;
   const R* asrc = OOP && A.ain ? A.ain : A.a;
-  int o[4] = {0, 0, 0, 0};
-  if (n.pinl) {
-    o[0] = n.poff[0];
-    o[1] = n.poff[1] >= 0 ? n.poff[1] : o[0];
-  } else if (n.pcnt > 0) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) o[k] = A.part_off[n.pstart + min(k, n.pcnt - 1)];
-  }
+  int o[4];
+  def_offsets<R>(A, n, o);
 #pragma unroll
   for (int c = 0; c < NDOF; ++c) {
     s.d[c] = dsrc[c * GS + g];
@@ -1300,6 +1307,300 @@ __global__ __launch_bounds__(256) void k_deferred(DefArgs<R> A) {
     def_store<R>(A, s, c, (size_t)c * A.GS + n.g, ak, n.rec);
     if (rr.at >= 0)
       rec_put(rows, A.rec, A.rec.def_q, A.rec.def_r, A.rec.ndefr, rr, q, c, rec_value<R>(A.rec, s, c, ak));
+  }
+}
+
+// Arguments of k_run_steps
+template <typename R>
+struct RunArgs {
+  TileArgs<R> T;
+  DefArgs<R> D;         // D.it: the first step
+  R* fpart2;            // partial forces of every second step
+  const int* nbr;       // [ntiles][8] tiles that share a node with a tile, or -1
+  const int* slot_def;  // [ntiles][SLOTS] deferred node of a partial force, or -1
+  unsigned* flag;       // [ntiles][FLAG_STRIDE] epoch + the steps whose partial forces a tile has stored
+  unsigned* arrived;    // tiles through with the steps; RUN_POISON added: a tile has given up
+  unsigned epoch;
+  int nsteps, spins;
+  int* fail;
+};
+constexpr int FLAG_STRIDE = 16;
+constexpr unsigned RUN_POISON = 1u << 24;
+
+// nsteps steps of a small grid in one launch, a workgroup per tile, all of them resident
+// together (cooperative launch): a step by its two launches is bound by their start and by
+// the reads and stores of a state that fits in the compute units (100 x 100 P-SV elements,
+// FP64: 14.2 us a step of two launches, 6.0 here).  The state is the predicted one, the
+// displacement in LDS, velocity and inverse mass in the registers of the node's lane.  After
+// the element phase a tile stores the partial forces of its perimeter and special nodes,
+// raises its flag, waits for the flags of the up to eight tiles that share nodes with it and
+// finishes those nodes itself, as k_deferred does; a node that several tiles share is
+// computed by each of them from the same values in the same order.  Partial forces alternate
+// between two arrays: a tile stores those of step s + 2 when its neighbours have raised their
+// flags for step s + 1, that is, have read those of step s.
+//
+// Partial forces, flags and the count go past the L2 caches of the XCDs (atomic accesses at
+// agent scope); a tile's stores are waited for before its flag is raised, so no cache is
+// written back or invalidated.
+//
+// A wait ends after `spins` polls.  Nothing of the state is stored before every tile is
+// through (a count at the end), so that a launch that has given up leaves the state it
+// started from, and the steps are then taken by the other kernels.
+template <typename R, int NDOF, int NELAST, int MODE>
+__global__ __launch_bounds__(TS_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_run_steps(RunArgs<R> A) {
+  constexpr int PS = PXM, NEL = TX * TZ;
+  constexpr bool NODEM = MODE == COEF_NODE, COMP = MODE == COEF_COMPACT;
+  using LV = typename LVec<R, NDOF>::T;
+  __shared__ LV Ud[PMAX];
+  __shared__ LV Ex[NEL * NP + 1];
+  __shared__ LV Mn[NODEM ? PMAX : 1];
+  __shared__ R Sa[MODE == COEF_SHARED ? NELAST * NP : 1];
+  __shared__ R Gm[NEL][3];
+  __shared__ R sW2[NP];
+  __shared__ int stop;
+  const TileArgs<R>& T = A.T;
+  const DefArgs<R>& D = A.D;
+  const int t = blockIdx.x, tid = threadIdx.x;
+  const int4 tg = T.tiles[t], gr = T.grids[t];
+  const int nxe = tg.z & 0xff, nze = (tg.z >> 8) & 0xff, nx = tg.z >> 16;
+  const int PX = 4 * nxe + 1, PZ = 4 * nze + 1, X0 = 4 * tg.x, Z0 = tg.w;
+  const int kL = tg.x / TX, kR = (tg.x + nxe + TX - 1) / TX;
+  const int ns = T.spec_cnt[t];
+  if (tid < NP) sW2[tid] = (R)c_W2[tid];
+  if (tid == 0) Ex[NEL * NP] = LV{}, stop = 0;
+
+  // this lane's patch nodes: storage index, slot of the partial force (-1: the node is
+  // finished here), velocity, inverse mass, first receiver
+  size_t g[TS_ITER];
+  int slot[TS_ITER], ir[TS_ITER];
+  bool in[TS_ITER];
+  NodeSlots sl[TS_ITER];
+  R vr[TS_ITER][NDOF], rm[TS_ITER];
+#pragma unroll
+  for (int r = 0; r < TS_ITER; ++r) {
+    const int p = tid + TS_NT * r, Z = p / PS, X = p - Z * PS;
+    in[r] = X < PX && Z < PZ;
+    g[r] = node_index(gr, min(X, PX - 1), min(Z, PZ - 1), PX, X0, Z0, kL, kR);
+    slot[r] = in[r] ? perim_slot(X, Z, PX, PZ) : -1;
+    for (int k = 0; k < ns; ++k)
+      if (T.spec_idx[t * MAXSPECIAL + k] == p) slot[r] = PERIM_MAX + k;
+    sl[r] = c_slots.node[min(p, PMAX - 1)];
+    rm[r] = T.rmass0[g[r]];
+    R u[NDOF], m[NDOF];
+#pragma unroll
+    for (int c = 0; c < NDOF; ++c) {
+      u[c] = T.d[c * T.S + g[r]];
+      vr[r][c] = T.v[c * T.S + g[r]];
+      if constexpr (NODEM) m[c] = T.coefs[c * T.S + g[r]];
+    }
+    if (p < PMAX) {
+      Ud[p] = lv_make<R, NDOF>(u);
+      if constexpr (NODEM) Mn[p] = lv_make<R, NDOF>(m);
+    }
+    ir[r] = -1;
+    if (D.rec.seis && in[r] && slot[r] < 0) {
+      int lo = 0, hi = D.rec.nint;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if ((size_t)D.rec.int_g[mid] < g[r]) lo = mid + 1;
+        else hi = mid;
+      }
+      if (lo < D.rec.nint && (size_t)D.rec.int_g[lo] == g[r]) ir[r] = lo;
+    }
+  }
+  if constexpr (MODE == COEF_SHARED) {
+    for (int k = tid; k < NELAST * NP; k += TS_NT) Sa[k] = T.coefs[gr.w + k];
+  } else {
+    if (tid < NEL * 3) {
+      const int e = tid / 3, k = tid - 3 * (tid / 3);
+      Gm[e][k] = T.geom[cell_index(gr, nx, tg.x, tg.y, min(e % TX, nxe - 1), min(e / TX, nze - 1)) * 3 + k];
+    }
+  }
+  const int lane = tid & 63;
+  const int e = (tid >> 6) * TS_EPW + lane / NG, s = lane % NG;
+  const int lx = e % TX, lz = e / TX;
+  const bool eslot = lane < TS_EPW * NG && e < NEL, on = eslot && lx < nxe && lz < nze;
+  const int base = 4 * lz * PS + 4 * lx;
+  LV* ex = Ex + min(e, NEL - 1) * NP;
+  R m[COMP ? NG : 1][NDOF];
+  if constexpr (COMP) {
+    const size_t cell = cell_index(gr, nx, tg.x, tg.y, min(lx, nxe - 1), min(lz, nze - 1));
+#pragma unroll
+    for (int i = 0; i < NG; ++i)
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) m[i][c] = T.coefs[(cell * NDOF + c) * NP + s * NG + i];
+  }
+
+  // the deferred node of this lane (one lane per slot), its values and its patch node
+  const int nper = 2 * PX + 2 * (PZ - 2);
+  const bool dl = tid < nper || (tid >= PERIM_MAX && tid < PERIM_MAX + ns);
+  int pp = 0, dq = 0, o[4] = {0, 0, 0, 0};
+  DefNode n{};
+  DefVals<R, NDOF> x{};
+  RecRef rr;
+  if (dl) {
+    if (tid < nper) {
+      const int w = tid - 2 * PX;
+      const int X = tid < 2 * PX ? tid % PX : (w < PZ - 2 ? 0 : PX - 1);
+      const int Z = tid < PX ? 0 : (tid < 2 * PX ? PZ - 1 : w % (PZ - 2) + 1);
+      pp = Z * PS + X;
+    } else {
+      pp = T.spec_idx[t * MAXSPECIAL + tid - PERIM_MAX];
+    }
+    dq = A.slot_def[t * SLOTS + tid];
+    n = def_unpack(D.defs, dq);
+    def_offsets<R>(D, n, o);
+    x = def_load<R, NDOF, false, true>(D, n, dq, D.it);
+    if (D.rec.seis) rr = rec_ref(D.rec.def_q, D.rec.def_r, D.rec.ndefr, n.rec_at);
+  }
+  const bool own = dl && o[0] / SLOTS == t;  // stores and records the node
+  const int nb = tid < 8 ? A.nbr[t * 8 + tid] : -1;
+  const R dt = T.dt, c1 = T.c1, c2 = T.c2, c3 = T.c3, c4 = T.c4;
+  const int field = D.rec.field;
+  R fa[TS_ITER][NDOF], fd[NDOF] = {};  // last step: the accelerations, for the stores
+#pragma unroll
+  for (int r = 0; r < TS_ITER; ++r)
+#pragma unroll
+    for (int c = 0; c < NDOF; ++c) fa[r][c] = 0;
+  __syncthreads();
+
+#pragma unroll 1
+  for (int k = 0; k < A.nsteps; ++k) {
+    const int it = D.it + k;
+    const bool last = k == A.nsteps - 1;
+    double* const rows = rec_rows(D.rec, NDOF, it);
+    if (dl && n.scnt > 0) x.am = it >= 1 && it <= D.nt ? D.ampl[(size_t)x.e.src * D.nt + (it - 1)] : 0.0;
+    {
+      const auto* hp = hconst<R>();
+      R H[NG][NG];
+#pragma unroll
+      for (int a = 0; a < NG; ++a)
+#pragma unroll
+        for (int b = 0; b < NG; ++b) H[a][b] = hp[a * NG + b];
+      el_gradient<R, NDOF, false>(on, base, s, e, ex, Ud, Ud, (const R*)nullptr, H);
+      wave_order();
+      R s1r[NG][NDOF];
+      el_flux<R, NDOF, NELAST, MODE, false>(on, base, s, e, ex, Ud, Ud, (const R*)nullptr, H, Gm, sW2, Sa, Mn, m,
+                                            [](int, int) { return R(0); }, s1r);
+      wave_order();
+      el_divergence<R, NDOF>(on, s, ex, H);
+      wave_order();
+      el_force<R, NDOF, false>(on, eslot, false, base, s, e, ex, Ud, Ud, (const R*)nullptr, (const R*)nullptr, s1r);
+    }
+    __syncthreads();
+    R* const fp = k & 1 ? A.fpart2 : T.fpart;
+    R F[TS_ITER][NDOF];
+#pragma unroll
+    for (int r = 0; r < TS_ITER; ++r) {
+      const LV f0 = Ex[sl[r].q[0]], f1 = Ex[sl[r].q[1]], f2 = Ex[sl[r].q[2]], f3 = Ex[sl[r].q[3]];
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        F[r][c] = ((lv_get<R, NDOF>(f0, c) + lv_get<R, NDOF>(f1, c)) + lv_get<R, NDOF>(f2, c)) + lv_get<R, NDOF>(f3, c);
+        if (slot[r] >= 0)
+          __hip_atomic_store(&fp[c * T.FPS + (size_t)t * SLOTS + slot[r]], F[r][c], __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    // nodes that are finished here
+#pragma unroll
+    for (int r = 0; r < TS_ITER; ++r)
+      if (in[r] && slot[r] < 0) {
+        const int p = tid + TS_NT * r;
+        const LV u = Ud[p];
+        R nu[NDOF];
+#pragma unroll
+        for (int c = 0; c < NDOF; ++c) {
+          const R ak = F[r][c] * rm[r];
+          const R vn = vr[r][c] + c3 * ak;
+          const R dn = lv_get<R, NDOF>(u, c) + c4 * ak;
+          vr[r][c] = last ? vn : vn + c2 * ak;
+          nu[c] = last ? dn : dn + dt * vn + c1 * ak;
+          if (last) fa[r][c] = ak;
+          if (rows && ir[r] >= 0)
+            for (int q = ir[r]; q < D.rec.nint && (size_t)D.rec.int_g[q] == g[r]; ++q)
+              rows[(size_t)c * D.rec.nrec + D.rec.int_r[q]] = (double)(field == 0 ? dn : (field == 1 ? vn : ak));
+        }
+        Ud[p] = lv_make<R, NDOF>(nu);
+      }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial forces are past the L2
+    __syncthreads();
+    if (tid == 0)
+      __hip_atomic_store(&A.flag[(size_t)t * FLAG_STRIDE], A.epoch + k + 1, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    if (nb >= 0) {
+      int left = A.spins;
+      while ((int)(__hip_atomic_load(&A.flag[(size_t)nb * FLAG_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) -
+                   (A.epoch + k + 1)) < 0) {
+        if (--left < 0) {
+          stop = 1;
+          break;
+        }
+      }
+    }
+    __syncthreads();
+    if (stop) break;
+    if (dl) {
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (q < 2 || !n.pinl)
+            x.f[q][c] = __hip_atomic_load(&fp[c * T.FPS + o[q]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      NodeState<R> st = def_state<R, NDOF, true>(D, n, x, it);
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        const R ak = st.f[c] * x.rm[c];
+        const R vn = st.v[c] + c3 * ak;
+        const R dn = st.d[c] + c4 * ak;
+        x.v[c] = last ? vn : vn + c2 * ak;
+        x.d[c] = last ? dn : dn + dt * vn + c1 * ak;
+        if (last) fd[c] = ak;
+        if (rows && own && rr.at >= 0)
+          rec_put(rows, D.rec, D.rec.def_q, D.rec.def_r, D.rec.ndefr, rr, dq, c,
+                  (double)(field == 0 ? dn : (field == 1 ? vn : ak)));
+      }
+      Ud[pp] = lv_make<R, NDOF>(x.d);
+    }
+    __syncthreads();
+  }
+
+  // the state is stored when every tile is through; a tile that gives up (or has waited too
+  // long here) takes the count past the number that the others wait for
+  if (tid == 0) {
+    const unsigned want = gridDim.x;
+    bool ok = !stop;
+    if (ok) {
+      unsigned at = __hip_atomic_fetch_add(A.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+      for (int left = A.spins; at < want && left > 0; --left)
+        at = __hip_atomic_load(A.arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (at < want) at = __hip_atomic_fetch_add(A.arrived, RUN_POISON, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      ok = at == want;
+    } else {
+      __hip_atomic_fetch_add(A.arrived, RUN_POISON, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!ok) *A.fail = 1;
+    stop = !ok;
+  }
+  __syncthreads();
+  if (stop) return;
+#pragma unroll
+  for (int r = 0; r < TS_ITER; ++r)
+    if (in[r] && slot[r] < 0) {
+      const LV u = Ud[tid + TS_NT * r];
+#pragma unroll
+      for (int c = 0; c < NDOF; ++c) {
+        T.a[c * T.S + g[r]] = fa[r][c];
+        T.v[c * T.S + g[r]] = vr[r][c];
+        T.d[c * T.S + g[r]] = lv_get<R, NDOF>(u, c);
+      }
+    }
+  if (own) {
+#pragma unroll
+    for (int c = 0; c < NDOF; ++c) {
+      T.a[c * T.S + n.g] = fd[c];
+      T.v[c * T.S + n.g] = x.v[c];
+      T.d[c * T.S + n.g] = x.d[c];
+    }
   }
 }
 
