@@ -354,8 +354,11 @@ __device__ inline PairOut fault_solve(const FaultDev& F, const PairData& P, int 
   }
 #pragma unroll
   for (int c = 0; c < nd; ++c) {
-    const double bt = P.B[c] * Tx[c];
-    n1.f[c] = (R)((double)n1.f[c] + bt);
+    // one rounding at node 1, two at node 2, however the compiler arranges the code around:
+    // with FP32 fields a bit here grows to 1e-5 of a rupture's tractions in a hundred steps
+    double bt = P.B[c] * Tx[c];
+    asm volatile("" : "+v"(bt));
+    n1.f[c] = (R)__builtin_fma(P.B[c], Tx[c], (double)n1.f[c]);
     if (two) n2.f[c] = (R)((double)n2.f[c] - bt);
   }
   F.sigma[k] = sigma;
