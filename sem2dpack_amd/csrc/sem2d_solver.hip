@@ -248,6 +248,40 @@ int upload_bulk(sem2d_solver* h, void** p, const double* src, size_t n) {
   return upload(h, (float**)p, tmp.data(), n);
 }
 
+// rows of `per` values, row e of src to row to[e] of dst, in the bulk type
+template <typename R>
+__global__ void k_scatter_rows(size_t n, int per, const double* __restrict__ src, const int* __restrict__ to,
+                               R* __restrict__ dst) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const size_t e = i / per;
+  dst[(size_t)to[e] * per + (i - e * per)] = (R)src[i];
+}
+// Uploads the rows of per-element arrays into another order of the elements: copied as they
+// are, in pieces, and put in their place on the device (the ten coefficients of 24,120
+// elements: a new solver 16 ms where the host ordered them first, 6 ms so).
+int upload_rows(sem2d_solver* h, void** p, const double* src, int nelem, int per, const std::vector<int>& to) {
+  int rc = dev_alloc(h, (char**)p, (size_t)nelem * per * rsize(h));
+  if (rc) return rc;
+  const int piece = std::min<int>(nelem, std::max<size_t>(1, ((size_t)64 << 20) / (per * sizeof(double))));
+  const size_t bytes = (size_t)piece * per * sizeof(double);
+  char* tmp = nullptr;
+  HIPCHK(h, hipMalloc((void**)&tmp, bytes + (size_t)nelem * sizeof(int)));
+  int* pos = (int*)(tmp + bytes);
+  hipError_t e = hipMemcpyAsync(pos, to.data(), (size_t)nelem * sizeof(int), hipMemcpyHostToDevice, h->stream);
+  for (int e0 = 0; e0 < nelem && e == hipSuccess; e0 += piece) {
+    const size_t n = (size_t)std::min(piece, nelem - e0) * per;
+    e = hipMemcpyAsync(tmp, src + (size_t)e0 * per, n * sizeof(double), hipMemcpyHostToDevice, h->stream);
+    const unsigned blocks = (unsigned)((n + 255) / 256);
+    if (h->fp32) k_scatter_rows<float><<<blocks, 256, 0, h->stream>>>(n, per, (double*)tmp, pos + e0, (float*)*p);
+    else k_scatter_rows<double><<<blocks, 256, 0, h->stream>>>(n, per, (double*)tmp, pos + e0, (double*)*p);
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  hipFree(tmp);
+  HIPCHK(h, e);
+  return 0;
+}
+
 int write_bulk(sem2d_solver* h, void* dst, const double* src, size_t n) {
   if (!h->fp32) {
     HIPCHK(h, hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, h->stream));
@@ -1808,15 +1842,11 @@ int sem2d_create(const sem2d_desc* s, sem2d_solver** out) {
     // per-element arrays follow the colour-sorted element order
     const size_t per = h->coef_mode == COEF_COMPACT ? (size_t)h->ndof * NP : (size_t)h->nelast * NP;
     const double* src = h->coef_mode == COEF_COMPACT ? s->lam_mu : s->coefs;
-    std::vector<double> co((size_t)s->nelem * per);
-    for (int k = 0; k < s->nelem; ++k)
-      std::memcpy(&co[(size_t)k * per], src + (size_t)h->elem_order[k] * per, per * sizeof(double));
-    if ((rc = upload_bulk(h, &h->coefs, co.data(), co.size()))) return rc;
+    std::vector<int> to(s->nelem);
+    for (int k = 0; k < s->nelem; ++k) to[h->elem_order[k]] = k;
+    if ((rc = upload_rows(h, &h->coefs, src, s->nelem, (int)per, to))) return rc;
     if (h->coef_mode == COEF_COMPACT) {
-      std::vector<double> ge((size_t)s->nelem * 3);
-      for (int k = 0; k < s->nelem; ++k)
-        for (int q = 0; q < 3; ++q) ge[(size_t)k * 3 + q] = s->geom[(size_t)h->elem_order[k] * 3 + q];
-      if ((rc = upload_bulk(h, &h->geom, ge.data(), ge.size()))) return rc;
+      if ((rc = upload_rows(h, &h->geom, s->geom, s->nelem, 3, to))) return rc;
     }
   }
   const size_t nf = (size_t)h->ndof * h->npoin;
@@ -1839,15 +1869,11 @@ int sem2d_create(const sem2d_desc* s, sem2d_solver** out) {
       // per-element arrays in cell order (iz*nx + ix)
       const size_t per = h->coef_mode == COEF_COMPACT ? (size_t)h->ndof * NP : (size_t)h->nelast * NP;
       const double* src = h->coef_mode == COEF_COMPACT ? s->lam_mu : s->coefs;
-      std::vector<double> co((size_t)s->nelem * per);
-      for (int cell = 0; cell < s->nelem; ++cell)
-        std::memcpy(&co[(size_t)cell * per], src + (size_t)(s->elem_of_cell[cell] - 1) * per, per * sizeof(double));
-      if ((rc = upload_bulk(h, &S.coefs, co.data(), co.size()))) return rc;
+      std::vector<int> to(s->nelem);
+      for (int cell = 0; cell < s->nelem; ++cell) to[S.cell_elem[cell]] = cell;
+      if ((rc = upload_rows(h, &S.coefs, src, s->nelem, (int)per, to))) return rc;
       if (h->coef_mode == COEF_COMPACT) {
-        std::vector<double> ge((size_t)s->nelem * 3);
-        for (int cell = 0; cell < s->nelem; ++cell)
-          for (int q = 0; q < 3; ++q) ge[(size_t)cell * 3 + q] = s->geom[(size_t)(s->elem_of_cell[cell] - 1) * 3 + q];
-        if ((rc = upload_bulk(h, &S.geom, ge.data(), ge.size()))) return rc;
+        if ((rc = upload_rows(h, &S.geom, s->geom, s->nelem, 3, to))) return rc;
         // the moduli once per node, if every element at a node holds bitwise the same
         // values there (a medium given as a function of position)
         const int nd = h->ndof;
