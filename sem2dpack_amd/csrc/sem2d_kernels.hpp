@@ -19,10 +19,11 @@ __constant__ double c_H[NP];
 __constant__ double c_W2[NP];
 __constant__ float c_Hf[NP];  // c_H in single precision
 
-// Coefficient storage modes (sem2d_desc.coef_mode).  COEF_NODE is internal to the
-// structured tile kernel: the compact moduli stored once per global node (in the field
-// layout) when every element sharing a node holds the same values there.
-enum { COEF_PER_ELEM = 0, COEF_SHARED = 1, COEF_COMPACT = 2, COEF_NODE = 3 };
+// Coefficient storage modes (sem2d_desc.coef_mode).  COEF_NODE and COEF_ELEM are internal to
+// the structured tile kernels: the compact moduli once per global node (in the field layout)
+// when every element sharing a node holds the same values there, or once per element when
+// all its points hold the same.
+enum { COEF_PER_ELEM = 0, COEF_SHARED = 1, COEF_COMPACT = 2, COEF_NODE = 3, COEF_ELEM = 4 };
 
 // h'_i(x_j) at [i*NG + j] in the bulk type, by a pointer the compiler cannot look through:
 // read at compile-time indices, the entries are scalar operands, loaded where this is

@@ -220,7 +220,7 @@ __device__ __forceinline__ void el_flux(bool on, int base, int s, int e, LV* ex,
       }
     }
     R g0 = 0, g1 = 0, g2 = 0;
-    if constexpr (MODE == COEF_COMPACT || MODE == COEF_NODE) {
+    if constexpr (MODE == COEF_COMPACT || MODE == COEF_NODE || MODE == COEF_ELEM) {
       g0 = Gm[e][0];
       g1 = Gm[e][1];
       g2 = Gm[e][2];
@@ -229,7 +229,7 @@ __device__ __forceinline__ void el_flux(bool on, int base, int s, int e, LV* ex,
     for (int i = 0; i < NG; ++i) {
       const int pt = s * NG + i;
       R A[NELAST];
-      if constexpr (MODE == COEF_COMPACT || MODE == COEF_NODE) {
+      if constexpr (MODE == COEF_COMPACT || MODE == COEF_NODE || MODE == COEF_ELEM) {
         const R w2 = sW2[pt];
         R m0, m1;
         if constexpr (MODE == COEF_NODE) {
@@ -237,8 +237,8 @@ __device__ __forceinline__ void el_flux(bool on, int base, int s, int e, LV* ex,
           m0 = lv_get<R, NDOF>(mm, 0);
           m1 = lv_get<R, NDOF>(mm, NDOF - 1);
         } else {
-          m0 = m[i][0];
-          m1 = m[i][NDOF - 1];
+          m0 = m[MODE == COEF_ELEM ? 0 : i][0];
+          m1 = m[MODE == COEF_ELEM ? 0 : i][NDOF - 1];
         }
         if constexpr (NDOF == 2) {
           const R la = m0, mu = m1, kx = la + 2 * mu;
@@ -454,7 +454,8 @@ k_tile_step(TileArgs<R> args) {
   constexpr int PS = PXM;        // patch row length
   constexpr int NEL = TX * TZ;   // element slots
   constexpr bool NODEM = MODE == COEF_NODE;
-  constexpr bool COMP = MODE == COEF_COMPACT;
+  constexpr bool COMP = MODE == COEF_COMPACT || MODE == COEF_ELEM;
+  constexpr int NM = MODE == COEF_COMPACT ? NG : 1;  // moduli of a row's points, or the element's
   // FULLPF: the registers admit the prefetch of everything a tile reads but per-element
   // moduli, and of a tile's forces until the next tile's loads have arrived.  Otherwise
   // (FP64 P-SV) the predicted velocity and the inverse mass, which only the stores need,
@@ -699,16 +700,17 @@ k_tile_step(TileArgs<R> args) {
 
     // the moduli of the points of this lane's row (element phase below), ahead of the waits
     // for the tile's node values
-    R m[COMP ? NG : 1][NDOF];
+    R m[NM][NDOF];
     if constexpr (COMP) {
       const int tl = lane_id(), lane = tl & 63;
       const int e = min((tl >> 6) * TS_EPW + lane / NG, NEL - 1), s = lane % NG;
       const R* bCo = ubase(P->coefs);
       const auto cell = cidx(gr, tg.z >> 16, G, min(e % TX, G.nxe - 1), min(e / TX, G.nze - 1));
 #pragma unroll
-      for (int i = 0; i < NG; ++i)
+      for (int i = 0; i < NM; ++i)
 #pragma unroll
-        for (int c = 0; c < NDOF; ++c) m[i][c] = fld(bCo, (cell * NDOF + c) * NP + s * NG + i);
+        for (int c = 0; c < NDOF; ++c)
+          m[i][c] = fld(bCo, NM == 1 ? cell * NDOF + c : (cell * NDOF + c) * NP + s * NG + i);
     }
 
     // predictor
@@ -1349,7 +1351,8 @@ constexpr unsigned RUN_POISON = 1u << 24;
 template <typename R, int NDOF, int NELAST, int MODE>
 __global__ __launch_bounds__(TS_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_run_steps(RunArgs<R> A) {
   constexpr int PS = PXM, NEL = TX * TZ;
-  constexpr bool NODEM = MODE == COEF_NODE, COMP = MODE == COEF_COMPACT;
+  constexpr bool NODEM = MODE == COEF_NODE, COMP = MODE == COEF_COMPACT || MODE == COEF_ELEM;
+  constexpr int NM = MODE == COEF_COMPACT ? NG : 1;
   using LV = typename LVec<R, NDOF>::T;
   __shared__ LV Ud[PMAX];
   __shared__ LV Ex[NEL * NP + 1];
@@ -1422,13 +1425,14 @@ __global__ __launch_bounds__(TS_NT) __attribute__((amdgpu_waves_per_eu(2))) void
   const bool eslot = lane < TS_EPW * NG && e < NEL, on = eslot && lx < nxe && lz < nze;
   const int base = 4 * lz * PS + 4 * lx;
   LV* ex = Ex + min(e, NEL - 1) * NP;
-  R m[COMP ? NG : 1][NDOF];
+  R m[NM][NDOF];
   if constexpr (COMP) {
     const size_t cell = cell_index(gr, nx, tg.x, tg.y, min(lx, nxe - 1), min(lz, nze - 1));
 #pragma unroll
-    for (int i = 0; i < NG; ++i)
+    for (int i = 0; i < NM; ++i)
 #pragma unroll
-      for (int c = 0; c < NDOF; ++c) m[i][c] = T.coefs[(cell * NDOF + c) * NP + s * NG + i];
+      for (int c = 0; c < NDOF; ++c)
+        m[i][c] = T.coefs[NM == 1 ? cell * NDOF + c : (cell * NDOF + c) * NP + s * NG + i];
   }
 
   // the deferred node of this lane (one lane per slot), its values and its patch node
@@ -1698,7 +1702,11 @@ struct AdjArgs {
 // added in row order.  HIST: the forward acceleration is the second difference of the
 // displacement history (fwd_accel).  The adjoint state of the interior nodes is read again
 // for the stores (a register each through the element phase would halve the wavefronts).
-template <typename R, bool HIST, bool W32>
+// ELEM: moduli per element (COEF_ELEM).  Bound by memory where the tiles fill the chip, by
+// the chain of a tile's phases where they do not: 400 x 400 elements, FP64, 113.6 us for 390
+// MB; 150 x 101 16.1 us.  (A lane per element point, with a workgroup barrier per colour and
+// three state arrays, in two launches: 162 and 18.8 + 16.9 us.)
+template <typename R, bool HIST, bool ELEM, bool W32>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_step(AdjArgs<R> args) {
   constexpr int NDOF = 2, PS = PXM, NEL = TX * TZ;
   using LV = typename LVec<R, NDOF>::T;
@@ -1882,13 +1890,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     }
     wave_order();
     // moduli of the row's points, the element's running sensitivities
-    R m[NG][NDOF];
+    constexpr int NM = ELEM ? 1 : NG;
+    R m[NM][NDOF];
     {
       const R* bco = ub(P->coefs);
 #pragma unroll
-      for (int i = 0; i < NG; ++i)
+      for (int i = 0; i < NM; ++i)
 #pragma unroll
-        for (int c = 0; c < NDOF; ++c) m[i][c] = at(bco, (cell * NDOF + c) * NP + s * NG + i);
+        for (int c = 0; c < NDOF; ++c)
+          m[i][c] = at(bco, ELEM ? cell * NDOF + c : (cell * NDOF + c) * NP + s * NG + i);
     }
     column(Uf);
     // the sensitivities first, then the fluxes: the gradient of d_n and the transposed
@@ -1935,7 +1945,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
       for (int i = 0; i < NG; ++i) {
         const int pt = s * NG + i;
         const R w = sW2[pt];
-        const R la = m[i][0], mu = m[i][1], kx = la + 2 * mu;
+        const R la = m[ELEM ? 0 : i][0], mu = m[ELEM ? 0 : i][1], kx = la + 2 * mu;
         const R A0 = w * kx * g0, A1 = w * la * g2, A2 = w * kx * g1;
         const R A3 = w * mu * g1, A4 = w * mu * g2, A5 = w * mu * g0;
         R pxi[NDOF];

@@ -32,9 +32,13 @@ def problem(nx, nz, ndof, medium, **kw):
     p = parfile.parse_par(par(nx, nz, ndof, **kw))
     if medium == "uniform":  # one set of point coefficients
         return builder.build(p)
-    if medium == "nodes":  # moduli continuous across elements
+    if medium != "elements":  # moduli continuous across elements, or but for one element
         grid = workloads.layered_random_grid((0.0, 100.0 * nx + 400.0), (0.0, 100.0 * nz + 400.0), dx=400.0)
-        return builder.build(p, material=workloads.hete1_material(*grid), per_element_coefs=False)
+        pb = builder.build(p, material=workloads.hete1_material(*grid), per_element_coefs=False)
+        if medium == "points":
+            pb.lam_mu = np.array(pb.lam_mu)
+            pb.lam_mu[0] *= 1.01
+        return pb
     n, rng = nx * nz, np.random.default_rng(nx)
     mu = 2670.0 * 3464.0 ** 2 * (1 + 0.1 * rng.random(n))
     return builder.build(p, elem_props=(2670.0 * np.ones(n), mu, mu), per_element_coefs=False)
@@ -57,7 +61,8 @@ def same(a, b):
 @pytest.mark.parametrize("fp32", [False, True])
 @pytest.mark.parametrize("nx,nz,ndof,medium", [(1, 1, 2, "uniform"), (9, 17, 2, "elements"), (24, 16, 2, "nodes"),
                                                (128, 128, 2, "uniform"), (130, 128, 2, "nodes"),
-                                               (7, 9, 1, "uniform"), (33, 25, 1, "elements"), (170, 178, 1, "nodes")])
+                                               (7, 9, 1, "uniform"), (33, 25, 1, "elements"), (170, 178, 1, "nodes"),
+                                               (24, 16, 2, "points"), (10, 9, 1, "points")])
 def test_runs(nx, nz, ndof, medium, fp32):
     print(f"\n[runs {nx}x{nz} ndof={ndof} {medium} fp32={fp32}]", flush=True)
     pb = problem(nx, nz, ndof, medium)
