@@ -260,24 +260,39 @@ __global__ void k_scatter_rows(size_t n, int per, const double* __restrict__ src
   const size_t e = i / per;
   dst[(size_t)to[e] * per + (i - e * per)] = (R)src[i];
 }
-// Uploads the rows of per-element arrays into another order of the elements: copied as they
-// are, in pieces, and put in their place on the device (the ten coefficients of 24,120
-// elements: a new solver 16 ms where the host ordered them first, 6 ms so).
-int upload_rows(sem2d_solver* h, void** p, const double* src, int nelem, int per, const std::vector<int>& to) {
-  int rc = dev_alloc(h, (char**)p, (size_t)nelem * per * rsize(h));
-  if (rc) return rc;
+// Uploads the rows of a per-element array into one or two other orders of the elements:
+// copied once as they are, in pieces, and put in their places on the device (the ten
+// coefficients of 24,120 elements: a new solver 16 ms where the host ordered them first, 6 ms
+// so).
+struct RowOrder {
+  void** p;
+  const std::vector<int>* to;
+};
+int upload_rows(sem2d_solver* h, const double* src, int nelem, int per, std::initializer_list<RowOrder> orders) {
+  int rc;
+  for (const RowOrder& o : orders)
+    if ((rc = dev_alloc(h, (char**)o.p, (size_t)nelem * per * rsize(h)))) return rc;
   const int piece = std::min<int>(nelem, std::max<size_t>(1, ((size_t)64 << 20) / (per * sizeof(double))));
   const size_t bytes = (size_t)piece * per * sizeof(double);
   char* tmp = nullptr;
-  HIPCHK(h, hipMalloc((void**)&tmp, bytes + (size_t)nelem * sizeof(int)));
-  int* pos = (int*)(tmp + bytes);
-  hipError_t e = hipMemcpyAsync(pos, to.data(), (size_t)nelem * sizeof(int), hipMemcpyHostToDevice, h->stream);
+  HIPCHK(h, hipMalloc((void**)&tmp, bytes + orders.size() * nelem * sizeof(int)));
+  int* const pos = (int*)(tmp + bytes);
+  hipError_t e = hipSuccess;
+  int k = 0;
+  for (const RowOrder& o : orders)
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(pos + (size_t)nelem * k++, o.to->data(), (size_t)nelem * sizeof(int),
+                         hipMemcpyHostToDevice, h->stream);
   for (int e0 = 0; e0 < nelem && e == hipSuccess; e0 += piece) {
     const size_t n = (size_t)std::min(piece, nelem - e0) * per;
     e = hipMemcpyAsync(tmp, src + (size_t)e0 * per, n * sizeof(double), hipMemcpyHostToDevice, h->stream);
     const unsigned blocks = (unsigned)((n + 255) / 256);
-    if (h->fp32) k_scatter_rows<float><<<blocks, 256, 0, h->stream>>>(n, per, (double*)tmp, pos + e0, (float*)*p);
-    else k_scatter_rows<double><<<blocks, 256, 0, h->stream>>>(n, per, (double*)tmp, pos + e0, (double*)*p);
+    k = 0;
+    for (const RowOrder& o : orders) {
+      const int* to = pos + (size_t)nelem * k++ + e0;
+      if (h->fp32) k_scatter_rows<float><<<blocks, 256, 0, h->stream>>>(n, per, (double*)tmp, to, (float*)*o.p);
+      else k_scatter_rows<double><<<blocks, 256, 0, h->stream>>>(n, per, (double*)tmp, to, (double*)*o.p);
+    }
   }
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
   hipFree(tmp);
@@ -1849,19 +1864,11 @@ int sem2d_create(const sem2d_desc* s, sem2d_solver** out) {
     for (int p = 0; p < NP; ++p) ib[(size_t)k * NP + p] = s->ibool[(size_t)e * NP + p] - 1;
   }
   if ((rc = upload(h, &h->ibool, ib.data(), ib.size()))) return rc;
-  if (h->coef_mode == COEF_SHARED) {
-    if ((rc = upload_bulk(h, &h->coefs, s->coefs, (size_t)h->nelast * NP))) return rc;
-  } else {
-    // per-element arrays follow the colour-sorted element order
-    const size_t per = h->coef_mode == COEF_COMPACT ? (size_t)h->ndof * NP : (size_t)h->nelast * NP;
-    const double* src = h->coef_mode == COEF_COMPACT ? s->lam_mu : s->coefs;
-    std::vector<int> to(s->nelem);
-    for (int k = 0; k < s->nelem; ++k) to[h->elem_order[k]] = k;
-    if ((rc = upload_rows(h, &h->coefs, src, s->nelem, (int)per, to))) return rc;
-    if (h->coef_mode == COEF_COMPACT) {
-      if ((rc = upload_rows(h, &h->geom, s->geom, s->nelem, 3, to))) return rc;
-    }
-  }
+  const size_t per = h->coef_mode == COEF_COMPACT ? (size_t)h->ndof * NP : (size_t)h->nelast * NP;
+  const double* rows = h->coef_mode == COEF_COMPACT ? s->lam_mu : s->coefs;
+  std::vector<int> to(s->nelem);  // per-element arrays follow the colour-sorted element order
+  for (int k = 0; k < s->nelem; ++k) to[h->elem_order[k]] = k;
+  if (h->coef_mode == COEF_SHARED && (rc = upload_bulk(h, &h->coefs, s->coefs, (size_t)h->nelast * NP))) return rc;
   const size_t nf = (size_t)h->ndof * h->npoin;
   if ((rc = upload_bulk(h, &h->rmass, s->rmass, nf))) return rc;
   h->rmass_host.assign(s->rmass, s->rmass + nf);
@@ -1879,14 +1886,12 @@ int sem2d_create(const sem2d_desc* s, sem2d_solver** out) {
     if (h->coef_mode == COEF_SHARED) {
       S.coefs = h->coefs;
     } else {
-      // per-element arrays in cell order (iz*nx + ix)
-      const size_t per = h->coef_mode == COEF_COMPACT ? (size_t)h->ndof * NP : (size_t)h->nelast * NP;
-      const double* src = h->coef_mode == COEF_COMPACT ? s->lam_mu : s->coefs;
-      std::vector<int> to(s->nelem);
-      for (int cell = 0; cell < s->nelem; ++cell) to[S.cell_elem[cell]] = cell;
-      if ((rc = upload_rows(h, &S.coefs, src, s->nelem, (int)per, to))) return rc;
+      // per-element arrays in cell order (iz*nx + ix) as well
+      std::vector<int> tc(s->nelem);
+      for (int cell = 0; cell < s->nelem; ++cell) tc[S.cell_elem[cell]] = cell;
+      if ((rc = upload_rows(h, rows, s->nelem, (int)per, {{&h->coefs, &to}, {&S.coefs, &tc}}))) return rc;
       if (h->coef_mode == COEF_COMPACT) {
-        if ((rc = upload_rows(h, &S.geom, s->geom, s->nelem, 3, to))) return rc;
+        if ((rc = upload_rows(h, s->geom, s->nelem, 3, {{&h->geom, &to}, {&S.geom, &tc}}))) return rc;
         // the moduli once per element, if its points hold bitwise the same values (a medium
         // given by element)
         const int nde = h->ndof;
@@ -1897,7 +1902,7 @@ int sem2d_create(const sem2d_desc* s, sem2d_solver** out) {
           for (int p = 1; p < NP && flat; ++p) flat = std::memcmp(x, x + p, sizeof *x) == 0;
           em[r] = x[0];
         }
-        if (flat && (rc = upload_rows(h, &S.elemmod, em.data(), s->nelem, nde, to))) return rc;
+        if (flat && (rc = upload_rows(h, em.data(), s->nelem, nde, {{&S.elemmod, &tc}}))) return rc;
         // the moduli once per node, if every element at a node holds bitwise the same
         // values there (a medium given as a function of position)
         const int nd = h->ndof;
@@ -1918,6 +1923,10 @@ int sem2d_create(const sem2d_desc* s, sem2d_solver** out) {
         if (same && (rc = upload_bulk(h, &S.nodemod, nm.data(), nm.size()))) return rc;
       }
     }
+  }
+  if (!h->st.on && h->coef_mode != COEF_SHARED) {
+    if ((rc = upload_rows(h, rows, s->nelem, (int)per, {{&h->coefs, &to}}))) return rc;
+    if (h->coef_mode == COEF_COMPACT && (rc = upload_rows(h, s->geom, s->nelem, 3, {{&h->geom, &to}}))) return rc;
   }
   const size_t nfs = (size_t)h->ndof * h->fstride;
   if ((rc = dev_alloc(h, (char**)&h->d, nfs * rsize(h)))) return rc;
