@@ -1,9 +1,10 @@
 // Dynamic fault boundary: pointwise traction solve on split-node pairs.
 // asinh, sinh and cosh follow the C library's decomposition (sem2d_libm.hpp).
 //
-// One lane per fault node pair.  All fault arithmetic is FP64 whatever the bulk
-// type, and floating-point contraction is disabled so that, given the same
-// nodal inputs, every operation rounds as in the reference.
+// One lane per fault node pair.  All fault arithmetic is FP64 whatever the bulk type.  The
+// pragmas below keep the front end from contracting products into sums; the backend, built
+// with -ffp-contract=fast, still does where a product's only use is a sum, so where a bit
+// matters the rounding is written out (fault_solve).
 //   BC_DYNFLT_apply      SRC/bc_dynflt.f90:569-739
 //   slip weakening       SRC/bc_dynflt_swf.f90:142-194
 //   rate and state       SRC/bc_dynflt_rsf.f90:165-568 (two-pass rsf_solver,

@@ -961,7 +961,7 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   for (int k : h->fault_n2) is_fault[k] = 1;
   // Dirichlet components per reference node: those applied by k_deferred (every
   // Dirichlet boundary at a node off the fault; at a fault node only those that act
-  // before the fault) and those k_fault applies after the fault solve
+  // before the fault) and those applied after the fault solve
   std::vector<unsigned char> dmask_def((size_t)h->npoin, 0), dmask_aft((size_t)h->npoin, 0);
   for (const auto& D : h->dirs)
     for (int k : D.node) {
@@ -1055,15 +1055,21 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
     X.fault_dmask[k] = dmask_aft[h->fault_n1[k]];
     if (!h->fault_n2.empty()) X.fault_dmask[k] |= (unsigned char)(dmask_aft[h->fault_n2[k]] << 2);
   }
-  std::vector<int> def_of((size_t)h->npoin, -1);  // reference node -> deferred node
-  for (size_t q = 0; q < ndef; ++q) def_of[def_ref[q]] = S.on ? (int)q : def_ref[q];
+  // places in defs of the fault's and the recorded nodes, by reference node
+  std::unordered_map<int, int> at;
+  for (size_t q = 0; q < ndef; ++q)
+    if (is_rec[def_ref[q]] || is_fault[def_ref[q]]) at[def_ref[q]] = (int)q;
+  auto def_of = [&](int ref) {  // as k_deferred counts them; -1: not deferred
+    const auto f = at.find(ref);
+    return f == at.end() ? -1 : (S.on ? f->second : ref);
+  };
   X.fault_def1.clear();
   X.fault_def2.clear();
   std::unordered_map<int, int> flt_of;  // reference node -> 2 * pair + side
   for (size_t k = 0; k < h->fault_n1.size(); ++k) {
     const int r1 = h->fault_n1[k], r2 = h->fault_n2.empty() ? -1 : h->fault_n2[k];
-    X.fault_def1.push_back(def_of[r1]);
-    X.fault_def2.push_back(r2 < 0 ? -1 : def_of[r2]);
+    X.fault_def1.push_back(def_of(r1));
+    X.fault_def2.push_back(r2 < 0 ? -1 : def_of(r2));
     flt_of[r1] = 2 * (int)k;
     if (r2 >= 0) flt_of[r2] = 2 * (int)k + 1;
   }
@@ -1075,14 +1081,12 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
       const int ref = h->rec_ref[r];
       const auto f = flt_of.find(ref);
       if (f != flt_of.end()) X.rec_flt.push_back({f->second, r});
-      else if (def_of[ref] >= 0) X.rec_def.push_back({def_of[ref], r});
+      else if (def_of(ref) >= 0) X.rec_def.push_back({def_of(ref), r});
       else X.rec_int.push_back({S.gmap[ref], r});
     }
   std::sort(X.rec_int.begin(), X.rec_int.end());
   std::sort(X.rec_def.begin(), X.rec_def.end());
   std::sort(X.rec_flt.begin(), X.rec_flt.end());
-  std::vector<int> at((size_t)h->npoin, -1);  // reference node -> its place in defs
-  for (size_t q = 0; q < ndef; ++q) at[def_ref[q]] = (int)q;
   for (int k = (int)X.rec_def.size() - 1; k >= 0; --k) X.defs[at[h->rec_ref[X.rec_def[k].second]]].rec_at = k;
   for (int k = (int)X.rec_flt.size() - 1; k >= 0; --k) X.defs[at[h->rec_ref[X.rec_flt[k].second]]].rec_at = k;
   X.fault_at.clear();
@@ -1095,7 +1099,7 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   if (S.on) {
     const int ncx = (S.nx + TX - 1) / TX;
     for (int ref : h->rec_ref) {
-      if (def_of[ref] >= 0) continue;
+      if (def_of(ref) >= 0) continue;
       const int Xg = S.gridx[ref] % S.NX1, Zg = S.gridx[ref] / S.NX1;
       const int band = S.ezflt > 0 && Zg > 4 * S.ezflt;
       const int zl = band ? Zg - (4 * S.ezflt + 1) : Zg;
@@ -1113,8 +1117,8 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
     }
   }
   // every split-fault node must be a deferred node: k_deferred leaves those nodes
-  // uncorrected and k_fault finishes both nodes of each pair; a fault node inside a
-  // tile would be corrected by the tile kernel and again by k_fault
+  // uncorrected and the lane of a fault pair finishes both its nodes; a fault node inside a
+  // tile would be corrected by the tile kernel and again there
   {
     size_t nfault_def = 0;
     for (const DefNode& n : X.defs) nfault_def += n.fault ? 1 : 0;
@@ -1895,13 +1899,13 @@ int sem2d_create(const sem2d_desc* s, sem2d_solver** out) {
         // the moduli once per element, if its points hold bitwise the same values (a medium
         // given by element)
         const int nde = h->ndof;
-        std::vector<double> em((size_t)s->nelem * nde);
+        const size_t nrow = (size_t)s->nelem * nde;
         bool flat = true;
-        for (size_t r = 0; r < em.size() && flat; ++r) {
-          const double* x = s->lam_mu + r * NP;
-          for (int p = 1; p < NP && flat; ++p) flat = std::memcmp(x, x + p, sizeof *x) == 0;
-          em[r] = x[0];
-        }
+        for (size_t r = 0; r < nrow && flat; ++r)
+          for (int p = 1; p < NP && flat; ++p)
+            flat = std::memcmp(s->lam_mu + r * NP, s->lam_mu + r * NP + p, sizeof(double)) == 0;
+        std::vector<double> em(flat ? nrow : 0);
+        for (size_t r = 0; r < em.size(); ++r) em[r] = s->lam_mu[r * NP];
         if (flat && (rc = upload_rows(h, em.data(), s->nelem, nde, {{&S.elemmod, &tc}}))) return rc;
         // the moduli once per node, if every element at a node holds bitwise the same
         // values there (a medium given as a function of position)

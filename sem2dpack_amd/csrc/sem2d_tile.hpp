@@ -5,7 +5,8 @@
 // cut into tiles of up to TX x TZ elements; one workgroup owns one tile and, in a
 // single pass over HBM, does for the tile's patch of (4*nxe+1) x (4*nze+1) nodes:
 //
-//   1. load d, v, a; Newmark predictor (SRC/solver.f90:59-60); predicted d in LDS;
+//   1. load d, v, a; Newmark predictor (SRC/solver.f90:59-60), or, between the steps of a
+//      call, the predicted state itself (StepOut); predicted d in LDS;
 //   2. element forces f = -K d (ELAST_KD2_*, SRC/mat_elastic.f90:589-641,739-775),
 //      summed per node in the order of the 2x2 checkerboard colours of the tile's
 //      elements (no atomics, the summation order is fixed);
@@ -16,7 +17,8 @@
 // k_deferred then finishes every perimeter / special node: it sums the partial
 // forces of the tiles that share it (fixed tile order), adds sources and absorbing
 // boundaries (in BC order) and applies the corrector; the nodes of a split fault get
-// there by pairs, with the traction solve in between.
+// there by pairs, with the traction solve in between.  k_run_steps does both for many
+// steps of a small grid in one launch.
 #pragma once
 #include <hip/hip_runtime.h>
 
