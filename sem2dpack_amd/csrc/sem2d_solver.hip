@@ -722,6 +722,22 @@ bool structured_map(sem2d_solver* h, const sem2d_desc* s) {
   return true;
 }
 
+// f(t) for every tile t whose patch holds grid node (X, Z).  The tiles of a split grid are two
+// bands, each cut from its own first element row, the upper one a node row further up.
+template <typename F>
+static void tiles_at(const StructState& S, int X, int Z, F f) {
+  const int W = 4 * TX, ncx = (S.nx + TX - 1) / TX;
+  int t0 = 0;
+  for (int b = 0; b < (S.ezflt > 0 ? 2 : 1); ++b) {
+    const int r0 = b ? S.ezflt : 0, r1 = S.ezflt > 0 && !b ? S.ezflt : S.nz;
+    const int nrow = (r1 - r0 + TZ - 1) / TZ, z = Z - (4 * r0 + b);
+    if (z >= 0 && z <= 4 * (r1 - r0))
+      for (int tz = std::max(z - 1, 0) / (4 * TZ); tz <= z / (4 * TZ) && tz < nrow; ++tz)
+        for (int tx = std::max(X - 1, 0) / W; tx <= X / W && tx < ncx; ++tx) f(t0 + tz * ncx + tx);
+    t0 += nrow * ncx;
+  }
+}
+
 // ngp, fps: field and partial-force component strides; ncoef: entries of the per-cell
 // coefficient array
 static bool fits32(size_t ngp, size_t fps, size_t ncoef, size_t rs) {
@@ -1097,13 +1113,11 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   X.mark_of.assign(S.on ? S.ntiles : 0, -1);
   X.marks.clear();
   if (S.on) {
-    const int ncx = (S.nx + TX - 1) / TX;
     for (int ref : h->rec_ref) {
       if (def_of(ref) >= 0) continue;
       const int Xg = S.gridx[ref] % S.NX1, Zg = S.gridx[ref] / S.NX1;
-      const int band = S.ezflt > 0 && Zg > 4 * S.ezflt;
-      const int zl = band ? Zg - (4 * S.ezflt + 1) : Zg;
-      const int t = (band ? (S.ezflt + TZ - 1) / TZ * ncx : 0) + zl / (4 * TZ) * ncx + Xg / (4 * TX);
+      int t = 0;
+      tiles_at(S, Xg, Zg, [&](int u) { t = u; });  // one: the node is not on a tile edge
       const int4 tg = S.tiles[t];
       const int Xn = Xg - 4 * tg.x, Zn = Zg - tg.w;
       if (Xn <= 0 || Zn <= 0 || Xn >= 4 * (tg.z & 0xff) || Zn >= 4 * ((tg.z >> 8) & 0xff))
@@ -4146,12 +4160,8 @@ int sem2d_adjoint_init(sem2d_solver* h, int nsteps, int seg) {
       if (it != u_at.end()) udef[q] = it->second;
     }
     std::vector<unsigned char> utile(S.ntiles, 0);
-    const int ncx = (S.nx + TX - 1) / TX, ncz = (S.nz + TZ - 1) / TZ;
-    for (int ref : h->rec_ref) {
-      const int Xg = S.gridx[ref] % S.NX1, Zg = S.gridx[ref] / S.NX1, W = 4 * TX;
-      for (int tz = (Zg > 0 ? (Zg - 1) / W : 0); tz <= Zg / W && tz < ncz; ++tz)
-        for (int tx = (Xg > 0 ? (Xg - 1) / W : 0); tx <= Xg / W && tx < ncx; ++tx) utile[(size_t)tz * ncx + tx] = 1;
-    }
+    for (int ref : h->rec_ref)
+      tiles_at(S, S.gridx[ref] % S.NX1, S.gridx[ref] / S.NX1, [&](int t) { utile[t] = 1; });
     if ((rc = adj_alloc(h, &q, udef.size() * sizeof(int)))) return rc;
     A.udef = (int*)q;
     if ((rc = adj_alloc(h, &q, utile.size()))) return rc;
