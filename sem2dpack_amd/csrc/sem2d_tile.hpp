@@ -24,6 +24,7 @@
 
 #include <type_traits>
 
+#include "sem2d_commit.hpp"
 #include "sem2d_fault.hpp"
 #include "sem2d_kernels.hpp"
 
@@ -1323,13 +1324,24 @@ struct RunArgs {
   const int* nbr;       // [ntiles][8] tiles that share a node with a tile, or -1
   const int* slot_def;  // [ntiles][SLOTS] deferred node of a partial force, or -1
   unsigned* flag;       // [ntiles][FLAG_STRIDE] epoch + the steps whose partial forces a tile has stored
-  unsigned* arrived;    // tiles through with the steps; RUN_POISON added: a tile has given up
+  unsigned* arrived;    // the word of run_commit
   unsigned epoch;
   int nsteps, spins;
   int* fail;
 };
 constexpr int FLAG_STRIDE = 16;
-constexpr unsigned RUN_POISON = 1u << 24;
+// run_commit's word, accessed past the L2 caches
+struct RunWord {
+  unsigned* p;
+  __device__ unsigned add(unsigned x) {
+    return __hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ unsigned load() { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+  __device__ bool cas(unsigned& e, unsigned d) {
+    return __hip_atomic_compare_exchange_strong(p, &e, d, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+  }
+};
 
 // nsteps steps of a small grid in one launch, a workgroup per tile, all of them resident
 // together (cooperative launch): a step by its two launches is bound by their start and by
@@ -1347,9 +1359,9 @@ constexpr unsigned RUN_POISON = 1u << 24;
 // agent scope); a tile's stores are waited for before its flag is raised, so no cache is
 // written back or invalidated.
 //
-// A wait ends after `spins` polls.  Nothing of the state is stored before every tile is
-// through (a count at the end), so that a launch that has given up leaves the state it
-// started from, and the steps are then taken by the other kernels.
+// A wait ends after `spins` polls.  Nothing of the state is stored before the tiles have
+// agreed that every one is through (run_commit), so that a launch that has given up leaves
+// the state it started from, and the steps are then taken by the other kernels.
 template <typename R, int NDOF, int NELAST, int MODE>
 __global__ __launch_bounds__(TS_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_run_steps(RunArgs<R> A) {
   constexpr int PS = PXM, NEL = TX * TZ;
@@ -1570,20 +1582,10 @@ __global__ __launch_bounds__(TS_NT) __attribute__((amdgpu_waves_per_eu(2))) void
     __syncthreads();
   }
 
-  // the state is stored when every tile is through; a tile that gives up (or has waited too
-  // long here) takes the count past the number that the others wait for
+  // the state is stored when every tile is through
   if (tid == 0) {
-    const unsigned want = gridDim.x;
-    bool ok = !stop;
-    if (ok) {
-      unsigned at = __hip_atomic_fetch_add(A.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-      for (int left = A.spins; at < want && left > 0; --left)
-        at = __hip_atomic_load(A.arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (at < want) at = __hip_atomic_fetch_add(A.arrived, RUN_POISON, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      ok = at == want;
-    } else {
-      __hip_atomic_fetch_add(A.arrived, RUN_POISON, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    RunWord word{A.arrived};
+    const bool ok = run_commit(word, !stop, gridDim.x, A.spins);
     if (!ok) *A.fail = 1;
     stop = !ok;
   }
