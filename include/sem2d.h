@@ -313,6 +313,12 @@ int sem2d_field_info(sem2d_solver *h, double *vmax, double *dmax, int *nonfinite
    on either (same summation order). */
 int sem2d_set_tile_config(sem2d_solver *h, int threads, int wg_per_cu);
 
+/* Launches that took many steps at once (small structured grids; no counterpart in the
+   reference): those whose steps were kept, and those that gave up waiting for a part of the
+   grid and left the state alone, their steps being taken one by one.  Results do not depend
+   on which. */
+int sem2d_run_counts(sem2d_solver *h, int *taken, int *given_up);
+
 /* Current step index (number of steps taken). */
 int sem2d_get_step(sem2d_solver *h, int *it);
 

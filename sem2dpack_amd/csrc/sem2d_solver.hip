@@ -107,12 +107,13 @@ struct StructState {
   void* elemmod = nullptr;
   // k_run_steps: neighbours of the tiles, deferred node of each partial force, the second
   // array of partial forces, flags and count, whether a launch has given up; run_ok: 0 not
-  // asked yet, 1 the grid's tiles are resident together, -1 not so or not a run's grid
+  // asked yet, 1 the grid's tiles are resident together, -1 not so or not a run's grid;
+  // launches kept and given up so far
   int *nbr = nullptr, *slot_def = nullptr, *run_fail = nullptr;
   unsigned *run_flag = nullptr, *run_count = nullptr;
   void* fpart2 = nullptr;
   unsigned epoch = 0;
-  int run_ok = -1;
+  int run_ok = -1, runs_taken = 0, runs_given_up = 0;
   std::vector<void*> prep_allocs;  // freed when the deferred tables are rebuilt
   std::vector<int> cell_elem;      // cell (iz*nx + ix) -> element (0-based)
   std::vector<int> def_ref;        // deferred node -> reference node (0-based)
@@ -1652,6 +1653,7 @@ int launch_run_k(sem2d_solver* h, const StepDev& X, int n, const StepCoefs<R>& K
   HIPCHK(h, hipMemcpyAsync(&fail, S.run_fail, sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   if (fail) S.run_ok = -1;  // the device is shared with something that keeps tiles waiting
+  ++(fail ? S.runs_given_up : S.runs_taken);
   *done = !fail;
   return 0;
 }
@@ -2786,6 +2788,13 @@ int sem2d_set_tile_config(sem2d_solver* h, int threads, int wg_per_cu) {
   if (wg_per_cu < 0) wg_per_cu = tile_wgs_per_cu(h->fp32, h->ndof);  // automatic: the measured defaults
   S.pipe_wgs = ncu * wg_per_cu;
   S.pipe_wgs = ((S.pipe_wgs + 7) / 8) * 8;
+  return 0;
+}
+
+int sem2d_run_counts(sem2d_solver* h, int* taken, int* given_up) {
+  if (!h) return 1;
+  if (taken) *taken = h->st.runs_taken;
+  if (given_up) *given_up = h->st.runs_given_up;
   return 0;
 }
 

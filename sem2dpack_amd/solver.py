@@ -348,6 +348,14 @@ class Solver:
         """Tile-kernel launch configuration (structured grids); results do not depend on it."""
         self._check(self.api.set_tile_config(self.h, int(threads), int(wg_per_cu)), "set_tile_config")
 
+    def run_counts(self):
+        """(taken, given_up): launches that took many steps at once (small structured grids)
+        and those that gave up, their steps being taken one by one; results do not depend on
+        which."""
+        t, g = C.c_int(), C.c_int()
+        self._check(self.api.run_counts(self.h, C.byref(t), C.byref(g)), "run_counts")
+        return t.value, g.value
+
     def close(self):
         if getattr(self, "h", None):
             self.api.destroy(self.h)

@@ -1,0 +1,44 @@
+"""Which calls are taken as a run of steps in one launch: those of 17 steps or more on a grid
+whose tiles are resident together."""
+import pytest
+
+from conftest import case_par
+from sem2dpack_amd import builder, solver
+from test_gpu_run_steps import NT, problem
+
+pytestmark = pytest.mark.gpu
+
+
+def counts(pb, steps=(NT,), **kw):
+    s = solver.Solver(pb, **kw)
+    for n in steps:
+        s.step(n)
+    return s.run_counts()
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("nx,nz,ndof,medium", [(1, 1, 2, "uniform"), (24, 16, 2, "points"), (33, 25, 1, "elements"),
+                                               (128, 128, 2, "nodes"), (121, 121, 1, "nodes")])
+def test_runs_are_taken(nx, nz, ndof, medium, fp32):
+    assert counts(problem(nx, nz, ndof, medium), bulk_fp32=fp32) == (1, 0)
+
+
+def test_no_runs_in_short_calls_and_beside_a_fault():
+    assert counts(problem(24, 16, 2, "uniform"), [16] * 3) == (0, 0)
+    assert counts(problem(24, 16, 2, "uniform"), structured=False) == (0, 0)
+    assert counts(builder.build(case_par("sh_swf"), nsteps=NT)) == (0, 0)
+
+
+def test_progress_rows_cut_runs():
+    assert counts(problem(24, 16, 2, "uniform"), itinfo=20) == (2, 0)
+
+
+def test_a_run_that_gives_up_is_not_tried_again(monkeypatch):
+    """waits of no poll at all: of several tiles the first one through finds the others missing"""
+    monkeypatch.setenv("SEM2D_RUN_SPINS", "0")
+    s = solver.Solver(problem(64, 64, 2, "uniform"))
+    s.step(NT)
+    assert s.run_counts() == (0, 1)
+    monkeypatch.delenv("SEM2D_RUN_SPINS")
+    s.step(NT)
+    assert s.run_counts() == (0, 1)
