@@ -1161,10 +1161,13 @@ void fault_waves(const FaultHost& F, int m, int k0, int o0, std::vector<int4>& w
   for (int o = 0; o < F.nout; ++o) slot[s0 + F.oix1 - 1 + (size_t)o * F.oixd] = o0 + o;
 }
 
-// Tiles a grid may have for its tiles to be asked whether they are resident together
-// (k_run_steps): one or two workgroups on each of the 256 compute units.  In larger grids a
-// workgroup has more than one tile, and two launches a step are no longer most of its time.
-constexpr int RUN_MAX_TILES = 512;
+// Tiles a grid may have for a run of steps in one launch (k_run_steps): as many as there are
+// compute units, one workgroup each.  A second one is not sure of a place on any of them: a
+// workgroup of six wavefronts takes up to two places on each SIMD, and at the 134 to 254
+// registers of the kernels a SIMD has two or three.  (The occupancy query says two workgroups
+// for those of SH grids, but they were not resident together: 200 x 150 elements, 475 tiles,
+// waited 443 ms to give up where two launches a step take 4.4 ms for 40 steps.)
+constexpr int RUN_MAX_TILES = 256;
 
 // Tables of k_run_steps for a grid without faults, element-point terms, Stacey terms,
 // receivers inside elements and boundaries that are not flat (other grids: nbr stays null)
@@ -1605,11 +1608,12 @@ __global__ void k_periodic(int n, const int* __restrict__ m, const int* __restri
   }
 }
 
-// Polls of one wait of k_run_steps before it gives up (0.5 us or more each); SEM2D_RUN_SPINS
-// sets it, 0 makes a launch give up where a neighbour is not there yet.
+// Polls of one wait of k_run_steps before it gives up (0.4 us or more each, 55 ms in all;
+// a neighbour that is running is there within microseconds); SEM2D_RUN_SPINS sets it, 0 makes
+// a launch give up where a neighbour is not there yet.
 int run_spins() {
   const char* env = getenv("SEM2D_RUN_SPINS");
-  return env ? std::max(0, atoi(env)) : 1 << 20;
+  return env ? std::max(0, atoi(env)) : 1 << 17;
 }
 
 // Steps from which a run of them is one launch of k_run_steps: the launch, its start and
@@ -1629,7 +1633,7 @@ int launch_run_k(sem2d_solver* h, const StepDev& X, int n, const StepCoefs<R>& K
     HIPCHK(h, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     HIPCHK(h, hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
     HIPCHK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, TS_NT, 0));
-    S.run_ok = coop && S.ntiles <= ncu * per ? 1 : -1;
+    S.run_ok = coop && per > 0 && S.ntiles <= ncu ? 1 : -1;
     if (S.run_ok < 0) return 0;
   }
   HIPCHK(h, hipMemsetAsync(S.run_count, 0, sizeof(unsigned), h->stream));

@@ -1,5 +1,6 @@
 """Which calls are taken as a run of steps in one launch: those of 17 steps or more on a grid
-whose tiles are resident together."""
+of at most one tile per compute unit.  A run of a larger grid is not tried: its tiles would
+wait for others that are not running until they give up."""
 import pytest
 
 from conftest import case_par
@@ -21,6 +22,17 @@ def counts(pb, steps=(NT,), **kw):
                                                (128, 128, 2, "nodes"), (121, 121, 1, "nodes")])
 def test_runs_are_taken(nx, nz, ndof, medium, fp32):
     assert counts(problem(nx, nz, ndof, medium), bulk_fp32=fp32) == (1, 0)
+
+
+# one tile more than the 256 compute units (a row of them), and the most that two
+# workgroups on each could hold
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("nx,nz,ndof,medium", [(8, 8 * 257, 1, "uniform"), (129, 128, 2, "uniform"),
+                                               (200, 150, 1, "nodes"), (170, 178, 1, "points"),
+                                               (170, 178, 1, "elements")])
+def test_no_runs_of_more_tiles_than_are_resident(nx, nz, ndof, medium, fp32):
+    print(f"\n[no runs {nx}x{nz} ndof={ndof} {medium} fp32={fp32}]", flush=True)
+    assert counts(problem(nx, nz, ndof, medium), bulk_fp32=fp32) == (0, 0)
 
 
 def test_no_runs_in_short_calls_and_beside_a_fault():
