@@ -60,7 +60,8 @@ struct AbsoHost {
 
 // Structured-mesh fast path (node-grid field order, fused tile kernel)
 struct StructState {
-  bool on = false, ready = false;
+  bool on = false;
+  int ready = 0;  // 1: the tables of the step kernels are there; -1: the general path has none
   int nx = 0, nz = 0, ezflt = 0, NX1 = 0, NZ1 = 0;
   int ROW = 0;                    // storage slots per node row (4*TX per tile column)
   std::vector<int> gmap;          // reference node (0-based) -> storage index
@@ -1350,8 +1351,19 @@ int prepare_structured(sem2d_solver* h) {
   }
   HIPCHK(h, hipStreamSynchronize(h->stream));
   if ((rc = run_tables(h, X))) return rc;
-  S.ready = true;
+  S.ready = 1;
   return 0;
+}
+
+// The general path goes without tables until what they are made from changes.
+void drop_tables(sem2d_solver* h) {
+  StructState& S = h->st;
+  hipStreamSynchronize(h->stream);
+  for (void* q : S.prep_allocs) hipFree(q);
+  S.prep_allocs.clear();
+  (void)hipGetLastError();
+  h->err.clear();
+  S.ready = -1;
 }
 
 // Everything one structured step launches on: the device tables of one grid (a
@@ -1691,15 +1703,21 @@ int do_steps(sem2d_solver* h, int nsteps) {
   // coefficients, 32 steps 2.2 ms against 1.7 by single launches, 64 steps 3.1 against 3.4,
   // 1000 steps 30 against 52; 800 elements NGLL 9, 64 steps 1.1 against 1.8 ms, 1000 steps 12
   // against 37.  Periodic boundaries, HHT-alpha, linear slip faults and incident waves keep
-  // the single launches.
-  bool tables = h->st.on || (!h->hht && !h->nper && !h->nlsf && (h->st.ready || nsteps >= 64));
+  // the single launches, and so does what the tables cannot hold.
+  bool tables = h->st.on || (!h->hht && !h->nper && !h->nlsf && (h->st.ready > 0 || (h->st.ready == 0 && nsteps >= 64)));
   for (auto& b : h->abso) tables = tables && !b.wxz;
   if (tables && !h->st.on && !h->st.ready) {  // room for the element forces and the node records
     const size_t pts = (size_t)h->nelem * h->np, need = pts * (h->ndof * rsize(h) + 8) + (size_t)h->npoin * 24;
     size_t fr = 0, tot = 0;
     tables = pts <= (size_t)65536 * 256 && hipMemGetInfo(&fr, &tot) == hipSuccess && need + need / 4 < fr;
   }
-  if (tables && !h->st.ready && (rc = prepare_structured(h))) return rc;
+  if (tables && !h->st.ready && (rc = prepare_structured(h))) {
+    if (h->st.on) return rc;
+    // the general path: more entries at a node than a record counts, a fault whose pairs
+    // share nodes, no memory left; the launches one by one need no tables
+    drop_tables(h);
+    tables = false;
+  }
   if (h->flt.on && (rc = potency_reserve(h, h->flt.pot_rows + nsteps))) return rc;
   if (h->itinfo > 0 && (rc = info_reserve(h, h->info_rows + (h->it + nsteps) / h->itinfo - h->it / h->itinfo)))
     return rc;
@@ -1987,7 +2005,7 @@ int sem2d_set_abso(sem2d_solver* h, int n, const int* node, const double* C) {
   ah.node = nd;
   ah.C.assign(C, C + (size_t)h->ndof * n);
   h->abso_host.push_back(ah);
-  h->st.ready = false;
+  h->st.ready = 0;
   return 0;
 }
 
@@ -2000,7 +2018,7 @@ int sem2d_set_abso_normals(sem2d_solver* h, int n, const double* nrm) {
   AbsoDev& ad = h->abso.back();
   if (!nrm || n != ad.n) return set_err(h, 3, "set_abso_normals: size differs from the boundary's");
   h->abso_host.back().nrm.assign(nrm, nrm + (size_t)2 * n);
-  h->st.ready = false;
+  h->st.ready = 0;
   return upload(h, &ad.nrm, nrm, (size_t)2 * n);
 }
 
@@ -2033,7 +2051,7 @@ int sem2d_set_abso_stacey(sem2d_solver* h, int nbe, const int* enode, const doub
   if ((rc = upload(h, &ad.soff, off.data(), off.size()))) return rc;
   if ((rc = upload(h, &ad.sidx, idx.data(), idx.size()))) return rc;
   ad.nbe = nbe;
-  h->st.ready = false;
+  h->st.ready = 0;
   return 0;
 }
 
@@ -2081,7 +2099,7 @@ int sem2d_set_force(sem2d_solver* h, int iglob, const double* dir, int* isrc) {
   }
   h->stf.emplace_back();
   h->src_dirty = true;
-  h->st.ready = false;
+  h->st.ready = 0;
   if (isrc) *isrc = s;
   return 0;
 }
@@ -2109,7 +2127,7 @@ int sem2d_set_moment(sem2d_solver* h, int nel, const int* ixi, const int* ieta, 
   }
   h->stf.emplace_back();
   h->src_dirty = true;
-  h->st.ready = false;
+  h->st.ready = 0;
   if (isrc) *isrc = s;
   return 0;
 }
@@ -2137,7 +2155,7 @@ int sem2d_set_receivers(sem2d_solver* h, int nrec, const int* iglob, int isamp, 
   if (rc) return rc;
   h->rec_w = nullptr;
   h->rec_ref = std::move(ref);
-  h->st.ready = false;  // the tables mark the recorded nodes
+  h->st.ready = 0;  // the tables mark the recorded nodes
   if ((rc = dev_alloc(h, &h->seis, (size_t)nsamp * h->ndof * nrec))) return rc;
   h->nrec = nrec;
   h->isamp = isamp;
@@ -2153,7 +2171,7 @@ int sem2d_set_receivers(sem2d_solver* h, int nrec, const int* iglob, int isamp, 
 // the fused tile kernels have neither the viscous nor the 2.5D term: a structured grid
 // with either uses the general element path, with the fields in the reference numbering
 static int use_general_path(sem2d_solver* h) {
-  h->st.ready = false;
+  h->st.ready = 0;
   if (h->st.on) {
     h->st.on = false;
     h->fstride = (size_t)h->npoin;
@@ -2187,7 +2205,7 @@ static int upload_cell_points(sem2d_solver* h, void** dst, const double* src) {
   int dev = 0, ncu = 256;
   if (hipGetDevice(&dev) == hipSuccess) hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   S.pipe_wgs = ((ncu + 7) / 8) * 8;
-  S.ready = false;
+  S.ready = 0;
   return 0;
 }
 
@@ -2258,7 +2276,7 @@ int sem2d_set_receivers_interp(sem2d_solver* h, int nrec, const int* elem, const
     }
   }
   h->rec_ref = std::move(ref);
-  h->st.ready = false;  // the tables mark the recorded nodes
+  h->st.ready = 0;  // the tables mark the recorded nodes
   int rc = upload(h, &h->rec_node, nd.data(), nd.size());
   if (rc) return rc;
   if ((rc = upload(h, &h->rec_w, interp, (size_t)nrec * NP))) return rc;
@@ -2304,7 +2322,7 @@ int sem2d_set_fault(sem2d_solver* h, const sem2d_fault_desc* f, int nsamp) {
   h->fault_n1 = n1;
   if (two) h->fault_n2 = n2;
   else h->fault_n2.clear();
-  h->st.ready = false;
+  h->st.ready = 0;
   if (h->st.on)
     for (int k = 0; k < np; ++k) {
       n1[k] = h->st.gmap[n1[k]];
@@ -2727,7 +2745,7 @@ int sem2d_set_dirichlet(sem2d_solver* h, int n, const int* node, int comp) {
   int rc = upload(h, &D.node_dev, dn.data(), dn.size());
   if (rc) return rc;
   h->dirs.push_back(std::move(D));
-  h->st.ready = false;
+  h->st.ready = 0;
   return 0;
 }
 
