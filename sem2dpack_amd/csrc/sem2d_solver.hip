@@ -42,6 +42,7 @@ struct AbsoDev {
   // [nbe][NG][2]; per boundary node the contributions e*NG+k (element order) soff/sidx
   int nbe = 0;
   int *enode = nullptr, *soff = nullptr, *sidx = nullptr;
+  bool ends = false;  // the end nodes take both ends' contributions (sem2d_set_abso_periodic)
   double* K = nullptr;
   double* nrm = nullptr;  // [2][n] node normals of a boundary that is not flat (general path)
   // incident plane wave (general path): node coordinates [2][n], unit-amplitude Vin and
@@ -1702,10 +1703,10 @@ int do_steps(sem2d_solver* h, int nsteps) {
   // or the call is long enough to pay for them: 24,120 elements NGLL 5 with ten
   // coefficients, 32 steps 2.2 ms against 1.7 by single launches, 64 steps 3.1 against 3.4,
   // 1000 steps 30 against 52; 800 elements NGLL 9, 64 steps 1.1 against 1.8 ms, 1000 steps 12
-  // against 37.  Periodic boundaries, HHT-alpha, linear slip faults and incident waves keep
-  // the single launches, and so does what the tables cannot hold.
+  // against 37.  Periodic boundaries, HHT-alpha, linear slip faults, incident waves and
+  // Stacey terms joined at the ends keep the single launches, and so does what the tables cannot hold.
   bool tables = h->st.on || (!h->hht && !h->nper && !h->nlsf && (h->st.ready > 0 || (h->st.ready == 0 && nsteps >= 64)));
-  for (auto& b : h->abso) tables = tables && !b.wxz;
+  for (auto& b : h->abso) tables = tables && !b.wxz && !b.ends;
   if (tables && !h->st.on && !h->st.ready) {  // room for the element forces and the node records
     const size_t pts = (size_t)h->nelem * h->np, need = pts * (h->ndof * rsize(h) + 8) + (size_t)h->npoin * 24;
     size_t fr = 0, tot = 0;
@@ -2083,6 +2084,7 @@ int sem2d_set_abso_periodic(sem2d_solver* h) {
   }
   if ((rc = upload(h, &ad.soff, off.data(), off.size()))) return rc;
   if ((rc = upload(h, &ad.sidx, idx.data(), idx.size()))) return rc;
+  ad.ends = true;
   return 0;
 }
 

@@ -65,3 +65,19 @@ def test_sources_added_between_calls(fp32):
     assert src["kind"] == "force"
     for x, y, nm in zip(run(NT), run(NT // 2), "dva"):
         assert np.array_equal(x, y), nm
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+def test_stacey_ends_of_a_periodic_boundary_without_its_pairs(fp32):
+    """sem2d_set_abso_periodic after a Stacey boundary, without sem2d_set_periodic"""
+    pb = builder.build(case_par("psv_stacey"), nsteps=2 * NT)
+    rng = np.random.default_rng(7)
+    for ab in pb.abso:
+        if ab.get("stacey") is not None:
+            ab["periodic_ends"] = True
+    # forces at the ends of the boundaries, where the terms differ
+    src = pb.sources[0]
+    pb.sources = [dict(src, kind="force", iglob=int(g), dir=rng.standard_normal(2),
+                       stf_table=rng.standard_normal(2 * NT))
+                  for ab in pb.abso for g in (ab["node"][0], ab["node"][-1])]
+    same(pb, bulk_fp32=fp32)
