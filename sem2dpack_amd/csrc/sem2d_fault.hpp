@@ -107,9 +107,10 @@ __device__ __forceinline__ PairData pair_load(const FaultDev& F, int k, bool two
   return P;
 }
 
-// the pair's state after the step
+// the pair's state after the step, and what its tractions add to the force of node 1 and take
+// from that of node 2
 struct PairOut {
-  double D0, V0, T[2], Ts0, mu;
+  double D0, V0, T[2], Ts0, mu, bt[2];
 };
 
 #pragma clang fp contract(off)
@@ -353,6 +354,7 @@ __device__ inline PairOut fault_solve(const FaultDev& F, const PairData& P, int 
     Tx[0] = nz * T[0] + nx * T[1];
     Tx[1] = -nx * T[0] + nz * T[1];
   }
+  PairOut out;
 #pragma unroll
   for (int c = 0; c < nd; ++c) {
     // one rounding at node 1, two at node 2, however the compiler arranges the code around:
@@ -361,6 +363,7 @@ __device__ inline PairOut fault_solve(const FaultDev& F, const PairData& P, int 
     asm volatile("" : "+v"(bt));
     n1.f[c] = (R)__builtin_fma(P.B[c], Tx[c], (double)n1.f[c]);
     if (two) n2.f[c] = (R)((double)n2.f[c] - bt);
+    out.bt[c] = bt;
   }
   F.sigma[k] = sigma;
   if (F.law != 3) F.theta[k] = th;
@@ -369,7 +372,6 @@ __device__ inline PairOut fault_solve(const FaultDev& F, const PairData& P, int 
   F.T[np + k] = T[1];
   F.Tstick[k] = Ts[0];
   F.Tstick[np + k] = Ts[1];
-  PairOut out;
   out.T[0] = T[0], out.T[1] = T[1], out.Ts0 = Ts[0], out.mu = mu;
 #pragma unroll
   for (int c = 0; c < nd; ++c) {
@@ -404,12 +406,13 @@ __global__ __launch_bounds__(64) void k_fault(FaultDev F, const R* d, const R* v
       n2.f[c] = f[o + i2];
     }
   }
-  fault_solve<R, nd>(F, pair_load<nd>(F, k, i2 >= 0), k, time, i2 >= 0, n1, n2);
+  const PairOut po = fault_solve<R, nd>(F, pair_load<nd>(F, k, i2 >= 0), k, time, i2 >= 0, n1, n2);
 #pragma unroll
   for (int c = 0; c < nd; ++c) {
     const size_t o = (size_t)c * npoin;
     f[o + i1] = n1.f[c];
-    if (i2 >= 0) f[o + i2] = n2.f[c];
+    // a pair whose two sides are one node: both act on it
+    if (i2 >= 0) f[o + i2] = i2 == i1 ? (R)((double)n1.f[c] - po.bt[c]) : n2.f[c];
   }
 }
 

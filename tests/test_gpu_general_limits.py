@@ -81,3 +81,30 @@ def test_stacey_ends_of_a_periodic_boundary_without_its_pairs(fp32):
                        stf_table=rng.standard_normal(2 * NT))
                   for ab in pb.abso for g in (ab["node"][0], ab["node"][-1])]
     same(pb, bulk_fp32=fp32)
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("case", ["sh_swf", "psv_rsf"])
+def test_a_fault_pair_of_one_node(case, fp32):
+    """Both sides of the last pair are the same node: its tractions cancel there, so the
+    fields are those without the pair (up to the roundings of adding and subtracting it:
+    one of the bulk type's a step, of a force no larger than the others)."""
+    pb = builder.build(case_par(case), nsteps=2 * NT)
+    without = solver.Solver(pb, structured=False)
+    f = pb.fault
+    lone = int(np.setdiff1d(np.arange(1, pb.npoin + 1), np.r_[f["node1"], f["node2"]])[pb.npoin // 3])
+    f = pb.fault = dict(f)
+    for k in ("node1", "node2"):
+        f[k] = np.r_[f[k], np.int32(lone)].astype(np.int32)
+    n = len(f["node1"])
+    for k, x in list(f.items()):
+        if isinstance(x, np.ndarray) and x.ndim and len(x) == n - 1:
+            f[k] = np.concatenate([x, x[n // 2:n // 2 + 1]])
+    f["invM2"][-1] = f["invM1"][-1]
+    one = same(pb, bulk_fp32=fp32)
+    assert np.any(one.fault_state()["T"][:, -1] != 0)  # it does slip
+    if not fp32:
+        without.step(NT)
+        without.step(3)
+        for x, y, nm in zip(one.fields(), without.fields(), "dva"):
+            assert np.linalg.norm(x - y) < 1e-9 * np.linalg.norm(y), nm
