@@ -295,6 +295,9 @@ __device__ inline PairOut fault_solve(const FaultDev& F, const PairData& P, int 
       dA[c] = -2.0 * P.iM1[c] * (double)n1.f[c];
     }
     T[c] = P.Z[c] * (dV[c] + F.a2v * dA[c]);
+    // rounded here: without the rotation (SH) the product would be fused with the addition of
+    // the initial stress
+    if (nd == 1) asm volatile("" : "+v"(T[c]));
   }
   const double nx = P.nx, nz = P.nz;
   if (nd == 2) {
