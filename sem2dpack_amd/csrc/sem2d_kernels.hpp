@@ -113,18 +113,18 @@ __device__ __forceinline__ void load_coefs(const R* __restrict__ coefs, const R*
 // the predicted fields (StepOut); otherwise they are formed here from d, v and a.
 template <typename R>
 struct ElemStep {
-  R* fe = nullptr;  // null: assembly into f (one colour)
+  R* fe = nullptr;
   size_t stride = 0;
   const R* a = nullptr;
   R dt = 0, c1 = 0, c2 = 0;
   int pin = 1;
 };
 
-// Element forces of one colour, or of all elements (E.fe).  With Kelvin-Voigt elements (kv != nullptr, [element
+// Element forces of one colour, assembled into f, or (STEP) of all elements.  With Kelvin-Voigt elements (kv != nullptr, [element
 // in colour order][NGLL^2]) the element displacement is d + eta v (MAT_KV_add_etav,
 // SRC/mat_kelvin_voigt.f90:139-150, applied by MAT_Fint, SRC/mat_gen.f90:435).  NGL is
 // NGLL; for NGL != 5, hg holds h'_i(x_j) at hg[i*NGL+j] (for NGL = 5 it is c_H).
-template <typename R, int NDOF, int NELAST, int MODE, int NGL = NG>
+template <typename R, int NDOF, int NELAST, int MODE, int NGL = NG, bool STEP = false>
 __global__ __launch_bounds__(256) void k_force_colour(int e0, int ne, const int* __restrict__ ibool,
                                                       const R* __restrict__ coefs, const R* __restrict__ geom,
                                                       const R* __restrict__ d, R* __restrict__ f,
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void k_force_colour(int e0, int ne, const int*
   int node = 0;
   if (active) {
     node = ibool[(size_t)e * NPL + p];
-    if (!E.pin) {
+    if (STEP && !E.pin) {
       const R eta = kv ? kv[(size_t)e * NPL + p] : R(0);
 #pragma unroll
       for (int c = 0; c < NDOF; ++c) {
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void k_force_colour(int e0, int ne, const int*
       R fe = s1 + s2;
       if (beta25)  // 2.5D: MAT_ELAST_add_25D_f (SRC/mat_elastic.f90:447-459)
         fe = (s1 + s2) - beta25[(size_t)e * NPL + p] * U[le][c][p];
-      if (E.fe) {
+      if constexpr (STEP) {
         E.fe[(size_t)c * E.stride + (size_t)e * NPL + p] = fe;
       } else {
         R* fp = f + (size_t)c * npoin + node;

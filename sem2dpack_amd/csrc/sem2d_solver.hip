@@ -433,7 +433,7 @@ void launch_force_t(sem2d_solver* h, const R* d, R* f, const R* v, const ElemSte
   const R* kv = v ? (const R*)h->kv_eta : nullptr;
   constexpr int EPB = fe_epb(NGL);
   if (E.fe) {
-    k_force_colour<R, NDOF, NELAST, MODE, NGL><<<(h->nelem + EPB - 1) / EPB, 256, 0, h->stream>>>(
+    k_force_colour<R, NDOF, NELAST, MODE, NGL, true><<<(h->nelem + EPB - 1) / EPB, 256, 0, h->stream>>>(
         0, h->nelem, h->ibool, (const R*)h->coefs, (const R*)h->geom, d, f, h->npoin, v, kv, (const R*)h->beta25,
         h->hg, E);
     return;
