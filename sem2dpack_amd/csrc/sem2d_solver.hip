@@ -802,6 +802,7 @@ struct StructTables {
   std::vector<int4> tiles, grids;
   std::vector<int> spec_cnt, spec_idx;
   std::vector<DefNode> defs;
+  std::vector<int> def_ref;      // their reference nodes (0-based)
   std::vector<int> part_off;
   std::vector<SrcEntry> dsrc;
   std::vector<double> dabso, dabson;
@@ -1029,7 +1030,8 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   bool skew = false;
   for (const AbsoHost& B : h->abso_host) skew |= !B.nrm.empty();
   X.part_off = std::move(P.off);
-  std::vector<int> def_ref(P.g.size());
+  std::vector<int>& def_ref = X.def_ref;
+  def_ref.resize(P.g.size());
   X.defs.reserve(P.g.size());
   for (size_t i = 0; i < P.g.size(); ++i) {
     DefNode n{};
@@ -1224,10 +1226,7 @@ int prepare_structured(sem2d_solver* h) {
   if (rc) return rc;
   S.ndef = S.on ? (int)X.defs.size() : h->npoin;
   if (S.on) {
-    S.def_ref.resize(S.ndef);
-    std::vector<int> ginv(S.NS, -1);  // storage index -> reference node (inverse of gmap)
-    for (int k = 0; k < h->npoin; ++k) ginv[S.gmap[k]] = k;
-    for (int q = 0; q < S.ndef; ++q) S.def_ref[q] = ginv[X.defs[q].g];
+    S.def_ref = X.def_ref;
     if ((rc = prep_upload(h, &S.tiles_dev, X.tiles.data(), X.tiles.size()))) return rc;
     if ((rc = prep_upload(h, &S.grids_dev, X.grids.data(), X.grids.size()))) return rc;
     if ((rc = prep_upload(h, &S.spec_cnt, X.spec_cnt.data(), X.spec_cnt.size()))) return rc;
