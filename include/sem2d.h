@@ -308,9 +308,9 @@ int sem2d_field_info(sem2d_solver *h, double *vmax, double *dmax, int *nonfinite
 
 /* Launch configuration of the structured-grid tile kernel (no counterpart in the
    reference, whose loop is serial): persistent workgroups per CU (0: one workgroup per
-   tile; < 0: automatic, 2, or 4 for SH with FP32 fields).  threads is 256 or 512 and is
-   kept for sem2d_batch_config: the kernel has one workgroup shape.  Results do not depend
-   on either (same summation order). */
+   tile; < 0: automatic, 2, or 4 for SH with FP32 fields).  threads must be 256 or 512
+   and has no effect: the kernel has one workgroup shape.  Results do not depend on either
+   (same summation order). */
 int sem2d_set_tile_config(sem2d_solver *h, int threads, int wg_per_cu);
 
 /* Launches that took many steps at once (small structured grids; no counterpart in the
@@ -392,15 +392,16 @@ int sem2d_batch_create(int n, sem2d_solver *const *members, sem2d_batch **out);
 int sem2d_batch_step(sem2d_batch *b, int nsteps);
 
 /* Autotuner: time trial_steps steps of each tile-kernel launch configuration
-   (persistent workgroups per CU, or one workgroup per tile), keep the fastest and restore the state.  *choice receives
-   the index of the chosen configuration. */
+   (persistent workgroups per CU, or one workgroup per tile), keep the fastest and restore
+   the state.  *choice receives the index of the chosen configuration. */
 int sem2d_batch_tune(sem2d_batch *b, int trial_steps, int *choice);
 
 /* Set the tile-kernel launch configuration explicitly (as sem2d_set_tile_config;
    0 <= wg_per_cu <= 4). */
 int sem2d_batch_set_config(sem2d_batch *b, int threads, int wg_per_cu);
 
-/* Current tile-kernel launch configuration and total tile count. */
+/* Current tile-kernel launch configuration (threads: those of a workgroup as launched) and
+   total tile count. */
 int sem2d_batch_config(sem2d_batch *b, int *threads, int *workgroups, int *ntiles);
 
 /* Per-member outputs, in the layouts of the single-scenario fetches. */

@@ -1152,7 +1152,6 @@ int struct_tables(sem2d_solver* h, StructTables& X) {
   return 0;
 }
 
-// Upload the structured tables of the solver's own grid.
 // Wavefronts of a fault's pairs (FaultOut): those of member m, whose pairs start at k0 and
 // whose record places start at o0
 void fault_waves(const FaultHost& F, int m, int k0, int o0, std::vector<int4>& wave, std::vector<int2>& member,
@@ -1216,6 +1215,7 @@ int run_tables(sem2d_solver* h, const StructTables& X) {
   return 0;
 }
 
+// Makes the tables of the step kernels and uploads them.
 int prepare_structured(sem2d_solver* h) {
   StructState& S = h->st;
   HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -2907,7 +2907,6 @@ struct sem2d_batch {
   std::vector<int> fault_base, rec_base, fout_base, src_base;
   StepDev X;
   int ncu = 256;
-  int threads = 512;  // as set by sem2d_batch_set_config (one kernel shape serves both values)
   // records
   int nrec = 0, isamp = 1, field = 1, nsamp = 0;
   int* rec_node = nullptr;
@@ -3179,10 +3178,8 @@ int batch_graph(sem2d_batch* b, int chunk) {
   return 0;
 }
 
-// launch configuration of the tile kernel: threads per workgroup (256: 10-element
-// batches, 512: 20-element batches) and workgroups per CU (0: one workgroup per tile)
-void batch_set_config(sem2d_batch* b, int threads, int per_cu) {
-  b->threads = threads;
+// launch configuration of the tile kernel: workgroups per CU (0: one workgroup per tile)
+void batch_set_config(sem2d_batch* b, int per_cu) {
   b->X.pipe_wgs = per_cu > 0 ? ((b->ncu * per_cu + 7) / 8) * 8 : 0;
   batch_drop_graph(b);
 }
@@ -3512,7 +3509,7 @@ int sem2d_batch_create(int n, sem2d_solver* const* members, sem2d_batch** out) {
     if ((rc = up2(&P.flt_q, &P.flt_r, &P.nfltr, A.rec_flt))) return rc;
   }
   // default launch configuration (sem2d_batch_tune measures the alternatives)
-  batch_set_config(b, 512, tile_wgs_per_cu(b->fp32, b->ndof));
+  batch_set_config(b, tile_wgs_per_cu(b->fp32, b->ndof));
   // records of step 0
   if (b->nrec || b->X.fault_on) {
     if (b->fp32) launch_batch_record<float>(b);
@@ -3560,12 +3557,12 @@ int sem2d_batch_tune(sem2d_batch* b, int trial_steps, int* choice) {
   for (auto& k : blks)
     if ((rc = keep(k.p, k.bytes))) break;
   const int it0 = b->it;
-  const int cand[][2] = {{512, 2}, {512, 3}, {512, 4}, {512, 1}, {512, 0}};
+  const int cand[] = {2, 3, 4, 1, 0};  // workgroups per CU
   const int ncand = sizeof(cand) / sizeof(cand[0]);
   double best = 1e30;
   int ibest = 0;
   for (int q = 0; q < ncand && !rc; ++q) {
-    batch_set_config(b, cand[q][0], cand[q][1]);
+    batch_set_config(b, cand[q]);
     rc = batch_run(b, 1, false);  // warm-up
     if (!rc) rc = batch_run(b, trial_steps, false);
     if (!rc && b->last_ms < best) {
@@ -3581,7 +3578,7 @@ int sem2d_batch_tune(sem2d_batch* b, int trial_steps, int* choice) {
   hipStreamSynchronize(b->stream);
   for (void* q : saved) hipFree(q);
   if (rc) return rc;
-  batch_set_config(b, cand[ibest][0], cand[ibest][1]);
+  batch_set_config(b, cand[ibest]);
   if (choice) *choice = ibest;
   return 0;
 }
@@ -3590,13 +3587,13 @@ int sem2d_batch_set_config(sem2d_batch* b, int threads, int wg_per_cu) {
   if (!b) return 1;
   if ((threads != 256 && threads != 512) || wg_per_cu < 0 || wg_per_cu > 4)
     return berr(b, 3, "batch_set_config: threads must be 256 or 512 and 0 <= wg_per_cu <= 4");
-  batch_set_config(b, threads, wg_per_cu);
+  batch_set_config(b, wg_per_cu);
   return 0;
 }
 
 int sem2d_batch_config(sem2d_batch* b, int* threads, int* wgs, int* ntiles) {
   if (!b) return 1;
-  if (threads) *threads = b->threads;
+  if (threads) *threads = TS_NT;
   if (wgs) *wgs = b->X.pipe_wgs > 0 ? b->X.pipe_wgs : (b->X.T.ntiles + 7) / 8 * 8;
   if (ntiles) *ntiles = b->X.T.ntiles;
   return 0;

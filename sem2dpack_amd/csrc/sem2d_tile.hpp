@@ -71,11 +71,6 @@ __device__ __forceinline__ size_t cell_index(const int4 gr, int nx, int tx0, int
   return (size_t)gr.w + (size_t)(tz0 + lz) * nx + tx0 + lx;
 }
 
-template <typename R, int MODE>
-__device__ __forceinline__ const R* grid_coefs(const R* coefs, const int4 gr) {
-  return MODE == COEF_SHARED ? coefs + gr.w : coefs;
-}
-
 __device__ __forceinline__ int perim_slot(int X, int Z, int PX, int PZ) {
   // branch-free form of: Z == 0 -> X; Z == PZ-1 -> PX + X; X == 0 -> 2PX + Z-1;
   // X == PX-1 -> 2PX + PZ-2 + Z-1; otherwise -1
@@ -1210,7 +1205,7 @@ __device__ __forceinline__ double rec_value(const RecOut& P, const NodeState<R>&
 
 // Everything a step does after the tile kernel, in one launch: the deferred nodes (those
 // of the tile perimeters and the sources), the receivers, and, FLT, the fault: the first
-// FLT_WG * fo.nwave lanes' wavefronts take the fault pairs, each lane both nodes of a pair
+// fo.nwave wavefronts take the fault pairs, each lane both nodes of a pair
 // from their partial forces to their stores, with the pair's traction solve, its record
 // and the step's potency row; the nodes' other lanes skip them.
 // PIN: the state read is the predicted one.
