@@ -46,7 +46,7 @@ module sem2d_hip
             sem2d_set_fields, sem2d_fetch_seismo, sem2d_fetch_fault, sem2d_fetch_fault_state, &
             sem2d_fetch_potency, &
             sem2d_compute_fint, sem2d_compute_fint_noalloc, sem2d_set_itinfo, sem2d_fetch_info, &
-            sem2d_field_info, sem2d_set_tile_config, sem2d_get_step, sem2d_last_step_ms, &
+            sem2d_field_info, sem2d_set_tile_config, sem2d_run_counts, sem2d_get_step, sem2d_last_step_ms, &
             sem2d_last_error, sem2d_destroy, sem2d_error_message, &
             sem2d_adjoint_init, sem2d_adjoint_forward, sem2d_adjoint_backward, sem2d_adjoint_fetch, &
             sem2d_adjoint_timing, sem2d_adjoint_plan, sem2d_adjoint_release, &
@@ -322,6 +322,13 @@ module sem2d_hip
       import :: c_int, c_ptr
       type(c_ptr), value :: h
       integer(c_int), value :: threads, wg_per_cu
+    end function
+
+    ! launches that took many steps at once: kept, and given up
+    integer(c_int) function sem2d_run_counts(h, taken, given_up) bind(C, name='sem2d_run_counts')
+      import :: c_int, c_ptr
+      type(c_ptr), value :: h
+      integer(c_int), intent(out) :: taken, given_up
     end function
 
     integer(c_int) function sem2d_get_step(h, it) bind(C, name='sem2d_get_step')
