@@ -12,10 +12,10 @@ Metric: GLL node-updates/s = npoin * steps / seconds (FP64 fields).  The same ru
 repeated with the FP32 bulk update (fault/time accumulators in FP64) and reported
 under "variants".
 
-Roofline: algorithmic bytes per step B = npoin*(6*ndof+1)*s + nelem*25*(4+2*s)
-(d, v, a read and written, one inverse-mass word per node, int32 ibool and two
-moduli per element-local point; s = 8 or 4), divided by the step time measured
-with HIP events on the solver's stream, against 8 TB/s.
+Roofline: the bytes a step between others cannot do without, B = npoin*(4*ndof+1+2)*s
+(the predicted displacement and velocity read and written, one inverse mass and two
+moduli per node; s = 8 or 4), divided by the step time measured with HIP events on the
+solver's stream, against 8 TB/s.  "traffic" is what the step's kernels move.
 
 CPU baseline: the reference SEM2DPACK Fortran solver (built from source by
 oracle/build_ref.py) on one core, on a 500 x 250-element window of the same medium
@@ -54,8 +54,8 @@ HBM_PEAK = 8.0e12
 CPU_SAMPLE = dict(nx=500, nz=250, lx=50e3, lz=25e3, steps=120)
 
 
-def alg_bytes(npoin, nelem, ndof, s, m=2):
-    return npoin * (6 * ndof + 1) * s + nelem * 25 * (4 + m * s)
+def alg_bytes(npoin, ndof, s, m=2):
+    return npoin * (4 * ndof + 1 + m) * s
 
 
 def host_cpu():
@@ -182,11 +182,10 @@ def run_gpu(pb, steps, warmup, fp32):
     return (t1 - t0), ev_ms, finite
 
 
-def batch_bytes(npoin, nelem, nflt, ndof=2, s=4):
-    """Algorithmic bytes of one batched step: fields and inverse mass per node, int32
-    ibool per element-local point (homogeneous scenarios: no per-point moduli) and
-    ~0.5 KB per FP64 fault pair."""
-    return npoin * (6 * ndof + 1) * s + nelem * 25 * 4 + nflt * 512
+def batch_bytes(npoin, nflt, ndof=2, s=4):
+    """Algorithmic bytes of one batched step: the state handed on and the inverse mass per
+    node (homogeneous scenarios: no moduli) and ~0.5 KB per FP64 fault pair."""
+    return npoin * (4 * ndof + 1) * s + nflt * 512
 
 
 # arrays of a built problem that the solver does not read (coordinates, material
@@ -272,7 +271,7 @@ def run_batch(pbs, steps, build_s):
     b.close()
     for m in members:
         m.close()
-    B = batch_bytes(npoin, nelem, nflt)
+    B = batch_bytes(npoin, nflt)
     return {
         "metric": "batched scenarios/s", "value": n / t_batch, "unit": "scenarios/s",
         "steps": steps, "ms_per_step": 1e3 * t_batch / steps,
@@ -469,7 +468,7 @@ def main():
     npoin, nelem, ndof = pb.npoin, pb.nelem, pb.ndof
     wall, ev_ms, finite = run_gpu(pb, steps, args.warmup, False)
     log(f"throughput fp64: {1e3 * wall / steps:.3f} ms/step")
-    B64 = alg_bytes(npoin, nelem, ndof, 8)
+    B64 = alg_bytes(npoin, ndof, 8)
     value = npoin * steps / wall
     ach = B64 / (ev_ms * 1e-3)
     traffic = None
@@ -504,7 +503,7 @@ def main():
     if not args.no_fp32:
         wall32, ev32, fin32 = run_gpu(pb, steps, args.warmup, True)
         log(f"throughput fp32 bulk: {1e3 * wall32 / steps:.3f} ms/step")
-        B32 = alg_bytes(npoin, nelem, ndof, 4)
+        B32 = alg_bytes(npoin, ndof, 4)
         line["variants"]["fp32_bulk"] = {
             "value": npoin * steps / wall32, "ms_per_step": 1e3 * wall32 / steps,
             "roofline_frac": B32 / (ev32 * 1e-3) / HBM_PEAK, "achieved_GBs": B32 / (ev32 * 1e-3) / 1e9,
